@@ -28,6 +28,7 @@
 namespace magace {
 
 static_assert(TermList::kLanes == kAdjointThreads, "the chunk order must be built for the adjoint's workgroup size");
+static_assert(kNodeTasks == kNodeTasksDev && kNodeQuantum == kNodeQuantumDev && kNodeQuantumG == kNodeQuantumGDev, "the plan must keep to the kernel's tasks");
 static_assert(TermList::kGroup == kCombGroup, "combine groups must match the kernel's");
 
 namespace {
@@ -94,6 +95,14 @@ struct Context {
     int2* ypair = nullptr;     // products of two A entries (body orders 5, 6), TermList::ypair
     int2* yft = nullptr;       // their gradient's way back to Z (TermList::yft, yfe)
     int2* yfe = nullptr;
+    // the adjoint's node plan on the device; d_w: the merged monomial weights that its record weights
+    // are taken from
+    NodeTab<double> n64;
+    NodeTab<float> n32;
+    NodeWeights node_w;
+    std::vector<void*> node_mem;
+    double* d_w = nullptr;
+    bool records_stale = true;  // the gradient records on the device are not those of the coefficients
     Buffers buf;
     std::vector<int> h_off;
     hipStream_t stream = nullptr;
@@ -185,6 +194,8 @@ Context::~Context() {
     dfree(crec64); dfree(crec32); dfree(crec16); dfree(crecu); dfree(crec16u); dfree(chunks); dfree(comb); dfree(comb2); dfree(fold); dfree(cw2_64);
     dfree(ypair); dfree(yft); dfree(yfe);
     dfree(cw2_32);
+    for (void*& p : node_mem) dfree(p);
+    dfree(d_w);
     dfree(buf.Z); dfree(buf.W); dfree(buf.ehc); dfree(buf.rho1); dfree(buf.dE); dfree(buf.edf); dfree(buf.rho);
     dfree(buf.Pt);
     dfree(buf.err);
@@ -306,6 +317,7 @@ int build_context(Potential&& pot, std::unique_ptr<Context>& out) {
                                     ">= 8192 partial sums)");
         return MAGACE_ERR_INPUT;
     }
+    M.nodes = build_nodes(M.z, M.terms, (int)((kNodeLdsMost - kNodeLdsTail) / 16));
     M.spl = build_splines(M.pot);
     fill_params(ctx->P64, M);
     fill_params(ctx->P32, M);
@@ -362,6 +374,100 @@ int upload_records(Context& c) {
     return 0;
 }
 
+// record weights of the node plan from the merged monomial weights
+int upload_node_weights(Context& c) {
+    if (c.node_w.n == 0) return 0;
+    const std::vector<double>& w = c.model.terms.w;
+    HIPCHK(hipMemcpy(c.d_w, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(fill_node_weights(c.node_w, c.d_w, nullptr));
+    HIPCHK(hipStreamSynchronize(nullptr));
+    return 0;
+}
+
+// the node plan's tables
+int upload_nodes(Context& c) {
+    auto alloc = [&](auto*& dst, size_t bytes) -> int {
+        void* p = nullptr;
+        HIPCHK(hipMalloc(&p, bytes + 64));
+        c.node_mem.push_back(p);
+        dst = (std::remove_reference_t<decltype(dst)>)p;
+        return 0;
+    };
+    auto up = [&](auto*& dst, const auto& v) -> int {
+        if (int rc = alloc(dst, v.size() * sizeof(v[0]))) return rc;
+        if (!v.empty()) HIPCHK(hipMemcpy((void*)dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
+        return 0;
+    };
+    // `n` steps of a lane side by side
+    auto grouped = [](const auto& v, size_t n) {
+        auto o = v;
+        for (size_t s = 0; s + 64 * n <= v.size(); s += 64 * n)
+            for (size_t k = 0; k < n; ++k)
+                for (size_t L = 0; L < 64; ++L) o[s + n * L + k] = v[s + 64 * k + L];
+        return o;
+    };
+    const NodePlan& N = c.model.nodes;
+    if (!N.ok) return 0;
+    HIPCHK(hipMalloc((void**)&c.d_w, c.model.terms.w.size() * sizeof(double) + 64));
+    NodeTab<double>& D = c.n64;
+    NodeTab<float>& F = c.n32;
+    int rc = up(D.core_z, N.core_z);
+    if (!rc) rc = up(D.pair, N.pair);
+    if (!rc) rc = up(D.head, N.head);
+    if (!rc) rc = up(D.row, N.row);
+    if (!rc) rc = up(D.col, grouped(N.col, 4));
+    if (!rc) rc = up(D.g_row, N.g_row);
+    if (!rc) rc = up(D.g_rec, grouped(N.g_rec, 2));
+    if (!rc) rc = up(D.a2_x, N.a2_x);
+    if (!rc) rc = up(D.a2_c, N.a2_c);
+    if (!rc) rc = up(D.d_slot, N.d_slot);
+    if (!rc) rc = up(D.d_x, N.d_x);
+    if (rc) return rc;
+    auto sizes = [&](auto& t) {
+        t.nw = N.nw;
+        t.slot_one = N.slot_one;
+        t.first_node = N.first_node;
+        t.npair = N.np + N.nq;
+        t.nslots = N.nslots;
+        t.na2 = (int)N.a2_x.size();
+        t.k2 = N.k2;
+        t.nd = (int)N.d_slot.size();
+        t.kd = N.kd;
+    };
+    sizes(D);
+    sizes(F);
+    F.core_z = D.core_z; F.pair = D.pair; F.head = D.head; F.row = D.row; F.col = D.col; F.g_row = D.g_row;
+    F.g_rec = D.g_rec; F.a2_x = D.a2_x; F.a2_c = D.a2_c; F.d_slot = D.d_slot; F.d_x = D.d_x;
+    // weights of the sparse product, of the A2 entries and of the sums over them, in one array
+    std::vector<int32_t> t(N.t);
+    t.insert(t.end(), N.a2_t.begin(), N.a2_t.end());
+    t.insert(t.end(), N.d_t.begin(), N.d_t.end());
+    NodeWeights w;
+    w.n = (int)t.size();
+    rc = up(w.t, t);
+    if (!rc) rc = alloc(w.w64, t.size() * sizeof(double));
+    if (!rc) rc = alloc(w.w32, t.size() * sizeof(float));
+    if (rc) return rc;
+    D.w = (const NodeTab<double>::W4*)w.w64;
+    D.a2_w = w.w64 + N.t.size();
+    D.d_w = D.a2_w + N.a2_t.size();
+    F.w = (const NodeTab<float>::W4*)w.w32;
+    F.a2_w = w.w32 + N.t.size();
+    F.d_w = F.a2_w + N.a2_t.size();
+    c.node_w = w;
+    return upload_node_weights(c);
+}
+
+// The gradient records serve what the node plan does not: potentials without one, and the accumulation
+// recipe.  Their device copy is brought up to date when one of these is in use.
+int ensure_records(Context& c) {
+    if (!c.records_stale || !(!c.model.nodes.ok || c.precision == MAGACE_MIXED_ACC)) return 0;
+    if (c.model.terms.ncontrib())
+        if (int rc = upload_records(c)) return rc;
+    c.records_stale = false;
+    return 0;
+}
+
 // merged weights w_t = sum_k c_k u_{k,t} and record weights after a coefficient change
 int refresh_weights(Context& c) {
     Potential& pot = c.model.pot;
@@ -385,8 +491,10 @@ int refresh_weights(Context& c) {
     set_c1(c.P64, c.model);
     set_c1(c.P32, c.model);
     bump_generation();  // c1 travels by value in the kernel arguments
-    if (c.uploaded && nr) return upload_records(c);
-    return 0;
+    c.records_stale = true;
+    if (!c.uploaded) return 0;
+    if (int rc = upload_node_weights(c)) return rc;
+    return ensure_records(c);
 }
 
 // device tables are uploaded on first use so the host model can be built without a GPU
@@ -431,9 +539,10 @@ int upload(Context& c) {
     if (int rc = up_int2(c.yft, M.terms.yft)) return rc;
     if (int rc = up_int2(c.yfe, M.terms.yfe)) return rc;
     if (nc) {
-        if (int rc = upload_records(c)) return rc;
         HIPCHK(hipMemcpy(c.chunks, M.terms.chunks.data(), nch * sizeof(int2), hipMemcpyHostToDevice));
     }
+    if (int rc = upload_nodes(c)) return rc;
+    if (int rc = ensure_records(c)) return rc;
     HIPCHK(hipMalloc((void**)&c.buf.err, sizeof(int)));
     HIPCHK(hipMemset(c.buf.err, 0, sizeof(int)));
     c.P64.lut_a = c.t64.lut_a; c.P64.lut_m = c.t64.lut_m;
@@ -516,10 +625,10 @@ hipError_t launch(Context& c, int natom, int atom_base, const int* off, const do
                   double* eout, double* flist, double* tlist, double* tlist0, Buffers& B, hipStream_t s,
                   hipEvent_t* ev) {
     if (c.precision == MAGACE_FP64)
-        return Launch<double>::run(c.P64, natom, atom_base, off, dlist, elist, dmomi, emomi, dmom, emom, eout, flist,
+        return Launch<double>::run(c.P64, c.n64, natom, atom_base, off, dlist, elist, dmomi, emomi, dmom, emom, eout, flist,
                                    tlist, tlist0, B, s, c.shape_class, ev, c.dvar[0]);
     // MAGACE_MIXED_ACC runs the FP32 kernels with the accumulation recipe and the mixed tuning
-    return Launch<float>::run(c.P32, natom, atom_base, off, dlist, elist, dmomi, emomi, dmom, emom, eout, flist,
+    return Launch<float>::run(c.P32, c.n32, natom, atom_base, off, dlist, elist, dmomi, emomi, dmom, emom, eout, flist,
                               tlist, tlist0, B, s, c.shape_class, ev, c.dvar[1], c.precision == MAGACE_MIXED_ACC);
 }
 
@@ -762,7 +871,7 @@ int magace_set_precision(int mode) {
     }
     if (g_ctx->precision != mode) bump_generation();
     g_ctx->precision = mode;
-    return 0;
+    return g_ctx->uploaded ? ensure_records(*g_ctx) : 0;
 }
 
 int magace_get_precision(void) { return g_ctx ? g_ctx->precision : -1; }
@@ -1391,7 +1500,7 @@ int magace_fit_backward(int natom, int nei, const int* offsets, const int* nlist
                         (int)bs.b6.size()};
     Buffers B = c.buf;
     B.Wd = F.Wd;
-    HIPCHK(fit_backward(c.P64, c.shape_class, natom, offsets, nlist, gF, dlist, elist, dlist_momi, dlist_mom,
+    HIPCHK(fit_backward(c.P64, !c.model.nodes.ok, c.shape_class, natom, offsets, nlist, gF, dlist, elist, dlist_momi, dlist_mom,
                         elist_mom, gE ? atom_struct : nullptr, gE, B, F, (int)T.nterms(), nbo, grad, s));
     return 0;
 }

@@ -7,8 +7,9 @@
 //              for a chunk of neighbours; threads then own (lm, n-block) columns of A and
 //              (l'm', n-block) columns of A2 and accumulate in registers.  Writes
 //              Z = [A | A2 | A0] per atom, the core sum and the B1 part of rho.
-//   k_adjoint  (prepB + forceweights, src/b_basis.F90:62-307, src/forces.F90:84-349)
-//              one workgroup per atom (two in FP32).  Z and dZ in LDS; each thread sums
+//   k_adjoint_nodes (prepB + forceweights, src/b_basis.F90:62-307, src/forces.F90:84-349; adjoint.hip)
+//              for one density and body orders up to 4; otherwise, and for the accumulation recipe,
+//   k_adjoint  one workgroup per atom (two in FP32).  Z and dZ in LDS; each thread sums
 //              chunks of gradient records w*Z[a]Z[b]Z[c] per target (the transposed
 //              monomial table), partial sums meet in a fixed order (no atomics); then rho,
 //              E_i, dE/drho and the scaled gradient W = dE/dZ are written.
@@ -24,6 +25,7 @@
 #include <cmath>
 
 #include "device.hpp"
+#include "kernels.hpp"
 
 namespace magace {
 
@@ -76,24 +78,6 @@ hipError_t upload_legendre_constants() {
 }
 
 // ---------------------------------------------------------------- small helpers
-template <typename T>
-__device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
-    return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-template <typename T>
-__device__ __forceinline__ void cfma(cplx<T>& acc, cplx<T> a, cplx<T> b) {
-    acc.re = fma(a.re, b.re, fma(-a.im, b.im, acc.re));
-    acc.im = fma(a.re, b.im, fma(a.im, b.re, acc.im));
-}
-template <typename T>
-__device__ __forceinline__ T re_mul(cplx<T> a, cplx<T> b) {  // Re(a*b)
-    return fma(a.re, b.re, -a.im * b.im);
-}
-template <typename T>
-__device__ __forceinline__ cplx<T> cconj_sign(cplx<T> a, int m) {  // (-1)^m conj(a)
-    return (m & 1) ? cplx<T>{-a.re, a.im} : cplx<T>{a.re, -a.im};
-}
-
 // Kahan step: s += x, with c holding minus the part of the running sum that s has lost
 // (the compensated sum is s - c)
 template <typename T>
@@ -710,79 +694,6 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     if (threadIdx.x == 0)
         for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += red[i];
     return s;  // valid on thread 0
-}
-
-// embedding F(rho) and F'(rho) (src/forces.F90:1134-1233, nfemb 0..2)
-__device__ inline void embed(int nfemb, double rho, double wpre, double mexp, double& F, double& dF) {
-    if (nfemb == 0) { F = rho; dF = 1.0; return; }
-    const double w = 10.0, eps = 1e-10;
-    const double s = nfemb == 2 ? 1.0 + rho : rho;
-    if (fabs(s) > eps) {
-        double y1 = w * s * s;
-        const double g = y1 > 30.0 ? 0.0 : exp(-y1);
-        const double omg = 1.0 - g, a = fabs(s), sg = s >= 0.0 ? 1.0 : -1.0;
-        y1 = pow(omg * a, mexp);
-        const double y2 = mexp * g * a;
-        F = nfemb == 2 ? wpre * (sg * (y1 + y2) - 1.0) : wpre * sg * (y1 + y2);
-        const double dg = -2.0 * w * s * g, da = sg;
-        const double dy = fabs(y1) < eps ? 0.0 : mexp * y1 / (omg * a);
-        dF = wpre * sg * (dy * (-dg * a + omg * da) + mexp * (dg * a + g * da));
-    } else {
-        F = nfemb == 2 ? wpre * mexp * (s - 1.0) : wpre * mexp * rho;
-        dF = wpre * mexp;
-    }
-}
-
-// An aligned vector at LDS byte address `off`. The adjoint kernels declare no static LDS (the
-// host checks this before launching them), so their dynamic LDS, and with it Z' at its start,
-// begins at address 0: a record's byte offset into Z' is the address itself, and reading it
-// this way saves the add of the dynamic base, which the compiler resolves only after
-// instruction selection and so cannot fold away.
-template <typename E, int N>
-__device__ __forceinline__ E __attribute__((ext_vector_type(N))) lds_at(uint32_t off) {
-    typedef E V __attribute__((ext_vector_type(N)));
-    return *(const __attribute__((address_space(3))) V*)(size_t)off;
-}
-__device__ __forceinline__ float4 lds_f4(uint32_t off) {
-    const auto v = lds_at<float, 4>(off);
-    return make_float4(v.x, v.y, v.z, v.w);
-}
-// one complex entry of Z' at a byte offset, as a single aligned vector read
-template <typename T> __device__ __forceinline__ cplx<T> lds_cplx(uint32_t off) {
-    const auto v = lds_at<T, 2>(off);
-    return {v.x, v.y};
-}
-
-// E_i = f_in(e_hc) sum_d F(rho_d) + e_hc (src/forces.F90:1066-1128) for nd densities whose
-// B parts sum to tots[d]; writes eout, dE_i/drho_d = fc F'(rho_d) (also into scale[d]), the
-// e_hc factor and rho
-template <typename T>
-__device__ inline void atom_energy(const DevParams<T>& P, int nd, int atom, const double* tots, double e,
-                                   const double* r1, double* __restrict__ eout, double* __restrict__ dEout,
-                                   double* __restrict__ edfout, double* __restrict__ rho_out, double* scale) {
-    // e = e_hc of the atom, r1[d] its B1 parts of rho (loaded by the caller ahead of time)
-    double Fs = 0.0, dF[2] = {0.0, 0.0};
-    for (int d = 0; d < nd; ++d) {
-        const double r = tots[d] + r1[d];
-        rho_out[(size_t)atom * nd + d] = r;
-        double F;
-        embed(P.nfemb, r, P.p1[d][0], P.p1[d][1], F, dF[d]);
-        Fs += F;
-    }
-    const double elow = P.ecut - P.decut;
-    double fc = 1.0, dfc = 0.0;
-    if (e >= P.ecut) { fc = 0.0; dfc = 0.0; }
-    else if (e > elow) {
-        const double pi = 3.14159265358979323846;
-        fc = 0.5 * (1.0 + cos(pi * (e - elow) / P.decut));
-        dfc = -0.5 * sin(pi * (e - elow) / P.decut) * pi / P.decut;
-    }
-    eout[atom] = fc * Fs + e;
-    for (int d = 0; d < nd; ++d) {
-        dEout[(size_t)atom * nd + d] = fc * dF[d];
-        scale[d] = fc * dF[d];
-    }
-    edfout[atom] = dfc * Fs + 1.0;
 }
 
 __device__ __forceinline__ float4 vadd(float4 a, float4 b) {
@@ -1460,7 +1371,7 @@ __global__ void __launch_bounds__(64) k_forces(DevParams<T> P, const int* __rest
                                                const double* __restrict__ emomi,
                                                const double* __restrict__ dmom,
                                                const double* __restrict__ emom,
-                                               const cplx<T>* __restrict__ Win,
+                                               const cplx<T>* __restrict__ Win, bool scaled,
                                                const double* __restrict__ dEin,
                                                const double* __restrict__ edfin,
                                                double* __restrict__ flist, double* __restrict__ tlist,
@@ -1475,6 +1386,8 @@ __global__ void __launch_bounds__(64) k_forces(DevParams<T> P, const int* __rest
         // forty loads in flight per lane: one trip to memory serves 2560 entries (all of W for
         // lmax 6), where a load followed by its store had waited for every 64
         const cplx<T>* __restrict__ Wg = Win + (size_t)atom * P.nz;
+        // W = dE/dRho dRho/dZ; the node adjoint leaves the first factor to this kernel
+        const T sc = scaled ? (T)1 : (T)dEin[atom];
         constexpr int U = 40;
         for (int i0 = 0; i0 < P.nz; i0 += 64 * U) {
             cplx<T> v[U];
@@ -1486,7 +1399,7 @@ __global__ void __launch_bounds__(64) k_forces(DevParams<T> P, const int* __rest
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int i = i0 + 64 * u + lane;
-                if (i < P.nz) sW[i] = v[u];
+                if (i < P.nz) sW[i] = {sc * v[u].re, sc * v[u].im};
             }
         }
         __syncthreads();
@@ -2193,10 +2106,10 @@ __device__ inline void inner_cutoff(double e, double ecut, double decut, double&
 // dL/dc_{k,d} for L = sum_s gE_s E_s - D_u E:
 //   alpha = gE fc F'_d - fc F''_d D_u rho_d - F'_d dfc D_u e_hc,  beta = -fc F'_d.
 // D_u rho_d = Re sum_x G_x Zdot_x over the representatives of conjugate pairs, G = drho_d/dZ
-// folded (the conjugate symmetry of Zdot allows it): with one density G = W / (fc F'), with two
-// the adjoint's per-density output Wd[atom][d].
+// folded (the conjugate symmetry of Zdot allows it): with one density G = W, or W / (fc F') where
+// the adjoint scaled it, with two the adjoint's per-density output Wd[atom][d].
 template <int ND>
-__global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, const cplx<double>* __restrict__ W,
+__global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, bool scaled, const cplx<double>* __restrict__ W,
                                                  const cplx<double>* __restrict__ Zdot,
                                                  const double* __restrict__ rho, const double* __restrict__ ehc,
                                                  const double* __restrict__ ehc_dot,
@@ -2211,7 +2124,8 @@ __global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, const cpl
     for (int d = 0; d < ND; ++d) {
         const cplx<double>* w = W + ((size_t)atom * ND + d) * P.nz;
         double s = 0.0;
-        for (int x = threadIdx.x; x < P.nz; x += blockDim.x) s += re_mul(w[x], zd[x]);
+        for (int x = threadIdx.x; x < P.nz; x += blockDim.x)
+            if (P.fold[x] >> 17 & 1) s += re_mul(w[x], zd[x]);
         tot[d] = block_sum<double>(s, red);
         __syncthreads();
     }
@@ -2224,7 +2138,7 @@ __global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, const cpl
             double F, dF, d2F;
             embed2(P.nfemb, rho[(size_t)atom * ND + d], P.p1[d][0], P.p1[d][1], F, dF, d2F);
             const double sc = fc * dF;
-            const double rho_dot = ND == 2 ? tot[d] : (sc != 0.0 ? tot[d] / sc : 0.0);
+            const double rho_dot = ND == 2 || !scaled ? tot[d] : (sc != 0.0 ? tot[d] / sc : 0.0);
             alpha[(size_t)atom * ND + d] = g * fc * dF - fc * d2F * rho_dot - dF * dfc * ehc_dot[atom];
             beta[(size_t)atom * ND + d] = -fc * dF;
         }
@@ -2409,7 +2323,7 @@ static hipError_t run_jvp_class(const DevParams<double>& P, int natom, const int
     return hipGetLastError();
 }
 
-hipError_t fit_backward(const DevParams<double>& P, int cls, int natom, const int* off, const int* nlist,
+hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int natom, const int* off, const int* nlist,
                         const double* du, const double* dlist, const double* elist, const double* dmomi,
                         const double* dmom, const double* emom, const int* atom_struct, const double* gE,
                         Buffers& B, FitBuffers& F, int nterms, const int* nbo5, double* grad, hipStream_t s) {
@@ -2427,10 +2341,10 @@ hipError_t fit_backward(const DevParams<double>& P, int cls, int natom, const in
                                                                  (cplx<double>*)F.Zdot, F.ehc_dot, B.err, s);
     if (e != hipSuccess) return e;
     if (nd == 2)
-        hipLaunchKernelGGL(k_fit_atom<2>, dim3(natom), dim3(256), 0, s, P, (const cplx<double>*)B.Wd,
+        hipLaunchKernelGGL(k_fit_atom<2>, dim3(natom), dim3(256), 0, s, P, scaled, (const cplx<double>*)B.Wd,
                            (const cplx<double>*)F.Zdot, B.rho, B.ehc, F.ehc_dot, atom_struct, gE, F.alpha, F.beta);
     else
-        hipLaunchKernelGGL(k_fit_atom<1>, dim3(natom), dim3(256), 0, s, P, (const cplx<double>*)B.W,
+        hipLaunchKernelGGL(k_fit_atom<1>, dim3(natom), dim3(256), 0, s, P, scaled, (const cplx<double>*)B.W,
                            (const cplx<double>*)F.Zdot, B.rho, B.ehc, F.ehc_dot, atom_struct, gE, F.alpha, F.beta);
     const size_t nM = 2 * (size_t)nterms * nd;
     hipLaunchKernelGGL(k_fill_double, dim3((unsigned)((nM + 255) / 256)), dim3(256), 0, s, F.M, nM);
@@ -2505,7 +2419,7 @@ int supported_nm3_class(int nm3, int nr2m, int nb_a, int l3a, int l2m, int nr3a)
 
 template <typename T, int L, int CH, bool SPLIT, bool TASKSPLIT, int NB, int NM3X, int NB2, int NR2X, int NRAX, int NBAX,
           bool ACC>
-static hipError_t run_class(const DevParams<T>& P, int natom, int atom_base, const int* off, const double* dlist,
+static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int natom, int atom_base, const int* off, const double* dlist,
                             const double* elist, const double* dmomi, const double* emomi,
                             const double* dmom, const double* emom, double* eout, double* flist,
                             double* tlist, double* tlist0, Buffers& B, hipStream_t s, hipEvent_t* ev) {
@@ -2565,24 +2479,28 @@ static hipError_t run_class(const DevParams<T>& P, int natom, int atom_base, con
     // FP32 with one density: two atoms per adjoint block (their Z and W interleaved in LDS)
     const bool pair = sizeof(T) == 4 && !nd2 && P.crec16 != nullptr;
     const size_t lds2p = 2 * (size_t)P.nzx * 16 + (2 * (kAdjointThreads / 64) + 2) * sizeof(double);
-    if (pair && lds2p > limit[3]) return hipErrorInvalidValue;
     const size_t lds2 =
         (nd2 ? 3 : 2) * (size_t)P.nzx * sizeof(cplx<T>) + (2 * (kAdjointThreads / 64) + 2) * sizeof(double);
     const size_t lds3 = (size_t)P.nz * sizeof(cplx<T>);
-    if (lds1 > limit[0] || lds2 > limit[nd2 ? 2 : 1] || lds3 > limit[q1 ? 5 + qi : 4])
+    // the node plan where the potential has one; the accumulation recipe keeps the record walk, whose
+    // FP64 sums over monomial products it is defined by
+    const bool nodes = N.nw > 0 && !ACC;
+    if (!nodes && pair && lds2p > limit[3]) return hipErrorInvalidValue;
+    if (lds1 > limit[0] || (!nodes && lds2 > limit[nd2 ? 2 : 1]) || lds3 > limit[q1 ? 5 + qi : 4])
         return hipErrorInvalidValue;
     if (ev) (void)hipEventRecord(ev[0], s);
     hipLaunchKernelGGL(k1, dim3(natom), dim3(256), lds1, s, P, off, dlist, elist, dmomi, emomi, dmom,
                        emom, (cplx<T>*)B.Z, B.ehc, B.rho1, B.err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[1], s);
+    if (nodes && (e = run_adjoint_nodes<T>(P, N, natom, B, eout, s)) != hipSuccess) return e;
     if constexpr (sizeof(T) == 4) {
-        if (pair)
+        if (!nodes && pair)
             hipLaunchKernelGGL(k_adjoint_pair<ACC>, dim3((natom + 1) / 2), dim3(kAdjointThreads), lds2p, s, P, atom_base,
                                ACC ? P.crec16 : P.crec16u, (const cplx<T>*)B.Z, (cplx<T>*)B.W, (char*)B.Pt, B.ehc, B.rho1, eout, B.dE,
                                B.edf, B.rho, natom);
     }
-    if (pair) {
+    if (nodes || pair) {
     } else if (nd2)
         hipLaunchKernelGGL((k_adjoint<T, true, ACC>), dim3(natom), dim3(kAdjointThreads), lds2, s, P, atom_base,
                            (const cplx<T>*)B.Z, (cplx<T>*)B.W, (cplx<T>*)B.Wd, (char*)B.Pt, B.ehc, B.rho1, eout,
@@ -2594,13 +2512,13 @@ static hipError_t run_class(const DevParams<T>& P, int natom, int atom_base, con
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[2], s);
     hipLaunchKernelGGL(k3, dim3(natom), dim3(64), lds3, s, P, off, dlist, elist, dmomi, emomi, dmom, emom,
-                       (const cplx<T>*)B.W, B.dE, B.edf, flist, tlist, tlist0, B.err);
+                       (const cplx<T>*)B.W, !nodes, B.dE, B.edf, flist, tlist, tlist0, B.err);
     if (ev) (void)hipEventRecord(ev[3], s);
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t Launch<T>::run(const DevParams<T>& P, int natom, int atom_base, const int* off, const double* dlist,
+hipError_t Launch<T>::run(const DevParams<T>& P, const NodeTab<T>& N, int natom, int atom_base, const int* off, const double* dlist,
                           const double* elist, const double* dmomi, const double* emomi,
                           const double* dmom, const double* emom, double* eout, double* flist,
                           double* tlist, double* tlist0, Buffers& B, hipStream_t s, int cls,
@@ -2614,13 +2532,13 @@ hipError_t Launch<T>::run(const DevParams<T>& P, int natom, int atom_base, const
     // 0.93 -> 0.81 ms; with lmax 6 the runtime split costs FP64 3%).
     const bool heavy = P.nb_a + P.nr3a * (P.l3a + 1) >= 40;
 #define MAGACE_RUN_ACC(CH, SPLIT, TS, ACC)                                                                     \
-    (cls == 0   ? run_class<T, 6, CH, SPLIT, TS, 4, 4, 4, 2, 8, 10, ACC>(P, natom, atom_base, off, dlist, elist,      \
+    (cls == 0   ? run_class<T, 6, CH, SPLIT, TS, 4, 4, 4, 2, 8, 10, ACC>(P, N, natom, atom_base, off, dlist, elist,      \
                                                                          dmomi, emomi, dmom, emom, eout, flist,      \
                                                                          tlist, tlist0, B, s, ev)                    \
-     : cls == 1 ? run_class<T, 2, CH, SPLIT, TS, 1, 27, 2, 5, 4, 16, ACC>(P, natom, atom_base, off, dlist, elist,     \
+     : cls == 1 ? run_class<T, 2, CH, SPLIT, TS, 1, 27, 2, 5, 4, 16, ACC>(P, N, natom, atom_base, off, dlist, elist,     \
                                                                           dmomi, emomi, dmom, emom, eout, flist,     \
                                                                           tlist, tlist0, B, s, ev)                   \
-                : run_class<T, 6, CH, SPLIT, TS, 4, 9, 4, 5, 8, 16, ACC>(P, natom, atom_base, off, dlist, elist,      \
+                : run_class<T, 6, CH, SPLIT, TS, 4, 9, 4, 5, 8, 16, ACC>(P, N, natom, atom_base, off, dlist, elist,      \
                                                                          dmomi, emomi, dmom, emom, eout, flist,      \
                                                                          tlist, tlist0, B, s, ev))
     // the accumulation recipe (MAGACE_MIXED_ACC) exists for the FP32 kernels only

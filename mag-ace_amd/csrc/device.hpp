@@ -92,6 +92,47 @@ struct Buffers {
 // bytes of Buffers::Pt per atom
 __host__ __device__ inline size_t partials_bytes(int nslot, int nd) { return (size_t)nslot * 16 * (size_t)nd; }
 
+// tasks of a wave whose sums wait in registers (kNodeTasks of the plan)
+constexpr int kNodeTasksDev = 2;
+// steps of a task come in multiples of these: the sparse product's and the gradient's (NodePlan)
+constexpr int kNodeQuantumDev = 4, kNodeQuantumGDev = 4;
+// The node plan of the adjoint on the device (NodePlan; adjoint.hip).  nw = 0: there is none for this
+// potential, and k_adjoint walks the gradient records.
+template <typename T>
+struct NodeTab {
+    struct W4 {
+        T v[4];
+    };
+    int nw = 0, slot_one = 0, first_node = 0, npair = 0, nslots = 0, na2 = 0, k2 = 0, nd = 0, kd = 0;
+    const unsigned short* core_z = nullptr;
+    const uint32_t* pair = nullptr;
+    const int4* head = nullptr;    // [waves][64]
+    const ushort4* row = nullptr;
+    const uint2* col = nullptr;    // LDS slots of four steps of a lane
+    const W4* w = nullptr;
+    const uint32_t* g_row = nullptr;
+    const uint2* g_rec = nullptr;  // two steps of a lane
+    const unsigned short* a2_x = nullptr;
+    const uint32_t* a2_c = nullptr;
+    const T* a2_w = nullptr;
+    const uint32_t* d_slot = nullptr;
+    const int* d_x = nullptr;
+    const T* d_w = nullptr;
+};
+// weights of a plan's records in both precisions, from the monomials' (t: monomial * 2 + (1: minus), -1: 0)
+struct NodeWeights {
+    int n = 0;
+    const int* t = nullptr;
+    double* w64 = nullptr;
+    float* w32 = nullptr;
+};
+hipError_t fill_node_weights(const NodeWeights& n, const double* w, hipStream_t s);
+// energies and the unscaled gradient dRho/dZ of the representatives (B.W; the entries between them are
+// not written), from B.Z
+template <typename T>
+hipError_t run_adjoint_nodes(const DevParams<T>& P, const NodeTab<T>& N, int natom, const Buffers& B, double* eout,
+                             hipStream_t s);
+
 // atom_base: the index of the launch's first atom in the whole system (even), which fixes the
 // adjoint's walk per atom, so that results do not depend on how the atoms are split into
 // launches
@@ -103,7 +144,7 @@ constexpr int kDensityVariants = 3;
 
 template <typename T>
 struct Launch {
-    static hipError_t run(const DevParams<T>& P, int natom, int atom_base, const int* offsets,
+    static hipError_t run(const DevParams<T>& P, const NodeTab<T>& N, int natom, int atom_base, const int* offsets,
                           const double* dlist, const double* elist, const double* dmomi,
                           const double* emomi, const double* dmom, const double* emom, double* eout,
                           double* flist, double* tlist, double* tlist0, Buffers& B, hipStream_t s,
@@ -123,7 +164,7 @@ struct FitBuffers {
     double* ub_u = nullptr;
     size_t cap_atoms = 0;
 };
-hipError_t fit_backward(const DevParams<double>& P, int cls, int natom, const int* off, const int* nlist,
+hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int natom, const int* off, const int* nlist,
                         const double* du, const double* dlist, const double* elist, const double* dmomi,
                         const double* dmom, const double* emom, const int* atom_struct, const double* gE,
                         Buffers& B, FitBuffers& F, int nterms, const int* nbo5, double* grad, hipStream_t s);

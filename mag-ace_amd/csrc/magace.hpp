@@ -132,6 +132,50 @@ struct TermList {
     size_t ncontrib() const { return rec_t.size(); }
 };
 
+// The adjoint's plan (nodes.cpp): the monomials as products of two nodes, p = A0 entry times A
+// entry and q = product of two A entries or one A entry, rho = Re sum w X_p X_q.  A workgroup keeps
+// the entries it needs in LDS slots: the core [the A and A0 entries in use | 1 | 0], the pair
+// products [p | q] and the sums over A2 entries.  The work is cut into tasks of one wave each,
+// assigned to the waves of a workgroup at build time (wave_ptr); records are stored step by step,
+// 64 lanes after one another.
+constexpr size_t kNodeLdsTail = 384;          // sums and scalars behind the slots
+constexpr size_t kNodeLdsMost = 160 * 1024;
+constexpr int kNodeSingle = 0x4000;           // NodeSide::row: a single entry, its Z index below
+constexpr uint32_t kNodeOwn = 1u << 24, kNodeConj = 1u << 25, kNodeMinus = 1u << 26, kNodeNone = 1u << 31;
+constexpr int kNodeQuantum = 4, kNodeQuantumG = 4;  // a task's steps are a multiple of these (product, gradient)
+constexpr int kNodeAhead = 16;                // steps that the kernel reads ahead
+constexpr int kNodeTasks = 2;                 // p tasks of a wave at most (their sums wait in registers)
+struct NodePlan {
+    bool ok = false;
+    int nw = 8;                      // waves of a workgroup
+    int slot_one = 0, slot_zero = 0, first_node = 0, np = 0, nq = 0, nslots = 0;
+    std::vector<uint16_t> core_z;    // Z index of core slot i
+    std::vector<uint32_t> pair;      // nodes: slots of the two factors
+    // [waves][64][4]: headers of a wave's tasks (steps, even; log2 of the lanes per block; first row), p
+    // tasks, then q tasks, then gradient tasks; entry 62: their numbers, entry 63: first steps of the
+    // wave's two record streams, which run through its tasks in order
+    std::vector<int32_t> head;
+    // G_p = sum w X_q, G_q (and single entries) = sum w X_p
+    std::vector<uint16_t> row;       // 4 per block: LDS slots of its rows, kNodeSingle | Z index, or 0xffff: none
+    std::vector<uint16_t> col;       // per step and lane: LDS slot of the column's entry
+    std::vector<int32_t> t;          // 4 per step and lane: monomial * 2 + (1: minus), -1: weight 0
+    // gradient of the representatives: per step and lane G slot | slot of the other factor << 16 | real
+    // part negative << 30 | imaginary part negative << 31; rows: Z index | conjugate partner << 12 |
+    // kNodeOwn (the entry's own single G is added), kNodeConj (the partner's, conjugated, with
+    // kNodeMinus negated)
+    std::vector<uint32_t> g_row;
+    std::vector<uint32_t> g_rec;
+    // two-factor monomials A0 A2: per A2 representative k2 records (A0 slot | conjugate << 31), one
+    // array after another; per A0 entry its A2 entries
+    int k2 = 0;
+    std::vector<uint16_t> a2_x;
+    std::vector<uint32_t> a2_c;
+    std::vector<int32_t> a2_t;
+    std::vector<uint32_t> d_slot;    // G slot | slot of the A0 entry << 16
+    int kd = 0;
+    std::vector<int32_t> d_x, d_t;   // [kd][A0 entries][8]: A2 entry, monomial * 2 or -1
+};
+
 // Spline tables in node-major layout: row n holds [4 coeffs] for every function family.
 struct Splines {
     int nlut = 10000;                    // src/radial.F90:43
@@ -148,6 +192,7 @@ struct Model {
     Potential pot;
     ZLayout z;
     TermList terms;
+    NodePlan nodes;
     Splines spl;
 };
 
@@ -178,6 +223,9 @@ Basis enumerate_basis(const Header& h);
 double clebsch_gordan(int j1, int j2, int J, int m1, int m2, int M);
 ZLayout make_layout(const Header& h);
 TermList build_terms(const Potential& pot, const ZLayout& z);
+// nodes.cpp: the adjoint's plan; not ok for monomials of other forms (body orders 5, 6), two densities,
+// or more than entry_limit LDS slots
+NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit);
 // splines.cpp
 void radial_basis(int radtype, double lambda, int nb, double cut, double dcut, double r,
                   double* g, double* dg);
