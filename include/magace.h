@@ -65,11 +65,12 @@ int magace_finalize(void);
 int magace_set_precision(int mode);
 int magace_get_precision(void);
 
-/* Kernel tuning (no counterpart in the reference).  The density kernel has variants of its
- * neighbour staging and of the split of its column tasks over idle threads; the choice
+/* Kernel tuning (no counterpart in the reference).  The density kernel of MAGACE_MIXED_ACC has variants
+ * of its neighbour staging and of the split of its column tasks over idle threads; the choice
  * changes timing and the order of floating-point sums (so results in the last bits), never
- * the arithmetic.  Defaults come from a table compiled into the library per potential header
- * (measured by mag-ace_amd/tune.py), else from a built-in rule.
+ * the arithmetic.  MAGACE_FP64 and MAGACE_MIXED sum on the matrix cores and have none: their values are
+ * kept and reported, and change nothing.  Defaults come from a table compiled into the library per
+ * potential header (measured by mag-ace_amd/tune.py), else from a built-in rule.
  * v[4] = {FP64 variant, FP64 split, mixed variant, mixed split}; variant -1 = built-in rule,
  * 0..2; split 0 = automatic, 1..8.
  * magace_tune times MAGACE_TUNE_CANDIDATES (variant, split) candidates on the caller's

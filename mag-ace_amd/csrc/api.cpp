@@ -67,6 +67,8 @@ template <typename T>
 struct DevTables {
     T* lut_a = nullptr;
     T* lut_m = nullptr;
+    T* lut_g = nullptr;
+    T* cperm = nullptr;
 };
 
 struct Context {
@@ -92,6 +94,7 @@ struct Context {
     int2* comb = nullptr;
     int2* comb2 = nullptr;
     uint32_t* fold = nullptr;
+    uint32_t* cols = nullptr;  // DevParams::cols
     int2* ypair = nullptr;     // products of two A entries (body orders 5, 6), TermList::ypair
     int2* yft = nullptr;       // their gradient's way back to Z (TermList::yft, yfe)
     int2* yfe = nullptr;
@@ -191,7 +194,8 @@ void dfree(T*& p) {
 
 Context::~Context() {
     dfree(t64.lut_a); dfree(t64.lut_m); dfree(t32.lut_a); dfree(t32.lut_m);
-    dfree(crec64); dfree(crec32); dfree(crec16); dfree(crecu); dfree(crec16u); dfree(chunks); dfree(comb); dfree(comb2); dfree(fold); dfree(cw2_64);
+    dfree(t64.lut_g); dfree(t64.cperm); dfree(t32.lut_g); dfree(t32.cperm);
+    dfree(crec64); dfree(crec32); dfree(crec16); dfree(crecu); dfree(crec16u); dfree(chunks); dfree(comb); dfree(comb2); dfree(fold); dfree(cols); dfree(cw2_64);
     dfree(ypair); dfree(yft); dfree(yfe);
     dfree(cw2_32);
     for (void*& p : node_mem) dfree(p);
@@ -228,6 +232,7 @@ void fill_params(DevParams<T>& P, const Model& M) {
     const Header& h = M.pot.h;
     P.stride_a = M.spl.atomic_stride;
     P.stride_m = M.spl.magnetic_stride;
+    P.stride_g = 4 * (h.nb_a + 1);
     P.nlut = M.spl.nlut;
     P.rs_a = M.spl.rs_a;
     P.rs_m = M.spl.rs_m;
@@ -275,6 +280,65 @@ int upload_table(T*& dst, const std::vector<double>& src) {
     HIPCHK(hipMalloc((void**)&dst, tmp.size() * sizeof(T) + 64));
     HIPCHK(hipMemcpy(dst, tmp.data(), tmp.size() * sizeof(T), hipMemcpyHostToDevice));
     return 0;
+}
+
+// the base functions' and the core term's part of the atomic table, and the radial coefficients as
+// operands of the matrix products
+template <typename T>
+int upload_base_tables(DevTables<T>& t, const Model& M) {
+    const Header& h = M.pot.h;
+    const int sg = 4 * (h.nb_a + 1), sa = M.spl.atomic_stride;
+    std::vector<double> g((size_t)M.spl.nlut * sg);
+    for (int n = 0; n < M.spl.nlut; ++n) {
+        const double* row = M.spl.atomic.data() + (size_t)n * sa;
+        std::copy(row, row + 4 * h.nb_a, g.begin() + (size_t)n * sg);
+        std::copy(row + sa - 4, row + sa, g.begin() + (size_t)n * sg + 4 * h.nb_a);
+    }
+    if (upload_table(t.lut_g, g)) return MAGACE_ERR_DEVICE;
+    std::vector<double> c((size_t)(h.l3a + 1) * 256, 0.0);
+    for (int l = 0; l <= h.l3a; ++l)
+        for (int r = 0; r < 4; ++r)
+            for (int lane = 0; lane < 64; ++lane) {
+                const int n = lane & 15, k = matrix_row(sizeof(T), lane >> 4, r);
+                if (n < h.nr3_a && k < h.nb_a)
+                    c[((size_t)l * 4 + r) * 64 + lane] = M.pot.crad_a[((size_t)n * (h.l3a + 1) + l) * h.nb_a + k];
+            }
+    return upload_table(t.cperm, c);
+}
+
+// DevParams::cols
+std::vector<uint32_t> density_columns(const Model& M) {
+    const Header& h = M.pot.h;
+    std::vector<uint32_t> v;
+    auto pad = [&] {
+        while (!v.empty() && v.size() % 16) v.push_back(v.back());
+    };
+    for (int l = 0; l <= h.l3a; ++l)
+        for (int m = 0; m <= l; ++m)
+            for (int q = 0; q < M.z.nm3; ++q) {
+                const int lq = q % M.z.lsm3;
+                int lp = 0;
+                while ((lp + 1) * (lp + 1) <= lq) ++lp;
+                const int mp = lq - lp * lp - lp;
+                v.push_back((uint32_t)(l * (l + 1) / 2 + m) | (uint32_t)q << 8 | (uint32_t)l << 16 | (uint32_t)m << 20 |
+                            (uint32_t)(mp + 8) << 24);
+            }
+    pad();
+    for (int np = 0; np < h.nr2_m; ++np)
+        for (int l = 0; l <= h.l2m; ++l)
+            for (int m = 0; m <= l; ++m)
+                v.push_back((uint32_t)(l * (l + 1) / 2 + m) | (uint32_t)(l * h.nr2_m + np) << 8 | (uint32_t)l << 16 |
+                            (uint32_t)m << 20 | (uint32_t)np << 24);
+    pad();
+    for (int np = 0; np < h.nr2_m; ++np)
+        for (int l = 0; l <= h.l2m; ++l)
+            for (int m = -l; m <= l; ++m) {
+                // Y_{l,-m} = (-1)^m conj(Y_lm)
+                const int am = m < 0 ? -m : m;
+                v.push_back((uint32_t)(l * (l + 1) / 2 + am) | (uint32_t)(l * h.nr2_m + np) << 8 |
+                            (m < 0 && (am & 1) ? 1u << 16 : 0u) | (m < 0 && !(am & 1) ? 1u << 17 : 0u));
+            }
+    return v;
 }
 
 int build_context(Potential&& pot, std::unique_ptr<Context>& out) {
@@ -515,6 +579,7 @@ int upload(Context& c) {
     if (upload_table(c.t64.lut_m, M.spl.magnetic)) return MAGACE_ERR_DEVICE;
     if (upload_table(c.t32.lut_a, M.spl.atomic)) return MAGACE_ERR_DEVICE;
     if (upload_table(c.t32.lut_m, M.spl.magnetic)) return MAGACE_ERR_DEVICE;
+    if (upload_base_tables(c.t64, M) || upload_base_tables(c.t32, M)) return MAGACE_ERR_DEVICE;
     const size_t nc = M.terms.ncontrib(), nch = M.terms.chunks.size() / 2;
     HIPCHK(hipMalloc((void**)&c.crec64, nc * sizeof(uint4) + 64));
     HIPCHK(hipMalloc((void**)&c.crec32, nc * sizeof(uint4) + 64));
@@ -530,6 +595,11 @@ int upload(Context& c) {
     if (ncomb2) HIPCHK(hipMemcpy(c.comb2, M.terms.comb2.data(), ncomb2 * sizeof(int2), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc((void**)&c.fold, M.terms.fold.size() * sizeof(uint32_t) + 64));
     HIPCHK(hipMemcpy(c.fold, M.terms.fold.data(), M.terms.fold.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    {
+        const std::vector<uint32_t> v = density_columns(M);
+        HIPCHK(hipMalloc((void**)&c.cols, v.size() * sizeof(uint32_t) + 64));
+        HIPCHK(hipMemcpy(c.cols, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    }
     auto up_int2 = [](int2*& d, const std::vector<int32_t>& v) -> int {
         HIPCHK(hipMalloc((void**)&d, v.size() * sizeof(int32_t) + 64));
         if (!v.empty()) HIPCHK(hipMemcpy(d, v.data(), v.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -547,6 +617,8 @@ int upload(Context& c) {
     HIPCHK(hipMemset(c.buf.err, 0, sizeof(int)));
     c.P64.lut_a = c.t64.lut_a; c.P64.lut_m = c.t64.lut_m;
     c.P32.lut_a = c.t32.lut_a; c.P32.lut_m = c.t32.lut_m;
+    c.P64.lut_g = c.t64.lut_g; c.P64.cperm = c.t64.cperm;
+    c.P32.lut_g = c.t32.lut_g; c.P32.cperm = c.t32.cperm;
     c.P64.crec = c.crec64;
     c.P32.crec = c.crec32;
     c.P32.crec16 = c.crec16;
@@ -556,6 +628,7 @@ int upload(Context& c) {
     c.P64.comb = c.P32.comb = c.comb;
     c.P64.comb2 = c.P32.comb2 = c.comb2;
     c.P64.fold = c.P32.fold = c.fold;
+    c.P64.cols = c.P32.cols = c.cols;
     c.P64.ypair = c.P32.ypair = c.ypair;
     c.P64.yft = c.P32.yft = c.yft;
     c.P64.yfe = c.P32.yfe = c.yfe;

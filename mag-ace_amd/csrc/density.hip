@@ -1,0 +1,490 @@
+// density.hip -- A, A2, A0 of every atom on the matrix cores, and their derivative along a displacement.
+//
+// k_density_mm does the work of prepA (src/a_basis.F90:59-359).  With R_{l,n} = sum_k C_{nlk} g_k the sums
+// over neighbours are taken for the base functions first,
+//   B[k][lm,q] = sum_j g_k(j) Y_lm(j) H_q(j),   A[n][lm][q] = sum_k C_{nlk} B[k][lm,q],
+//   A2[k][n'][l'm'] = sum_j g_k(j) M_{l',n'}(j) Y_l'm'(j),
+// which is one product G^T F of the pairs' base functions (at most 16 rows) with all columns, and a small
+// one with C whose B operand is the first one's result as it lies in the registers.  Only the g_k (10 for
+// the lmax-6 header) are looked up for a pair, in a table of their own that stays in L2, where the 49
+// R_{l,n} had to come from a table six times as large.
+//
+// Measured against the kernel that staged all R_{l,n} and summed on the vector units (us): 16000 atoms
+// lmax 6 mixed 403 -> 328, FP64 735 -> 545; 27648 atoms lmax 4 mixed 494 -> 370, FP64 855 -> 535; 4394 atoms
+// of the example potential's shape 161 -> 89 and 338 -> 110; 128 atoms lmax 4 FP64 24.4 -> 14.5.  Of the 328
+// the staging is 90, the products 110 (69 at the matrix cores' rate) and the stores of Z 100.
+#include <hip/hip_runtime.h>
+
+#include "device.hpp"
+#include "kernels.hpp"
+#include "matrix.hpp"
+
+namespace magace {
+
+namespace {
+
+constexpr int kPairs = 60;  // pairs of a round: 15 steps of four; lane 60 of the staging is the central atom
+
+// pairs summed before they join the atom's sum: one chain of all 57 would round 57 times at the size of
+// the whole sum (FP32 errors of E and of the forces against 64 bits, lmax-4 header: 60 pairs a chain
+// 5.4e-7 and 3.5e-7, 20 pairs 3.2e-7 and 2.5e-7, and shorter chains less)
+template <typename T> constexpr int kChain = sizeof(T) == 4 ? 12 : kPairs;
+
+struct DensityLds {  // strides and offsets (in T) of the staging arrays
+    int sY, sYm, sH, sM;          // row lengths: Y, Y' and H in complex entries, M in values; odd
+    int oYm, oH, oG, oM, oYd, oGd, size;
+    __host__ __device__ DensityLds(int lha, int lhm, int nm3, int nfm, bool jvp) {
+        sY = lha | 1, sYm = lhm | 1, sH = nm3 | 1, sM = nfm | 1;
+        oYm = 2 * kPairs * sY;
+        oH = oYm + 2 * (kPairs + 1) * sYm;
+        oG = (oH + 2 * kPairs * sH + 3) & ~3;
+        oM = oG + 16 * kPairs;
+        oYd = (oM + (kPairs + 1) * sM + 3) & ~3;
+        oGd = oYd + (jvp ? 2 * kPairs * sY : 0);
+        size = oGd + (jvp ? 16 * kPairs : 0);
+    }
+};
+
+// items (row j, function k), j < rows, k < nf, one a lane and step: value(j, k, flags, coefficients, fraction)
+// with flags >> 16 set where the function is 0 or 1 and flags >> 17 where it is 1; lane j has row j's number
+template <typename T, typename F>
+__device__ __forceinline__ void spline_items(const T* __restrict__ lut, int stride, int first, int nf, int rows,
+                                             int row, T w, int lane, F&& value) {
+    constexpr int U = sizeof(T) == 4 ? 7 : 4;  // loads in flight
+    const int dj = 64 / nf, dk = 64 - dj * nf;
+    int j = lane / nf, k = lane - j * nf;
+    const T* __restrict__ base = lut + 4 * first;
+    while (__any(j < rows)) {
+        Coef<T> c[U];
+        T wj[U];
+        int at[U];  // row | function << 8 | absent << 16 | one << 17
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int src = j < rows ? j : 0, r = __shfl(row, src, 64);
+            wj[u] = __shfl(w, src, 64);
+            c[u] = coef_at(base + (uint32_t)(r < 0 ? 0 : r) * (uint32_t)stride + 4 * k);
+            at[u] = (j < rows ? j : 255) | k << 8 | (r < 0 ? 1 << 16 : 0) | (r == kRowOne ? 1 << 17 : 0);
+            j += dj;
+            k += dk;
+            if (k >= nf) {
+                k -= nf;
+                ++j;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int ju = at[u] & 0xff;
+            if (ju < rows) value(ju, at[u] >> 8 & 0xff, at[u], c[u], wj[u]);
+        }
+    }
+}
+
+}  // namespace
+
+// One workgroup of four waves an atom, rounds of up to kPairs pairs.  Staging, a wave each: Y_lm of the
+// bonds and the core term; Y_l'm' of the moments and H_q = M_{l',n'} Y_l'm'; the g_k; the M_{l',n'}.  Then
+// wave w takes the column tiles w, w + 4, ... (16 columns of A or A2, real and imaginary parts: two
+// products a step of four pairs).  TA, T2: tiles of A and of A2 of a wave at most.  JVP: the derivative of A and A2 along
+// the pairs' displacements u_i - u_j (k_density_jvp's work in a fit) in place of the values.
+// Waves per SIMD: what the LDS of the usual headers lets in.
+template <typename T, int L, int TA, int T2, bool JVP>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TA > 2 ? 2 : sizeof(T) == 4 ? 4 : L <= 4 ? 3 : 2, 8)))
+k_density_mm(DevParams<T> P, const int* __restrict__ off,
+                                                    const double* __restrict__ dlist, const double* __restrict__ elist,
+                                                    const double* __restrict__ dmomi, const double* __restrict__ emomi,
+                                                    const double* __restrict__ dmom, const double* __restrict__ emom,
+                                                    const int* __restrict__ nlist, const double* __restrict__ du,
+                                                    cplx<T>* __restrict__ Zout, double* __restrict__ ehc_out,
+                                                    double* __restrict__ rho1_out, int* err) {
+    typedef typename Mm<T>::V V;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int atom = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nfm = P.nr2m * (P.l2m + 1);
+    const DensityLds D(P.lha, P.lhm, P.nm3, nfm, JVP);
+    T* lds = (T*)smem;
+    cplx<T>*sY = (cplx<T>*)lds, *sYm = (cplx<T>*)(lds + D.oYm), *sH = (cplx<T>*)(lds + D.oH);
+    T *sG = lds + D.oG, *sM = lds + D.oM;
+    cplx<T>* sYd = (cplx<T>*)(lds + D.oYd);
+    T* sGd = lds + D.oGd;
+    const int p0 = off[atom], nn = off[atom + 1] - p0;
+    Zout += (size_t)atom * P.nz;
+
+    // this lane's columns (P.cols): wave w has the tiles w, w + 4, ... of those of A followed by those of A2
+    const int nA = P.lha * P.nm3, nA2 = P.nr2m * P.lhm;
+    const int tA = (nA + 15) >> 4, tAll = tA + ((nA2 + 15) >> 4);
+    const int ci = lane & 15, g = lane >> 4;
+    const int na = (tA - wave + 3) >> 2, n2 = ((tAll - wave + 3) >> 2) - na;
+    V ar[TA], ai[TA], a2r[T2], a2i[T2];
+    uint32_t ca[TA], c2[T2];
+#pragma unroll
+    for (int t = 0; t < TA; ++t) {
+        ar[t] = (V)(T)0;
+        ai[t] = (V)(T)0;
+        ca[t] = P.cols[min(wave + 4 * t, tA - 1) * 16 + ci];
+    }
+#pragma unroll
+    for (int t = 0; t < T2; ++t) {
+        a2r[t] = (V)(T)0;
+        a2i[t] = (V)(T)0;
+        c2[t] = P.cols[min(wave + 4 * (na + t), tAll - 1) * 16 + ci];
+    }
+    // rows past nb_a of the base functions stay zero
+    for (int i = tid; i < kPairs * 16; i += 256) {
+        sG[i] = (T)0;
+        if (JVP) sGd[i] = (T)0;
+    }
+    double ux = 0, uy = 0, uz = 0;
+    if constexpr (JVP) {
+        ux = du[3 * (size_t)atom];
+        uy = du[3 * (size_t)atom + 1];
+        uz = du[3 * (size_t)atom + 2];
+    }
+    double core = 0.0;
+    for (int c0 = 0; c0 == 0 || c0 < nn; c0 += kPairs) {
+        const int nj = min(nn - c0, kPairs), nj4 = (nj + 3) & ~3;
+        const bool live = lane < nj, centre = !JVP && lane == kPairs && c0 == 0;
+        const size_t p = (size_t)p0 + c0 + (live ? lane : 0);
+        __syncthreads();
+        if (wave == 0) {
+            if (lane < nj4) {
+                T w = 0;
+                const int row = live ? atomic_index(P, dlist[p], w, err) : kRowZero;
+                const T x = live ? (T)elist[3 * p] : (T)0, y = live ? (T)elist[3 * p + 1] : (T)0,
+                        z = live ? (T)elist[3 * p + 2] : (T)1;
+                const Coef<T> cc = coef_at(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g + 4 * P.nb_a);
+                if constexpr (!JVP) {
+                    harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
+                        sY[lane * D.sY + k] = {pl * ph.re, pl * ph.im};
+                    });
+                    core += row < 0 ? 0.0 : (double)coef_value(cc, w);
+                } else {
+                    T dx = 0, dy = 0, dz = 0;
+                    if (live) {
+                        const size_t jn = 3 * (size_t)nlist[p];
+                        dx = ux - du[jn];
+                        dy = uy - du[jn + 1];
+                        dz = uz - du[jn + 2];
+                    }
+                    const T rdot = x * dx + y * dy + z * dz;
+                    const T invr = live ? (T)(1.0 / dlist[p]) : (T)0;
+                    // the displacement's part across the bond, over r: D_u Y = grad Y . t
+                    const T tx = (dx - rdot * x) * invr, ty = (dy - rdot * y) * invr, tz = (dz - rdot * z) * invr;
+                    harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T dpl, cplx<T> ph, cplx<T> ph1, int m) {
+                        sY[lane * D.sY + k] = {pl * ph.re, pl * ph.im};
+                        // Y = P(z) (x + iy)^m
+                        const T a = dpl * tz, b = (T)m * pl;
+                        const cplx<T> e = cmul(ph1, cplx<T>{tx, ty});
+                        sYd[lane * D.sY + k] = {fma(a, ph.re, b * e.re), fma(a, ph.im, b * e.im)};
+                    });
+                    core += row < 0 ? 0.0 : (double)(coef_slope(cc, w, (T)P.rs_a) * rdot);
+                }
+            }
+        } else if (wave == 1) {
+            if (lane < nj4 || centre) {
+                const bool any = live || centre;
+                T w = 0;
+                const int row = live ? magnetic_index(P, dmom[p], w, err) : kRowZero;
+                const double* v = centre ? emomi + 3 * (size_t)atom : emom + 3 * p;
+                const T x = any ? (T)v[0] : (T)0, y = any ? (T)v[1] : (T)0, z = any ? (T)v[2] : (T)1;
+                const T* mrow = P.lut_m + (size_t)(row < 0 ? 0 : row) * P.stride_m + 4 * P.nb_m;
+                // the first M of H, so that their trip to memory passes during the Y_l'm'
+                constexpr int U = 2;
+                Coef<T> cm[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) cm[u] = coef_at(mrow + 4 * (u <= P.l3m ? u * P.nr2m : 0));
+                harmonics<T, L>(x, y, z, P.l2m, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
+                    sYm[lane * D.sYm + k] = {pl * ph.re, pl * ph.im};
+                });
+                if (lane < nj4)
+                    for (int np = 0; np * P.lsm3 < P.nm3; ++np)
+                        for (int lp = 0; lp <= P.l3m; ++lp) {
+                            Coef<T> c;
+                            if (np > 0 || lp >= U)
+                                c = coef_at(mrow + 4 * (lp * P.nr2m + np));
+                            else
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) c.c[u] = lp ? cm[1].c[u] : cm[0].c[u];
+                            const T mv = row == kRowOne ? (T)1 : row < 0 ? (T)0 : coef_value(c, w);
+                            for (int mp = -lp; mp <= lp; ++mp) {
+                                const cplx<T> h = sYm[lane * D.sYm + lp * (lp + 1) / 2 + (mp < 0 ? -mp : mp)];
+                                const cplx<T> yv = mp < 0 ? cconj_sign(h, -mp) : h;
+                                sH[lane * D.sH + np * P.lsm3 + lp * lp + lp + mp] = {mv * yv.re, mv * yv.im};
+                            }
+                        }
+            }
+        } else if (wave == 2) {
+            T w = 0;
+            const int row = live ? atomic_index(P, dlist[p], w, err) : kRowZero;
+            T rdot = 0;
+            if constexpr (JVP) {
+                if (live) {
+                    const size_t jn = 3 * (size_t)nlist[p];
+                    rdot = elist[3 * p] * (ux - du[jn]) + elist[3 * p + 1] * (uy - du[jn + 1]) +
+                           elist[3 * p + 2] * (uz - du[jn + 2]);
+                }
+            }
+            spline_items<T>(P.lut_g, P.stride_g, 0, P.nb_a, nj4, row, w, lane,
+                            [&](int j, int k, int r, const Coef<T>& c, T wj) {
+                                sG[j * 16 + k] = r >> 16 ? (T)0 : coef_value(c, wj);
+                                if constexpr (JVP) sGd[j * 16 + k] = r >> 16 ? (T)0 : coef_slope(c, wj, (T)P.rs_a);
+                            });
+            if constexpr (JVP) {
+                // g'_k (u_i - u_j) . e: each lane scales its own pair's row, after the wave's writes above
+                __builtin_amdgcn_wave_barrier();
+                if (lane < nj4)
+                    for (int k = 0; k < P.nb_a; ++k) sGd[lane * 16 + k] *= rdot;
+            }
+        } else {
+            T w = 0;
+            const int row = centre ? magnetic_index(P, dmomi[atom], w, err)
+                                   : live ? magnetic_index(P, dmom[p], w, err) : kRowZero;
+            // the central atom's row follows the pairs' (lane kPairs -> row nj4 of the items)
+            const bool first = !JVP && c0 == 0;
+            const int src = first && lane == nj4 ? kPairs : lane;
+            const int rowi = __shfl(row, src, 64);
+            const T wi = __shfl(w, src, 64);
+            if (nfm > 0)
+                spline_items<T>(P.lut_m, P.stride_m, P.nb_m, nfm, nj4 + (first ? 1 : 0), rowi, wi, lane,
+                            [&](int j, int k, int r, const Coef<T>& c, T wj) {
+                                sM[(j == nj4 ? kPairs : j) * D.sM + k] =
+                                    r >> 17 ? (T)1 : r >> 16 ? (T)0 : coef_value(c, wj);
+                            });
+            if (first) {
+                // B1 part of rho (b_basis.F90:62-83): lane k has g^m_k of the central moment
+                const int rc = __shfl(row, kPairs, 64);
+                const T wc = __shfl(w, kPairs, 64);
+                double b0 = 0.0, b1 = 0.0;
+                if (lane < P.nb_m) {
+                    const Coef<T> c = coef_at(P.lut_m + (size_t)(rc < 0 ? 0 : rc) * P.stride_m + 4 * lane);
+                    const double v = (double)(rc == kRowOne ? (T)1 : rc < 0 ? (T)0 : coef_value(c, wc)) - 1.0;
+                    b0 = P.c1[0][lane] * v;
+                    b1 = P.c1[1][lane] * v;
+                }
+                double s0 = 0.0, s1 = 0.0;
+                for (int k = 0; k < P.nb_m; ++k) {  // in the order of the functions
+                    s0 += __shfl(b0, k, 64);
+                    s1 += __shfl(b1, k, 64);
+                }
+                if (lane < P.nd) rho1_out[(size_t)atom * P.nd + lane] = lane ? s1 : s0;
+            }
+        }
+        __syncthreads();
+        if (c0 == 0) {
+            // A0 (src/a_basis.F90:90-106); it does not depend on positions
+            for (int t = tid; t < P.nr2m * P.lsm; t += 256) {
+                cplx<T> z = {0, 0};
+                if constexpr (!JVP) {
+                    const uint32_t d = P.cols[tAll * 16 + t];
+                    const cplx<T> h = sYm[kPairs * D.sYm + (d & 0xff)];
+                    const T mv = sM[kPairs * D.sM + (d >> 8 & 0xff)];
+                    z = {(d >> 16 & 1 ? -mv : mv) * h.re, (d >> 17 & 1 ? -mv : mv) * h.im};
+                }
+                Zout[P.oA0 + t] = z;
+            }
+        }
+        for (int s0 = 0; s0 < nj4; s0 += kChain<T>) {
+            V sr[TA], si[TA], s2r[T2], s2i[T2];  // the sums of kChain pairs, in FP32
+            constexpr bool kPart = kChain<T> < kPairs;
+            V(&br)[TA] = kPart ? sr : ar;
+            V(&bi)[TA] = kPart ? si : ai;
+            V(&b2r)[T2] = kPart ? s2r : a2r;
+            V(&b2i)[T2] = kPart ? s2i : a2i;
+            if constexpr (kPart) {
+#pragma unroll
+                for (int t = 0; t < TA; ++t) sr[t] = si[t] = (V)(T)0;
+#pragma unroll
+                for (int t = 0; t < T2; ++t) s2r[t] = s2i[t] = (V)(T)0;
+            }
+            for (int s = s0; s < min(s0 + kChain<T>, nj4); s += 4) {
+                const int j = s + g;
+                // the step's operands of every tile first, so that one trip to LDS serves them all
+                const T a = sG[j * 16 + ci];
+                T ad = 0;
+                if constexpr (JVP) ad = sGd[j * 16 + ci];
+                cplx<T> y[TA], h[TA], yd[JVP ? TA : 1], y2[T2];
+                T m2[T2];
+#pragma unroll
+                for (int t = 0; t < TA; ++t) {
+                    y[t] = sY[j * D.sY + (ca[t] & 0xff)];
+                    h[t] = sH[j * D.sH + (ca[t] >> 8 & 0xff)];
+                    if constexpr (JVP) yd[JVP ? t : 0] = sYd[j * D.sY + (ca[t] & 0xff)];
+                }
+#pragma unroll
+                for (int t = 0; t < T2; ++t) {
+                    y2[t] = sYm[j * D.sYm + (c2[t] & 0xff)];
+                    m2[t] = sM[j * D.sM + (c2[t] >> 8 & 0xff)];
+                }
+#pragma unroll
+                for (int t = 0; t < TA; ++t)
+                    if (t < na) {
+                        const cplx<T> v = cmul(y[t], h[t]);
+                        br[t] = Mm<T>::mul(JVP ? ad : a, v.re, br[t]);
+                        bi[t] = Mm<T>::mul(JVP ? ad : a, v.im, bi[t]);
+                        if constexpr (JVP) {
+                            const cplx<T> vd = cmul(yd[JVP ? t : 0], h[t]);
+                            br[t] = Mm<T>::mul(a, vd.re, br[t]);
+                            bi[t] = Mm<T>::mul(a, vd.im, bi[t]);
+                        }
+                    }
+#pragma unroll
+                for (int t = 0; t < T2; ++t)
+                    if (t < n2) {
+                        b2r[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].re, b2r[t]);
+                        b2i[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].im, b2i[t]);
+                    }
+            }
+            if constexpr (kPart) {
+#pragma unroll
+                for (int t = 0; t < TA; ++t) {
+                    ar[t] += sr[t];
+                    ai[t] += si[t];
+                }
+#pragma unroll
+                for (int t = 0; t < T2; ++t) {
+                    a2r[t] += s2r[t];
+                    a2i[t] += s2i[t];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TA; ++t)
+        if (t < na) {
+            // A = C B for each l that the tile's columns have
+            const int l = ca[t] >> 16 & 15, m = ca[t] >> 20 & 15, q = ca[t] >> 8 & 0xff, mp = (int)(ca[t] >> 24 & 31) - 8;
+            const int l0 = __builtin_amdgcn_readlane(l, 0), l1 = __builtin_amdgcn_readlane(l, 15);
+            V zr = (V)(T)0, zi = (V)(T)0;
+            T k[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) k[r] = P.cperm[(size_t)l0 * 256 + 64 * r + lane];
+            for (int ll = l0; ll <= l1; ++ll) {
+                V br = (V)(T)0, bi = (V)(T)0;
+                T kn[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) kn[r] = P.cperm[(size_t)min(ll + 1, l1) * 256 + 64 * r + lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    br = Mm<T>::mul(k[r], ar[t][r], br);
+                    bi = Mm<T>::mul(k[r], ai[t][r], bi);
+                    k[r] = kn[r];
+                }
+                if (l == ll) {
+                    zr = br;
+                    zi = bi;
+                }
+            }
+            const T sg = ((m + mp) & 1) ? (T)-1 : (T)1;
+            if ((wave + 4 * t) * 16 + ci < nA) {
+                cplx<T>* z0 = Zout + (l * l + l + m) * P.nm3 + q;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int n = Mm<T>::row(g, r);
+                    if (n < P.nr3a) {
+                        cplx<T>* z = z0 + n * P.lsa * P.nm3;
+                        *z = {zr[r], zi[r]};
+                        // A[n][l,-m][qbar] = (-1)^(m+m') conj(A[n][l,m][q])
+                        if (m > 0) z[-2 * m * P.nm3 - 2 * mp] = {sg * zr[r], -sg * zi[r]};
+                    }
+                }
+            }
+        }
+#pragma unroll
+    for (int t = 0; t < T2; ++t)
+        if (t < n2 && (wave + 4 * (na + t) - tA) * 16 + ci < nA2) {
+            const int l = c2[t] >> 16 & 15, m = c2[t] >> 20 & 15, np = c2[t] >> 24;
+            const T sg = (m & 1) ? (T)-1 : (T)1;
+            cplx<T>* z0 = Zout + P.oA2 + np * P.lsm + l * l + l + m;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = Mm<T>::row(g, r);
+                if (k < P.nb_a) {
+                    cplx<T>* z = z0 + k * P.nr2m * P.lsm;
+                    *z = {a2r[t][r], a2i[t][r]};
+                    if (m > 0) z[-2 * m] = {sg * a2r[t][r], -sg * a2i[t][r]};
+                }
+            }
+        }
+    if (wave == 0) {
+        for (int o = 32; o > 0; o >>= 1) core += __shfl_xor(core, o, 64);
+        if (lane == 0) ehc_out[atom] = core;
+    }
+}
+
+namespace {
+
+template <typename T, int L, int TA, int T2, bool JVP>
+hipError_t launch_density(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
+                          const double* dmomi, const double* emomi, const double* dmom, const double* emom,
+                          const int* nlist, const double* du, void* Z, double* ehc, double* rho1, int* err,
+                          hipStream_t s) {
+    auto k = k_density_mm<T, L, TA, T2, JVP>;
+    const size_t lds = (size_t)DensityLds(P.lha, P.lhm, P.nm3, P.nr2m * (P.l2m + 1), JVP).size * sizeof(T);
+    static bool set = false;
+    static size_t limit = 0;
+    hipError_t e;
+    if (!set) {
+        int dev = 0, most = 0;
+        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+        if ((e = hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) != hipSuccess) return e;
+        if ((e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, most)) != hipSuccess)
+            return e;
+        limit = (size_t)most;
+        set = true;
+    }
+    if (lds > limit) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k, dim3(natom), dim3(256), lds, s, P, off, dlist, elist, dmomi, emomi, dmom, emom, nlist, du,
+                       (cplx<T>*)Z, ehc, rho1, err);
+    return hipGetLastError();
+}
+
+template <typename T, int L, bool JVP, typename... A>
+hipError_t by_tiles(const DevParams<T>& P, A... a) {
+    const int tA = (P.lha * P.nm3 + 15) >> 4, tAll = tA + ((P.nr2m * P.lhm + 15) >> 4);
+    int ta = 0, t2 = 0;
+    for (int w = 0; w < 4; ++w) {
+        const int na = (tA - w + 3) >> 2;
+        ta = ta > na ? ta : na;
+        const int n2 = ((tAll - w + 3) >> 2) - na;
+        t2 = t2 > n2 ? t2 : n2;
+    }
+    if (tA < 1) return hipErrorInvalidValue;
+    if (ta <= 1 && t2 <= 1) return launch_density<T, L, 1, 1, JVP>(P, a...);
+    if (ta <= 2 && t2 <= 1) return launch_density<T, L, 2, 1, JVP>(P, a...);
+    if (ta <= 4 && t2 <= 3) return launch_density<T, L, 4, 3, JVP>(P, a...);
+    return hipErrorInvalidValue;  // no header of the supported classes has more
+}
+
+}  // namespace
+
+template <typename T>
+hipError_t run_density(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
+                       const double* dmomi, const double* emomi, const double* dmom, const double* emom,
+                       const Buffers& B, hipStream_t s) {
+    const int l = P.l3a > P.l2m ? P.l3a : P.l2m;
+    const int* no_list = nullptr;
+    const double* no_u = nullptr;
+    if (l <= 2) return by_tiles<T, 2, false>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+    if (l <= 4) return by_tiles<T, 4, false>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+    return by_tiles<T, 6, false>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+}
+
+hipError_t run_density_jvp(const DevParams<double>& P, int natom, const int* off, const int* nlist, const double* du,
+                           const double* dlist, const double* elist, const double* dmom, const double* emom, void* Zdot,
+                           double* ehc_dot, int* err, hipStream_t s) {
+    const int l = P.l3a > P.l2m ? P.l3a : P.l2m;
+    const double* none = nullptr;
+    double* no_rho = nullptr;
+    if (l <= 2) return by_tiles<double, 2, true>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+    if (l <= 4) return by_tiles<double, 4, true>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+    return by_tiles<double, 6, true>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+}
+
+template hipError_t run_density<double>(const DevParams<double>&, int, const int*, const double*, const double*,
+                                        const double*, const double*, const double*, const double*, const Buffers&,
+                                        hipStream_t);
+template hipError_t run_density<float>(const DevParams<float>&, int, const int*, const double*, const double*,
+                                       const double*, const double*, const double*, const double*, const Buffers&,
+                                       hipStream_t);
+
+}  // namespace magace

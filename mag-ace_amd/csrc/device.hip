@@ -126,25 +126,6 @@ __device__ __forceinline__ void spline_values(const T* __restrict__ row, const T
     }
 }
 
-// The same with horner's derivative as well: put(k, v, dv), dv = 0 where the row is absent
-template <typename T, typename F>
-__device__ __forceinline__ void spline_values_dv(const T* __restrict__ row, const T* __restrict__ safe, T w, T rs,
-                                                 int k0, int k1, int koff, T dflt, F&& put) {
-    constexpr int B = sizeof(T) == 4 ? 8 : 4;
-    for (int k = k0; k < k1; k += B) {
-        T c[B][4];
-#pragma unroll
-        for (int u = 0; u < B; ++u) load_coef(row && k + u < k1 ? row + 4 * (koff + k + u) : safe, c[u]);
-#pragma unroll
-        for (int u = 0; u < B; ++u)
-            if (k + u < k1) {
-                const T v = row ? fma(w, fma(w, fma(w, c[u][3], c[u][2]), c[u][1]), c[u][0]) : dflt;
-                const T dv = row ? fma(w, fma(w, (T)3 * c[u][3], (T)2 * c[u][2]), c[u][1]) * rs : (T)0;
-                put(k + u, v, dv);
-            }
-    }
-}
-
 // Spline row and fraction for the atomic table (src/radial.F90:68-84).
 // Returns nullptr when the pair is beyond the table (all functions zero).
 template <typename T>
@@ -303,10 +284,10 @@ __device__ __forceinline__ void store_a2_half(const DevParams<T>& P, const cplx<
     }
 }
 
-// ACC (FP32 only): A and A2 summed with Kahan compensation (the accumulation recipe of
-// MAGACE_MIXED_ACC); twice the accumulator registers, so one wave per SIMD less
-template <typename T, int L, int CH, int NB, int NM3X, int NB2, int NR2X, bool SPLIT, bool TASKSPLIT, bool ACC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6 && NM3X <= 4 ? (sizeof(T) == 4 ? (ACC ? 3 : 4) : 3) : (sizeof(T) == 4 && !ACC ? 3 : 2), 8))) k_density(DevParams<T> P, const int* __restrict__ off,
+// The density of the accumulation recipe (MAGACE_MIXED_ACC): A and A2 summed over the neighbours with
+// Kahan compensation, which the matrix cores of density.hip cannot do.
+template <typename T, int L, int CH, int NB, int NM3X, int NB2, int NR2X, bool SPLIT, bool TASKSPLIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6 && NM3X <= 4 ? 3 : 2, 8))) k_density(DevParams<T> P, const int* __restrict__ off,
                                                 const double* __restrict__ dlist,
                                                 const double* __restrict__ elist,
                                                 const double* __restrict__ dmomi,
@@ -405,7 +386,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
         for (int a = 0; a < (NB > NB2 ? NB : NB2); ++a)
 #pragma unroll
             for (int b = 0; b < (NM3X > NR2X ? NM3X : NR2X); ++b) acc[a][b] = {0, 0};
-        constexpr int kCa = ACC ? (NB > NB2 ? NB : NB2) : 1, kCq = ACC ? (NM3X > NR2X ? NM3X : NR2X) : 1;
+        constexpr int kCa = NB > NB2 ? NB : NB2, kCq = NM3X > NR2X ? NM3X : NR2X;
         cplx<T> cmp[kCa][kCq];
 #pragma unroll
         for (int a = 0; a < kCa; ++a)
@@ -586,13 +567,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         const T r = kEarly ? rv[kEarly ? b : 0] : rr[b];
 #pragma unroll
                         for (int q = 0; q < NM3X; ++q) {
-                            if constexpr (ACC) {
-                                kahan_add(acc[b][q].re, cmp[ACC ? b : 0][ACC ? q : 0].re, r * yh[q].re);
-                                kahan_add(acc[b][q].im, cmp[ACC ? b : 0][ACC ? q : 0].im, r * yh[q].im);
-                            } else {
-                                acc[b][q].re = fma(r, yh[q].re, acc[b][q].re);
-                                acc[b][q].im = fma(r, yh[q].im, acc[b][q].im);
-                            }
+                            kahan_add(acc[b][q].re, cmp[b][q].re, r * yh[q].re);
+                            kahan_add(acc[b][q].im, cmp[b][q].im, r * yh[q].im);
                         }
                     }
                 }
@@ -617,27 +593,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         const T g = kEarly ? gv[kEarly ? b : 0] : gr[b];
 #pragma unroll
                         for (int q = 0; q < NR2X; ++q) {
-                            if constexpr (ACC) {
-                                kahan_add(acc[b][q].re, cmp[ACC ? b : 0][ACC ? q : 0].re, g * my[q].re);
-                                kahan_add(acc[b][q].im, cmp[ACC ? b : 0][ACC ? q : 0].im, g * my[q].im);
-                            } else {
-                                acc[b][q].re = fma(g, my[q].re, acc[b][q].re);
-                                acc[b][q].im = fma(g, my[q].im, acc[b][q].im);
-                            }
+                            kahan_add(acc[b][q].re, cmp[b][q].re, g * my[q].re);
+                            kahan_add(acc[b][q].im, cmp[b][q].im, g * my[q].im);
                         }
                     }
                 }
             }
         }
-        if constexpr (ACC) {  // the compensated sums
+        // the compensated sums
 #pragma unroll
-            for (int a = 0; a < kCa; ++a)
+        for (int a = 0; a < kCa; ++a)
 #pragma unroll
-                for (int b = 0; b < kCq; ++b) {
-                    acc[a][b].re -= cmp[a][b].re;
-                    acc[a][b].im -= cmp[a][b].im;
-                }
-        }
+            for (int b = 0; b < kCq; ++b) {
+                acc[a][b].re -= cmp[a][b].re;
+                acc[a][b].im -= cmp[a][b].im;
+            }
         if (kSplit && sa > 1) {  // one round only: every thread of the block reaches these barriers
             cplx<T>* scr = (cplx<T>*)smem;  // [SA - 1][nTA][NB][NM3X]
             __syncthreads();
@@ -1872,203 +1842,6 @@ __global__ void __launch_bounds__(64) k_forces(DevParams<T> P, const int* __rest
 // P_t = prod Z[idx_t]; D_u P_t follows from Zdot = D_u Z, the forward-mode derivative of the
 // density along u.  FP64 only.
 
-// Y_lm (m >= 0) and D_u Y_lm = (grad Y . du) / r for a bond of unit vector (x, y, z)
-template <int L>
-__device__ __forceinline__ void ylm_half_jvp(double x, double y, double z, int lmax, double dux, double duy,
-                                             double duz, double invr, cplx<double>* out, cplx<double>* dout) {
-    double P[(L + 1) * (L + 2) / 2], dP[(L + 1) * (L + 2) / 2];
-    legendre<double, L>(z, P, dP);
-    cplx<double> ph[L + 1];
-    ph[0] = {1, 0};
-#pragma unroll
-    for (int m = 1; m <= L; ++m) ph[m] = cmul(ph[m - 1], cplx<double>{x, y});
-#pragma unroll
-    for (int l = 0; l <= L; ++l)
-#pragma unroll
-        for (int m = 0; m <= l; ++m) {
-            if (l > lmax) continue;
-            const int k = l * (l + 1) / 2 + m;
-            cplx<double> Y, g[3];
-            ylm_grad<double>(m, P[k], dP[k], ph[m], ph[m > 0 ? m - 1 : 0], x, y, z, Y, g);
-            out[k] = Y;
-            dout[k] = {(g[0].re * dux + g[1].re * duy + g[2].re * duz) * invr,
-                       (g[0].im * dux + g[1].im * duy + g[2].im * duz) * invr};
-        }
-}
-
-// Zdot = D_u Z and D_u e_hc, the pair vector of pair p = (i -> j) moving by u_i - u_j.
-// Same task layout as k_density; A0 does not depend on positions.
-// The wide class (27 magnetic columns) runs at 2 waves per SIMD: 256 registers with a spill
-// instead of 294 at 1 wave (fit step on the shape of the example potential 41.3 -> 37.3 ms).
-template <int L, int CH, int NB, int NM3X, int NB2, int NR2X>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM3X > 8 ? 2 : 1, 8)))
-k_density_jvp(DevParams<double> P, const int* __restrict__ off,
-              const int* __restrict__ nlist, const double* __restrict__ du,
-              const double* __restrict__ dlist,
-              const double* __restrict__ elist,
-              const double* __restrict__ dmom,
-              const double* __restrict__ emom,
-              cplx<double>* __restrict__ Zdot,
-              double* __restrict__ ehc_dot, int* err) {
-    using T = double;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int atom = blockIdx.x;
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int nfa = P.nr3a * (P.l3a + 1), nfm = P.nr2m * (P.l2m + 1);
-    cplx<T>* sY = (cplx<T>*)smem;        // [CH][lha]
-    cplx<T>* sYd = sY + CH * P.lha;      // [CH][lha]
-    cplx<T>* sYm = sYd + CH * P.lha;     // [CH][lhm]
-    cplx<T>* sH = sYm + CH * P.lhm;      // [CH][nm3]
-    T* sR = (T*)(sH + CH * P.nm3);       // [CH][nfa]
-    T* sRd = sR + CH * nfa;              // [CH][nfa]
-    T* sGd = sRd + CH * nfa;             // [CH][nb_a]
-    T* sM = sGd + CH * P.nb_a;           // [CH][nfm]
-    T* sCrd = sM + CH * nfm;             // [CH]
-    double* sE = sCrd + CH;              // [1]
-
-    const int p0 = off[atom], nn = off[atom + 1] - p0;
-    Zdot += (size_t)atom * P.nz;
-    const double uix = du[3 * (size_t)atom], uiy = du[3 * (size_t)atom + 1], uiz = du[3 * (size_t)atom + 2];
-    for (int t = tid; t < P.nr2m * P.lsm; t += nthr) Zdot[P.oA0 + t] = {0, 0};
-    if (tid == 0) *sE = 0.0;
-
-    const int nblkA = (P.nr3a + NB - 1) / NB, nblkA2 = (P.nb_a + NB2 - 1) / NB2;
-    // tasks cover m >= 0 only; the m < 0 entries are conjugates (see k_density)
-    const int nTA = P.lha * nblkA, nTA2 = P.lhm * nblkA2;
-    // A2 tasks start at a wave boundary when that fits in one round (no wave runs both loops)
-    const int a2base = ((nTA + 63) & ~63) + nTA2 <= nthr ? (nTA + 63) & ~63 : nTA;
-    for (int round = 0; round * nthr < a2base + nTA2; ++round) {
-        const int task = round * nthr + tid;
-        cplx<T> acc[NB > NB2 ? NB : NB2][NM3X > NR2X ? NM3X : NR2X];
-#pragma unroll
-        for (int a = 0; a < (NB > NB2 ? NB : NB2); ++a)
-#pragma unroll
-            for (int b = 0; b < (NM3X > NR2X ? NM3X : NR2X); ++b) acc[a][b] = {0, 0};
-        const bool isA = task < nTA, isA2 = task >= a2base && task < a2base + nTA2;
-        int lh = 0, l = 0, n0 = 0;
-        if (isA) { lh = task % P.lha; n0 = (task / P.lha) * NB; }
-        if (isA2) { lh = (task - a2base) % P.lhm; n0 = ((task - a2base) / P.lhm) * NB2; }
-        while ((l + 1) * (l + 2) / 2 <= lh) ++l;
-        const int m = lh - l * (l + 1) / 2;  // >= 0
-        const int lm = l * l + l + m;
-        for (int c0 = 0; c0 < nn; c0 += CH) {
-            const int nj = nn - c0 < CH ? nn - c0 : CH;
-            __syncthreads();
-            // staging of pair c0 + j spread over the block (as in k_density): role 0 the bond
-            // Y_lm and D_u Y_lm and the core term, roles 1..nsplit shares of the radial
-            // functions and their derivatives along u, role nsplit + 1 the magnetic side
-            const int j = tid % CH, role = tid / CH, nsplit = nthr / CH - 2;
-            const bool live = j < nj;
-            const int p = p0 + c0 + (live ? j : 0);
-            if (role <= nsplit) {
-                if (live) {
-                    const int jn = nlist[p];
-                    const double dux = uix - du[3 * (size_t)jn], duy = uiy - du[3 * (size_t)jn + 1],
-                                 duz = uiz - du[3 * (size_t)jn + 2];
-                    const double ex = elist[3 * p], ey = elist[3 * p + 1], ez = elist[3 * p + 2];
-                    const double rdot = ex * dux + ey * duy + ez * duz;
-                    T w;
-                    const T* row = atomic_row(P, dlist[p], w, err);
-                    if (role == 0) {
-                        T cr = 0, dcr = 0;
-                        if (row) horner(row + 4 * (P.nb_a + nfa), w, (T)P.rs_a, cr, dcr);
-                        sCrd[j] = dcr * rdot;
-                        ylm_half_jvp<L>(ex, ey, ez, P.l3a, dux, duy, duz, 1.0 / dlist[p], sY + j * P.lha,
-                                        sYd + j * P.lha);
-                    } else {
-                        const int nf = P.nb_a + nfa, per = (nf + nsplit - 1) / nsplit;
-                        const int k0 = (role - 1) * per, k1 = min(nf, k0 + per);
-                        spline_values_dv<T>(row, P.lut_a, w, (T)P.rs_a, k0, k1, 0, (T)0, [&](int k, T v, T dv) {
-                            if (k < P.nb_a) {
-                                sGd[j * P.nb_a + k] = dv * rdot;
-                            } else {
-                                sR[j * nfa + (k - P.nb_a)] = v;
-                                sRd[j * nfa + (k - P.nb_a)] = dv * rdot;
-                            }
-                        });
-                    }
-                } else if (role == 0) {
-                    sCrd[j] = 0;
-                }
-            } else if (role == nsplit + 1) {  // magnetic side (does not move with positions)
-                if (live) {
-                    T w = 0;
-                    bool unit;
-                    const T* row = magnetic_row(P, dmom[p], w, unit, err);
-                    spline_values<T>(row, P.lut_m, w, 0, nfm, P.nb_m, unit ? (T)1 : (T)0,
-                                     [&](int k, T v) { sM[j * nfm + k] = v; });
-                    cplx<T>* yh = sYm + j * P.lhm;
-                    ylm_half<T, L>(emom[3 * p], emom[3 * p + 1], emom[3 * p + 2], P.l2m, yh);
-                    for (int q = 0; q < P.nm3; ++q) {
-                        const int np = q / P.lsm3, lmp = q % P.lsm3;
-                        int lp = 0;
-                        while ((lp + 1) * (lp + 1) <= lmp) ++lp;
-                        const int mp = lmp - lp * lp - lp;
-                        const cplx<T> y = yfull(yh, lp, mp);
-                        const T mv = sM[j * nfm + lp * P.nr2m + np];
-                        sH[j * P.nm3 + q] = {mv * y.re, mv * y.im};
-                    }
-                }
-            }
-            __syncthreads();
-            if (round == 0 && tid == 0) {
-                double sum = 0.0;
-                for (int j = 0; j < nj; ++j) sum += sCrd[j];
-                *sE += sum;
-            }
-            if (isA) {
-                // unused columns and radial indices are read without a test, as in k_density
-                for (int j = 0; j < nj; ++j) {
-                    const cplx<T> y = sY[j * P.lha + lh], yd = sYd[j * P.lha + lh];
-                    cplx<T> h[NM3X];
-#pragma unroll
-                    for (int q = 0; q < NM3X; ++q) h[q] = sH[j * P.nm3 + q];
-                    const T* rr = sR + j * nfa + l * P.nr3a + n0;
-                    const T* rdr = sRd + j * nfa + l * P.nr3a + n0;
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) {
-                        const T r = rr[b], rd = rdr[b];
-                        const cplx<T> ry = {rd * y.re + r * yd.re, rd * y.im + r * yd.im};
-#pragma unroll
-                        for (int q = 0; q < NM3X; ++q) cfma(acc[b][q], ry, h[q]);
-                    }
-                }
-            } else if (isA2) {
-                for (int j = 0; j < nj; ++j) {
-                    const cplx<T> y = sYm[j * P.lhm + lh];
-                    const T* mr = sM + j * nfm + l * P.nr2m;
-                    cplx<T> my[NR2X];
-#pragma unroll
-                    for (int q = 0; q < NR2X; ++q) my[q] = {mr[q] * y.re, mr[q] * y.im};
-                    const T* gr = sGd + j * P.nb_a + n0;
-#pragma unroll
-                    for (int b = 0; b < NB2; ++b) {
-                        const T gd = gr[b];
-#pragma unroll
-                        for (int q = 0; q < NR2X; ++q) {
-                            acc[b][q].re = fma(gd, my[q].re, acc[b][q].re);
-                            acc[b][q].im = fma(gd, my[q].im, acc[b][q].im);
-                        }
-                    }
-                }
-            }
-        }
-        if (isA)
-            store_a_half<T, NB, NM3X>(P, acc, n0, l, m, Zdot);
-        else if (isA2)
-            store_a2_half<T, NB2, NR2X>(P, acc, n0, m, lm, Zdot);
-    }
-    __syncthreads();
-    if (tid == 0) ehc_dot[atom] = *sE;
-}
-
-size_t density_jvp_lds_bytes(const DevParams<double>& Pd, int CH) {
-    const int nfa = Pd.nr3a * (Pd.l3a + 1), nfm = Pd.nr2m * (Pd.l2m + 1);
-    const size_t n = 16 * ((size_t)CH * 2 * Pd.lha + (size_t)CH * Pd.lhm + (size_t)CH * Pd.nm3) +
-                     8 * ((size_t)CH * 2 * nfa + (size_t)CH * Pd.nb_a + (size_t)CH * nfm + CH + 1);
-    return ((n + 15) & ~(size_t)15) + 16;
-}
-
 // F, F' and F'' of the embedding (src/forces.F90:1134-1233)
 __device__ inline void embed2(int nfemb, double rho, double wpre, double mexp, double& F, double& dF,
                               double& d2F) {
@@ -2295,34 +2068,6 @@ __global__ void k_fill_double(double* __restrict__ p, size_t n) {
     if (i < n) p[i] = 0.0;
 }
 
-template <int L, int CH, int NB, int NM3X, int NB2, int NR2X>
-static hipError_t run_jvp_class(const DevParams<double>& P, int natom, const int* off, const int* nlist,
-                                const double* du, const double* dlist, const double* elist, const double* dmom,
-                                const double* emom, cplx<double>* Zdot, double* ehc_dot, int* err, hipStream_t s) {
-    auto k = k_density_jvp<L, CH, NB, NM3X, NB2, NR2X>;
-    const size_t lds = density_jvp_lds_bytes(P, CH);
-    static bool set = false;
-    static size_t limit = 0;
-    hipError_t e;
-    if (!set) {
-        int dev = 0, maxsh = 0;
-        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-        if ((e = hipDeviceGetAttribute(&maxsh, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) != hipSuccess)
-            return e;
-        hipFuncAttributes fa;
-        if ((e = hipFuncGetAttributes(&fa, (const void*)k)) != hipSuccess) return e;
-        limit = (size_t)maxsh - fa.sharedSizeBytes;
-        if ((e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit)) !=
-            hipSuccess)
-            return e;
-        set = true;
-    }
-    if (lds > limit) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k, dim3(natom), dim3(256), lds, s, P, off, nlist, du, dlist, elist, dmom, emom, Zdot,
-                       ehc_dot, err);
-    return hipGetLastError();
-}
-
 hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int natom, const int* off, const int* nlist,
                         const double* du, const double* dlist, const double* elist, const double* dmomi,
                         const double* dmom, const double* emom, const int* atom_struct, const double* gE,
@@ -2333,12 +2078,7 @@ hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int na
     OrderCounts nbo;
     int nb234 = 0;
     for (int o = 0; o < 5; ++o) nb234 += (nbo.n[o] = nbo5[o]);
-    hipError_t e = cls == 0   ? run_jvp_class<6, 32, 4, 4, 4, 2>(P, natom, off, nlist, du, dlist, elist, dmom, emom,
-                                                                 (cplx<double>*)F.Zdot, F.ehc_dot, B.err, s)
-                   : cls == 1 ? run_jvp_class<2, 32, 1, 27, 2, 5>(P, natom, off, nlist, du, dlist, elist, dmom, emom,
-                                                                  (cplx<double>*)F.Zdot, F.ehc_dot, B.err, s)
-                              : run_jvp_class<6, 32, 4, 9, 4, 5>(P, natom, off, nlist, du, dlist, elist, dmom, emom,
-                                                                 (cplx<double>*)F.Zdot, F.ehc_dot, B.err, s);
+    hipError_t e = run_density_jvp(P, natom, off, nlist, du, dlist, elist, dmom, emom, F.Zdot, F.ehc_dot, B.err, s);
     if (e != hipSuccess) return e;
     if (nd == 2)
         hipLaunchKernelGGL(k_fit_atom<2>, dim3(natom), dim3(256), 0, s, P, scaled, (const cplx<double>*)B.Wd,
@@ -2428,7 +2168,9 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
     Pd.lhm = P.lhm; Pd.nm3 = P.nm3; Pd.nb_a = P.nb_a; Pd.nb_m = P.nb_m;
     const size_t lds1 = density_lds_bytes(Pd, CH, sizeof(T));
     static_assert(!ACC || sizeof(T) == 4, "the accumulation recipe belongs to the FP32 kernels");
-    auto k1 = k_density<T, L, CH, NB, NM3X, NB2, NR2X, SPLIT, TASKSPLIT, ACC>;
+    // the accumulation recipe's density; the others run on the matrix cores (density.hip)
+    const void* k1 = nullptr;
+    if constexpr (ACC) k1 = (const void*)k_density<T, L, CH, NB, NM3X, NB2, NR2X, SPLIT, TASKSPLIT>;
     const bool nd2 = P.nd == 2;
     // the Q1 instantiation exists only for the four-column class.  Q1 visits every radial index
     // up to its compile-time bound, so the bounds 4 (for nr3a <= 4), 5, 6, 7 and NRAX each have
@@ -2458,7 +2200,7 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
         if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
         if ((e = hipDeviceGetAttribute(&maxsh, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) != hipSuccess)
             return e;
-        const void* ks[10] = {(const void*)k1, (const void*)k_adjoint<T, false, ACC>,
+        const void* ks[10] = {k1, (const void*)k_adjoint<T, false, ACC>,
                               (const void*)k_adjoint<T, true, ACC>, nullptr, (const void*)k3g,
                               (const void*)k3qs[0], (const void*)k3qs[1], (const void*)k3qs[2],
                               (const void*)k3qs[3], (const void*)k3qs[4]};
@@ -2486,12 +2228,16 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
     // FP64 sums over monomial products it is defined by
     const bool nodes = N.nw > 0 && !ACC;
     if (!nodes && pair && lds2p > limit[3]) return hipErrorInvalidValue;
-    if (lds1 > limit[0] || (!nodes && lds2 > limit[nd2 ? 2 : 1]) || lds3 > limit[q1 ? 5 + qi : 4])
+    if ((ACC && lds1 > limit[0]) || (!nodes && lds2 > limit[nd2 ? 2 : 1]) || lds3 > limit[q1 ? 5 + qi : 4])
         return hipErrorInvalidValue;
     if (ev) (void)hipEventRecord(ev[0], s);
-    hipLaunchKernelGGL(k1, dim3(natom), dim3(256), lds1, s, P, off, dlist, elist, dmomi, emomi, dmom,
-                       emom, (cplx<T>*)B.Z, B.ehc, B.rho1, B.err);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if constexpr (ACC) {
+        hipLaunchKernelGGL((k_density<T, L, CH, NB, NM3X, NB2, NR2X, SPLIT, TASKSPLIT>), dim3(natom), dim3(256), lds1, s, P,
+                           off, dlist, elist, dmomi, emomi, dmom, emom, (cplx<T>*)B.Z, B.ehc, B.rho1, B.err);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    } else if ((e = run_density<T>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, B, s)) != hipSuccess) {
+        return e;
+    }
     if (ev) (void)hipEventRecord(ev[1], s);
     if (nodes && (e = run_adjoint_nodes<T>(P, N, natom, B, eout, s)) != hipSuccess) return e;
     if constexpr (sizeof(T) == 4) {
@@ -2541,15 +2287,17 @@ hipError_t Launch<T>::run(const DevParams<T>& P, const NodeTab<T>& N, int natom,
                 : run_class<T, 6, CH, SPLIT, TS, 4, 9, 4, 5, 8, 16, ACC>(P, N, natom, atom_base, off, dlist, elist,      \
                                                                          dmomi, emomi, dmom, emom, eout, flist,      \
                                                                          tlist, tlist0, B, s, ev))
-    // the accumulation recipe (MAGACE_MIXED_ACC) exists for the FP32 kernels only
-#define MAGACE_RUN(CH, SPLIT, TS) \
-    (sizeof(T) == 4 && acc ? MAGACE_RUN_ACC(CH, SPLIT, TS, (sizeof(T) == 4)) : MAGACE_RUN_ACC(CH, SPLIT, TS, false))
-    // a density variant chosen by the tuner (kDensityVariants) replaces the rule above
-    if (dvar < 0) dvar = heavy ? 0 : (sizeof(T) == 8 ? 1 : 2);
-    if (dvar == 0) return MAGACE_RUN(32, true, false);
-    if (dvar == 1) return MAGACE_RUN(32, true, true);
-    return MAGACE_RUN(64, false, true);
-#undef MAGACE_RUN
+    if constexpr (sizeof(T) == 4) {
+        if (acc) {
+            // the accumulation recipe's density staging: a variant chosen by the tuner (kDensityVariants)
+            // replaces the rule
+            if (dvar < 0) dvar = heavy ? 0 : 2;
+            if (dvar == 0) return MAGACE_RUN_ACC(32, true, false, true);
+            if (dvar == 1) return MAGACE_RUN_ACC(32, true, true, true);
+            return MAGACE_RUN_ACC(64, false, true, true);
+        }
+    }
+    return MAGACE_RUN_ACC(32, true, false, false);
 #undef MAGACE_RUN_ACC
 }
 

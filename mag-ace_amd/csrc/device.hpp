@@ -23,7 +23,13 @@ template <typename T>
 struct DevParams {
     const T* lut_a = nullptr;  // atomic spline rows [nlut][stride_a]
     const T* lut_m = nullptr;  // magnetic spline rows [nlut][stride_m]
-    int stride_a = 0, stride_m = 0, nlut = 0;
+    const T* lut_g = nullptr;  // rows of the base functions g_1..g_nb and the core term alone [nlut][stride_g]
+    const T* cperm = nullptr;  // radial coefficients C_{nlk} as A operands, [l3a + 1][4][64] (density.hip)
+    // columns of the density's products, 16 a tile, of A (Y entry | q << 8 | l << 16 | m << 20 | m' + 8 << 24),
+    // then of A2 (Y' entry | M entry << 8 | l << 16 | m << 20 | n' << 24), then the A0 entries (Y' entry |
+    // M entry << 8 | real part negative << 16 | imaginary part negative << 17)
+    const uint32_t* cols = nullptr;
+    int stride_a = 0, stride_m = 0, stride_g = 0, nlut = 0;
     double rs_a = 0, rs_m = 0;  // nlut / cutoff (index arithmetic stays FP64)
     int nb_a = 0, nb_m = 0, nr2m = 0, l2m = 0, nr3a = 0, nr3m = 0, l3a = 0, l3m = 0;
     int lsa = 0, lsm = 0, lsm3 = 0, nm3 = 0, oA2 = 0, oA0 = 0, nz = 0;
@@ -170,6 +176,18 @@ hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int na
                         Buffers& B, FitBuffers& F, int nterms, const int* nbo5, double* grad, hipStream_t s);
 hipError_t fit_assemble(int natom, const int* off, const int* nlist, const double* flist, const double* eout,
                         const int* atom_struct, int nstruc, double* f, double* estruct, hipStream_t s);
+
+// Z, e_hc and the B1 part of rho (density.hip)
+template <typename T>
+hipError_t run_density(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
+                       const double* dmomi, const double* emomi, const double* dmom, const double* emom,
+                       const Buffers& B, hipStream_t s);
+// their derivative along the displacements du of the atoms (fitting)
+hipError_t run_density_jvp(const DevParams<double>& P, int natom, const int* off, const int* nlist, const double* du,
+                           const double* dlist, const double* elist, const double* dmom, const double* emom, void* Zdot,
+                           double* ehc_dot, int* err, hipStream_t s);
+// row of a 16x16x4 product's result in register r of lane group g, by the size of a value (matrix.hpp)
+inline int matrix_row(size_t bytes, int g, int r) { return bytes == 4 ? 4 * g + r : g + 4 * r; }
 
 hipError_t upload_legendre_constants();
 hipError_t clear_flags(int* p, hipStream_t s);
