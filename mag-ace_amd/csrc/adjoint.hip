@@ -137,15 +137,16 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
     double* red = (double*)(smem + (size_t)N.nslots * 16);  // [NA][NT / 64]
     const cplx<T>* __restrict__ Z0 = Zin + (size_t)a0 * P.nz;
     const cplx<T>* __restrict__ Z1 = two ? Z0 + P.nz : Z0;  // an odd last atom is paired with itself
-    auto load = [&](int x) {
+    auto load = [&](uint32_t e) {  // a ZLayout::half entry
         V v;
+        const uint32_t x = e & 0xfff;
         const cplx<T> a = Z0[x];
         v[0] = a.re, v[1] = a.im;
         if constexpr (NA == 2) {
             const cplx<T> b = Z1[x];
             v[2] = b.re, v[3] = b.im;
         }
-        return v;
+        return slot_flip(v, (e << 17) & 0x80000000u, (e << 16) & 0x80000000u);
     };
     // the atoms' e_hc and B1 part of rho, read ahead by the threads that evaluate their energies
     const int eatom = tid == NT - 64 ? a0 : NA == 2 && tid == NT - 63 && two ? a0 + 1 : -1;
@@ -298,7 +299,7 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
         if (lane == 0) red[a * (NT / 64) + wave] = rho[a];
     }
     __syncthreads();
-    // the gradient of the representatives; what the other entries of W hold is never read
+    // the gradient of the stored entries (0 where the conjugate partner stands for the pair)
     auto fetch = [&](int x) {
         V v;
         const cplx<T> a = W0[x];

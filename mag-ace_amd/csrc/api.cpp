@@ -69,6 +69,8 @@ struct DevTables {
     T* lut_m = nullptr;
     T* lut_g = nullptr;
     T* cperm = nullptr;
+    T* crow = nullptr;
+    uint2* vcol = nullptr;
 };
 
 struct Context {
@@ -94,7 +96,9 @@ struct Context {
     int2* comb = nullptr;
     int2* comb2 = nullptr;
     uint32_t* fold = nullptr;
-    uint32_t* cols = nullptr;  // DevParams::cols
+    uint32_t* cols = nullptr;  // DevParams::cols, steps, zmap
+    double* steps = nullptr;
+    uint16_t* zmap = nullptr;
     int2* ypair = nullptr;     // products of two A entries (body orders 5, 6), TermList::ypair
     int2* yft = nullptr;       // their gradient's way back to Z (TermList::yft, yfe)
     int2* yfe = nullptr;
@@ -194,7 +198,9 @@ void dfree(T*& p) {
 
 Context::~Context() {
     dfree(t64.lut_a); dfree(t64.lut_m); dfree(t32.lut_a); dfree(t32.lut_m);
-    dfree(t64.lut_g); dfree(t64.cperm); dfree(t32.lut_g); dfree(t32.cperm);
+    dfree(t64.lut_g); dfree(t64.cperm); dfree(t64.crow); dfree(t64.vcol);
+    dfree(t32.lut_g); dfree(t32.cperm); dfree(t32.crow); dfree(t32.vcol);
+    dfree(steps); dfree(zmap);
     dfree(crec64); dfree(crec32); dfree(crec16); dfree(crecu); dfree(crec16u); dfree(chunks); dfree(comb); dfree(comb2); dfree(fold); dfree(cols); dfree(cw2_64);
     dfree(ypair); dfree(yft); dfree(yfe);
     dfree(cw2_32);
@@ -240,12 +246,7 @@ void fill_params(DevParams<T>& P, const Model& M) {
     P.nr3a = h.nr3_a; P.nr3m = h.nr3_m; P.l3a = h.l3a; P.l3m = M.z.lAm;  // the magnetic l range of A
     P.lsa = M.z.lsa; P.lsm = M.z.lsm; P.lsm3 = M.z.lsm3; P.nm3 = M.z.nm3;
     P.oA2 = M.z.oA2; P.oA0 = M.z.oA0; P.nz = M.z.nz;
-    for (int q = 0; q < M.z.nm3 && q < 32; ++q) {
-        const int lq = q % M.z.lsm3;
-        int lp = 0;
-        while ((lp + 1) * (lp + 1) <= lq) ++lp;
-        P.mpq[q] = (signed char)(lq - lp * lp - lp);
-    }
+    P.hA2 = M.z.hA2; P.hA0 = M.z.hA0; P.nzh = M.z.nh;
     P.lha = (h.l3a + 1) * (h.l3a + 2) / 2;
     P.lhm = (h.l2m + 1) * (h.l2m + 2) / 2;
     P.nchunks = (int)(M.terms.chunks.size() / 2);
@@ -303,7 +304,13 @@ int upload_base_tables(DevTables<T>& t, const Model& M) {
                 if (n < h.nr3_a && k < h.nb_a)
                     c[((size_t)l * 4 + r) * 64 + lane] = M.pot.crad_a[((size_t)n * (h.l3a + 1) + l) * h.nb_a + k];
             }
-    return upload_table(t.cperm, c);
+    if (upload_table(t.cperm, c)) return MAGACE_ERR_DEVICE;
+    std::vector<double> r((size_t)(h.l3a + 1) * 8 * 16, 0.0);
+    for (int l = 0; l <= h.l3a; ++l)
+        for (int n = 0; n < h.nr3_a; ++n)
+            for (int k = 0; k < h.nb_a; ++k)
+                r[((size_t)l * 8 + n) * 16 + k] = M.pot.crad_a[((size_t)n * (h.l3a + 1) + l) * h.nb_a + k];
+    return upload_table(t.crow, r);
 }
 
 // DevParams::cols
@@ -315,29 +322,111 @@ std::vector<uint32_t> density_columns(const Model& M) {
     };
     for (int l = 0; l <= h.l3a; ++l)
         for (int m = 0; m <= l; ++m)
-            for (int q = 0; q < M.z.nm3; ++q) {
-                const int lq = q % M.z.lsm3;
-                int lp = 0;
-                while ((lp + 1) * (lp + 1) <= lq) ++lp;
-                const int mp = lq - lp * lp - lp;
-                v.push_back((uint32_t)(l * (l + 1) / 2 + m) | (uint32_t)q << 8 | (uint32_t)l << 16 | (uint32_t)m << 20 |
-                            (uint32_t)(mp + 8) << 24);
-            }
+            for (int q = 0; q < M.z.nm3; ++q)
+                v.push_back((uint32_t)(l * (l + 1) / 2 + m) | (uint32_t)q << 8 | (uint32_t)l << 16);
     pad();
     for (int np = 0; np < h.nr2_m; ++np)
         for (int l = 0; l <= h.l2m; ++l)
             for (int m = 0; m <= l; ++m)
-                v.push_back((uint32_t)(l * (l + 1) / 2 + m) | (uint32_t)(l * h.nr2_m + np) << 8 | (uint32_t)l << 16 |
-                            (uint32_t)m << 20 | (uint32_t)np << 24);
+                v.push_back((uint32_t)(l * (l + 1) / 2 + m) | (uint32_t)(l * h.nr2_m + np) << 8);
     pad();
-    for (int np = 0; np < h.nr2_m; ++np)
-        for (int l = 0; l <= h.l2m; ++l)
-            for (int m = -l; m <= l; ++m) {
-                // Y_{l,-m} = (-1)^m conj(Y_lm)
-                const int am = m < 0 ? -m : m;
-                v.push_back((uint32_t)(l * (l + 1) / 2 + am) | (uint32_t)(l * h.nr2_m + np) << 8 |
-                            (m < 0 && (am & 1) ? 1u << 16 : 0u) | (m < 0 && !(am & 1) ? 1u << 17 : 0u));
+    return v;
+}
+
+// Walks of the four lane groups through the harmonics l <= lmax, m >= 0 (forces.hip), walk[g][t] = (l, m):
+// every order m is walked by one group, the longest first, each by the group with the shortest walk; or all
+// orders by every group.
+typedef std::array<std::vector<std::pair<int, int>>, 4> Walks;
+Walks harmonic_walks(int lmax, bool all) {
+    Walks walk;
+    for (int m = 0; m <= lmax; ++m) {
+        int g = 0;
+        for (int k = 1; k < 4; ++k)
+            if (walk[k].size() < walk[g].size()) g = k;
+        for (int l = m; l <= lmax; ++l)
+            for (int k = 0; k < 4; ++k)
+                if (all || k == g) walk[k].emplace_back(l, m);
+    }
+    return walk;
+}
+int walk_steps(const Walks& walk) {
+    size_t n = 0;
+    for (const auto& w : walk) n = std::max(n, w.size());
+    return (int)n;
+}
+
+// DevParams::qsplit: whichever gives fewer products, all harmonics in every group and 16 columns q a round, or
+// the orders spread over the groups and 4 (27 columns at l <= 2: 12 instead of 21 tiles; 4 at l <= 6: 28 or 7)
+bool split_columns(const Model& M) {
+    const int nq4 = (M.z.nm3 + 3) / 4, l = M.pot.h.l3a;
+    return (nq4 + 3) / 4 * walk_steps(harmonic_walks(l, true)) < nq4 * walk_steps(harmonic_walks(l, false));
+}
+
+// DevParams::steps of one side: 4 numbers a step and group; sq_a etc. as src/spherical.F90:18-49
+// and returns the steps that are some group's first of an order
+uint32_t append_steps(const Walks& walk, int nr2m, std::vector<double>& out) {
+    uint32_t first = 0;
+    for (int t = 0; t < walk_steps(walk); ++t)
+        for (int g = 0; g < 4; ++g) {
+            double a = 0.0, b = 0.0, c = 0.0;
+            int lm = 0;
+            if (t < (int)walk[g].size()) {
+                const int l = walk[g][t].first, m = walk[g][t].second;
+                lm = l | m << 8 | (l == m ? 1 << 16 : 0) | 1 << 17 | l * nr2m << 18;
+                if (l == m) first |= 1u << t;
+                if (l == m) {  // P_m^m
+                    c = 1.0;
+                    for (int k = 1; k <= m; ++k) c *= -std::sqrt(1.0 + 0.5 / k);
+                } else if (l == m + 1) {
+                    a = std::sqrt(2.0 * m + 3.0);
+                } else {
+                    const double ll = (double)l * l, l1 = (double)(l - 1) * (l - 1), mm = (double)m * m;
+                    a = std::sqrt((4.0 * ll - 1.0) / (ll - mm));
+                    b = -a * std::sqrt((l1 - mm) / (4.0 * l1 - 1.0));
+                }
             }
+            out.insert(out.end(), {a, b, c, (double)lm});
+        }
+    return first;
+}
+
+// rows of the tiles of V for results of `bytes` a value (DevParams::vcol)
+std::vector<uint2> force_columns(const Model& M, size_t bytes, bool qsplit) {
+    const Header& h = M.pot.h;
+    const Walks wa = harmonic_walks(h.l3a, qsplit), wm = harmonic_walks(h.l2m, false);
+    const int sta = walk_steps(wa), stm = walk_steps(wm), lhm = (h.l2m + 1) * (h.l2m + 2) / 2, nq4 = (M.z.nm3 + 3) / 4;
+    std::vector<uint2> v;
+    auto tile = [&](auto&& column) {
+        uint2 rows[16];
+        for (int g = 0; g < 4; ++g)
+            for (int r = 0; r < 4; ++r) rows[matrix_row(bytes, g, r)] = column(g, r);
+        v.insert(v.end(), rows, rows + 16);
+    };
+    const uint2 none = make_uint2(~0u, 0);
+    for (int rd = 0; rd < (qsplit ? (nq4 + 3) / 4 : nq4); ++rd)
+        for (int t = 0; t < sta; ++t)
+            tile([&](int g, int r) {
+                const int q = 4 * (qsplit ? 4 * rd + g : rd) + r;
+                if (t >= (int)wa[g].size() || q >= M.z.nm3) return none;
+                const int l = wa[g][t].first, c = (l * (l + 1) / 2 + wa[g][t].second) * M.z.nm3;
+                int lp = 0;
+                const int x = q % M.z.lsm3;
+                while ((lp + 1) * (lp + 1) <= x) ++lp;
+                const int mp = x - lp * lp - lp, plus = q + (mp < 0 ? -2 * mp : 0), minus = q - (mp > 0 ? 2 * mp : 0);
+                if (mp == 0) return make_uint2((uint32_t)(c + q) | (uint32_t)l << 16, 0);
+                // H_-m' = (-1)^m' conj(H_m'): W_+ H_+ + W_- H_- = (W_+ + s W_-) Re H_+ + i (W_+ - s W_-) Im H_+
+                const bool sine = mp < 0, minus_sign = ((mp & 1) != 0) != sine;
+                return make_uint2((uint32_t)(c + plus) | (uint32_t)l << 16 | 1u << 25 | (sine ? 1u << 26 : 0u) |
+                                      (minus_sign ? 1u << 27 : 0u),
+                                  (uint32_t)(c + minus));
+            });
+    for (int s0 = 0; s0 < stm * h.nr2_m; s0 += 4)
+        tile([&](int g, int r) {
+            const int t = (s0 + r) / h.nr2_m, np = (s0 + r) % h.nr2_m;
+            if (t >= (int)wm[g].size()) return none;
+            const int l = wm[g][t].first, m = wm[g][t].second;
+            return make_uint2((uint32_t)(np * lhm + l * (l + 1) / 2 + m) | 1u << 24, 0);
+        });
     return v;
 }
 
@@ -595,10 +684,28 @@ int upload(Context& c) {
     if (ncomb2) HIPCHK(hipMemcpy(c.comb2, M.terms.comb2.data(), ncomb2 * sizeof(int2), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc((void**)&c.fold, M.terms.fold.size() * sizeof(uint32_t) + 64));
     HIPCHK(hipMemcpy(c.fold, M.terms.fold.data(), M.terms.fold.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    auto up_vec = [](auto*& d, const auto& v) -> int {
+        HIPCHK(hipMalloc((void**)&d, v.size() * sizeof(v[0]) + 64));
+        if (!v.empty()) HIPCHK(hipMemcpy(d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
+        return 0;
+    };
     {
-        const std::vector<uint32_t> v = density_columns(M);
-        HIPCHK(hipMalloc((void**)&c.cols, v.size() * sizeof(uint32_t) + 64));
-        HIPCHK(hipMemcpy(c.cols, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        const bool qsplit = split_columns(M);
+        const Walks wa = harmonic_walks(M.pot.h.l3a, qsplit), wm = harmonic_walks(M.pot.h.l2m, false);
+        std::vector<double> steps;
+        c.P64.firsta = c.P32.firsta = append_steps(wa, M.pot.h.nr2_m, steps);
+        c.P64.firstm = c.P32.firstm = append_steps(wm, M.pot.h.nr2_m, steps);
+        c.P64.sta = c.P32.sta = walk_steps(wa);
+        c.P64.stm = c.P32.stm = walk_steps(wm);
+        for (const auto& w : wm)
+            for (int t = 0; t < (int)w.size(); ++t)
+                if (w[t].first <= M.pot.h.l3m) c.P64.sth = c.P32.sth = std::max(c.P64.sth, t + 1);
+        c.P64.qsplit = c.P32.qsplit = qsplit;
+        if (int rc = up_vec(c.cols, density_columns(M))) return rc;
+        if (int rc = up_vec(c.steps, steps)) return rc;
+        if (int rc = up_vec(c.zmap, M.z.half)) return rc;
+        if (int rc = up_vec(c.t64.vcol, force_columns(M, 8, qsplit))) return rc;
+        if (int rc = up_vec(c.t32.vcol, force_columns(M, 4, qsplit))) return rc;
     }
     auto up_int2 = [](int2*& d, const std::vector<int32_t>& v) -> int {
         HIPCHK(hipMalloc((void**)&d, v.size() * sizeof(int32_t) + 64));
@@ -629,6 +736,10 @@ int upload(Context& c) {
     c.P64.comb2 = c.P32.comb2 = c.comb2;
     c.P64.fold = c.P32.fold = c.fold;
     c.P64.cols = c.P32.cols = c.cols;
+    c.P64.steps = c.P32.steps = c.steps;
+    c.P64.zmap = c.P32.zmap = c.zmap;
+    c.P64.vcol = c.t64.vcol; c.P32.vcol = c.t32.vcol;
+    c.P64.crow = c.t64.crow; c.P32.crow = c.t32.crow;
     c.P64.ypair = c.P32.ypair = c.ypair;
     c.P64.yft = c.P32.yft = c.yft;
     c.P64.yfe = c.P32.yfe = c.yfe;

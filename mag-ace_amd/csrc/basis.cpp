@@ -344,6 +344,35 @@ ZLayout make_layout(const Header& h) {
     z.oA2 = h.nr3_a * z.lsa * z.nm3;
     z.oA0 = z.oA2 + h.nb_a * h.nr2_m * z.lsm;
     z.nz = z.oA0 + h.nr2_m * z.lsm;
+    // the stored half (ZLayout::half)
+    const int lha = (h.l3a + 1) * (h.l3a + 2) / 2, lhm = (h.l2m + 1) * (h.l2m + 2) / 2;
+    z.hA2 = h.nr3_a * lha * z.nm3;
+    z.hA0 = z.hA2 + h.nb_a * h.nr2_m * lhm;
+    z.nh = z.hA0 + h.nr2_m * lhm;
+    z.half.assign(z.nz, 0);
+    z.stored.assign(z.nz, 0);
+    auto put = [&](int x, int place, bool conj, int order) {
+        // X_bar = (-1)^order conj(X)
+        z.stored[x] = !conj;
+        z.half[x] = (uint16_t)(place | (conj ? (order & 1 ? 1 << 14 : 1 << 15) : 0));
+    };
+    for (int n = 0; n < h.nr3_a; ++n)
+        for (int l = 0; l <= h.l3a; ++l)
+            for (int m = -l; m <= l; ++m)
+                for (int np = 0; np < h.nr3_m; ++np)
+                    for (int lp = 0; lp <= z.lAm; ++lp)
+                        for (int mp = -lp; mp <= lp; ++mp) {
+                            const bool conj = m < 0;
+                            const int am = conj ? -m : m, q = np * z.lsm3 + lp * lp + lp + (conj ? -mp : mp);
+                            put(z.a(n, l, m, np, lp, mp), (n * lha + l * (l + 1) / 2 + am) * z.nm3 + q, conj, m + mp);
+                        }
+    for (int np = 0; np < h.nr2_m; ++np)
+        for (int lp = 0; lp <= h.l2m; ++lp)
+            for (int mp = -lp; mp <= lp; ++mp) {
+                const int am = mp < 0 ? -mp : mp, c = np * lhm + lp * (lp + 1) / 2 + am;
+                put(z.a0(np, lp, mp), z.hA0 + c, mp < 0, mp);
+                for (int n = 0; n < h.nb_a; ++n) put(z.a2(n, np, lp, mp), z.hA2 + n * h.nr2_m * lhm + c, mp < 0, mp);
+            }
     return z;
 }
 
@@ -1037,7 +1066,7 @@ TermList build_terms(const Potential& pot, const ZLayout& z) {
         for (int d = 1; d < nd; ++d)
             for (size_t r = 0; r < nr; ++r) T.cw[d * nr + r] = T.rec_t[r] >= 0 ? T.w[d * nt + T.rec_t[r]] : 0.0;
     }
-    // representatives: A entries with m' > 0, or m' = 0 and m >= 0; A2/A0 entries with m' >= 0
+    // representatives: A entries with m > 0, or m = 0 and m' >= 0; A2/A0 entries with m' >= 0
     T.fold.assign(z.nz, 0u);
     for (int n = 0; n < h.nr3_a; ++n)
         for (int l = 0; l <= h.l3a; ++l)
@@ -1046,7 +1075,7 @@ TermList build_terms(const Potential& pot, const ZLayout& z) {
                     for (int lp = 0; lp <= z.lAm; ++lp)
                         for (int mp = -lp; mp <= lp; ++mp) {
                             const int x = z.a(n, l, m, np, lp, mp);
-                            const bool rep = mp > 0 || (mp == 0 && m >= 0);
+                            const bool rep = m > 0 || (m == 0 && mp >= 0);
                             const bool self = m == 0 && mp == 0;
                             T.fold[x] = (uint32_t)cj.partner[x] | ((cj.sign[x] < 0 ? 1u : 0u) << 16) |
                                         ((rep ? 1u : 0u) << 17) | ((self ? 1u : 0u) << 18);
@@ -1059,6 +1088,7 @@ TermList build_terms(const Potential& pot, const ZLayout& z) {
         T.fold[x] = (uint32_t)cj.partner[x] | ((cj.sign[x] < 0 ? 1u : 0u) << 16) |
                     ((mp >= 0 ? 1u : 0u) << 17) | ((mp == 0 ? 1u : 0u) << 18);
     }
+    for (int x = 0; x < z.nz; ++x) T.fold[x] |= z.stored[x] ? 1u << 19 : 0u;
     return T;
 }
 

@@ -272,15 +272,15 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
         __syncthreads();
         if (c0 == 0) {
             // A0 (src/a_basis.F90:90-106); it does not depend on positions
-            for (int t = tid; t < P.nr2m * P.lsm; t += 256) {
+            for (int t = tid; t < nA2; t += 256) {
                 cplx<T> z = {0, 0};
                 if constexpr (!JVP) {
-                    const uint32_t d = P.cols[tAll * 16 + t];
+                    const uint32_t d = P.cols[tA * 16 + t];
                     const cplx<T> h = sYm[kPairs * D.sYm + (d & 0xff)];
                     const T mv = sM[kPairs * D.sM + (d >> 8 & 0xff)];
-                    z = {(d >> 16 & 1 ? -mv : mv) * h.re, (d >> 17 & 1 ? -mv : mv) * h.im};
+                    z = {mv * h.re, mv * h.im};
                 }
-                Zout[P.oA0 + t] = z;
+                Zout[P.hA0 + t] = z;
             }
         }
         for (int s0 = 0; s0 < nj4; s0 += kChain<T>) {
@@ -352,7 +352,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
     for (int t = 0; t < TA; ++t)
         if (t < na) {
             // A = C B for each l that the tile's columns have
-            const int l = ca[t] >> 16 & 15, m = ca[t] >> 20 & 15, q = ca[t] >> 8 & 0xff, mp = (int)(ca[t] >> 24 & 31) - 8;
+            const int l = ca[t] >> 16 & 15;
             const int l0 = __builtin_amdgcn_readlane(l, 0), l1 = __builtin_amdgcn_readlane(l, 15);
             V zr = (V)(T)0, zi = (V)(T)0;
             T k[4];
@@ -374,37 +374,24 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                     zi = bi;
                 }
             }
-            const T sg = ((m + mp) & 1) ? (T)-1 : (T)1;
-            if ((wave + 4 * t) * 16 + ci < nA) {
-                cplx<T>* z0 = Zout + (l * l + l + m) * P.nm3 + q;
+            const int c = (wave + 4 * t) * 16 + ci;
+            if (c < nA)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int n = Mm<T>::row(g, r);
-                    if (n < P.nr3a) {
-                        cplx<T>* z = z0 + n * P.lsa * P.nm3;
-                        *z = {zr[r], zi[r]};
-                        // A[n][l,-m][qbar] = (-1)^(m+m') conj(A[n][l,m][q])
-                        if (m > 0) z[-2 * m * P.nm3 - 2 * mp] = {sg * zr[r], -sg * zi[r]};
-                    }
+                    if (n < P.nr3a) Zout[n * nA + c] = {zr[r], zi[r]};
                 }
-            }
         }
 #pragma unroll
-    for (int t = 0; t < T2; ++t)
-        if (t < n2 && (wave + 4 * (na + t) - tA) * 16 + ci < nA2) {
-            const int l = c2[t] >> 16 & 15, m = c2[t] >> 20 & 15, np = c2[t] >> 24;
-            const T sg = (m & 1) ? (T)-1 : (T)1;
-            cplx<T>* z0 = Zout + P.oA2 + np * P.lsm + l * l + l + m;
+    for (int t = 0; t < T2; ++t) {
+        const int c = (wave + 4 * (na + t) - tA) * 16 + ci;
+        if (t < n2 && c < nA2)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int k = Mm<T>::row(g, r);
-                if (k < P.nb_a) {
-                    cplx<T>* z = z0 + k * P.nr2m * P.lsm;
-                    *z = {a2r[t][r], a2i[t][r]};
-                    if (m > 0) z[-2 * m] = {sg * a2r[t][r], -sg * a2i[t][r]};
-                }
+                if (k < P.nb_a) Zout[P.hA2 + k * nA2 + c] = {a2r[t][r], a2i[t][r]};
             }
-        }
+    }
     if (wave == 0) {
         for (int o = 32; o > 0; o >>= 1) core += __shfl_xor(core, o, 64);
         if (lane == 0) ehc_out[atom] = core;

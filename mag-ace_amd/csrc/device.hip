@@ -182,29 +182,6 @@ __device__ __forceinline__ void legendre(T z, T* P, T* dP) {
     }
 }
 
-// Y_lm (m >= 0) and its tangential gradient (src/spherical.F90:185-260), from the Legendre
-// values and the phase powers ph[m] = (x+iy)^m.
-template <typename T>
-__device__ __forceinline__ void ylm_grad(int m, T Plm, T dPlm, cplx<T> phm, cplx<T> phm1, T x, T y,
-                                         T z, cplx<T>& Y, cplx<T> (&g)[3]) {
-    Y = {Plm * phm.re, Plm * phm.im};
-    cplx<T> gx, gy, gz;
-    if (m == 0) {
-        gx = {0, 0};
-        gy = {0, 0};
-        gz = {dPlm, 0};
-    } else {
-        const T s = (T)m * Plm;
-        gx = {s * phm1.re, s * phm1.im};
-        gy = {-gx.im, gx.re};
-        gz = {dPlm * phm.re, dPlm * phm.im};
-    }
-    const cplx<T> rdy = {x * gx.re + y * gy.re + z * gz.re, x * gx.im + y * gy.im + z * gz.im};
-    g[0] = {gx.re - rdy.re * x, gx.im - rdy.im * x};
-    g[1] = {gy.re - rdy.re * y, gy.im - rdy.im * y};
-    g[2] = {gz.re - rdy.re * z, gz.im - rdy.im * z};
-}
-
 // half set of Y_lm (m >= 0) written to out[lh]
 template <typename T, int L>
 __device__ __forceinline__ void ylm_half(T x, T y, T z, int lmax, cplx<T>* out) {
@@ -240,47 +217,30 @@ __device__ __forceinline__ cplx<T> yfull(const cplx<T>* half, int l, int m) {
 // magnetic columns): 3 waves per SIMD in FP32 (168 registers, a 12-byte spill; on the shape
 // of the example potential 0.75 -> 0.57 ms) and 2 in FP64 (256 registers with a 192-byte
 // spill instead of 302 registers at 1 wave: 2.06 -> 1.33 ms).
-// Stores of the m >= 0 density tasks (k_density, k_density_jvp): A[n][l,m][q] for the task's
-// radial block and, for m > 0, the conjugate partners
-// A[n][l,-m][qbar] = (-1)^(m+m') conj(A[n][l,m][q]) with q = n' lsm3 + l'^2 + l' + m' and
-// qbar = n' lsm3 + l'^2 + l' - m'; A2[n][n'][l',m'] and A2[n][n'][l',-m'] = (-1)^m' conj(.).
+// Stores of the m >= 0 density tasks: A[n][l,m][q] for the task's radial block, A2[n][n'][l',m'], in the
+// places of ZLayout::half.
 template <typename T, int NB, int NM3X, int NACC, int NQ>
-__device__ __forceinline__ void store_a_half(const DevParams<T>& P, const cplx<T> (&acc)[NACC][NQ], int n0, int l,
-                                             int m, cplx<T>* __restrict__ Z) {
-    const int lm = l * l + l + m;
+__device__ __forceinline__ void store_a_half(const DevParams<T>& P, const cplx<T> (&acc)[NACC][NQ], int n0, int lh,
+                                             cplx<T>* __restrict__ Z) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         const int n = n0 + b;
         if (n < P.nr3a)
 #pragma unroll
             for (int q = 0; q < NM3X; ++q)
-                if (q < P.nm3) {
-                    Z[(n * P.lsa + lm) * P.nm3 + q] = acc[b][q];
-                    if (m > 0) {
-                        // m' of column q (a kernel argument: q is a compile-time index); its
-                        // partner is column q - 2 m'
-                        const int mp = P.mpq[q];
-                        const T sg = ((m + mp) & 1) ? (T)-1 : (T)1;
-                        Z[(n * P.lsa + lm - 2 * m) * P.nm3 + q - 2 * mp] = {sg * acc[b][q].re, -sg * acc[b][q].im};
-                    }
-                }
+                if (q < P.nm3) Z[(n * P.lha + lh) * P.nm3 + q] = acc[b][q];
     }
 }
 template <typename T, int NB2, int NR2X, int NACC, int NQ>
-__device__ __forceinline__ void store_a2_half(const DevParams<T>& P, const cplx<T> (&acc)[NACC][NQ], int n0, int m,
-                                              int lm, cplx<T>* __restrict__ Z) {
-    const T s = (m & 1) ? (T)-1 : (T)1;
+__device__ __forceinline__ void store_a2_half(const DevParams<T>& P, const cplx<T> (&acc)[NACC][NQ], int n0, int lh,
+                                              cplx<T>* __restrict__ Z) {
 #pragma unroll
     for (int b = 0; b < NB2; ++b) {
         const int n = n0 + b;
         if (n < P.nb_a)
 #pragma unroll
             for (int q = 0; q < NR2X; ++q)
-                if (q < P.nr2m) {
-                    cplx<T>* z = Z + P.oA2 + (n * P.nr2m + q) * P.lsm;
-                    z[lm] = acc[b][q];
-                    if (m > 0) z[lm - 2 * m] = {s * acc[b][q].re, -s * acc[b][q].im};
-                }
+                if (q < P.nr2m) Z[P.hA2 + (n * P.nr2m + q) * P.lhm + lh] = acc[b][q];
     }
 }
 
@@ -346,21 +306,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
         }
         for (int d = 0; d < P.nd; ++d) rho1_out[(size_t)atom * P.nd + d] = rho1[d];
     }
-    for (int t = tid; t < P.nr2m * P.lsm; t += nthr) {
-        const int np = t / P.lsm, lm = t % P.lsm;
+    for (int t = tid; t < P.nr2m * P.lhm; t += nthr) {
+        const int np = t / P.lhm, lh = t % P.lhm;
         int l = 0;
-        while ((l + 1) * (l + 1) <= lm) ++l;
-        const int m = lm - l * l - l;
-        const cplx<T> y = yfull(sYc, l, m);
+        while ((l + 1) * (l + 2) / 2 <= lh) ++l;
+        const cplx<T> y = sYc[lh];
         const T mv = sMc[l * P.nr2m + np];
-        Zout[P.oA0 + np * P.lsm + lm] = {mv * y.re, mv * y.im};
+        Zout[P.hA0 + t] = {mv * y.re, mv * y.im};
     }
 
     // Tasks cover m >= 0 only (P.lha and P.lhm entries per radial block): since R, M and g are
     // real and Y_{l,-m} = (-1)^m conj(Y_lm),
     //   A[n][l,-m][n',l',-m'] = (-1)^(m+m') conj(A[n][l,m][n',l',m'])  and
     //   A2[n][n'][l',-m'] = (-1)^m' conj(A2[n][n'][l',m']),
-    // which are written at the store from the m > 0 sums (m = 0 tasks hold all their columns).
+    // which are not stored.
     const int nblkA = (P.nr3a + NB - 1) / NB, nblkA2 = (P.nb_a + NB2 - 1) / NB2;
     const int nTA = P.lha * nblkA, nTA2 = P.lhm * nblkA2;
     // TASKSPLIT: when the A and A2 column tasks leave threads idle, each A task's neighbours
@@ -629,9 +588,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         }
         }
         if (isA && part == 0) {
-            store_a_half<T, NB, NM3X>(P, acc, n0, l, m, Zout);
+            store_a_half<T, NB, NM3X>(P, acc, n0, lh, Zout);
         } else if (isA2) {
-            store_a2_half<T, NB2, NR2X>(P, acc, n0, m, lm, Zout);
+            store_a2_half<T, NB2, NR2X>(P, acc, n0, lh, Zout);
         }
     }
     __syncthreads();
@@ -648,6 +607,13 @@ size_t density_lds_bytes(const DevParams<double>& Pd, int CH, size_t tsize) {
 }
 
 // ============================================================================ k_adjoint
+// entry of the full feature vector from its place in memory (ZLayout::half)
+template <typename T>
+__device__ __forceinline__ cplx<T> full_entry(const cplx<T>* __restrict__ Z, uint32_t e) {
+    const cplx<T> v = Z[e & 0xfff];
+    return {e >> 14 & 1 ? -v.re : v.re, e >> 15 & 1 ? -v.im : v.im};
+}
+
 template <typename T> __device__ __forceinline__ T rec_weight(uint4 r);
 template <> __device__ __forceinline__ double rec_weight<double>(uint4 r) {
     return __hiloint2double((int)r.w, (int)r.z);
@@ -751,7 +717,7 @@ __global__ void __launch_bounds__(kAdjointThreads) k_adjoint(DevParams<T> P, int
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int x = tid + u * kAdjointThreads;
-            v[u] = x < P.nz ? Zin[x] : cplx<T>{0, 0};
+            v[u] = x < P.nz ? full_entry(Zin, P.zmap[x]) : cplx<T>{0, 0};
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -990,10 +956,12 @@ __global__ void __launch_bounds__(kAdjointThreads) k_adjoint(DevParams<T> P, int
                 }
             }
         }
-        Wout[x] = ND2 ? cplx<T>{sc * w.re + sc2 * w2.re, sc * w.im + sc2 * w2.im} : cplx<T>{sc * w.re, sc * w.im};
+        if (!(f & (1u << 19))) continue;  // not stored
+        const int h = P.zmap[x];
+        Wout[h] = ND2 ? cplx<T>{sc * w.re + sc2 * w2.re, sc * w.im + sc2 * w2.im} : cplx<T>{sc * w.re, sc * w.im};
         if (wd) {
-            wd[x] = w;
-            wd[P.nz + x] = w2;
+            wd[h] = w;
+            wd[P.nz + h] = w2;
         }
     }
 }
@@ -1029,8 +997,9 @@ __global__ void __launch_bounds__(kAdjointThreads) k_adjoint_pair(DevParams<floa
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int x = tid + u * kAdjointThreads;
-            a[u] = x < P.nz ? Z0[x] : cplx<T>{0, 0};
-            b[u] = x < P.nz ? Z1[x] : cplx<T>{0, 0};
+            const uint32_t e = x < P.nz ? P.zmap[x] : 0u;
+            a[u] = x < P.nz ? full_entry(Z0, e) : cplx<T>{0, 0};
+            b[u] = x < P.nz ? full_entry(Z1, e) : cplx<T>{0, 0};
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -1229,606 +1198,10 @@ __global__ void __launch_bounds__(kAdjointThreads) k_adjoint_pair(DevParams<floa
                 w.w -= sg * b.w;
             }
         }
-        W0[x] = cplx<T>{sc0 * w.x, sc0 * w.y};
-        if (two) W1[x] = cplx<T>{sc1 * w.z, sc1 * w.w};
-    }
-}
-
-// ============================================================================ k_forces
-// Legendre rows streamed one l at a time (src/spherical.F90:55-155): row l of P_lm and
-// dP_lm/dz for m = 0..l from rows l-1 and l-2.  m is unrolled, l is a runtime loop, so the
-// rows stay in registers without indexing them dynamically.
-template <typename T, int L>
-struct LegRows {
-    T P[L + 1], dP[L + 1], P1[L + 1], dP1[L + 1], P2[L + 1], dP2[L + 1];
-    __device__ __forceinline__ void step(int l, T z) {
-#pragma unroll
-        for (int m = 0; m <= L; ++m) {
-            P2[m] = P1[m]; dP2[m] = dP1[m];
-            P1[m] = P[m]; dP1[m] = dP[m];
-        }
-        if (l == 0) {
-#pragma unroll
-            for (int m = 0; m <= L; ++m) { P[m] = (T)0; dP[m] = (T)0; }
-            P[0] = (T)1;
-            return;
-        }
-        if (l == 1) {
-            P[0] = (T)1.73205080756887719318 * z;
-            dP[0] = (T)1.73205080756887719318;
-            if (L >= 1) { P[L >= 1 ? 1 : 0] = -(T)1.22474487139158894067; dP[L >= 1 ? 1 : 0] = (T)0; }
-            return;
-        }
-        const int base = l * (l + 1) / 2;
-#pragma unroll
-        for (int m = 0; m <= L; ++m) {
-            if (m <= l - 2) {
-                const T a = LegC<T>::a(base + m), b = LegC<T>::b(base + m);
-                const T pm = a * fma(z, P1[m], b * P2[m]);
-                dP[m] = a * (P1[m] + fma(z, dP1[m], b * dP2[m]));
-                P[m] = pm;
-            } else if (m == l - 1) {
-                const T t = LegC<T>::d(l) * P1[m];
-                P[m] = t * z;
-                dP[m] = t;
-            } else if (m == l) {
-                P[m] = LegC<T>::c(l) * P1[m > 0 ? m - 1 : 0];
-                dP[m] = (T)0;
-            }
-        }
-    }
-};
-
-// one entry P_l^m, dP_l^m/dz of the rows above (l <= L): P_m^m = prod_{k<=m} c(k), then
-// P_{m+1}^m = d(m+1) z P_m^m and the three-term recurrence up to l.  The constants are loaded
-// first, to the compile-time bound (factors past m are 1 and steps past l are skipped), so
-// that one trip to memory serves them all instead of one per factor and step.
-template <typename T, int L>
-__device__ __forceinline__ void legendre_one(int l, int m, T z, T& p, T& dp) {
-    static_assert(L >= 1 && L < kLmaxC, "the constant tables cover l <= kLmaxC");
-    T cf[L], ca[L], cb[L];
-#pragma unroll
-    for (int k = 1; k <= L; ++k) cf[k - 1] = LegC<T>::c(k);  // every index is in the table
-    const T dm = LegC<T>::d(m + 1);
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-        const int ll = min(m + 2 + i, L), k = ll * (ll + 1) / 2 + m;
-        ca[i] = LegC<T>::a(k);
-        cb[i] = LegC<T>::b(k);
-    }
-    // every step is computed and kept or dropped by a select: with early exits the compiler
-    // moved each load into its branch, one trip to memory per step again
-    T pmm = (T)1;
-#pragma unroll
-    for (int k = 1; k <= L; ++k) pmm *= k <= m ? cf[k - 1] : (T)1;
-    T p2 = pmm, dp2 = (T)0;
-    T p1 = dm * pmm * z, dp1 = dm * pmm;
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-        const T a = ca[i], b = cb[i];
-        const T pn = a * fma(z, p1, b * p2);
-        const T dpn = a * (p1 + fma(z, dp1, b * dp2));
-        const bool on = m + 2 + i <= l;
-        p2 = on ? p1 : p2;
-        dp2 = on ? dp1 : dp2;
-        p1 = on ? pn : p1;
-        dp1 = on ? dpn : dp1;
-    }
-    p = l == m ? pmm : p1;
-    dp = l == m ? (T)0 : dp1;
-}
-
-template <typename T>
-__device__ __forceinline__ void conj_all(cplx<T>& Y, cplx<T> (&g)[3], int am) {
-    Y = cconj_sign(Y, am);
-    g[0] = cconj_sign(g[0], am);
-    g[1] = cconj_sign(g[1], am);
-    g[2] = cconj_sign(g[2], am);
-}
-
-// lane = pair.  LA/LM: compile-time bounds of l3a/l2m; NM3X: magnetic columns of A;
-// NBAX: atomic radial base bound; NRAX: nr3a bound; NR2X: nr2m bound.
-// W is folded onto representatives of conjugate pairs (A: m' > 0, or m' = 0 and m >= 0;
-// A2, A0: m' >= 0), so only those index pairs are visited.
-// Q1: the magnetic columns of A are (l', m') = (0,0), (1,-1), (1,0), (1,1) (l3m = 1, one radial
-// function), so the representative columns are known at compile time: 0, 2, 3 for m >= 0 and
-// 3 for m < 0, and no other W entry is read.
-template <typename T, int LA, int LM, int NM3X, int NBAX, int NRAX, int NR2X, bool Q1>
-__global__ void __launch_bounds__(64) k_forces(DevParams<T> P, const int* __restrict__ off,
-                                               const double* __restrict__ dlist,
-                                               const double* __restrict__ elist,
-                                               const double* __restrict__ dmomi,
-                                               const double* __restrict__ emomi,
-                                               const double* __restrict__ dmom,
-                                               const double* __restrict__ emom,
-                                               const cplx<T>* __restrict__ Win, bool scaled,
-                                               const double* __restrict__ dEin,
-                                               const double* __restrict__ edfin,
-                                               double* __restrict__ flist, double* __restrict__ tlist,
-                                               double* __restrict__ tlist0, int* err) {
-    const int atom = blockIdx.x, lane = threadIdx.x;
-    const int p0 = off[atom], nn = off[atom + 1] - p0;
-    // W of this atom staged in LDS with coalesced loads: every lane reads the same entries
-    // (broadcast), which as scalar loads would thrash the scalar cache with 20-40 KB per atom
-    extern __shared__ __align__(16) unsigned char smem_f[];
-    cplx<T>* sW = reinterpret_cast<cplx<T>*>(smem_f);
-    {
-        // forty loads in flight per lane: one trip to memory serves 2560 entries (all of W for
-        // lmax 6), where a load followed by its store had waited for every 64
-        const cplx<T>* __restrict__ Wg = Win + (size_t)atom * P.nz;
-        // W = dE/dRho dRho/dZ; the node adjoint leaves the first factor to this kernel
-        const T sc = scaled ? (T)1 : (T)dEin[atom];
-        constexpr int U = 40;
-        for (int i0 = 0; i0 < P.nz; i0 += 64 * U) {
-            cplx<T> v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = i0 + 64 * u + lane;
-                v[u] = i < P.nz ? Wg[i] : cplx<T>{0, 0};
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = i0 + 64 * u + lane;
-                if (i < P.nz) sW[i] = {sc * v[u].re, sc * v[u].im};
-            }
-        }
-        __syncthreads();
-    }
-    const cplx<T>* W = sW;
-    const int nfa = P.nr3a * (P.l3a + 1);
-    const double edf = edfin[atom];
-    // magnetic column q of A -> m' (for the representative test): column q takes part with
-    // m >= 0 (use0) when m' >= 0, with m < 0 (use1, the conjugated half) when m' > 0
-    bool use0[NM3X], use1[NM3X];
-#pragma unroll
-    for (int q = 0; q < NM3X; ++q) {
-        const int lq = q % P.lsm3;
-        int lp = 0;
-        while ((lp + 1) * (lp + 1) <= lq) ++lp;
-        const int mp = lq - lp * lp - lp;
-        use0[q] = q < P.nm3 && mp >= 0;
-        use1[q] = q < P.nm3 && mp > 0;
-    }
-    static_assert(!Q1 || NM3X == 4, "Q1 needs four magnetic columns");
-    auto used = [&](int q, int sg) -> bool {
-        if constexpr (Q1) return sg ? q == 3 : q != 1;
-        return sg ? use1[q] : use0[q];
-    };
-
-    for (int c0 = 0; c0 < nn; c0 += 64) {
-        const int j = c0 + lane;
-        const bool active = j < nn;
-        const int p = p0 + (active ? j : 0);
-        T Fx = 0, Fy = 0, Fz = 0, Tx = 0, Ty = 0, Tz = 0;
-        T wa = 0;
-        // the pair's inputs, all loads issued before the first is used
-        const double r_d = dlist[p], mu_d = dmom[p];
-        const double ex_d = elist[3 * p], ey_d = elist[3 * p + 1], ez_d = elist[3 * p + 2];
-        const double sx_d = emom[3 * p], sy_d = emom[3 * p + 1], sz_d = emom[3 * p + 2];
-        const T* rowa = active ? atomic_row(P, r_d, wa, err) : nullptr;
-        if (rowa) {
-            const T invr = (T)(1.0 / r_d);
-            const T ex = (T)ex_d, ey = (T)ey_d, ez = (T)ez_d;
-            const T sx = (T)sx_d, sy = (T)sy_d, sz = (T)sz_d;
-            T wm = 0;
-            bool unit = false;
-            const T* rowm = magnetic_row(P, mu_d, wm, unit, err);
-            const T rsa = (T)P.rs_a, rsm = (T)P.rs_m;
-            // the atomic loop's first spline coefficients (row l = 0); each later row is loaded
-            // one l ahead in the loop.  Q1 loads row 0 here, so that it comes in the same trip
-            // to memory as the M values below (the wide classes load it at the loop, where
-            // their registers allow)
-            T cq0[Q1 ? NRAX : 1][4];
-            if constexpr (Q1)
-#pragma unroll
-                for (int n = 0; n < NRAX; ++n) load_coef(n < P.nr3a ? rowa + 4 * (P.nb_a + n) : P.lut_a, cq0[n]);
-            // H_q = M_{l',n'}(mu_j) Y_{l'm'}(s_j), m' >= 0, for the magnetic columns of A
-            cplx<T> H[NM3X], U[NM3X];
-#pragma unroll
-            for (int q = 0; q < NM3X; ++q) {
-                H[q] = {0, 0};
-                U[q] = {0, 0};
-            }
-            {
-                // M_{l',n'}(mu_j) of the columns' (l', n'), entry n' (l3m + 1) + l' (at most nm3
-                // of them), with their coefficient loads issued together
-                T Mh[NM3X];
-                {
-                    const int nl = P.l3m + 1, nh = nl * P.nr3m;
-                    T c[NM3X][4];
-#pragma unroll
-                    for (int i = 0; i < NM3X; ++i)
-                        load_coef(rowm && i < nh ? rowm + 4 * (P.nb_m + (i % nl) * P.nr2m + i / nl) : P.lut_m, c[i]);
-#pragma unroll
-                    for (int i = 0; i < NM3X; ++i)
-                        Mh[i] = rowm ? fma(wm, fma(wm, fma(wm, c[i][3], c[i][2]), c[i][1]), c[i][0]) : unit ? (T)1 : (T)0;
-                }
-                cplx<T> ph = {1, 0};
-                LegRows<T, LM> Lr;
-                for (int lp = 0; lp <= P.l3m; ++lp) {
-                    Lr.step(lp, sz);
-                    ph = {1, 0};
-#pragma unroll
-                    for (int am = 0; am <= LM; ++am) {
-                        if (am > lp) break;
-                        const cplx<T> y = {Lr.P[am] * ph.re, Lr.P[am] * ph.im};
-                        for (int np = 0; np < P.nr3m; ++np) {
-                            T v = 0;
-                            const int ih = np * (P.l3m + 1) + lp;
-#pragma unroll
-                            for (int i = 0; i < NM3X; ++i)
-                                if (i == ih) v = Mh[i];
-                            const int q = np * P.lsm3 + lp * lp + lp + am;
-#pragma unroll
-                            for (int qq = 0; qq < NM3X; ++qq)
-                                if (qq == q) H[qq] = {v * y.re, v * y.im};
-                        }
-                        ph = cmul(ph, cplx<T>{sx, sy});
-                    }
-                }
-            }
-            // ---- atomic loop: F from A and U_q = sum W_A R Y (src/forces.F90:497-620, 836-957)
-            {
-                cplx<T> pha[LA + 1];
-                pha[0] = {1, 0};
-#pragma unroll
-                for (int m = 1; m <= LA; ++m) pha[m] = cmul(pha[m - 1], cplx<T>{ex, ey});
-                LegRows<T, LA> Lr;
-                // spline coefficients of row l are loaded one iteration ahead, so the gathers
-                // from the table overlap the arithmetic of the previous l
-                T cq[NRAX][4];
-#pragma unroll
-                for (int n = 0; n < NRAX; ++n) {
-                    if constexpr (Q1) {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) cq[n][k] = cq0[Q1 ? n : 0][k];
-                    } else {
-                        load_coef(n < P.nr3a ? rowa + 4 * (P.nb_a + n) : P.lut_a, cq[n]);
-                    }
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) cq[n][k] = n < P.nr3a ? cq[n][k] : (T)0;
-                }
-                for (int l = 0; l <= P.l3a; ++l) {
-                    Lr.step(l, ez);
-                    T R[NRAX], dR[NRAX];
-#pragma unroll
-                    for (int n = 0; n < NRAX; ++n) {
-                        R[n] = fma(wa, fma(wa, fma(wa, cq[n][3], cq[n][2]), cq[n][1]), cq[n][0]);
-                        dR[n] = fma(wa, fma(wa, (T)3 * cq[n][3], (T)2 * cq[n][2]), cq[n][1]) * rsa;
-                    }
-                    if (l < P.l3a) {
-                        const T* nrow = rowa + 4 * (P.nb_a + (l + 1) * P.nr3a);
-#pragma unroll
-                        for (int n = 0; n < NRAX; ++n) {
-                            load_coef(n < P.nr3a ? nrow + 4 * n : P.lut_a, cq[n]);
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) cq[n][k] = n < P.nr3a ? cq[n][k] : (T)0;
-                        }
-                    }
-#pragma unroll
-                    for (int am = 0; am <= LA; ++am) {
-                        if (am > l) break;
-                        cplx<T> Y0, g0[3];
-                        ylm_grad<T>(am, Lr.P[am], Lr.dP[am], pha[am], pha[am > 0 ? am - 1 : 0], ex, ey, ez, Y0, g0);
-#pragma unroll
-                        for (int sg = 0; sg < 2; ++sg) {
-                            if (sg == 1 && am == 0) break;
-                            cplx<T> Y = Y0, g[3] = {g0[0], g0[1], g0[2]};
-                            if (sg) conj_all(Y, g, am);
-                            const int lm = l * l + l + (sg ? -am : am);
-                            // V_n = sum_q W[n][lm][q] H_q.  The force needs
-                            // sum_n Re[V_n (R'_n Y e + R_n/r grad Y)], the torque
-                            // sum_n W[n][lm][q] R_n Y: both are summed over n first
-                            // (S1 = sum_n R'_n V_n, S2 = sum_n R_n V_n, Tq = sum_n R_n W[n][lm][q])
-                            // and meet Y and grad Y once per (l, m).  With the columns in
-                            // registers (NM3X <= 8) the sums over n run per column instead,
-                            // Tq and Dq = sum_n R'_n W[n][lm][q], and S1 = sum_q Dq H_q,
-                            // S2 = sum_q Tq H_q follow after the loop: four operations per
-                            // column and n in place of six, and none per n for S1, S2
-                            constexpr int NTQ = NM3X <= 8 ? NM3X : 1;
-                            cplx<T> S1 = {0, 0}, S2 = {0, 0}, Tq[NTQ], Dq[NTQ];
-#pragma unroll
-                            for (int q = 0; q < NTQ; ++q) Tq[q] = Dq[q] = {0, 0};
-                            if constexpr (Q1 && sizeof(T) == 4) {
-                                // FP32 rows are 32 bytes, 16-byte aligned: columns 2, 3 in one
-                                // ds_read_b128 and column 0 (m >= 0 only) in another.  Each row's
-                                // reads are issued kAhead rows before its sums, so that their
-                                // latency passes during the sums of the rows before it (read and
-                                // used at once, every row had waited for its own reads).  The
-                                // loop runs to the compile-time bound, as below.
-                                constexpr int kAhead = 2, kRing = kAhead + 1;
-                                float4 r23[kRing], r01[kRing];
-#pragma unroll
-                                for (int n = 0; n < NRAX + kAhead; ++n) {
-                                    if (n < NRAX) {
-                                        const int nw = n >= P.nr3a ? 0 : n;
-                                        const float4* Wn = (const float4*)(W + (nw * P.lsa + lm) * P.nm3);
-                                        r23[n % kRing] = Wn[1];
-                                        if (sg == 0) r01[n % kRing] = Wn[0];
-                                    }
-                                    const int k = n - kAhead;  // the row summed now
-                                    if (k < 0) continue;
-                                    cplx<T> wv[NM3X];
-                                    wv[2] = {r23[k % kRing].x, r23[k % kRing].y};
-                                    wv[3] = {r23[k % kRing].z, r23[k % kRing].w};
-                                    if (sg == 0) wv[0] = {r01[k % kRing].x, r01[k % kRing].y};
-#pragma unroll
-                                    for (int q = 0; q < NM3X; ++q) {
-                                        if (used(q, sg)) {
-                                            Tq[q].re = fma(R[k], wv[q].re, Tq[q].re);
-                                            Tq[q].im = fma(R[k], wv[q].im, Tq[q].im);
-                                            Dq[q].re = fma(dR[k], wv[q].re, Dq[q].re);
-                                            Dq[q].im = fma(dR[k], wv[q].im, Dq[q].im);
-                                        }
-                                    }
-                                }
-                            } else
-#pragma unroll
-                            for (int n = 0; n < NRAX; ++n) {
-                                // Q1 runs to the compile-time bound (past nr3a, R = R' = 0 and
-                                // row 0 is read), so that each (l, m) body is one straight block
-                                // the scheduler can interleave (lmax-6 FP32 0.963 -> 0.919 ms);
-                                // the general instance keeps the exit, as without it it spills
-                                if constexpr (!Q1) {
-                                    if (n >= P.nr3a) break;
-                                }
-                                const int nw = Q1 && n >= P.nr3a ? 0 : n;
-                                const cplx<T>* Wn = W + (nw * P.lsa + lm) * P.nm3;
-                                // the row's reads are issued together, outside the uniform
-                                // branches, so their LDS latency overlaps (a read inside each
-                                // branch waited for its own result)
-                                // (wide classes, 27 columns, read inside the branches: the
-                                // hoisted values would not fit in registers)
-                                constexpr bool kHoist = NM3X <= 8;
-                                cplx<T> wv[kHoist ? NM3X : 1];
-                                if constexpr (kHoist) {
-#pragma unroll
-                                    for (int q = 0; q < NM3X; ++q)
-                                        if (!Q1 || used(q, sg)) wv[q] = Wn[q < P.nm3 ? q : 0];
-                                }
-                                if constexpr (kHoist) {
-#pragma unroll
-                                    for (int q = 0; q < NM3X; ++q) {
-                                        if (used(q, sg)) {
-                                            const cplx<T> wq = wv[kHoist ? q : 0];
-                                            const int qt = kHoist ? q : 0;
-                                            Tq[qt].re = fma(R[n], wq.re, Tq[qt].re);
-                                            Tq[qt].im = fma(R[n], wq.im, Tq[qt].im);
-                                            Dq[qt].re = fma(dR[n], wq.re, Dq[qt].re);
-                                            Dq[qt].im = fma(dR[n], wq.im, Dq[qt].im);
-                                        }
-                                    }
-                                } else {
-                                    // wide classes: per-column sums would not fit
-                                    cplx<T> V = {0, 0};
-                                    const cplx<T> ry = {R[n] * Y.re, R[n] * Y.im};
-#pragma unroll
-                                    for (int q = 0; q < NM3X; ++q) {
-                                        if (used(q, sg)) {
-                                            const cplx<T> wq = Wn[q];
-                                            cfma(V, wq, H[q]);
-                                            cfma(U[q], wq, ry);
-                                        }
-                                    }
-                                    S1.re = fma(dR[n], V.re, S1.re);
-                                    S1.im = fma(dR[n], V.im, S1.im);
-                                    S2.re = fma(R[n], V.re, S2.re);
-                                    S2.im = fma(R[n], V.im, S2.im);
-                                }
-                            }
-                            if constexpr (NM3X <= 8) {
-#pragma unroll
-                                for (int q = 0; q < NTQ; ++q)
-                                    if (used(q, sg)) {
-                                        cfma(S1, Dq[q], H[q]);
-                                        cfma(S2, Tq[q], H[q]);
-                                        cfma(U[q], Tq[q], Y);
-                                    }
-                            }
-                            // Re[S1 Y] e + Re[S2 grad Y] / r
-                            const T a = re_mul(S1, Y);
-                            Fx += fma(a, ex, invr * re_mul(S2, g[0]));
-                            Fy += fma(a, ey, invr * re_mul(S2, g[1]));
-                            Fz += fma(a, ez, invr * re_mul(S2, g[2]));
-                        }
-                    }
-                }
-            }
-            // ---- magnetic loop over m' >= 0: A2 part of F and T, A part of T
-            // (src/forces.F90:460-491, 793-957)
-            {
-                const T invmu = (T)(1.0 / mu_d);
-                T ga[NBAX], dga[NBAX];
-                T cc[4];  // the core term's coefficients, loaded with the g_n (used after this loop)
-                {
-                    T c[NBAX][4];  // one 16-byte load per function, issued together
-#pragma unroll
-                    for (int n = 0; n < NBAX; ++n) load_coef(n < P.nb_a ? rowa + 4 * n : P.lut_a, c[n]);
-                    load_coef(rowa + 4 * (P.nb_a + nfa), cc);
-#pragma unroll
-                    for (int n = 0; n < NBAX; ++n) {
-                        ga[n] = n < P.nb_a ? fma(wa, fma(wa, fma(wa, c[n][3], c[n][2]), c[n][1]), c[n][0]) : (T)0;
-                        dga[n] = n < P.nb_a ? fma(wa, fma(wa, (T)3 * c[n][3], (T)2 * c[n][2]), c[n][1]) * rsa : (T)0;
-                    }
-                }
-                T sf = 0;  // sum_n g'_n Re(W2 H2)
-                cplx<T> phm[LM + 1];
-                phm[0] = {1, 0};
-#pragma unroll
-                for (int m = 1; m <= LM; ++m) phm[m] = cmul(phm[m - 1], cplx<T>{sx, sy});
-                LegRows<T, LM> Lr;
-                // the coefficients of row l' are loaded one iteration ahead, as in the atomic loop
-                T cm[NR2X][4];
-#pragma unroll
-                for (int np = 0; np < NR2X; ++np)
-                    load_coef(rowm && np < P.nr2m ? rowm + 4 * (P.nb_m + np) : P.lut_m, cm[np]);
-                for (int lp = 0; lp <= P.l2m; ++lp) {
-                    Lr.step(lp, sz);
-                    T Mv[NR2X], dMv[NR2X];
-#pragma unroll
-                    for (int np = 0; np < NR2X; ++np) {
-                        const bool f = rowm && np < P.nr2m;
-                        Mv[np] = f ? fma(wm, fma(wm, fma(wm, cm[np][3], cm[np][2]), cm[np][1]), cm[np][0]) : unit ? (T)1 : (T)0;
-                        dMv[np] = f ? fma(wm, fma(wm, (T)3 * cm[np][3], (T)2 * cm[np][2]), cm[np][1]) * rsm : (T)0;
-                    }
-                    if (lp < P.l2m) {
-#pragma unroll
-                        for (int np = 0; np < NR2X; ++np)
-                            load_coef(rowm && np < P.nr2m ? rowm + 4 * (P.nb_m + (lp + 1) * P.nr2m + np) : P.lut_m, cm[np]);
-                    }
-#pragma unroll
-                    for (int am = 0; am <= LM; ++am) {
-                        if (am > lp) break;
-                        cplx<T> Y, g[3];
-                        ylm_grad<T>(am, Lr.P[am], Lr.dP[am], phm[am], phm[am > 0 ? am - 1 : 0], sx, sy, sz, Y, g);
-                        const int lmp = lp * lp + lp + am;
-                        // Q1 in FP32: the W2 entries of every n' of this (l', m') are read
-                        // before the first sum, so that one LDS round trip serves all n' (read
-                        // per n', each n' had waited for its own reads)
-                        constexpr bool kW2B = Q1 && sizeof(T) == 4;
-                        cplx<T> w2b[kW2B ? NR2X : 1][kW2B ? NBAX : 1];
-                        if constexpr (kW2B) {
-#pragma unroll
-                            for (int np = 0; np < NR2X; ++np) {
-                                const cplx<T>* W2r = W + P.oA2 + (np < P.nr2m ? np : 0) * P.lsm + lmp;
-#pragma unroll
-                                for (int n = 0; n < NBAX; ++n)
-                                    w2b[np][n] = W2r[(size_t)(n < P.nb_a ? n : 0) * P.nr2m * P.lsm];
-                            }
-                        }
-#pragma unroll
-                        for (int np = 0; np < NR2X; ++np) {
-                            if (np >= P.nr2m) break;
-                            const cplx<T> H2 = {Mv[np] * Y.re, Mv[np] * Y.im};
-                            // U2 = sum_n g_n W2[n], D2 = sum_n g'_n W2[n]; the force's
-                            // sum_n g'_n Re(W2[n] H2) is Re(D2 H2)
-                            cplx<T> U2 = {0, 0}, D2 = {0, 0};
-                            const cplx<T>* W2 = W + P.oA2 + np * P.lsm + lmp;
-#pragma unroll
-                            for (int n = 0; n < NBAX; ++n) {
-                                // no early exit: entries n >= nb_a have ga = dga = 0, and a
-                                // loop bounded at run time was left rolled, its register
-                                // arrays indexed indirectly (FP32 forces 1.46 -> 1.30 ms)
-                                const cplx<T> wv = kW2B ? w2b[kW2B ? np : 0][kW2B ? n : 0]
-                                                        : W2[(size_t)(n < P.nb_a ? n : 0) * P.nr2m * P.lsm];
-                                D2.re = fma(wv.re, dga[n], D2.re);
-                                D2.im = fma(wv.im, dga[n], D2.im);
-                                U2.re = fma(wv.re, ga[n], U2.re);
-                                U2.im = fma(wv.im, ga[n], U2.im);
-                            }
-                            sf += re_mul(D2, H2);
-                            if (lp <= P.l3m && np < P.nr3m) {
-                                const int q = np * P.lsm3 + lmp;
-#pragma unroll
-                                for (int qq = 0; qq < NM3X; ++qq)
-                                    if (qq == q) {
-                                        U2.re += U[qq].re;
-                                        U2.im += U[qq].im;
-                                    }
-                            }
-                            // d(M Y)/dm = M' s Y + M/mu grad Y
-                            const T a = dMv[np] * re_mul(U2, Y), b = Mv[np] * invmu;
-                            Tx += fma(a, sx, b * re_mul(U2, g[0]));
-                            Ty += fma(a, sy, b * re_mul(U2, g[1]));
-                            Tz += fma(a, sz, b * re_mul(U2, g[2]));
-                        }
-                    }
-                }
-                // F from A2 (g'_n e) and the core term (src/forces.F90:464-494)
-                const T dcr = fma(wa, fma(wa, (T)3 * cc[3], (T)2 * cc[2]), cc[1]) * rsa;
-                const T s = sf + (T)edf * dcr;
-                Fx = fma(s, ex, Fx);
-                Fy = fma(s, ey, Fy);
-                Fz = fma(s, ez, Fz);
-            }
-        }
-        // store transposed across the wave: lane L writes element L + 64 r of the 64 pairs'
-        // 192 consecutive doubles of flist (and of tlist), so that every store instruction
-        // covers whole lines, also when the outputs live in host memory and the stores cross
-        // PCIe.  Element i belongs to pair i / 3, component i % 3.
-        const int cnt = 3 * min(64, nn - c0);
-        double* __restrict__ fo = flist + 3 * (size_t)(p0 + c0);
-        double* __restrict__ to = tlist + 3 * (size_t)(p0 + c0);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const int i = lane + 64 * r, src = i / 3, comp = i - 3 * src;
-            const T f0 = __shfl(Fx, src), f1 = __shfl(Fy, src), f2 = __shfl(Fz, src);
-            const T t0 = __shfl(Tx, src), t1 = __shfl(Ty, src), t2 = __shfl(Tz, src);
-            if (i < cnt) {
-                fo[i] = (double)(comp == 0 ? f0 : comp == 1 ? f1 : f2);
-                to[i] = (double)(comp == 0 ? t0 : comp == 1 ? t1 : t2);
-            }
-        }
-    }
-    // ---- self term T0 = dE_i/dm_i over m' >= 0 (src/forces.F90:712-749), spread over the
-    // wave: lane k takes B1 function k (nb_m <= 32) and entry k of the (l', m' >= 0) half set
-    // (at most 28 entries for l2m <= LM <= 6; each lane with its own Legendre recurrence), and
-    // the wave sums the three components in a fixed butterfly order.  The global loads come in
-    // two batches, the atom's moment, direction and dE first, then every coefficient a lane
-    // needs (its B1 function and c1, and the M rows of its (l', m')): loaded where each was
-    // used, they had taken seven trips to memory at the end of every workgroup.
-    static_assert((LM + 1) * (LM + 2) / 2 <= 64, "one half-set entry per lane");
-    {
-        const double mu_d = dmomi[atom];
-        const double sxd = emomi[3 * atom], syd = emomi[3 * atom + 1], szd = emomi[3 * atom + 2];
-        const double dE0 = dEin[(size_t)atom * P.nd], dE1 = P.nd > 1 ? dEin[(size_t)atom * P.nd + 1] : 0.0;
-        const bool b1 = lane < P.nb_m, hs = lane < P.lhm;
-        const double c10 = P.c1[0][b1 ? lane : 0], c11 = P.c1[1][b1 ? lane : 0];
-        const T invmu = (T)(1.0 / mu_d);
-        const T sx = (T)sxd, sy = (T)syd, sz = (T)szd;
-        T wm = 0;
-        bool unit = false;
-        const T* rowm = magnetic_row(P, mu_d, wm, unit, err);
-        const T rsm = (T)P.rs_m;
-        int lp = 0;
-        while ((lp + 1) * (lp + 2) / 2 <= lane) ++lp;
-        const int am = lane - lp * (lp + 1) / 2;
-        T cb[4], cm[NR2X][4];
-        load_coef(rowm && b1 ? rowm + 4 * lane : P.lut_m, cb);
-#pragma unroll
-        for (int np = 0; np < NR2X; ++np)
-            load_coef(rowm && hs && np < P.nr2m ? rowm + 4 * (P.nb_m + lp * P.nr2m + np) : P.lut_m, cm[np]);
-        T Tx = 0, Ty = 0, Tz = 0;
-        if (b1) {  // B1: dE/dg^m_n = dE/drho c1_n
-            T v = unit ? (T)1 : (T)0, dv = 0;
-            if (rowm) horner(cb, wm, rsm, v, dv);
-            const T s1 = (T)(dE0 * c10 + dE1 * c11) * dv;
-            Tx = fma(s1, sx, Tx);
-            Ty = fma(s1, sy, Ty);
-            Tz = fma(s1, sz, Tz);
-        }
-        if (hs) {
-            T pl, dpl;
-            legendre_one<T, LM>(lp, am, sz, pl, dpl);
-            cplx<T> ph = {1, 0}, ph1 = {1, 0};
-            for (int k = 0; k < am; ++k) {
-                ph1 = ph;
-                ph = cmul(ph, cplx<T>{sx, sy});
-            }
-            cplx<T> Y, g[3];
-            ylm_grad<T>(am, pl, dpl, ph, ph1, sx, sy, sz, Y, g);
-#pragma unroll
-            for (int np = 0; np < NR2X; ++np) {
-                if (np >= P.nr2m) break;
-                T v = unit ? (T)1 : (T)0, dv = 0;
-                if (rowm) horner(cm[np], wm, rsm, v, dv);
-                const cplx<T> w0 = W[P.oA0 + np * P.lsm + lp * lp + lp + am];
-                const T a = dv * re_mul(w0, Y), b = v * invmu;
-                Tx += fma(a, sx, b * re_mul(w0, g[0]));
-                Ty += fma(a, sy, b * re_mul(w0, g[1]));
-                Tz += fma(a, sz, b * re_mul(w0, g[2]));
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            Tx += __shfl_xor(Tx, o, 64);
-            Ty += __shfl_xor(Ty, o, 64);
-            Tz += __shfl_xor(Tz, o, 64);
-        }
-        if (lane == 0) {
-            tlist0[3 * (size_t)atom] = (double)Tx;
-            tlist0[3 * (size_t)atom + 1] = (double)Ty;
-            tlist0[3 * (size_t)atom + 2] = (double)Tz;
-        }
+        if (!(f & (1u << 19))) continue;  // not stored
+        const int h = P.zmap[x];
+        W0[h] = cplx<T>{sc0 * w.x, sc0 * w.y};
+        if (two) W1[h] = cplx<T>{sc1 * w.z, sc1 * w.w};
     }
 }
 
@@ -1897,8 +1270,7 @@ __global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, bool scal
     for (int d = 0; d < ND; ++d) {
         const cplx<double>* w = W + ((size_t)atom * ND + d) * P.nz;
         double s = 0.0;
-        for (int x = threadIdx.x; x < P.nz; x += blockDim.x)
-            if (P.fold[x] >> 17 & 1) s += re_mul(w[x], zd[x]);
+        for (int x = threadIdx.x; x < P.nzh; x += blockDim.x) s += re_mul(w[x], zd[x]);
         tot[d] = block_sum<double>(s, red);
         __syncthreads();
     }
@@ -1924,7 +1296,8 @@ __global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, bool scal
 // [ND][nterms] complex
 constexpr int kFitMpt = 8;
 template <int ND>
-__global__ void __launch_bounds__(256) k_fit_accum(int nterms, int nz, int ny, const int2* __restrict__ ypair,
+__global__ void __launch_bounds__(256) k_fit_accum(int nterms, int nz, const unsigned short* __restrict__ zmap, int ny,
+                                                  const int2* __restrict__ ypair,
                                                   const ushort4* __restrict__ idx,
                                                   const cplx<double>* __restrict__ Z,
                                                   const cplx<double>* __restrict__ Zdot,
@@ -1948,8 +1321,8 @@ __global__ void __launch_bounds__(256) k_fit_accum(int nterms, int nz, int ny, c
     for (int a = a0; a < a1; ++a) {
         __syncthreads();
         for (int x = threadIdx.x; x < nz; x += blockDim.x) {
-            sZ[x] = Z[(size_t)a * nz + x];
-            sD[x] = Zdot[(size_t)a * nz + x];
+            sZ[x] = full_entry(Z + (size_t)a * nz, zmap[x]);
+            sD[x] = full_entry(Zdot + (size_t)a * nz, zmap[x]);
         }
         if (threadIdx.x == 0) {
             sZ[nz] = {1, 0};
@@ -2109,11 +1482,11 @@ hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int na
     }
     dim3 grid((unsigned)((nterms + 256 * kFitMpt - 1) / (256 * kFitMpt)), (unsigned)((natom + chunk - 1) / chunk));
     if (nd == 2)
-        hipLaunchKernelGGL(k_fit_accum<2>, grid, dim3(256), lds, s, nterms, P.nz, P.ny, P.ypair, (const ushort4*)F.idx,
+        hipLaunchKernelGGL(k_fit_accum<2>, grid, dim3(256), lds, s, nterms, P.nz, P.zmap, P.ny, P.ypair, (const ushort4*)F.idx,
                            (const cplx<double>*)B.Z, (const cplx<double>*)F.Zdot, F.alpha, F.beta, natom, chunk,
                            F.M);
     else
-        hipLaunchKernelGGL(k_fit_accum<1>, grid, dim3(256), lds, s, nterms, P.nz, P.ny, P.ypair, (const ushort4*)F.idx,
+        hipLaunchKernelGGL(k_fit_accum<1>, grid, dim3(256), lds, s, nterms, P.nz, P.zmap, P.ny, P.ypair, (const ushort4*)F.idx,
                            (const cplx<double>*)B.Z, (const cplx<double>*)F.Zdot, F.alpha, F.beta, natom, chunk,
                            F.M);
     hipLaunchKernelGGL(k_fit_b1, dim3((natom + 255) / 256), dim3(256), 0, s, P, natom, nd, dmomi, F.alpha, grad,
@@ -2172,40 +1545,20 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
     const void* k1 = nullptr;
     if constexpr (ACC) k1 = (const void*)k_density<T, L, CH, NB, NM3X, NB2, NR2X, SPLIT, TASKSPLIT>;
     const bool nd2 = P.nd == 2;
-    // the Q1 instantiation exists only for the four-column class.  Q1 visits every radial index
-    // up to its compile-time bound, so the bounds 4 (for nr3a <= 4), 5, 6, 7 and NRAX each have
-    // an instance; without Q1 all five name the general kernel
-    constexpr bool kQ1 = NM3X == 4;
-    const bool q1 = kQ1 && P.nm3 == 4 && P.lsm3 == 4;
-    auto k3g = k_forces<T, L, L, NM3X, NBAX, NRAX, NR2X, false>;
-    constexpr int kB4 = kQ1 && NRAX > 4 ? 4 : NRAX, kB5 = kQ1 && NRAX > 5 ? 5 : NRAX,
-                  kB6 = kQ1 && NRAX > 6 ? 6 : NRAX, kB7 = kQ1 && NRAX > 7 ? 7 : NRAX;
-    constexpr int kQB[5] = {kB4, kB5, kB6, kB7, NRAX};
-    const decltype(k3g) k3qs[5] = {
-        k_forces<T, L, L, NM3X, NBAX, kB4, NR2X, kQ1>, k_forces<T, L, L, NM3X, NBAX, kB5, NR2X, kQ1>,
-        k_forces<T, L, L, NM3X, NBAX, kB6, NR2X, kQ1>, k_forces<T, L, L, NM3X, NBAX, kB7, NR2X, kQ1>,
-        k_forces<T, L, L, NM3X, NBAX, NRAX, NR2X, kQ1>};
-    int qi = 0;  // the smallest bound that covers nr3a
-    while (qi < 4 && kQB[qi] < P.nr3a) ++qi;
-    auto k3 = q1 ? k3qs[qi] : k3g;
     hipError_t e = hipSuccess;
     // the dynamic-LDS limit is raised once per kernel instantiation (to the workgroup
     // maximum), so that evaluations can be captured into graphs without further API calls.
-    // limit[]: 0 density, 1 adjoint, 2 adjoint with two densities, 3 two-atom adjoint,
-    // 4 general forces, 5 + i the Q1 forces of bound kQB[i]
+    // limit[]: 0 density, 1 adjoint, 2 adjoint with two densities, 3 two-atom adjoint
     static bool attributes_set = false;
-    static size_t limit[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    static size_t limit[4] = {0, 0, 0, 0};
     if (!attributes_set) {
         int dev = 0, maxsh = 0;
         if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
         if ((e = hipDeviceGetAttribute(&maxsh, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) != hipSuccess)
             return e;
-        const void* ks[10] = {k1, (const void*)k_adjoint<T, false, ACC>,
-                              (const void*)k_adjoint<T, true, ACC>, nullptr, (const void*)k3g,
-                              (const void*)k3qs[0], (const void*)k3qs[1], (const void*)k3qs[2],
-                              (const void*)k3qs[3], (const void*)k3qs[4]};
+        const void* ks[4] = {k1, (const void*)k_adjoint<T, false, ACC>, (const void*)k_adjoint<T, true, ACC>, nullptr};
         if constexpr (sizeof(T) == 4) ks[3] = (const void*)k_adjoint_pair<ACC>;
-        for (int i = 0; i < 10; ++i) {
+        for (int i = 0; i < 4; ++i) {
             if (!ks[i]) continue;
             hipFuncAttributes fa;
             if ((e = hipFuncGetAttributes(&fa, ks[i])) != hipSuccess) return e;
@@ -2223,12 +1576,11 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
     const size_t lds2p = 2 * (size_t)P.nzx * 16 + (2 * (kAdjointThreads / 64) + 2) * sizeof(double);
     const size_t lds2 =
         (nd2 ? 3 : 2) * (size_t)P.nzx * sizeof(cplx<T>) + (2 * (kAdjointThreads / 64) + 2) * sizeof(double);
-    const size_t lds3 = (size_t)P.nz * sizeof(cplx<T>);
     // the node plan where the potential has one; the accumulation recipe keeps the record walk, whose
     // FP64 sums over monomial products it is defined by
     const bool nodes = N.nw > 0 && !ACC;
     if (!nodes && pair && lds2p > limit[3]) return hipErrorInvalidValue;
-    if ((ACC && lds1 > limit[0]) || (!nodes && lds2 > limit[nd2 ? 2 : 1]) || lds3 > limit[q1 ? 5 + qi : 4])
+    if ((ACC && lds1 > limit[0]) || (!nodes && lds2 > limit[nd2 ? 2 : 1]))
         return hipErrorInvalidValue;
     if (ev) (void)hipEventRecord(ev[0], s);
     if constexpr (ACC) {
@@ -2257,8 +1609,9 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
                            B.dE, B.edf, B.rho);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[2], s);
-    hipLaunchKernelGGL(k3, dim3(natom), dim3(64), lds3, s, P, off, dlist, elist, dmomi, emomi, dmom, emom,
-                       (const cplx<T>*)B.W, !nodes, B.dE, B.edf, flist, tlist, tlist0, B.err);
+    if ((e = run_forces<T>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, B, !nodes, flist, tlist, tlist0, s)) !=
+        hipSuccess)
+        return e;
     if (ev) (void)hipEventRecord(ev[3], s);
     return hipGetLastError();
 }

@@ -25,16 +25,30 @@ struct DevParams {
     const T* lut_m = nullptr;  // magnetic spline rows [nlut][stride_m]
     const T* lut_g = nullptr;  // rows of the base functions g_1..g_nb and the core term alone [nlut][stride_g]
     const T* cperm = nullptr;  // radial coefficients C_{nlk} as A operands, [l3a + 1][4][64] (density.hip)
-    // columns of the density's products, 16 a tile, of A (Y entry | q << 8 | l << 16 | m << 20 | m' + 8 << 24),
-    // then of A2 (Y' entry | M entry << 8 | l << 16 | m << 20 | n' << 24), then the A0 entries (Y' entry |
-    // M entry << 8 | real part negative << 16 | imaginary part negative << 17)
+    // columns of the density's products, 16 a tile: of A (Y entry | q << 8 | l << 16), then of A2 (Y' entry | M
+    // entry << 8)
     const uint32_t* cols = nullptr;
+    // forces (forces.hip): walks through the harmonics, four lane groups a step, of the bonds (sta steps; all
+    // groups the same if qsplit, each with columns q of its own) and of the moments (stm, of which the first
+    // sth meet l' <= l3m): a, b, c, l | m << 8 | first of its order << 16 | harmonic << 17 |
+    // l nr2m << 18, firsta and firstm the steps that are some group's first of an order; rows of the tiles of
+    // V: column of A | l << 16 | it and y are a pair +m', -m' << 25 | its sine << 26 | its odd m' << 27, column of
+    // A2 | 1 << 24, or ~0; radial coefficients [l3a + 1][8][16]
+    const double* steps = nullptr;
+    const uint2* vcol = nullptr;
+    const T* crow = nullptr;
+    int sta = 0, stm = 0, sth = 0;
+    uint32_t firsta = 0, firstm = 0;
+    bool qsplit = false;
+    // places of Z and W in memory (ZLayout::half): offsets of A2 and A0, entries, and the place of every
+    // full index
+    int hA2 = 0, hA0 = 0, nzh = 0;
+    const unsigned short* zmap = nullptr;
     int stride_a = 0, stride_m = 0, stride_g = 0, nlut = 0;
     double rs_a = 0, rs_m = 0;  // nlut / cutoff (index arithmetic stays FP64)
     int nb_a = 0, nb_m = 0, nr2m = 0, l2m = 0, nr3a = 0, nr3m = 0, l3a = 0, l3m = 0;
     int lsa = 0, lsm = 0, lsm3 = 0, nm3 = 0, oA2 = 0, oA0 = 0, nz = 0;
     int lha = 0, lhm = 0;  // (l+1)(l+2)/2 for l3a, l2m
-    signed char mpq[32] = {0};  // m' of the magnetic column q of A (q < nm3 <= 32)
     int sa = 0;                 // k_density: neighbour split of the A tasks (0 = automatic)
     // gradient contributions, one 16-byte record each: x = a | b << 16, y = c as byte offsets
     // of the factors in the adjoint's LDS copy of Z (index * sizeof(cplx<T>)), (z, w) = weight
@@ -81,8 +95,8 @@ enum : int {
 };
 
 struct Buffers {
-    void* Z = nullptr;       // [natom][nz] complex
-    void* W = nullptr;       // [natom][nz] complex
+    void* Z = nullptr;       // [natom][nz] complex, in the places of ZLayout::half
+    void* W = nullptr;       // [natom][nz] complex, likewise
     double* ehc = nullptr;   // core sum
     double* rho1 = nullptr;  // B1 part of rho, [natom][nd]
     double* dE = nullptr;    // fcut * F'(rho), [natom][nd]
@@ -186,6 +200,11 @@ hipError_t run_density(const DevParams<T>& P, int natom, const int* off, const d
 hipError_t run_density_jvp(const DevParams<double>& P, int natom, const int* off, const int* nlist, const double* du,
                            const double* dlist, const double* elist, const double* dmom, const double* emom, void* Zdot,
                            double* ehc_dot, int* err, hipStream_t s);
+// pair forces, pair torques and self torques from B.W; scaled: W holds dE/dZ, else dRho/dZ (forces.hip)
+template <typename T>
+hipError_t run_forces(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
+                      const double* dmomi, const double* emomi, const double* dmom, const double* emom, const Buffers& B,
+                      bool scaled, double* flist, double* tlist, double* tlist0, hipStream_t s);
 // row of a 16x16x4 product's result in register r of lane group g, by the size of a value (matrix.hpp)
 inline int matrix_row(size_t bytes, int g, int r) { return bytes == 4 ? 4 * g + r : g + 4 * r; }
 

@@ -72,6 +72,13 @@ struct ZLayout {
     int a2(int n, int np, int lp, int mp) const { return oA2 + (n * nr2m_ + np) * lsm + lp * lp + lp + mp; }
     int a0(int np, int lp, int mp) const { return oA0 + np * lsm + lp * lp + lp + mp; }
     int nr2m_ = 0;
+    // Z and W in device memory hold the entries of m >= 0 (A) and m' >= 0 (A2, A0) only, the others being
+    // conjugates: [A: n][l, m >= 0][q] at 0, [A2: n][n'][l', m' >= 0] at hA2, [A0: n'][l', m' >= 0] at hA0, nh
+    // in all.  half[x] of a full index: its place | real part negative << 14 | imaginary part negative
+    // << 15 (an entry with `stored` has neither flag).
+    int hA2 = 0, hA0 = 0, nh = 0;
+    std::vector<uint16_t> half;
+    std::vector<char> stored;
 };
 
 // rho = Re sum_t w_t prod_{s<4} Z[i_ts] with Z[nz] == 1 padding lower-degree terms.
@@ -105,7 +112,8 @@ struct TermList {
     std::vector<int32_t> comb, comb2;
     int nslot = 0;
     // folding of the gradient onto representatives of conjugate pairs (x, xbar):
-    // partner | sign << 16 (1 = odd m+m') | representative << 17 | self-conjugate << 18
+    // partner | sign << 16 (1 = odd m+m') | representative << 17 | self-conjugate << 18 | stored << 19
+    // (ZLayout::half); representatives are the stored entries, of A's m = 0 those of m' >= 0 only
     std::vector<uint32_t> fold;
     // Products of two A entries for monomials of five or six factors (body orders 5 and 6):
     // entry i is Y_i = Z[a] Z[b] at index nz + 1 + i of the extended vector Z' = [Z | 1 | Y],
@@ -140,7 +148,7 @@ struct TermList {
 // 64 lanes after one another.
 constexpr size_t kNodeLdsTail = 384;          // sums and scalars behind the slots
 constexpr size_t kNodeLdsMost = 160 * 1024;
-constexpr int kNodeSingle = 0x4000;           // NodeSide::row: a single entry, its Z index below
+constexpr int kNodeSingle = 0x4000;           // NodePlan::row: a single entry, its place in the row of W below
 constexpr uint32_t kNodeOwn = 1u << 24, kNodeConj = 1u << 25, kNodeMinus = 1u << 26, kNodeNone = 1u << 31;
 constexpr int kNodeQuantum = 4, kNodeQuantumG = 4;  // a task's steps are a multiple of these (product, gradient)
 constexpr int kNodeAhead = 16;                // steps that the kernel reads ahead
@@ -149,20 +157,20 @@ struct NodePlan {
     bool ok = false;
     int nw = 8;                      // waves of a workgroup
     int slot_one = 0, slot_zero = 0, first_node = 0, np = 0, nq = 0, nslots = 0;
-    std::vector<uint16_t> core_z;    // Z index of core slot i
+    std::vector<uint16_t> core_z;    // Z entry of core slot i (ZLayout::half)
     std::vector<uint32_t> pair;      // nodes: slots of the two factors
     // [waves][64][4]: headers of a wave's tasks (steps, even; log2 of the lanes per block; first row), p
     // tasks, then q tasks, then gradient tasks; entry 62: their numbers, entry 63: first steps of the
     // wave's two record streams, which run through its tasks in order
     std::vector<int32_t> head;
     // G_p = sum w X_q, G_q (and single entries) = sum w X_p
-    std::vector<uint16_t> row;       // 4 per block: LDS slots of its rows, kNodeSingle | Z index, or 0xffff: none
+    std::vector<uint16_t> row;       // 4 per block: LDS slots of its rows, kNodeSingle | place in W, or 0xffff: none
     std::vector<uint16_t> col;       // per step and lane: LDS slot of the column's entry
     std::vector<int32_t> t;          // 4 per step and lane: monomial * 2 + (1: minus), -1: weight 0
     // gradient of the representatives: per step and lane G slot | slot of the other factor << 16 | real
-    // part negative << 30 | imaginary part negative << 31; rows: Z index | conjugate partner << 12 |
-    // kNodeOwn (the entry's own single G is added), kNodeConj (the partner's, conjugated, with
-    // kNodeMinus negated)
+    // part negative << 30 | imaginary part negative << 31; rows: place in W | place of the conjugate
+    // partner's single G << 12 | kNodeOwn (the entry's own single G, which waits in its place, is added),
+    // kNodeConj (the partner's, conjugated, with kNodeMinus negated)
     std::vector<uint32_t> g_row;
     std::vector<uint32_t> g_rec;
     // two-factor monomials A0 A2: per A2 representative k2 records (A0 slot | conjugate << 31), one
@@ -173,7 +181,7 @@ struct NodePlan {
     std::vector<int32_t> a2_t;
     std::vector<uint32_t> d_slot;    // G slot | slot of the A0 entry << 16
     int kd = 0;
-    std::vector<int32_t> d_x, d_t;   // [kd][A0 entries][8]: A2 entry, monomial * 2 or -1
+    std::vector<int32_t> d_x, d_t;   // [kd][A0 entries][8]: A2 entry (ZLayout::half), monomial * 2 or -1
 };
 
 // Spline tables in node-major layout: row n holds [4 coeffs] for every function family.

@@ -93,17 +93,6 @@ __device__ __forceinline__ void harmonics(T x, T y, T z, int lmax, F&& put) {
     }
 }
 
-__device__ __forceinline__ int half_l(int lh) {  // l of the entry l(l+1)/2 + m
-    int l = 0;
-    while ((l + 1) * (l + 2) / 2 <= lh) ++l;
-    return l;
-}
-__device__ __forceinline__ int full_l(int lm) {  // l of the entry l^2 + l + m
-    int l = 0;
-    while ((l + 1) * (l + 1) <= lm) ++l;
-    return l;
-}
-
 // ---------------------------------------------------------------- spline rows
 // Row number and fraction of a distance or moment (src/radial.F90:68-84, 126-158); row < 0: every function
 // is 0 (kRowZero: beyond the table) or, for moments below the first node, 1 (kRowOne)

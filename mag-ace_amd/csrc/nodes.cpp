@@ -380,11 +380,20 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
                 minus = cj.sign(c) * cj.sign(a) * cj.sign(b) < 0;
                 b = cj.partner(b);
             }
-            single[b].slot = kNodeSingle | b;
+            single[b];
             edges.push_back({id_of(pnode, P, pp), -1, b, 2 * item[i] + minus});
             break;
         }
     }
+    // where a single entry's sum waits: a representative's in its place in W, the others' behind the stored
+    // entries (a row of W has room for all nz)
+    std::map<int, int> wait;
+    int behind = z.nh;
+    for (auto& s : single) {
+        wait[s.first] = T.fold[s.first] >> 17 & 1 ? z.half[s.first] : behind++;
+        s.second.slot = kNodeSingle | wait[s.first];
+    }
+    if (behind > z.nz) return N;
     // core slots: the A and A0 entries that the plan reads, then 1 and 0
     std::vector<char> used(z.nz, 0);
     for (const Pair& p : P) used[p.first] = used[p.second] = 1;
@@ -396,7 +405,7 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
     for (int x = 0; x < z.nz; ++x)
         if (used[x]) {
             slot[x] = (int)N.core_z.size();
-            N.core_z.push_back((uint16_t)x);
+            N.core_z.push_back(z.half[x]);
         }
     N.slot_one = (int)N.core_z.size();
     N.slot_zero = N.slot_one + 1;
@@ -419,7 +428,7 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
         for (const auto& d : dcol)
             for (size_t i = 8 * (size_t)k; i < 8 * (size_t)k + 8; ++i) {
                 const bool have = i < d.second.size();
-                N.d_x.push_back(have ? d.second[i].first : z.oA0);
+                N.d_x.push_back(z.half[have ? d.second[i].first : z.oA0]);
                 N.d_t.push_back(have ? 2 * d.second[i].second : -1);
             }
     N.nslots = next;
@@ -480,22 +489,25 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
     }
     for (const auto& d : dslot) g[d.first].emplace_back(d.second, N.slot_one);
     std::vector<std::vector<uint32_t>> lists;
-    std::vector<uint32_t> target;  // Z index | conjugate partner << 12, kNodeOwn, kNodeConj, kNodeMinus
+    std::vector<uint32_t> target;  // NodePlan::g_row
     for (int x = 0; x < z.nz; ++x) {
         if (x >= z.oA2 && x < z.oA0) continue;
-        if (!(T.fold[x] >> 17 & 1)) continue;
+        if (!z.stored[x]) continue;
+        const bool rep = T.fold[x] >> 17 & 1;  // the others (m = 0, m' < 0) are written as zeros
         std::vector<uint32_t> l;
-        for (const auto& e : g[x]) l.push_back((uint32_t)e.first | (uint32_t)e.second << 16);
-        if (!(T.fold[x] >> 18 & 1)) {
+        if (rep)
+            for (const auto& e : g[x]) l.push_back((uint32_t)e.first | (uint32_t)e.second << 16);
+        if (rep && !(T.fold[x] >> 18 & 1)) {
             const int xb = cj.partner(x), s = cj.sign(x);
             // s conj(G Z): the real part times s, the imaginary part times -s
             for (const auto& e : g[xb])
                 l.push_back((uint32_t)e.first | (uint32_t)e.second << 16 | (s < 0 ? 1u << 30 : 0u) | (s < 0 ? 0u : 1u << 31));
         }
         const int xb = cj.partner(x);
-        uint32_t row = (uint32_t)x | (uint32_t)xb << 12;
-        if (single.count(x)) row |= kNodeOwn;
-        if (!(T.fold[x] >> 18 & 1) && single.count(xb)) row |= kNodeConj | (cj.sign(x) < 0 ? kNodeMinus : 0u);
+        uint32_t row = z.half[x];
+        if (rep && single.count(x)) row |= kNodeOwn;
+        if (rep && !(T.fold[x] >> 18 & 1) && single.count(xb))
+            row |= kNodeConj | (uint32_t)wait[xb] << 12 | (cj.sign(x) < 0 ? kNodeMinus : 0u);
         lists.push_back(std::move(l));
         target.push_back(row);
     }
@@ -541,7 +553,7 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
     std::vector<std::vector<std::pair<uint32_t, int>>> al;
     size_t k2 = 0;
     for (int x = z.oA2; x < z.oA0; ++x) {
-        if (!(T.fold[x] >> 17 & 1)) continue;
+        if (!z.stored[x]) continue;
         std::vector<std::pair<uint32_t, int>> l;
         for (const auto& e : acol[x]) l.emplace_back((uint32_t)slot[e.first], 2 * e.second);
         if (!(T.fold[x] >> 18 & 1)) {
@@ -550,7 +562,7 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
         }
         k2 = std::max(k2, l.size());
         al.push_back(std::move(l));
-        N.a2_x.push_back((uint16_t)x);
+        N.a2_x.push_back(z.half[x]);
     }
     N.k2 = (int)k2;
     for (size_t k = 0; k < k2; ++k)

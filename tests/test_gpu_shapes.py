@@ -8,7 +8,7 @@ import sys
 import numpy as np
 import pytest
 
-from helpers import PKG, relerr, write_potential
+from helpers import HEADERS, PKG, relerr, write_potential
 
 capi, systems = PKG.capi, PKG.systems
 torch = pytest.importorskip("torch")
@@ -18,6 +18,10 @@ if not torch.cuda.is_available():
     pytest.skip("no GPU visible", allow_module_level=True)
 
 import oracle as O  # noqa: E402
+
+# thirteen atomic and five magnetic radial functions at lmax 6 with nine magnetic columns: the largest tables of
+# the forces, whose workgroups have two waves in FP64
+HEADERS["HLDS"] = dict(PKG.potgen.H6W, nb_a=13, nb_m=5, nr2_m=5, nr3_a=1, nr4_a=1)
 
 
 def cut_list(counts, seed):
@@ -48,7 +52,7 @@ def cut_list(counts, seed):
 COUNTS = ([57], [0, 1], [15, 16, 17], [31, 32, 33, 47, 48], [63, 64, 65, 0, 100, 2, 58])
 
 
-@pytest.mark.parametrize("header", ["HTINY", "H500", "H2000", "HFE", "H6W", "H500M0", "H500CORE"])
+@pytest.mark.parametrize("header", ["HTINY", "H500", "H2000", "HFE", "H6W", "H4W", "H500M0", "H500CORE", "HLDS"])
 @pytest.mark.parametrize("counts", COUNTS, ids=lambda c: "-".join(map(str, c)))
 def test_edges_of_tiles(header, counts, tmp_path):
     pot = write_potential(str(tmp_path / "p.in"), header, 77)
