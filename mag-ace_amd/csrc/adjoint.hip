@@ -64,11 +64,50 @@ __device__ __forceinline__ Slot<double>::V slot_flip(Slot<double>::V v, uint32_t
     r.x = flip(v.x, re), r.y = flip(v.y, im);
     return r;
 }
-template <typename V> __device__ __forceinline__ V slot_xor(V v, int o) {
-    V r;
+// +-1 with the sign of bit 31
+__device__ __forceinline__ float unit(uint32_t b, float) { return __uint_as_float((b & 0x80000000u) | 0x3f800000u); }
+__device__ __forceinline__ double unit(uint32_t b, double) {
+    return __hiloint2double((int)((b & 0x80000000u) | 0x3ff00000u), 0);
+}
+// s + t with the signs of a gradient record
+template <typename V> __device__ __forceinline__ V slot_add(V s, V t, uint32_t rec) {
+    const auto re = unit(rec << 1, s[0]), im = unit(rec, s[0]);
 #pragma unroll
-    for (int i = 0; i < (int)(sizeof(V) / sizeof(v[0])); ++i) r[i] = __shfl_xor(v[i], o, 64);
-    return r;
+    for (int i = 0; i < (int)(sizeof(V) / sizeof(s[0])); ++i) s[i] = fma(i & 1 ? im : re, t[i], s[i]);
+    return s;
+}
+// sums over the 2^s lanes of a block, every lane with the result: rows of 16 by the vector units' lane
+// permutations (7 - i and 15 - i do for i + 4 and i + 8, as 4 and 8 lanes hold one value by then), where shuffles
+// through LDS had been half of its instructions at lmax 4
+template <int CTRL> __device__ __forceinline__ float lane_mov(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double lane_mov(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+template <typename F> __device__ __forceinline__ void sum_lanes(int s, F&& each) {
+    // each(f): v = f(v) for all values
+    if (s < 1) return;
+    each([](auto x) { return x + lane_mov<0xb1>(x); });  // quads 1 0 3 2
+    if (s < 2) return;
+    each([](auto x) { return x + lane_mov<0x4e>(x); });  // quads 2 3 0 1
+    if (s < 3) return;
+    each([](auto x) { return x + lane_mov<0x141>(x); });  // 7 - i
+    if (s < 4) return;
+    each([](auto x) { return x + lane_mov<0x140>(x); });  // 15 - i
+    if (s < 5) return;
+    each([](auto x) { return fold16(x, x); });
+    if (s < 6) return;
+    each([](auto x) { return fold32(x, x); });
+}
+template <int N, typename V> __device__ __forceinline__ void sum_slots(int s, V (&v)[N]) {
+    sum_lanes(s, [&](auto f) {
+#pragma unroll
+        for (int r = 0; r < N; ++r)
+#pragma unroll
+            for (int i = 0; i < (int)(sizeof(V) / sizeof(v[r][0])); ++i) v[r][i] = f(v[r][i]);
+    });
 }
 
 // A lane's records, read four steps ahead of their use: the tasks of a wave are one stream in memory,
@@ -92,8 +131,7 @@ struct Ring {
     }
 };
 
-// four rows' sums over the columns of one task; the lanes of a block meet by shuffles, every lane
-// then holds the block's sums
+// four rows' sums over the columns of one task; every lane of a block ends with the block's sums
 template <typename T>
 __device__ __forceinline__ void side_task(Ring<T>& R, int steps, int s, typename Slot<T>::V (&acc)[4]) {
     typedef typename Slot<T>::V V;
@@ -112,9 +150,7 @@ __device__ __forceinline__ void side_task(Ring<T>& R, int steps, int s, typename
             R.wt[u] = R.w[u * 64];
         }
     }
-    for (int o = 0; o < s; ++o)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] += slot_xor(acc[r], 1 << o);
+    sum_slots(s, acc);
 }
 
 }  // namespace
@@ -184,14 +220,13 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
         slot_put<T>(16 * (N.slot_one + tid), v);
     }
     for (int i = tid >> 3; i < N.nd; i += NT / 8) {
-        V s = (V)(T)0;
+        V s[1] = {(V)(T)0};
         for (int k = 0; k < N.kd; ++k) {
             const int r = (k * N.nd + i) * 8 + (tid & 7);
-            s = N.d_w[r] * load(N.d_x[r]) + s;
+            s[0] = N.d_w[r] * load(N.d_x[r]) + s[0];
         }
-#pragma unroll
-        for (int o = 1; o < 8; o <<= 1) s += slot_xor(s, o);
-        if ((tid & 7) == 0) slot_put<T>(16 * (N.d_slot[i] & 0xffff), s);
+        sum_slots(3, s);
+        if ((tid & 7) == 0) slot_put<T>(16 * (N.d_slot[i] & 0xffff), s[0]);
     }
     const int3 cnt = head_of(62), first = head_of(63);
     const int npt = cnt.x, nqt = cnt.y, ngt = cnt.z;
@@ -295,7 +330,7 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
     }
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
-        for (int o = 32; o > 0; o >>= 1) rho[a] += __shfl_xor(rho[a], o, 64);
+        sum_lanes(6, [&](auto f) { rho[a] = f(rho[a]); });
         if (lane == 0) red[a * (NT / 64) + wave] = rho[a];
     }
     __syncthreads();
@@ -315,7 +350,7 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
         const bool lead = (lane & ((1 << h.y) - 1)) == 0;
         const uint32_t row = lead ? N.g_row[h.z + (lane >> h.y)] : 0x80000000u;
         const int x = row & 0xfff, xb = row >> 12 & 0xfff;
-        V s = (V)(T)0, own = (V)(T)0, part = (V)(T)0;
+        V s[1] = {(V)(T)0}, own = (V)(T)0, part = (V)(T)0;
         if (row & (1u << 24)) own = fetch(x);
         if (row & (1u << 25)) part = fetch(xb);
         for (int k = 0; k < h.x; k += 2 * DG) {
@@ -325,16 +360,16 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
                 gn[u] = rec[(DG + u) * 64];
                 const V t0 = slot_mul(slot_get<T>((r.x & 0x3fff) << 4), slot_get<T>((r.x >> 12) & 0x3fff0));
                 const V t1 = slot_mul(slot_get<T>((r.y & 0x3fff) << 4), slot_get<T>((r.y >> 12) & 0x3fff0));
-                s += slot_flip(t0, (r.x << 1) & 0x80000000u, r.x & 0x80000000u);
-                s += slot_flip(t1, (r.y << 1) & 0x80000000u, r.y & 0x80000000u);
+                s[0] = slot_add(s[0], t0, r.x);
+                s[0] = slot_add(s[0], t1, r.y);
             }
             rec += 64 * DG;
         }
-        for (int o = 0; o < h.y; ++o) s += slot_xor(s, 1 << o);
+        sum_slots(h.y, s);
         if (!(row >> 31)) {
             // the conjugate partner's single sum enters as s conj(G)
             const uint32_t minus = row & (1u << 26) ? 0x80000000u : 0u;
-            store(x, s + own + slot_flip(part, minus, minus ^ 0x80000000u));
+            store(x, s[0] + own + slot_flip(part, minus, minus ^ 0x80000000u));
         }
     }
     if (eatom >= 0) {

@@ -81,26 +81,6 @@ __device__ __forceinline__ void put_powers(cplx<T>* e, int g, T x, T y) {
     if (g < 3) e[g + 4] = cmul(a, e4);
 }
 
-// sums of a and b over the two halves of the wave, a's in the lower half and b's in the upper; the same over
-// pairs of 16 lanes
-__device__ __forceinline__ float fold32(float a, float b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float fold16(float a, float b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ double fold32(double a, double b) {
-    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
-    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
-    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
-}
-__device__ __forceinline__ double fold16(double a, double b) {
-    const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
-    const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
-    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
-}
 // lane group g: the sum of u[g] over the four groups
 template <typename T>
 __device__ __forceinline__ T fold_groups(const T (&u)[4]) {
@@ -132,14 +112,14 @@ struct ForceLds {  // offsets in T
 // functions.
 //
 // Bound by issue: at 16000 atoms of lmax 6 a wave has 1670 vector instructions and 132 products of 32 cycles
-// (FP32; 64 in FP64), about 11000 cycles of a SIMD, which measures 294 us (FP64 633 us).  One lane a pair, with W
+// (FP32; 64 in FP64), about 11000 cycles of a SIMD, which measures 294 us (FP64 622 us).  One lane a pair, with W
 // in LDS and sums over n, columns and the harmonics in vector instructions, took 449 us (1093 us); at lmax 4
-// and 27648 atoms 419 -> 324 us (901 -> 584 us), with 27 magnetic columns and 4394 atoms 213 -> 130 us (454 ->
-// 327 us), at 128 atoms of lmax 4 in FP64, where a wave's length counts, 36 -> 15 us.  Five waves a SIMD in
+// and 27648 atoms 419 -> 324 us (901 -> 590 us), with 27 magnetic columns and 4394 atoms 213 -> 130 us (454 ->
+// 320 us), at 128 atoms of lmax 4 in FP64, where a wave's length counts, 36 -> 15 us.  Five waves a SIMD in
 // FP32 need at most 96 registers and 32000 bytes of LDS a workgroup, which the layout below keeps at lmax 6;
 // loading the pairs' inputs before V is made costs the fifth wave and was slower (323 us).
 template <typename T, int NK>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 2, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 2, sizeof(T) == 4 ? 5 : 3)))
 k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restrict__ dlist,
             const double* __restrict__ elist, const double* __restrict__ dmomi, const double* __restrict__ emomi,
             const double* __restrict__ dmom, const double* __restrict__ emom, const cplx<T>* __restrict__ Win, bool scaled,
@@ -245,8 +225,8 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
                 const bool sine = vc.x >> 26 & 1;
                 // NB of n at a time, all their loads before the first use (the coefficients past nr3a are 0).  With
                 // 4 the FP32 kernel had room for 4 waves on a SIMD instead of 5: 305 instead of 294 us at
-                // 16000 atoms, lmax 6.
-                constexpr int NB = 2;
+                // 16000 atoms, lmax 6; in FP64, with room for 3 either way, 2 took 634 instead of 622 us.
+                constexpr int NB = sizeof(T) == 4 ? 2 : 4;
                 for (int n0 = 0; n0 < P.nr3a; n0 += NB) {
                     cplx<T> w[NB], wb[NB];
                     Coef<T> k[NB][NK];
