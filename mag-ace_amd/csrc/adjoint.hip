@@ -197,36 +197,53 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
         return make_int3(__builtin_amdgcn_readlane(head.x, t), __builtin_amdgcn_readlane(head.y, t),
                          __builtin_amdgcn_readlane(head.z, t));
     };
-    // entries of Z, four in flight a thread; the sums over A2 entries, eight lanes an A0 entry
-    for (int i0 = 0; i0 < N.slot_one; i0 += 4 * NT) {
-        V v[4];
+    // Entries of Z, four in flight a thread, and the sums over A2 entries, eight lanes an A0 entry: all places are
+    // loaded before the first entry, so that the phase is two trips to memory.
+    constexpr int UZ = 4, KD = 2;
+    {
+        uint32_t cz[UZ], dx[KD];
+        T dw[KD];
+        V v[UZ], dv[KD];
+        const int di = tid >> 3;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = i0 + u * NT + tid;
-            v[u] = load(N.core_z[i < N.slot_one ? i : 0]);
+        for (int u = 0; u < UZ; ++u) cz[u] = N.core_z[u * NT + tid < N.slot_one ? u * NT + tid : 0];
+#pragma unroll
+        for (int k = 0; k < KD; ++k) {
+            const bool on = di < N.nd && k < N.kd;
+            const int r = on ? (k * N.nd + di) * 8 + (tid & 7) : 0;
+            dx[k] = N.nd > 0 ? N.d_x[r] : 0u;
+            dw[k] = on ? N.d_w[r] : (T)0;
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = i0 + u * NT + tid;
-            if (i < N.slot_one) slot_put<T>(16 * i, v[u]);
+        for (int u = 0; u < UZ; ++u) v[u] = load(cz[u]);
+#pragma unroll
+        for (int k = 0; k < KD; ++k) dv[k] = load(dx[k]);
+#pragma unroll
+        for (int u = 0; u < UZ; ++u)
+            if (u * NT + tid < N.slot_one) slot_put<T>(16 * (u * NT + tid), v[u]);
+        for (int i = UZ * NT + tid; i < N.slot_one; i += NT) slot_put<T>(16 * i, load(N.core_z[i]));
+        if (tid < 2) {
+            V o = (V)(T)0;
+            if (tid == 0) {
+                o[0] = (T)1;
+                if constexpr (NA == 2) o[2] = (T)1;
+            }
+            slot_put<T>(16 * (N.slot_one + tid), o);
         }
-    }
-    if (tid < 2) {
-        V v = (V)(T)0;
-        if (tid == 0) {
-            v[0] = (T)1;
-            if constexpr (NA == 2) v[2] = (T)1;
+        for (int i = di; i < N.nd; i += NT / 8) {
+            V s[1] = {(V)(T)0};
+            if (i == di) {
+#pragma unroll
+                for (int k = 0; k < KD; ++k)
+                    if (k < N.kd) s[0] = dw[k] * dv[k] + s[0];
+            }
+            for (int k = i == di ? KD : 0; k < N.kd; ++k) {
+                const int r = (k * N.nd + i) * 8 + (tid & 7);
+                s[0] = N.d_w[r] * load(N.d_x[r]) + s[0];
+            }
+            sum_slots(3, s);
+            if ((tid & 7) == 0) slot_put<T>(16 * (N.d_slot[i] & 0xffff), s[0]);
         }
-        slot_put<T>(16 * (N.slot_one + tid), v);
-    }
-    for (int i = tid >> 3; i < N.nd; i += NT / 8) {
-        V s[1] = {(V)(T)0};
-        for (int k = 0; k < N.kd; ++k) {
-            const int r = (k * N.nd + i) * 8 + (tid & 7);
-            s[0] = N.d_w[r] * load(N.d_x[r]) + s[0];
-        }
-        sum_slots(3, s);
-        if ((tid & 7) == 0) slot_put<T>(16 * (N.d_slot[i] & 0xffff), s[0]);
     }
     const int3 cnt = head_of(62), first = head_of(63);
     const int npt = cnt.x, nqt = cnt.y, ngt = cnt.z;
@@ -236,6 +253,16 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
     uint32_t ab[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) ab[u] = u * NT + tid < N.npair ? N.pair[u * NT + tid] : 0u;
+    constexpr int K2 = 2;  // an A2 entry's terms read ahead
+    uint32_t a2c[K2];
+    T a2w[K2];
+#pragma unroll
+    for (int k = 0; k < K2; ++k) {
+        const bool on = tid < N.na2 && k < N.k2;
+        a2c[k] = on ? N.a2_c[k * N.na2 + tid] : 0u;
+        a2w[k] = on ? N.a2_w[k * N.na2 + tid] : (T)0;
+    }
+    const int a2x = tid < N.na2 ? N.a2_x[tid] : 0;
     __syncthreads();
     cplx<T>* __restrict__ W0 = Wout + (size_t)a0 * P.nz;
     auto store = [&](int x, V v) {
@@ -244,14 +271,18 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
             if (two) W0[P.nz + x] = {v[2], v[3]};
     };
     // A2 entries need the A0 entries only
+    auto a2_term = [&](V s, uint32_t c, T w) {
+        return w * slot_flip(slot_get<T>((c & 0x3fff) << 4), 0u, c & 0x80000000u) + s;
+    };
     for (int i = tid; i < N.na2; i += NT) {
         V s = (V)(T)0;
-        for (int k = 0; k < N.k2; ++k) {
-            const uint32_t c = N.a2_c[k * N.na2 + i];
-            const T w = N.a2_w[k * N.na2 + i];
-            s = w * slot_flip(slot_get<T>((c & 0x3fff) << 4), 0u, c & 0x80000000u) + s;
+        if (i == tid) {
+#pragma unroll
+            for (int k = 0; k < K2; ++k)
+                if (k < N.k2) s = a2_term(s, a2c[k], a2w[k]);
         }
-        store(N.a2_x[i], s);
+        for (int k = i == tid ? K2 : 0; k < N.k2; ++k) s = a2_term(s, N.a2_c[k * N.na2 + i], N.a2_w[k * N.na2 + i]);
+        store(i == tid ? a2x : (int)N.a2_x[i], s);
     }
     for (int i0 = 0; i0 < N.npair; i0 += U * NT) {
         uint32_t nb[U];
