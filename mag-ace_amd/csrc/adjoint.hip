@@ -207,13 +207,16 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
         const int di = tid >> 3;
 #pragma unroll
         for (int u = 0; u < UZ; ++u) cz[u] = N.core_z[u * NT + tid < N.slot_one ? u * NT + tid : 0];
+        auto places = [&](int i, int k0) {
 #pragma unroll
-        for (int k = 0; k < KD; ++k) {
-            const bool on = di < N.nd && k < N.kd;
-            const int r = on ? (k * N.nd + di) * 8 + (tid & 7) : 0;
-            dx[k] = N.nd > 0 ? N.d_x[r] : 0u;
-            dw[k] = on ? N.d_w[r] : (T)0;
-        }
+            for (int k = 0; k < KD; ++k) {
+                const bool on = i < N.nd && k0 + k < N.kd;
+                const int r = on ? ((k0 + k) * N.nd + i) * 8 + (tid & 7) : 0;
+                dx[k] = N.nd > 0 ? N.d_x[r] : 0u;
+                dw[k] = on ? N.d_w[r] : (T)0;
+            }
+        };
+        places(di, 0);
 #pragma unroll
         for (int u = 0; u < UZ; ++u) v[u] = load(cz[u]);
 #pragma unroll
@@ -232,14 +235,17 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
         }
         for (int i = di; i < N.nd; i += NT / 8) {
             V s[1] = {(V)(T)0};
-            if (i == di) {
+            if (i != di) places(i, 0);
+            for (int k0 = 0; k0 < N.kd; k0 += KD) {
+                if (k0 > 0 || i != di)
 #pragma unroll
-                for (int k = 0; k < KD; ++k)
-                    if (k < N.kd) s[0] = dw[k] * dv[k] + s[0];
-            }
-            for (int k = i == di ? KD : 0; k < N.kd; ++k) {
-                const int r = (k * N.nd + i) * 8 + (tid & 7);
-                s[0] = N.d_w[r] * load(N.d_x[r]) + s[0];
+                    for (int k = 0; k < KD; ++k) dv[k] = load(dx[k]);
+                T w[KD];
+#pragma unroll
+                for (int k = 0; k < KD; ++k) w[k] = dw[k];
+                if (k0 + KD < N.kd) places(i, k0 + KD);
+#pragma unroll
+                for (int k = 0; k < KD; ++k) s[0] = w[k] * dv[k] + s[0];
             }
             sum_slots(3, s);
             if ((tid & 7) == 0) slot_put<T>(16 * (N.d_slot[i] & 0xffff), s[0]);
@@ -281,7 +287,18 @@ k_adjoint_nodes(DevParams<T> P, NodeTab<T> N, const cplx<T>* __restrict__ Zin, c
             for (int k = 0; k < K2; ++k)
                 if (k < N.k2) s = a2_term(s, a2c[k], a2w[k]);
         }
-        for (int k = i == tid ? K2 : 0; k < N.k2; ++k) s = a2_term(s, N.a2_c[k * N.na2 + i], N.a2_w[k * N.na2 + i]);
+        for (int k0 = i == tid ? K2 : 0; k0 < N.k2; k0 += 4) {
+            uint32_t c[4];
+            T w[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int r = (k0 + k < N.k2 ? k0 + k : k0) * N.na2 + i;
+                c[k] = N.a2_c[r];
+                w[k] = k0 + k < N.k2 ? N.a2_w[r] : (T)0;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s = a2_term(s, c[k], w[k]);
+        }
         store(i == tid ? a2x : (int)N.a2_x[i], s);
     }
     for (int i0 = 0; i0 < N.npair; i0 += U * NT) {
