@@ -29,6 +29,9 @@ constexpr int kPairs = 60;  // pairs of a round: 15 steps of four; lane 60 of th
 // the whole sum (FP32 errors of E and of the forces against 64 bits, lmax-4 header: 60 pairs a chain
 // 5.4e-7 and 3.5e-7, 20 pairs 3.2e-7 and 2.5e-7, and shorter chains less)
 template <typename T> constexpr int kChain = sizeof(T) == 4 ? 12 : kPairs;
+template <typename T> constexpr int kRound = sizeof(T) == 4 ? 12 : 4;  // pairs of an unrolled turn; divides kPairs
+
+constexpr int kG = 17;  // row of a pair's base functions: 16, and one for the banks
 
 struct DensityLds {  // strides and offsets (in T) of the staging arrays
     int sY, sYm, sH, sM;          // row lengths: Y, Y' and H in complex entries, M in values; odd
@@ -38,44 +41,24 @@ struct DensityLds {  // strides and offsets (in T) of the staging arrays
         oYm = 2 * kPairs * sY;
         oH = oYm + 2 * (kPairs + 1) * sYm;
         oG = (oH + 2 * kPairs * sH + 3) & ~3;
-        oM = oG + 16 * kPairs;
+        oM = oG + kG * kPairs;
         oYd = (oM + (kPairs + 1) * sM + 3) & ~3;
         oGd = oYd + (jvp ? 2 * kPairs * sY : 0);
-        size = oGd + (jvp ? 16 * kPairs : 0);
+        size = oGd + (jvp ? kG * kPairs : 0);
     }
 };
 
-// items (row j, function k), j < rows, k < nf, one a lane and step: value(j, k, flags, coefficients, fraction)
-// with flags >> 16 set where the function is 0 or 1 and flags >> 17 where it is 1; lane j has row j's number
+// functions first .. first + nf - 1 of a row, value(k, coefficients), U loads in flight
 template <typename T, typename F>
-__device__ __forceinline__ void spline_items(const T* __restrict__ lut, int stride, int first, int nf, int rows,
-                                             int row, T w, int lane, F&& value) {
-    constexpr int U = sizeof(T) == 4 ? 7 : 4;  // loads in flight
-    const int dj = 64 / nf, dk = 64 - dj * nf;
-    int j = lane / nf, k = lane - j * nf;
-    const T* __restrict__ base = lut + 4 * first;
-    while (__any(j < rows)) {
+__device__ __forceinline__ void spline_row(const T* __restrict__ row, int first, int nf, F&& value) {
+    constexpr int U = sizeof(T) == 4 ? 8 : 4;
+    for (int k0 = 0; k0 < nf; k0 += U) {
         Coef<T> c[U];
-        T wj[U];
-        int at[U];  // row | function << 8 | absent << 16 | one << 17
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int src = j < rows ? j : 0, r = __shfl(row, src, 64);
-            wj[u] = __shfl(w, src, 64);
-            c[u] = coef_at(base + (uint32_t)(r < 0 ? 0 : r) * (uint32_t)stride + 4 * k);
-            at[u] = (j < rows ? j : 255) | k << 8 | (r < 0 ? 1 << 16 : 0) | (r == kRowOne ? 1 << 17 : 0);
-            j += dj;
-            k += dk;
-            if (k >= nf) {
-                k -= nf;
-                ++j;
-            }
-        }
+        for (int u = 0; u < U; ++u) c[u] = coef_at(row + 4 * (first + min(k0 + u, nf - 1)));
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int ju = at[u] & 0xff;
-            if (ju < rows) value(ju, at[u] >> 8 & 0xff, at[u], c[u], wj[u]);
-        }
+        for (int u = 0; u < U; ++u)
+            if (k0 + u < nf) value(k0 + u, c[u]);
     }
 }
 
@@ -130,7 +113,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
         c2[t] = P.cols[min(wave + 4 * (na + t), tAll - 1) * 16 + ci];
     }
     // rows past nb_a of the base functions stay zero
-    for (int i = tid; i < kPairs * 16; i += 256) {
+    for (int i = tid; i < kPairs * kG; i += 256) {
         sG[i] = (T)0;
         if (JVP) sGd[i] = (T)0;
     }
@@ -142,12 +125,13 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
     }
     double core = 0.0;
     for (int c0 = 0; c0 == 0 || c0 < nn; c0 += kPairs) {
-        const int nj = min(nn - c0, kPairs), nj4 = (nj + 3) & ~3;
+        // whole chains of pairs; those past the end have g = 0
+        const int nj = min(nn - c0, kPairs), nr = (nj + kRound<T> - 1) / kRound<T> * kRound<T>;
         const bool live = lane < nj, centre = !JVP && lane == kPairs && c0 == 0;
         const size_t p = (size_t)p0 + c0 + (live ? lane : 0);
         __syncthreads();
         if (wave == 0) {
-            if (lane < nj4) {
+            if (lane < nr) {
                 T w = 0;
                 const int row = live ? atomic_index(P, dlist[p], w, err) : kRowZero;
                 const T x = live ? (T)elist[3 * p] : (T)0, y = live ? (T)elist[3 * p + 1] : (T)0,
@@ -181,7 +165,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 }
             }
         } else if (wave == 1) {
-            if (lane < nj4 || centre) {
+            if (lane < nr || centre) {
                 const bool any = live || centre;
                 T w = 0;
                 const int row = live ? magnetic_index(P, dmom[p], w, err) : kRowZero;
@@ -196,7 +180,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 harmonics<T, L>(x, y, z, P.l2m, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
                     sYm[lane * D.sYm + k] = {pl * ph.re, pl * ph.im};
                 });
-                if (lane < nj4)
+                if (lane < nr)
                     for (int np = 0; np * P.lsm3 < P.nm3; ++np)
                         for (int lp = 0; lp <= P.l3m; ++lp) {
                             Coef<T> c;
@@ -224,32 +208,24 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                            elist[3 * p + 2] * (uz - du[jn + 2]);
                 }
             }
-            spline_items<T>(P.lut_g, P.stride_g, 0, P.nb_a, nj4, row, w, lane,
-                            [&](int j, int k, int r, const Coef<T>& c, T wj) {
-                                sG[j * 16 + k] = r >> 16 ? (T)0 : coef_value(c, wj);
-                                if constexpr (JVP) sGd[j * 16 + k] = r >> 16 ? (T)0 : coef_slope(c, wj, (T)P.rs_a);
-                            });
-            if constexpr (JVP) {
-                // g'_k (u_i - u_j) . e: each lane scales its own pair's row, after the wave's writes above
-                __builtin_amdgcn_wave_barrier();
-                if (lane < nj4)
-                    for (int k = 0; k < P.nb_a; ++k) sGd[lane * 16 + k] *= rdot;
-            }
+            if (lane < nr)
+                spline_row<T>(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g, 0, P.nb_a,
+                              [&](int k, const Coef<T>& c) {
+                                  sG[lane * kG + k] = row < 0 ? (T)0 : coef_value(c, w);
+                                  // g'_k (u_i - u_j) . e
+                                  if constexpr (JVP)
+                                      sGd[lane * kG + k] = row < 0 ? (T)0 : coef_slope(c, w, (T)P.rs_a) * rdot;
+                              });
         } else {
             T w = 0;
             const int row = centre ? magnetic_index(P, dmomi[atom], w, err)
                                    : live ? magnetic_index(P, dmom[p], w, err) : kRowZero;
-            // the central atom's row follows the pairs' (lane kPairs -> row nj4 of the items)
             const bool first = !JVP && c0 == 0;
-            const int src = first && lane == nj4 ? kPairs : lane;
-            const int rowi = __shfl(row, src, 64);
-            const T wi = __shfl(w, src, 64);
-            if (nfm > 0)
-                spline_items<T>(P.lut_m, P.stride_m, P.nb_m, nfm, nj4 + (first ? 1 : 0), rowi, wi, lane,
-                            [&](int j, int k, int r, const Coef<T>& c, T wj) {
-                                sM[(j == nj4 ? kPairs : j) * D.sM + k] =
-                                    r >> 17 ? (T)1 : r >> 16 ? (T)0 : coef_value(c, wj);
-                            });
+            if (lane < nr || centre)
+                spline_row<T>(P.lut_m + (size_t)(row < 0 ? 0 : row) * P.stride_m, P.nb_m, nfm,
+                              [&](int k, const Coef<T>& c) {
+                                  sM[lane * D.sM + k] = row == kRowOne ? (T)1 : row < 0 ? (T)0 : coef_value(c, w);
+                              });
             if (first) {
                 // B1 part of rho (b_basis.F90:62-83): lane k has g^m_k of the central moment
                 const int rc = __shfl(row, kPairs, 64);
@@ -283,25 +259,26 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 Zout[P.hA0 + t] = z;
             }
         }
-        for (int s0 = 0; s0 < nj4; s0 += kChain<T>) {
-            V sr[TA], si[TA], s2r[T2], s2i[T2];  // the sums of kChain pairs, in FP32
-            constexpr bool kPart = kChain<T> < kPairs;
-            V(&br)[TA] = kPart ? sr : ar;
-            V(&bi)[TA] = kPart ? si : ai;
-            V(&b2r)[T2] = kPart ? s2r : a2r;
-            V(&b2i)[T2] = kPart ? s2i : a2i;
-            if constexpr (kPart) {
+        for (int s0 = 0; s0 < nr; s0 += kRound<T>) {
+            constexpr bool kPart = kChain<T> < kPairs;  // the sums of kChain pairs join the atom's
+            V br[TA], bi[TA], b2r[T2], b2i[T2];
 #pragma unroll
-                for (int t = 0; t < TA; ++t) sr[t] = si[t] = (V)(T)0;
-#pragma unroll
-                for (int t = 0; t < T2; ++t) s2r[t] = s2i[t] = (V)(T)0;
+            for (int t = 0; t < TA; ++t) {
+                br[t] = kPart ? (V)(T)0 : ar[t];
+                bi[t] = kPart ? (V)(T)0 : ai[t];
             }
-            for (int s = s0; s < min(s0 + kChain<T>, nj4); s += 4) {
-                const int j = s + g;
+#pragma unroll
+            for (int t = 0; t < T2; ++t) {
+                b2r[t] = kPart ? (V)(T)0 : a2r[t];
+                b2i[t] = kPart ? (V)(T)0 : a2i[t];
+            }
+#pragma unroll
+            for (int s = 0; s < kRound<T>; s += 4) {
+                const int j = s0 + s + g;
                 // the step's operands of every tile first, so that one trip to LDS serves them all
-                const T a = sG[j * 16 + ci];
+                const T a = sG[j * kG + ci];
                 T ad = 0;
-                if constexpr (JVP) ad = sGd[j * 16 + ci];
+                if constexpr (JVP) ad = sGd[j * kG + ci];
                 cplx<T> y[TA], h[TA], yd[JVP ? TA : 1], y2[T2];
                 T m2[T2];
 #pragma unroll
@@ -334,17 +311,15 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                         b2i[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].im, b2i[t]);
                     }
             }
-            if constexpr (kPart) {
 #pragma unroll
-                for (int t = 0; t < TA; ++t) {
-                    ar[t] += sr[t];
-                    ai[t] += si[t];
-                }
+            for (int t = 0; t < TA; ++t) {
+                ar[t] = kPart ? ar[t] + br[t] : br[t];
+                ai[t] = kPart ? ai[t] + bi[t] : bi[t];
+            }
 #pragma unroll
-                for (int t = 0; t < T2; ++t) {
-                    a2r[t] += s2r[t];
-                    a2i[t] += s2i[t];
-                }
+            for (int t = 0; t < T2; ++t) {
+                a2r[t] = kPart ? a2r[t] + b2r[t] : b2r[t];
+                a2i[t] = kPart ? a2i[t] + b2i[t] : b2i[t];
             }
         }
     }
