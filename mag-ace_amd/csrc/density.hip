@@ -15,6 +15,8 @@
 // the staging is 90, the products 110 (69 at the matrix cores' rate) and the stores of Z 100.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device.hpp"
 #include "kernels.hpp"
 #include "matrix.hpp"
@@ -33,11 +35,19 @@ template <typename T> constexpr int kRound = sizeof(T) == 4 ? 12 : 4;  // pairs 
 
 constexpr int kG = 17;  // row of a pair's base functions: 16, and one for the banks
 
+// Harmonics in a pair's row of Y or Y'.  In FP32 those of the instance's lmax, so that the rows' addresses are known
+// when it is compiled; in FP64 the longer rows of headers below it cost a workgroup of a compute unit (4394 atoms
+// of the example potential's shape 111 -> 128 us).
+template <typename T, int L> __host__ __device__ constexpr int harmonics_row(int n) {
+    return sizeof(T) == 4 ? (L + 1) * (L + 2) / 2 : n;
+}
+
 struct DensityLds {  // strides and offsets (in T) of the staging arrays
     int sY, sYm, sH, sM;          // row lengths: Y, Y' and H in complex entries, M in values; odd
     int oYm, oH, oG, oM, oYd, oGd, size;
-    __host__ __device__ DensityLds(int lha, int lhm, int nm3, int nfm, bool jvp) {
-        sY = lha | 1, sYm = lhm | 1, sH = nm3 | 1, sM = nfm | 1;
+    // lha, lhm: harmonics_row
+    __host__ __device__ constexpr DensityLds(int lha, int lhm, int nm3, int nfm, bool jvp)
+        : sY(lha | 1), sYm(lhm | 1), sH(nm3 | 1), sM(nfm | 1), oYm(0), oH(0), oG(0), oM(0), oYd(0), oGd(0), size(0) {
         oYm = 2 * kPairs * sY;
         oH = oYm + 2 * (kPairs + 1) * sYm;
         oG = (oH + 2 * kPairs * sH + 3) & ~3;
@@ -48,17 +58,17 @@ struct DensityLds {  // strides and offsets (in T) of the staging arrays
     }
 };
 
-// functions first .. first + nf - 1 of a row, value(k, coefficients), U loads in flight
+// functions first .. first + nf - 1 of a row: value(k, coefficients), some more than once
 template <typename T, typename F>
 __device__ __forceinline__ void spline_row(const T* __restrict__ row, int first, int nf, F&& value) {
-    constexpr int U = sizeof(T) == 4 ? 8 : 4;
+    constexpr int U = 4;
+    row += 4 * first;
     for (int k0 = 0; k0 < nf; k0 += U) {
-        Coef<T> c[U];
+        Coef<T> n[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) c[u] = coef_at(row + 4 * (first + min(k0 + u, nf - 1)));
+        for (int u = 0; u < U; ++u) n[u] = coef_at(row + 4 * min(k0 + u, nf - 1));
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (k0 + u < nf) value(k0 + u, c[u]);
+        for (int u = 0; u < U; ++u) value(min(k0 + u, nf - 1), n[u]);
     }
 }
 
@@ -84,7 +94,8 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
     const int atom = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nfm = P.nr2m * (P.l2m + 1);
-    const DensityLds D(P.lha, P.lhm, P.nm3, nfm, JVP);
+    const int SY = harmonics_row<T, L>(P.lha) | 1, SYM = harmonics_row<T, L>(P.lhm) | 1;  // DensityLds::sY and sYm
+    const DensityLds D(harmonics_row<T, L>(P.lha), harmonics_row<T, L>(P.lhm), P.nm3, nfm, JVP);
     T* lds = (T*)smem;
     cplx<T>*sY = (cplx<T>*)lds, *sYm = (cplx<T>*)(lds + D.oYm), *sH = (cplx<T>*)(lds + D.oH);
     T *sG = lds + D.oG, *sM = lds + D.oM;
@@ -139,7 +150,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 const Coef<T> cc = coef_at(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g + 4 * P.nb_a);
                 if constexpr (!JVP) {
                     harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
-                        sY[lane * D.sY + k] = {pl * ph.re, pl * ph.im};
+                        sY[lane * SY + k] = {pl * ph.re, pl * ph.im};
                     });
                     core += row < 0 ? 0.0 : (double)coef_value(cc, w);
                 } else {
@@ -155,11 +166,11 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                     // the displacement's part across the bond, over r: D_u Y = grad Y . t
                     const T tx = (dx - rdot * x) * invr, ty = (dy - rdot * y) * invr, tz = (dz - rdot * z) * invr;
                     harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T dpl, cplx<T> ph, cplx<T> ph1, int m) {
-                        sY[lane * D.sY + k] = {pl * ph.re, pl * ph.im};
+                        sY[lane * SY + k] = {pl * ph.re, pl * ph.im};
                         // Y = P(z) (x + iy)^m
                         const T a = dpl * tz, b = (T)m * pl;
                         const cplx<T> e = cmul(ph1, cplx<T>{tx, ty});
-                        sYd[lane * D.sY + k] = {fma(a, ph.re, b * e.re), fma(a, ph.im, b * e.im)};
+                        sYd[lane * SY + k] = {fma(a, ph.re, b * e.re), fma(a, ph.im, b * e.im)};
                     });
                     core += row < 0 ? 0.0 : (double)(coef_slope(cc, w, (T)P.rs_a) * rdot);
                 }
@@ -178,7 +189,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
 #pragma unroll
                 for (int u = 0; u < U; ++u) cm[u] = coef_at(mrow + 4 * (u <= P.l3m ? u * P.nr2m : 0));
                 harmonics<T, L>(x, y, z, P.l2m, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
-                    sYm[lane * D.sYm + k] = {pl * ph.re, pl * ph.im};
+                    sYm[lane * SYM + k] = {pl * ph.re, pl * ph.im};
                 });
                 if (lane < nr)
                     for (int np = 0; np * P.lsm3 < P.nm3; ++np)
@@ -191,7 +202,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                                 for (int u = 0; u < 4; ++u) c.c[u] = lp ? cm[1].c[u] : cm[0].c[u];
                             const T mv = row == kRowOne ? (T)1 : row < 0 ? (T)0 : coef_value(c, w);
                             for (int mp = -lp; mp <= lp; ++mp) {
-                                const cplx<T> h = sYm[lane * D.sYm + lp * (lp + 1) / 2 + (mp < 0 ? -mp : mp)];
+                                const cplx<T> h = sYm[lane * SYM + lp * (lp + 1) / 2 + (mp < 0 ? -mp : mp)];
                                 const cplx<T> yv = mp < 0 ? cconj_sign(h, -mp) : h;
                                 sH[lane * D.sH + np * P.lsm3 + lp * lp + lp + mp] = {mv * yv.re, mv * yv.im};
                             }
@@ -221,7 +232,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
             const int row = centre ? magnetic_index(P, dmomi[atom], w, err)
                                    : live ? magnetic_index(P, dmom[p], w, err) : kRowZero;
             const bool first = !JVP && c0 == 0;
-            if (lane < nr || centre)
+            if (nfm > 0 && (lane < nr || centre))
                 spline_row<T>(P.lut_m + (size_t)(row < 0 ? 0 : row) * P.stride_m, P.nb_m, nfm,
                               [&](int k, const Coef<T>& c) {
                                   sM[lane * D.sM + k] = row == kRowOne ? (T)1 : row < 0 ? (T)0 : coef_value(c, w);
@@ -252,49 +263,64 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 cplx<T> z = {0, 0};
                 if constexpr (!JVP) {
                     const uint32_t d = P.cols[tA * 16 + t];
-                    const cplx<T> h = sYm[kPairs * D.sYm + (d & 0xff)];
+                    const cplx<T> h = sYm[kPairs * SYM + (d & 0xff)];
                     const T mv = sM[kPairs * D.sM + (d >> 8 & 0xff)];
                     z = {mv * h.re, mv * h.im};
                 }
                 Zout[P.hA0 + t] = z;
             }
         }
-        for (int s0 = 0; s0 < nr; s0 += kRound<T>) {
+        // NA tiles of A and N2 of A2
+        auto products = [&](auto NA_, auto N2_) {
+            constexpr int NA = NA_, N2 = N2_;
             constexpr bool kPart = kChain<T> < kPairs;  // the sums of kChain pairs join the atom's
-            V br[TA], bi[TA], b2r[T2], b2i[T2];
+            int iy[TA], ih[TA], iy2[T2], im[T2];
 #pragma unroll
-            for (int t = 0; t < TA; ++t) {
-                br[t] = kPart ? (V)(T)0 : ar[t];
-                bi[t] = kPart ? (V)(T)0 : ai[t];
+            for (int t = 0; t < NA; ++t) {
+                iy[t] = g * SY + (ca[t] & 0xff);
+                ih[t] = g * D.sH + (ca[t] >> 8 & 0xff);
             }
 #pragma unroll
-            for (int t = 0; t < T2; ++t) {
-                b2r[t] = kPart ? (V)(T)0 : a2r[t];
-                b2i[t] = kPart ? (V)(T)0 : a2i[t];
+            for (int t = 0; t < N2; ++t) {
+                iy2[t] = g * SYM + (c2[t] & 0xff);
+                im[t] = g * D.sM + (c2[t] >> 8 & 0xff);
             }
+            int ig = g * kG + ci;
+            for (int s0 = 0; s0 < nr; s0 += kRound<T>) {
+                V br[TA], bi[TA], b2r[T2], b2i[T2];
 #pragma unroll
-            for (int s = 0; s < kRound<T>; s += 4) {
-                const int j = s0 + s + g;
-                // the step's operands of every tile first, so that one trip to LDS serves them all
-                const T a = sG[j * kG + ci];
-                T ad = 0;
-                if constexpr (JVP) ad = sGd[j * kG + ci];
-                cplx<T> y[TA], h[TA], yd[JVP ? TA : 1], y2[T2];
-                T m2[T2];
-#pragma unroll
-                for (int t = 0; t < TA; ++t) {
-                    y[t] = sY[j * D.sY + (ca[t] & 0xff)];
-                    h[t] = sH[j * D.sH + (ca[t] >> 8 & 0xff)];
-                    if constexpr (JVP) yd[JVP ? t : 0] = sYd[j * D.sY + (ca[t] & 0xff)];
+                for (int t = 0; t < NA; ++t) {
+                    br[t] = kPart ? (V)(T)0 : ar[t];
+                    bi[t] = kPart ? (V)(T)0 : ai[t];
                 }
 #pragma unroll
-                for (int t = 0; t < T2; ++t) {
-                    y2[t] = sYm[j * D.sYm + (c2[t] & 0xff)];
-                    m2[t] = sM[j * D.sM + (c2[t] >> 8 & 0xff)];
+                for (int t = 0; t < N2; ++t) {
+                    b2r[t] = kPart ? (V)(T)0 : a2r[t];
+                    b2i[t] = kPart ? (V)(T)0 : a2i[t];
                 }
 #pragma unroll
-                for (int t = 0; t < TA; ++t)
-                    if (t < na) {
+                for (int s = 0; s < kRound<T>; s += 4) {
+                    // the step's operands of every tile first, so that one trip to LDS serves them all
+                    const T a = sG[ig + s * kG];
+                    T ad = 0;
+                    if constexpr (JVP) ad = sGd[ig + s * kG];
+                    cplx<T> y[TA], h[TA], yd[JVP ? TA : 1], y2[T2];
+                    T m2[T2];
+#pragma unroll
+                    for (int t = 0; t < NA; ++t) {
+                        y[t] = sY[iy[t] + s * SY];
+                        h[t] = sH[ih[t]];
+                        ih[t] += 4 * D.sH;
+                        if constexpr (JVP) yd[JVP ? t : 0] = sYd[iy[t] + s * SY];
+                    }
+#pragma unroll
+                    for (int t = 0; t < N2; ++t) {
+                        y2[t] = sYm[iy2[t] + s * SYM];
+                        m2[t] = sM[im[t]];
+                        im[t] += 4 * D.sM;
+                    }
+#pragma unroll
+                    for (int t = 0; t < NA; ++t) {
                         const cplx<T> v = cmul(y[t], h[t]);
                         br[t] = Mm<T>::mul(JVP ? ad : a, v.re, br[t]);
                         bi[t] = Mm<T>::mul(JVP ? ad : a, v.im, bi[t]);
@@ -305,22 +331,39 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                         }
                     }
 #pragma unroll
-                for (int t = 0; t < T2; ++t)
-                    if (t < n2) {
+                    for (int t = 0; t < N2; ++t) {
                         b2r[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].re, b2r[t]);
                         b2i[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].im, b2i[t]);
                     }
-            }
+                }
+                ig += kRound<T> * kG;
 #pragma unroll
-            for (int t = 0; t < TA; ++t) {
-                ar[t] = kPart ? ar[t] + br[t] : br[t];
-                ai[t] = kPart ? ai[t] + bi[t] : bi[t];
-            }
+                for (int t = 0; t < NA; ++t) {
+                    ar[t] = kPart ? ar[t] + br[t] : br[t];
+                    ai[t] = kPart ? ai[t] + bi[t] : bi[t];
+                    iy[t] += kRound<T> * SY;
+                }
 #pragma unroll
-            for (int t = 0; t < T2; ++t) {
-                a2r[t] = kPart ? a2r[t] + b2r[t] : b2r[t];
-                a2i[t] = kPart ? a2i[t] + b2i[t] : b2i[t];
+                for (int t = 0; t < N2; ++t) {
+                    a2r[t] = kPart ? a2r[t] + b2r[t] : b2r[t];
+                    a2i[t] = kPart ? a2i[t] + b2i[t] : b2i[t];
+                    iy2[t] += kRound<T> * SYM;
+                }
             }
+        };
+        // The loops have no branch on a wave's tiles: a tile that it does not have repeats the last one and is not
+        // stored.
+        using std::integral_constant;
+        if (na >= TA) {
+            if (n2 >= T2)
+                products(integral_constant<int, TA>(), integral_constant<int, T2>());
+            else
+                products(integral_constant<int, TA>(), integral_constant<int, T2 - 1>());
+        } else {
+            if (n2 >= T2)
+                products(integral_constant<int, TA - 1>(), integral_constant<int, T2>());
+            else
+                products(integral_constant<int, TA - 1>(), integral_constant<int, T2 - 1>());
         }
     }
 #pragma unroll
@@ -381,7 +424,8 @@ hipError_t launch_density(const DevParams<T>& P, int natom, const int* off, cons
                           const int* nlist, const double* du, void* Z, double* ehc, double* rho1, int* err,
                           hipStream_t s) {
     auto k = k_density_mm<T, L, TA, T2, JVP>;
-    const size_t lds = (size_t)DensityLds(P.lha, P.lhm, P.nm3, P.nr2m * (P.l2m + 1), JVP).size * sizeof(T);
+    const size_t lds = (size_t)DensityLds(harmonics_row<T, L>(P.lha), harmonics_row<T, L>(P.lhm), P.nm3,
+                                         P.nr2m * (P.l2m + 1), JVP).size * sizeof(T);
     static bool set = false;
     static size_t limit = 0;
     hipError_t e;
@@ -413,6 +457,7 @@ hipError_t by_tiles(const DevParams<T>& P, A... a) {
     if (tA < 1) return hipErrorInvalidValue;
     if (ta <= 1 && t2 <= 1) return launch_density<T, L, 1, 1, JVP>(P, a...);
     if (ta <= 2 && t2 <= 1) return launch_density<T, L, 2, 1, JVP>(P, a...);
+    if (ta <= 4 && t2 <= 1) return launch_density<T, L, 4, 1, JVP>(P, a...);
     if (ta <= 4 && t2 <= 3) return launch_density<T, L, 4, 3, JVP>(P, a...);
     return hipErrorInvalidValue;  // no header of the supported classes has more
 }
