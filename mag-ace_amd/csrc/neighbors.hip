@@ -5,17 +5,21 @@
 //
 // Pipeline (one stream, one host synchronisation to learn the pair count):
 //   k_nb_bbox     bounding box of open clusters                neilist.F90:313-336
-//   k_nb_frac     fractional coordinates wrapped into the cell neilist.F90:354-368
-//   k_nb_flag     image candidates inside the slab of width rc neilist.F90:382-434
-//   scan          cluster index of every kept candidate (stable: identity block first,
-//                 then shifts in (k1,k2,k3) order, atoms ascending inside a shift)
-//   k_nb_cluster  cluster positions + grid box of edge rc       neilist.F90:385-421, 576-588
+//   k_nb_frac     fractional coordinates wrapped into the cell neilist.F90:354-368; counters cleared
+//   k_nb_flag     image candidates inside the slab of width rc neilist.F90:382-434, counted per tile
+//   k_nb_cluster  cluster index of every kept candidate (stable: identity block first, then shifts in (k1,k2,k3)
+//                 order, atoms ascending inside a shift), position + grid box of edge rc, atoms per box
+//                                                               neilist.F90:385-421, 576-588
 //   scan, k_nb_bfill, k_nb_bsort   atoms grouped by box, ascending cluster index inside a
 //                 box (the reference's counting sort order)     neilist.F90:591-604
 //   k_nb_pairs<0> one wavefront per central atom: 27-box stencil in the reference order
 //                 (own box, then (k1,k2,k3) ascending), fastdist, ballot-compacted count
 //   scan          CSR offsets
-//   k_nb_pairs<1> same walk, writes the pairs in order          neilist.F90:693-793
+//   k_nb_tail     totals into host memory
+//   k_nb_pairs<1> same walk; the hits gather in LDS and 64 at a time are written in order  neilist.F90:693-793
+//
+// Bound by launches, the gaps between them and the one synchronisation at small sizes: 16000 atoms 211 -> 107 us
+// with ten launches and one copy to the device in place of twenty launches and six copies.
 //
 // Contraction of multiply-add is off in this file: every FP64 expression is evaluated in
 // the reference's operation order with IEEE rounding, so positions, distances and unit
@@ -25,6 +29,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -38,7 +43,9 @@ namespace magace {
 namespace {
 
 constexpr double kEps = 1.0e-9;  // neilist/neilist.F90:9
+constexpr long long kTilesAdded = 4096;  // tiles that each add up the counts before theirs (k_nb_cluster)
 constexpr int kScanThreads = 256, kScanItems = 4, kScanTile = kScanThreads * kScanItems;
+constexpr int kCandItems = 1, kCandTile = kScanThreads * kCandItems;
 
 enum : int { kNbErrBox = 1, kNbErrIdentical = 2 };
 
@@ -146,9 +153,28 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(const int* __restri
     }
 }
 
-__global__ void k_fill_int(int* __restrict__ p, long long n, int v) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+// the same in one launch for short arrays: every tile adds up all entries before it (16001 offsets: 13.5 us in the
+// three kernels above, 5 us here, 16 us in one workgroup)
+constexpr long long kScanEach = 64 * kScanTile;
+__global__ __launch_bounds__(kScanThreads) void k_scan_each(const int* __restrict__ in, int n, int* __restrict__ out) {
+    __shared__ int sh[kScanThreads / 64];
+    const int tile = blockIdx.x * kScanTile, base = tile + threadIdx.x * kScanItems;
+    int before = 0, v[kScanItems], s = 0;
+#pragma unroll 8
+    for (int i = threadIdx.x; i < tile; i += kScanThreads) before += in[i];
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) v[k] = base + k < n ? in[base + k] : 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) s += v[k];
+    int carry, total;
+    (void)block_exclusive(before, sh, carry);
+    int e = carry + block_exclusive(s, sh, total);
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (base + k < n) out[base + k] = e;
+        e += v[k];
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = carry + total;
 }
 
 // ---------------------------------------------------------------- kernels of the build
@@ -186,8 +212,11 @@ __global__ __launch_bounds__(256) void k_nb_bbox(const NbGeom* __restrict__ G, c
 // fractional coordinates wrapped into [0,1) (periodic) -- neilist.F90:356-367
 // afl = the integer part removed by the wrap (image bookkeeping for pair shifts)
 __global__ void k_nb_frac(const NbGeom* __restrict__ G, const int* __restrict__ atom_off, int nstruc, int ntot,
-                          const double* __restrict__ pos, double* __restrict__ frac, int* __restrict__ afl) {
+                          const double* __restrict__ pos, double* __restrict__ frac, int* __restrict__ afl, int nbox,
+                          int* __restrict__ bcount, int* __restrict__ err) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a == 0) *err = 0;
+    if (a < nbox) bcount[a] = 0;
     if (a >= ntot) return;
     const NbGeom& g = G[find_struct(atom_off, nstruc, a)];
     const double p0 = pos[3 * (size_t)a], p1 = pos[3 * (size_t)a + 1], p2 = pos[3 * (size_t)a + 2];
@@ -231,39 +260,53 @@ __device__ __forceinline__ Cand decode(const NbGeom* __restrict__ G, const long 
 }
 
 // image candidate kept?  neilist.F90:394-418
-__global__ void k_nb_flag(const NbGeom* __restrict__ G, const long long* __restrict__ cand_off, int nstruc,
-                          long long ncand, const double* __restrict__ frac, int* __restrict__ flag) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ncand) return;
-    const Cand c = decode(G, cand_off, nstruc, i);
-    int keep = 1;
-    if (!c.identity) {
-        const NbGeom& g = G[c.s];
-        const double r1[3] = {frac[3 * (size_t)c.a] + (double)c.k0, frac[3 * (size_t)c.a + 1] + (double)c.k1,
-                              frac[3 * (size_t)c.a + 2] + (double)c.k2};
-        keep = r1[0] > g.dxl[0] && r1[0] <= g.dxh[0] && r1[1] > g.dxl[1] && r1[1] <= g.dxh[1] &&
-               r1[2] > g.dxl[2] && r1[2] <= g.dxh[2];
-        if (keep) {
-            double r2[3];
-            for (int n = 0; n < 3; ++n) r2[n] = g.cell[n] * r1[0] + g.cell[n + 3] * r1[1] + g.cell[n + 6] * r1[2];
-            keep = r2[0] > g.lcc[0] && r2[0] <= g.hcc[0] && r2[1] > g.lcc[1] && r2[1] <= g.hcc[1] &&
-                   r2[2] > g.lcc[2] && r2[2] <= g.hcc[2];
-        }
+__device__ __forceinline__ bool kept(const NbGeom* __restrict__ G, const Cand& c, const double* __restrict__ frac) {
+    if (c.identity) return true;
+    const NbGeom& g = G[c.s];
+    const double r1[3] = {frac[3 * (size_t)c.a] + (double)c.k0, frac[3 * (size_t)c.a + 1] + (double)c.k1,
+                          frac[3 * (size_t)c.a + 2] + (double)c.k2};
+    if (!(r1[0] > g.dxl[0] && r1[0] <= g.dxh[0] && r1[1] > g.dxl[1] && r1[1] <= g.dxh[1] && r1[2] > g.dxl[2] &&
+          r1[2] <= g.dxh[2]))
+        return false;
+    double r2[3];
+    for (int n = 0; n < 3; ++n) r2[n] = g.cell[n] * r1[0] + g.cell[n + 3] * r1[1] + g.cell[n + 6] * r1[2];
+    return r2[0] > g.lcc[0] && r2[0] <= g.hcc[0] && r2[1] > g.lcc[1] && r2[1] <= g.hcc[1] && r2[2] > g.lcc[2] &&
+           r2[2] <= g.hcc[2];
+}
+
+// kept candidates of every tile of kCandTile (one a thread: few are kept, and a wave's lanes wait for those)
+__global__ __launch_bounds__(kScanThreads) void k_nb_flag(const NbGeom* __restrict__ G,
+                                                          const long long* __restrict__ cand_off, int nstruc,
+                                                          long long ncand, const double* __restrict__ frac,
+                                                          unsigned char* __restrict__ flag, int* __restrict__ sums) {
+    __shared__ int sh[kScanThreads / 64];
+    int n = 0;
+    for (int k = 0; k < kCandItems; ++k) {
+        const long long i = (long long)blockIdx.x * kCandTile + k * kScanThreads + threadIdx.x;
+        const bool keep = i < ncand && kept(G, decode(G, cand_off, nstruc, i), frac);
+        if (i < ncand) flag[i] = keep;
+        n += __popcll(__ballot(keep));
     }
-    flag[i] = keep;
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int w = 0; w < kScanThreads / 64; ++w) t += sh[w];
+        sums[blockIdx.x] = t;
+    }
 }
 
 // cluster arrays and grid box of every kept candidate -- neilist.F90:385-421, 576-588
-__global__ void k_nb_cluster(const NbGeom* __restrict__ G, const long long* __restrict__ cand_off, int nstruc,
-                             long long ncand, const double* __restrict__ frac, const int* __restrict__ flag,
-                             const int* __restrict__ cidx, double invrc, double* __restrict__ cpos,
-                             int* __restrict__ corg, int* __restrict__ cbox, int* __restrict__ cshift,
-                             int* __restrict__ bcount, int* __restrict__ err) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ncand || !flag[i]) return;
+struct ClusterOut {
+    double* pos;
+    int *org, *box, *shift, *slot;  // slot: the atom's place in its box, in no order
+    int *bcount, *err;
+};
+__device__ __forceinline__ void put_cluster(const NbGeom* __restrict__ G, const long long* __restrict__ cand_off,
+                                            int nstruc, long long i, int ci, const double* __restrict__ frac,
+                                            double invrc, const ClusterOut& o) {
     const Cand c = decode(G, cand_off, nstruc, i);
     const NbGeom& g = G[c.s];
-    const int ci = cidx[i];
     double r2[3];
     if (g.periodic) {
         // identity atoms: cell * wrapped fraction; images: cell * (fraction + shift)
@@ -288,39 +331,84 @@ __global__ void k_nb_cluster(const NbGeom* __restrict__ G, const long long* __re
     if (inside)
         box = g.box_off + ((int)gb[0] * g.ng[1] + (int)gb[1]) * g.ng[2] + (int)gb[2];
     else
-        atomicOr(err, kNbErrBox);
-    for (int n = 0; n < 3; ++n) cpos[3 * (size_t)ci + n] = r2[n];
-    cshift[3 * (size_t)ci] = c.k0;
-    cshift[3 * (size_t)ci + 1] = c.k1;
-    cshift[3 * (size_t)ci + 2] = c.k2;
-    corg[ci] = c.a;
-    cbox[ci] = box;
-    if (box >= 0) atomicAdd(&bcount[box], 1);
+        atomicOr(o.err, kNbErrBox);
+    for (int n = 0; n < 3; ++n) o.pos[3 * (size_t)ci + n] = r2[n];
+    o.shift[3 * (size_t)ci] = c.k0;
+    o.shift[3 * (size_t)ci + 1] = c.k1;
+    o.shift[3 * (size_t)ci + 2] = c.k2;
+    o.org[ci] = c.a;
+    o.box[ci] = box;
+    if (box >= 0) o.slot[ci] = atomicAdd(&o.bcount[box], 1);
+}
+
+// sums: candidates kept in every tile, or (scanned) in those before it
+__global__ __launch_bounds__(kScanThreads) void k_nb_cluster(const NbGeom* __restrict__ G,
+                                                             const long long* __restrict__ cand_off, int nstruc,
+                                                             long long ncand, const double* __restrict__ frac,
+                                                             const unsigned char* __restrict__ flag,
+                                                             const int* __restrict__ sums, bool scanned,
+                                                             int* __restrict__ cidx, double invrc, ClusterOut o) {
+    constexpr int NW = kScanThreads / 64;
+    __shared__ int sh[NW * (kCandItems + 1)];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int before = 0;
+    if (!scanned) {
+        for (int t = threadIdx.x; t < (int)blockIdx.x; t += kScanThreads) before += sums[t];
+        for (int k = 32; k > 0; k >>= 1) before += __shfl_xor(before, k, 64);
+    }
+    bool keep[kCandItems];
+    int rank[kCandItems];
+#pragma unroll
+    for (int k = 0; k < kCandItems; ++k) {
+        const long long i = (long long)blockIdx.x * kCandTile + k * kScanThreads + threadIdx.x;
+        keep[k] = i < ncand && flag[i];
+        const unsigned long long m = __ballot(keep[k]);
+        rank[k] = __popcll(m & ((1ull << lane) - 1ull));
+        if (lane == 0) sh[k * NW + w] = __popcll(m);
+    }
+    if (lane == 0) sh[kCandItems * NW + w] = before;
+    __syncthreads();
+    int ci = scanned ? sums[blockIdx.x] : 0;
+    if (!scanned)
+        for (int v = 0; v < NW; ++v) ci += sh[kCandItems * NW + v];
+#pragma unroll
+    for (int k = 0; k < kCandItems; ++k) {
+        const long long i = (long long)blockIdx.x * kCandTile + k * kScanThreads + threadIdx.x;
+        int at = ci + rank[k];
+        for (int v = 0; v < NW; ++v) {
+            if (v < w) at += sh[k * NW + v];
+            ci += sh[k * NW + v];
+        }
+        if (i < ncand) cidx[i] = at;
+        if (keep[k]) put_cluster(G, cand_off, nstruc, i, at, frac, invrc, o);
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) cidx[ncand] = ci;
 }
 
 __global__ void k_nb_bfill(const int* __restrict__ cidx_total, const int* __restrict__ cbox,
-                           const int* __restrict__ bstart, int* __restrict__ bcur, int* __restrict__ batoms) {
+                           const int* __restrict__ slot, const int* __restrict__ bstart, int* __restrict__ bmixed) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= *cidx_total) return;
     const int b = cbox[c];
-    if (b < 0) return;
-    const int slot = atomicAdd(&bcur[b], 1);
-    batoms[bstart[b] + slot] = c;
+    if (b >= 0) bmixed[bstart[b] + slot[c]] = c;
 }
 
-// ascending cluster index inside each box (the reference fills boxes in cluster order)
-__global__ void k_nb_bsort(int nbox, const int* __restrict__ bstart, int* __restrict__ batoms) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+// ascending cluster index inside each box (the reference fills boxes in cluster order): a wave a box, an atom's place
+// is the number of smaller ones (one lane a box moved them one by one: 26 us for 2200 boxes, 4 us here)
+__global__ __launch_bounds__(256) void k_nb_bsort(int nbox, const int* __restrict__ bstart,
+                                                  const int* __restrict__ bmixed, int* __restrict__ batoms) {
+    const int lane = threadIdx.x & 63;
+    const int b = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (b >= nbox) return;
     const int lo = bstart[b], hi = bstart[b + 1];
-    for (int i = lo + 1; i < hi; ++i) {
-        const int v = batoms[i];
-        int j = i - 1;
-        while (j >= lo && batoms[j] > v) {
-            batoms[j + 1] = batoms[j];
-            --j;
+    for (int i0 = lo; i0 < hi; i0 += 64) {
+        const int v = i0 + lane < hi ? bmixed[i0 + lane] : 0;
+        int less = 0;
+        for (int k0 = lo; k0 < hi; k0 += 64) {
+            const int u = k0 == i0 ? v : k0 + lane < hi ? bmixed[k0 + lane] : 0;
+            for (int k = 0; k < min(64, hi - k0); ++k) less += __shfl(u, k, 64) < v;
         }
-        batoms[j + 1] = v;
+        if (i0 + lane < hi) batoms[lo + less] = v;
     }
 }
 
@@ -376,8 +464,35 @@ __global__ __launch_bounds__(256) void k_nb_pairs(const NbGeom* __restrict__ G, 
     const int total = __shfl(incl, 26, 64);
     const double r1x = cpos[3 * (size_t)c1], r1y = cpos[3 * (size_t)c1 + 1], r1z = cpos[3 * (size_t)c1 + 2];
     const double rcsq = rcut * rcut;
-    int base_out = FILL ? out.offsets[a] : 0;
-    int found = 0;
+    const int base_out = FILL ? out.offsets[a] : 0;
+    // FILL: cluster indices of the hits that wait to be written, fewer than 64 and the latest 64
+    __shared__ int wait_all[FILL ? 4 : 1][FILL ? 128 : 1];
+    int* wait = wait_all[FILL ? threadIdx.x >> 6 : 0];
+    auto write = [&](int p, int c2) {
+        const double v0 = cpos[3 * (size_t)c2] - r1x, v1 = cpos[3 * (size_t)c2 + 1] - r1y,
+                     v2 = cpos[3 * (size_t)c2 + 2] - r1z;
+        const double d = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
+        const int j = corg[c2];
+        out.nlist[p] = j;
+        out.dl[p] = d;
+        // the boundary's convention (x_i - x_j)/r is the negated reference eist
+        out.el[3 * (size_t)p] = -(v0 / d);
+        out.el[3 * (size_t)p + 1] = -(v1 / d);
+        out.el[3 * (size_t)p + 2] = -(v2 / d);
+        if (out.shifts)
+            for (int n = 0; n < 3; ++n)
+                out.shifts[3 * (size_t)p + n] = cshift[3 * (size_t)c2 + n] - afl[3 * (size_t)j + n] +
+                                                afl[3 * (size_t)a + n];
+        const double mx = mag[3 * (size_t)j], my = mag[3 * (size_t)j + 1], mz = mag[3 * (size_t)j + 2];
+        const double mm = sqrt(mx * mx + my * my + mz * mz);
+        out.dm[p] = mm;
+        if (mm == 0.0) {
+            out.em[3 * (size_t)p] = 0.0; out.em[3 * (size_t)p + 1] = 0.0; out.em[3 * (size_t)p + 2] = 1.0;
+        } else {
+            out.em[3 * (size_t)p] = mx / mm; out.em[3 * (size_t)p + 1] = my / mm; out.em[3 * (size_t)p + 2] = mz / mm;
+        }
+    };
+    int found = 0, written = 0;
     for (int q0 = 0; q0 < total; q0 += 64) {
         const int q = q0 + lane;
         // largest stencil slot t with pre[t] <= q (empty slots share their successor's start)
@@ -389,46 +504,34 @@ __global__ __launch_bounds__(256) void k_nb_pairs(const NbGeom* __restrict__ G, 
         }
         const int pt = __shfl(pre, t, 64), bt = __shfl(bs, t, 64);
         bool pass = false;
-        double v0 = 0, v1 = 0, v2 = 0;
         int c2 = -1;
         if (q < total) {
             c2 = batoms[bt + (q - pt)];
             if (c2 != c1) {
-                v0 = cpos[3 * (size_t)c2] - r1x;
-                v1 = cpos[3 * (size_t)c2 + 1] - r1y;
-                v2 = cpos[3 * (size_t)c2 + 2] - r1z;
+                const double v0 = cpos[3 * (size_t)c2] - r1x, v1 = cpos[3 * (size_t)c2 + 1] - r1y,
+                             v2 = cpos[3 * (size_t)c2 + 2] - r1z;
                 // fastdist: neilist.F90:825-848
                 if (fabs(v0) < rcut && fabs(v1) < rcut && fabs(v2) < rcut) pass = v0 * v0 + v1 * v1 + v2 * v2 < rcsq;
+                if (pass && fabs(v0) + fabs(v1) + fabs(v2) < kEps) atomicOr(err, kNbErrIdentical);
             }
         }
         const unsigned long long m = __ballot(pass);
-        if (pass) {
-            if (fabs(v0) + fabs(v1) + fabs(v2) < kEps) atomicOr(err, kNbErrIdentical);
-            if (FILL) {
-                const int p = base_out + found + __popcll(m & ((1ull << lane) - 1ull));
-                const double d = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
-                const int j = corg[c2];
-                out.nlist[p] = j;
-                out.dl[p] = d;
-                // the boundary's convention (x_i - x_j)/r is the negated reference eist
-                out.el[3 * (size_t)p] = -(v0 / d);
-                out.el[3 * (size_t)p + 1] = -(v1 / d);
-                out.el[3 * (size_t)p + 2] = -(v2 / d);
-                if (out.shifts)
-                    for (int n = 0; n < 3; ++n)
-                        out.shifts[3 * (size_t)p + n] = cshift[3 * (size_t)c2 + n] - afl[3 * (size_t)j + n] +
-                                                        afl[3 * (size_t)a + n];
-                const double mx = mag[3 * (size_t)j], my = mag[3 * (size_t)j + 1], mz = mag[3 * (size_t)j + 2];
-                const double mm = sqrt(mx * mx + my * my + mz * mz);
-                out.dm[p] = mm;
-                if (mm == 0.0) {
-                    out.em[3 * (size_t)p] = 0.0; out.em[3 * (size_t)p + 1] = 0.0; out.em[3 * (size_t)p + 2] = 1.0;
-                } else {
-                    out.em[3 * (size_t)p] = mx / mm; out.em[3 * (size_t)p + 1] = my / mm; out.em[3 * (size_t)p + 2] = mz / mm;
-                }
+        if (FILL) {
+            if (pass) wait[found - written + __popcll(m & ((1ull << lane) - 1ull))] = c2;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (found - written + __popcll(m) >= 64) {
+                write(base_out + written + lane, wait[lane]);
+                const int next = wait[64 + lane];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                wait[lane] = next;
+                written += 64;
             }
         }
         found += __popcll(m);
+    }
+    if (FILL) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (lane < found - written) write(base_out + written + lane, wait[lane]);
     }
     if (lane == 0) {
         if (!FILL) {
@@ -447,11 +550,15 @@ __global__ __launch_bounds__(256) void k_nb_pairs(const NbGeom* __restrict__ G, 
     }
 }
 
-__global__ void k_nb_gather_clusters(int nstruc, const NbGeom* __restrict__ G, const int* __restrict__ cidx,
-                                     long long ncand, int* __restrict__ out) {
+// totals for the host: pairs, errors, clusters before every structure
+__global__ void k_nb_tail(int nstruc, const NbGeom* __restrict__ G, const int* __restrict__ cidx, long long ncand,
+                          const int* __restrict__ npairs, const int* __restrict__ err, int* __restrict__ tail) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s > nstruc) return;
-    out[s] = cidx[s < nstruc ? G[s].cand_off : ncand];
+    if (s == 0) {
+        tail[0] = *npairs;
+        tail[1] = *err;
+    }
+    if (s <= nstruc) tail[2 + s] = cidx[s < nstruc ? G[s].cand_off : ncand];
 }
 
 // ---------------------------------------------------------------- host side
@@ -468,13 +575,23 @@ bool grow(T*& p, size_t& cap, size_t n) {
     return true;
 }
 
+template <typename T>
+bool grow_host(T*& p, size_t& cap, size_t n) {
+    if (n <= cap && p) return true;
+    if (p) (void)hipHostFree((void*)p);
+    p = nullptr;
+    cap = 0;
+    const size_t want = n + n / 4 + 64;
+    if (hipHostMalloc((void**)&p, want * sizeof(T)) != hipSuccess) return false;
+    cap = want;
+    return true;
+}
+
 struct NbWork {
-    NbGeom* geom = nullptr; size_t c_geom = 0;
-    long long* cand_off = nullptr; size_t c_cand_off = 0;
-    int* atom_off = nullptr; size_t c_atom_off = 0;
+    unsigned char* geom = nullptr; size_t c_geom = 0;  // NbGeom [S], first candidates [S + 1], first atoms [S + 1]
     double* frac = nullptr; size_t c_frac = 0;
     double* bbox = nullptr; size_t c_bbox = 0;
-    int* flag = nullptr; size_t c_flag = 0;
+    unsigned char* flag = nullptr; size_t c_flag = 0;
     int* cidx = nullptr; size_t c_cidx = 0;
     double* cpos = nullptr; size_t c_cpos = 0;
     int* corg = nullptr; size_t c_corg = 0;
@@ -483,12 +600,15 @@ struct NbWork {
     int* afl = nullptr; size_t c_afl = 0;
     int* bcount = nullptr; size_t c_bcount = 0;
     int* bstart = nullptr; size_t c_bstart = 0;
-    int* bcur = nullptr; size_t c_bcur = 0;
+    int* slot = nullptr; size_t c_slot = 0;
+    int* bmixed = nullptr; size_t c_bmixed = 0;
     int* batoms = nullptr; size_t c_batoms = 0;
     int* counts = nullptr; size_t c_counts = 0;
     int* sums = nullptr; size_t c_sums = 0;
     int* err = nullptr; size_t c_err = 0;
-    int* clus = nullptr; size_t c_clus = 0;
+    // host memory that the device reaches: the geometry on its way there, the totals on theirs
+    unsigned char* h_geom = nullptr; size_t c_h_geom = 0;
+    int* h_tail = nullptr; size_t c_h_tail = 0;
     // staging for the host-pointer entry point
     double *pos = nullptr, *mag = nullptr; size_t c_pos = 0, c_mag = 0;
     int *off = nullptr, *nl = nullptr; size_t c_off = 0, c_nl = 0;
@@ -518,10 +638,21 @@ int fail_hip(hipError_t e, const char* what) {
             return fail_hip(hipErrorOutOfMemory, "neighbour workspace " #ptr);     \
     } while (0)
 
+#define NBHOST(ptr, n)                                                            \
+    do {                                                                          \
+        if (!grow_host(g_nb.ptr, g_nb.c_##ptr, (size_t)(n)))                       \
+            return fail_hip(hipErrorOutOfMemory, "neighbour workspace " #ptr);     \
+    } while (0)
+
 unsigned nblocks(long long n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
 // out[0..n] = exclusive scan of in[0..n-1], out[n] = total
 int scan(const int* in, long long n, int* out, hipStream_t s) {
+    if (n <= kScanEach) {
+        k_scan_each<<<(unsigned)std::max(1ll, (n + kScanTile - 1) / kScanTile), kScanThreads, 0, s>>>(in, (int)n, out);
+        NBCHK(hipGetLastError());
+        return 0;
+    }
     const long long ntiles = (n + kScanTile - 1) / kScanTile;
     if (ntiles > (1ll << 30)) {
         report_error(MAGACE_ERR_INPUT, "neighbour build: array too large to scan");
@@ -619,7 +750,8 @@ struct Request {
     hipStream_t s;
 };
 
-int build(const Request& R) {
+// queued: work that reads the host's copy of the geometry may be on the stream
+int build_queued(const Request& R, bool& queued) {
     if (!(R.rcut >= 1.0e-6 && R.rcut <= 100.0)) {  // neilist.F90:206-213
         report_error(MAGACE_ERR_INPUT, R.rcut < 1.0e-6 ? "value for rcut to small." : "value for rcut to large.");
         return MAGACE_ERR_INPUT;
@@ -661,16 +793,21 @@ int build(const Request& R) {
         return MAGACE_ERR_INPUT;
     }
     hipStream_t s = R.s;
-    NBGROW(geom, S + 1);
-    NBGROW(atom_off, S + 1);
-    NBGROW(cand_off, S + 1);
+    const size_t at_cand = sizeof(NbGeom) * S, at_atom = at_cand + sizeof(long long) * (S + 1),
+                 geom_bytes = at_atom + sizeof(int) * (S + 1);
+    NBGROW(geom, geom_bytes);
+    NBHOST(h_geom, geom_bytes);
+    NBHOST(h_tail, S + 3);
     NBGROW(err, 4);
+    NbGeom* const d_geom = (NbGeom*)g_nb.geom;
+    const long long* const d_cand = (const long long*)(g_nb.geom + at_cand);
+    const int* const d_atom = (const int*)(g_nb.geom + at_atom);
     std::vector<double> bbox;
     if (any_open) {
         // open clusters: the grid spans their bounding box (neilist.F90:313-352)
         NBGROW(bbox, 6 * (size_t)S);
-        NBCHK(hipMemcpyAsync(g_nb.geom, hg.data(), sizeof(NbGeom) * S, hipMemcpyHostToDevice, s));
-        k_nb_bbox<<<S, 256, 0, s>>>(g_nb.geom, R.pos, g_nb.bbox);
+        NBCHK(hipMemcpyAsync(d_geom, hg.data(), sizeof(NbGeom) * S, hipMemcpyHostToDevice, s));
+        k_nb_bbox<<<S, 256, 0, s>>>(d_geom, R.pos, g_nb.bbox);
         NBCHK(hipGetLastError());
         bbox.resize(6 * (size_t)S);
         NBCHK(hipMemcpyAsync(bbox.data(), g_nb.bbox, sizeof(double) * 6 * S, hipMemcpyDeviceToHost, s));
@@ -730,52 +867,52 @@ int build(const Request& R) {
     NBGROW(afl, 3 * (size_t)ntot + 1);
     NBGROW(bcount, nbox + 1);
     NBGROW(bstart, nbox + 1);
-    NBGROW(bcur, nbox + 1);
+    NBGROW(slot, ncand + 1);
+    NBGROW(bmixed, ncand + 1);
     NBGROW(batoms, ncand + 1);
     NBGROW(counts, ntot + 1);
-    NBGROW(clus, S + 1);
-    NBCHK(hipMemcpyAsync(g_nb.geom, hg.data(), sizeof(NbGeom) * S, hipMemcpyHostToDevice, s));
-    NBCHK(hipMemcpyAsync(g_nb.atom_off, ha.data(), sizeof(int) * (S + 1), hipMemcpyHostToDevice, s));
-    NBCHK(hipMemcpyAsync(g_nb.cand_off, hc.data(), sizeof(long long) * (S + 1), hipMemcpyHostToDevice, s));
-    k_fill_int<<<1, 64, 0, s>>>(g_nb.err, 1, 0);
-    if (nbox > 0) {
-        k_fill_int<<<nblocks(nbox, 256), 256, 0, s>>>(g_nb.bcount, nbox, 0);
-        k_fill_int<<<nblocks(nbox, 256), 256, 0, s>>>(g_nb.bcur, nbox, 0);
-    }
-    if (ntot > 0)
-        k_nb_frac<<<nblocks(ntot, 256), 256, 0, s>>>(g_nb.geom, g_nb.atom_off, S, (int)ntot, R.pos, g_nb.frac,
-                                                      g_nb.afl);
-    if (ncand > 0)
-        k_nb_flag<<<nblocks(ncand, 256), 256, 0, s>>>(g_nb.geom, g_nb.cand_off, S, ncand, g_nb.frac, g_nb.flag);
+    std::memcpy(g_nb.h_geom, hg.data(), sizeof(NbGeom) * S);
+    std::memcpy(g_nb.h_geom + at_cand, hc.data(), sizeof(long long) * (S + 1));
+    std::memcpy(g_nb.h_geom + at_atom, ha.data(), sizeof(int) * (S + 1));
+    const long long ntiles = (ncand + kCandTile - 1) / kCandTile;
+    NBGROW(sums, ntiles + 1);
+    queued = true;
+    NBCHK(hipMemcpyAsync(g_nb.geom, g_nb.h_geom, geom_bytes, hipMemcpyHostToDevice, s));
+    k_nb_frac<<<nblocks(std::max(std::max(ntot, nbox), 1ll), 256), 256, 0, s>>>(d_geom, d_atom, S, (int)ntot, R.pos, g_nb.frac,
+                                                                       g_nb.afl, (int)nbox, g_nb.bcount, g_nb.err);
     NBCHK(hipGetLastError());
-    if (int rc = scan(g_nb.flag, ncand, g_nb.cidx, s)) return rc;
     const double invrc = 1.0 / R.rcut;
-    if (ncand > 0)
-        k_nb_cluster<<<nblocks(ncand, 256), 256, 0, s>>>(g_nb.geom, g_nb.cand_off, S, ncand, g_nb.frac, g_nb.flag,
-                                                         g_nb.cidx, invrc, g_nb.cpos, g_nb.corg, g_nb.cbox,
-                                                         g_nb.cshift, g_nb.bcount, g_nb.err);
-    NBCHK(hipGetLastError());
+    if (ncand > 0) {
+        k_nb_flag<<<(unsigned)ntiles, kScanThreads, 0, s>>>(d_geom, d_cand, S, ncand, g_nb.frac, g_nb.flag, g_nb.sums);
+        // every tile adds up those before it unless they are many
+        const bool scanned = ntiles > kTilesAdded;
+        if (scanned) k_scan_sums<<<1, kScanThreads, 0, s>>>(g_nb.sums, (int)ntiles, g_nb.cidx, ncand);
+        k_nb_cluster<<<(unsigned)ntiles, kScanThreads, 0, s>>>(
+            d_geom, d_cand, S, ncand, g_nb.frac, g_nb.flag, g_nb.sums, scanned, g_nb.cidx, invrc,
+            ClusterOut{g_nb.cpos, g_nb.corg, g_nb.cbox, g_nb.cshift, g_nb.slot, g_nb.bcount, g_nb.err});
+        NBCHK(hipGetLastError());
+    } else if (int rc = scan(nullptr, 0, g_nb.cidx, s)) {
+        return rc;
+    }
     if (int rc = scan(g_nb.bcount, nbox, g_nb.bstart, s)) return rc;
     if (ncand > 0)
-        k_nb_bfill<<<nblocks(ncand, 256), 256, 0, s>>>(g_nb.cidx + ncand, g_nb.cbox, g_nb.bstart, g_nb.bcur,
-                                                       g_nb.batoms);
-    if (nbox > 0) k_nb_bsort<<<nblocks(nbox, 256), 256, 0, s>>>((int)nbox, g_nb.bstart, g_nb.batoms);
+        k_nb_bfill<<<nblocks(ncand, 256), 256, 0, s>>>(g_nb.cidx + ncand, g_nb.cbox, g_nb.slot, g_nb.bstart,
+                                                       g_nb.bmixed);
+    if (nbox > 0)
+        k_nb_bsort<<<nblocks(nbox, 4), 256, 0, s>>>((int)nbox, g_nb.bstart, g_nb.bmixed, g_nb.batoms);
     PairOut none{};
     if (ntot > 0)
-        k_nb_pairs<false><<<nblocks(ntot, 4), 256, 0, s>>>(g_nb.geom, g_nb.atom_off, S, (int)ntot, g_nb.cidx,
+        k_nb_pairs<false><<<nblocks(ntot, 4), 256, 0, s>>>(d_geom, d_atom, S, (int)ntot, g_nb.cidx,
                                                             g_nb.cpos, g_nb.corg, g_nb.cbox, g_nb.bstart,
                                                             g_nb.batoms, R.mag, g_nb.cshift, g_nb.afl, R.rcut,
                                                             g_nb.counts, none, g_nb.err);
     NBCHK(hipGetLastError());
     if (int rc = scan(g_nb.counts, ntot, R.offsets, s)) return rc;
-    k_nb_gather_clusters<<<nblocks(S + 1, 64), 64, 0, s>>>(S, g_nb.geom, g_nb.cidx, ncand, g_nb.clus);
+    k_nb_tail<<<nblocks(S + 1, 64), 64, 0, s>>>(S, d_geom, g_nb.cidx, ncand, R.offsets + ntot, g_nb.err, g_nb.h_tail);
     NBCHK(hipGetLastError());
-    int tail[2] = {0, 0};
-    std::vector<int> clus(S + 1);
-    NBCHK(hipMemcpyAsync(&tail[0], R.offsets + ntot, sizeof(int), hipMemcpyDeviceToHost, s));
-    NBCHK(hipMemcpyAsync(&tail[1], g_nb.err, sizeof(int), hipMemcpyDeviceToHost, s));
-    NBCHK(hipMemcpyAsync(clus.data(), g_nb.clus, sizeof(int) * (S + 1), hipMemcpyDeviceToHost, s));
+    queued = false;
     NBCHK(hipStreamSynchronize(s));
+    const int *tail = g_nb.h_tail, *clus = tail + 2;
     if (tail[1] & kNbErrBox) {
         report_error(MAGACE_ERR_INPUT, "neighbour build: atom outside the grid (non-finite position?)");
         return MAGACE_ERR_INPUT;
@@ -796,13 +933,20 @@ int build(const Request& R) {
     if (ntot > 0) {
         PairOut o = R.out;
         o.offsets = R.offsets;
-        k_nb_pairs<true><<<nblocks(ntot, 4), 256, 0, s>>>(g_nb.geom, g_nb.atom_off, S, (int)ntot, g_nb.cidx,
+        k_nb_pairs<true><<<nblocks(ntot, 4), 256, 0, s>>>(d_geom, d_atom, S, (int)ntot, g_nb.cidx,
                                                            g_nb.cpos, g_nb.corg, g_nb.cbox, g_nb.bstart,
                                                            g_nb.batoms, R.mag, g_nb.cshift, g_nb.afl, R.rcut,
                                                            g_nb.counts, o, g_nb.err);
         NBCHK(hipGetLastError());
     }
     return 0;
+}
+
+int build(const Request& R) {
+    bool queued = false;
+    const int rc = build_queued(R, queued);
+    if (queued) (void)hipStreamSynchronize(R.s);  // an error in between
+    return rc;
 }
 
 }  // namespace
