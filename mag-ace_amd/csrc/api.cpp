@@ -107,7 +107,7 @@ struct Context {
     NodeTab<double> n64;
     NodeTab<float> n32;
     NodeWeights node_w;
-    std::vector<void*> node_mem;
+    std::vector<void*> node_mem, fit_mem;  // fit_mem: the fitting plan's arrays (FitBuffers::plan)
     double* d_w = nullptr;
     bool records_stale = true;  // the gradient records on the device are not those of the coefficients
     Buffers buf;
@@ -209,7 +209,8 @@ Context::~Context() {
     dfree(buf.Z); dfree(buf.W); dfree(buf.ehc); dfree(buf.rho1); dfree(buf.dE); dfree(buf.edf); dfree(buf.rho);
     dfree(buf.Pt);
     dfree(buf.err);
-    dfree(fit.Zdot); dfree(fit.ehc_dot); dfree(fit.alpha); dfree(fit.beta); dfree(fit.M); dfree(fit.idx);
+    dfree(fit.Zdot); dfree(fit.ehc_dot); dfree(fit.alpha); dfree(fit.beta); dfree(fit.M);
+    for (void*& p : fit_mem) dfree(p);
     dfree(fit.ub_ptr); dfree(fit.ub_t); dfree(fit.ub_u); dfree(fit.Wd);
     dfree(f_fl); dfree(f_tl); dfree(f_t0); dfree(f_eout);
     for (auto& sl : slots) {
@@ -537,20 +538,42 @@ int upload_node_weights(Context& c) {
     return 0;
 }
 
+// device memory that `kept` frees, and a copy of v in it
+template <typename D>
+int alloc_kept(std::vector<void*>& kept, D*& dst, size_t bytes) {
+    void* p = nullptr;
+    HIPCHK(hipMalloc(&p, bytes + 64));
+    kept.push_back(p);
+    dst = (D*)p;
+    return 0;
+}
+template <typename D, typename V>
+int upload_kept(std::vector<void*>& kept, D*& dst, const V& v) {
+    if (int rc = alloc_kept(kept, dst, v.size() * sizeof(v[0]))) return rc;
+    if (!v.empty()) HIPCHK(hipMemcpy((void*)dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
+    return 0;
+}
+
+// the fitting plan, built when a fit asks for its first gradient
+int upload_fit_plan(Context& c) {
+    const FitPlan F = build_fit_plan(c.model.z, c.model.terms);
+    FitTab& D = c.fit.plan;
+    D.groups = F.groups;
+    D.slots = F.slots;
+    D.most = (F.tiles + kFitWaves - 1) / kFitWaves;
+    int rc = upload_kept(c.fit_mem, D.head, F.head);
+    if (!rc) rc = upload_kept(c.fit_mem, D.entry, F.entry);
+    if (!rc) rc = upload_kept(c.fit_mem, D.prod, F.prod);
+    if (!rc) rc = upload_kept(c.fit_mem, D.node, F.node);
+    if (!rc) rc = upload_kept(c.fit_mem, D.place, F.place);
+    if (!rc) rc = upload_kept(c.fit_mem, D.t, F.t);
+    return rc;
+}
+
 // the node plan's tables
 int upload_nodes(Context& c) {
-    auto alloc = [&](auto*& dst, size_t bytes) -> int {
-        void* p = nullptr;
-        HIPCHK(hipMalloc(&p, bytes + 64));
-        c.node_mem.push_back(p);
-        dst = (std::remove_reference_t<decltype(dst)>)p;
-        return 0;
-    };
-    auto up = [&](auto*& dst, const auto& v) -> int {
-        if (int rc = alloc(dst, v.size() * sizeof(v[0]))) return rc;
-        if (!v.empty()) HIPCHK(hipMemcpy((void*)dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice));
-        return 0;
-    };
+    auto alloc = [&](auto*& dst, size_t bytes) { return alloc_kept(c.node_mem, dst, bytes); };
+    auto up = [&](auto*& dst, const auto& v) { return upload_kept(c.node_mem, dst, v); };
     // `n` steps of a lane side by side
     auto grouped = [](const auto& v, size_t n) {
         auto o = v;
@@ -1659,16 +1682,15 @@ int magace_fit_backward(int natom, int nei, const int* offsets, const int* nlist
     const TermList& T = c.model.terms;
     FitBuffers& F = c.fit;
     const size_t nd = (size_t)c.model.pot.h.ndensity;
-    if (!F.idx) {
-        HIPCHK(hipMalloc((void**)&F.idx, T.idx.size() * sizeof(uint16_t) + 64));
-        HIPCHK(hipMemcpy(F.idx, T.idx.data(), T.idx.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+    if (!F.M) {
+        if (int rc = upload_fit_plan(c)) return rc;
         HIPCHK(hipMalloc((void**)&F.ub_ptr, T.ub_ptr.size() * sizeof(int32_t) + 64));
         HIPCHK(hipMalloc((void**)&F.ub_t, T.ub_t.size() * sizeof(int32_t) + 64));
         HIPCHK(hipMalloc((void**)&F.ub_u, T.ub_u.size() * sizeof(double) + 64));
         HIPCHK(hipMemcpy(F.ub_ptr, T.ub_ptr.data(), T.ub_ptr.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(F.ub_t, T.ub_t.data(), T.ub_t.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(F.ub_u, T.ub_u.data(), T.ub_u.size() * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(hipMalloc((void**)&F.M, 2 * T.nterms() * nd * sizeof(double) + 64));
+        HIPCHK(hipMalloc((void**)&F.M, T.nterms() * nd * sizeof(double) + 64));
     }
     if ((size_t)natom > F.cap_atoms) {
         dfree(F.Zdot); dfree(F.ehc_dot); dfree(F.alpha); dfree(F.beta);

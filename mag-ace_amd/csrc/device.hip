@@ -1290,95 +1290,6 @@ __global__ void __launch_bounds__(256) k_fit_atom(DevParams<double> P, bool scal
     }
 }
 
-// M_{t,d} += sum_i alpha_{i,d} P_t,i + beta_{i,d} D_u P_t,i over a chunk of atoms (Z, Zdot of one
-// atom in LDS at a time); each thread owns kFitMpt monomials so that an atom's Z and Zdot are
-// staged once per kFitMpt * 256 monomials; grid = (monomial tiles, atom chunks); M is
-// [ND][nterms] complex
-constexpr int kFitMpt = 8;
-template <int ND>
-__global__ void __launch_bounds__(256) k_fit_accum(int nterms, int nz, const unsigned short* __restrict__ zmap, int ny,
-                                                  const int2* __restrict__ ypair,
-                                                  const ushort4* __restrict__ idx,
-                                                  const cplx<double>* __restrict__ Z,
-                                                  const cplx<double>* __restrict__ Zdot,
-                                                  const double* __restrict__ alpha, const double* __restrict__ beta,
-                                                  int natom, int chunk, double* __restrict__ M) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int nzx = nz + 1 + ny;              // Z' = [Z | 1 | Y] as in the adjoint
-    cplx<double>* sZ = (cplx<double>*)smem;  // [nzx]
-    cplx<double>* sD = sZ + nzx;              // [nzx]
-    const int t0 = blockIdx.x * blockDim.x * kFitMpt + threadIdx.x;
-    ushort4 ix[kFitMpt];
-    double accr[ND][kFitMpt], acci[ND][kFitMpt];
-#pragma unroll
-    for (int j = 0; j < kFitMpt; ++j) {
-        const int t = t0 + j * blockDim.x;
-        ix[j] = t < nterms ? idx[t] : ushort4{0, 0, 0, 0};
-#pragma unroll
-        for (int d = 0; d < ND; ++d) accr[d][j] = acci[d][j] = 0.0;
-    }
-    const int a0 = blockIdx.y * chunk, a1 = min(natom, a0 + chunk);
-    for (int a = a0; a < a1; ++a) {
-        __syncthreads();
-        for (int x = threadIdx.x; x < nz; x += blockDim.x) {
-            sZ[x] = full_entry(Z + (size_t)a * nz, zmap[x]);
-            sD[x] = full_entry(Zdot + (size_t)a * nz, zmap[x]);
-        }
-        if (threadIdx.x == 0) {
-            sZ[nz] = {1, 0};
-            sD[nz] = {0, 0};
-        }
-        if (ny > 0) {  // Y = Z[a] Z[b], D_u Y = D_u Z[a] Z[b] + Z[a] D_u Z[b]
-            __syncthreads();
-            for (int i = threadIdx.x; i < ny; i += blockDim.x) {
-                const int2 pr = ypair[i];
-                const cplx<double> za = sZ[pr.x], zb = sZ[pr.y];
-                sZ[nz + 1 + i] = cmul(za, zb);
-                cplx<double> d = cmul(sD[pr.x], zb);
-                cfma(d, za, sD[pr.y]);
-                sD[nz + 1 + i] = d;
-            }
-        }
-        __syncthreads();
-        double al[ND], be[ND];
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            al[d] = alpha[(size_t)a * ND + d];
-            be[d] = beta[(size_t)a * ND + d];
-        }
-#pragma unroll
-        for (int j = 0; j < kFitMpt; ++j) {
-            if (t0 + j * (int)blockDim.x >= nterms) break;
-            const cplx<double> z0 = sZ[ix[j].x], z1 = sZ[ix[j].y], z2 = sZ[ix[j].z], z3 = sZ[ix[j].w];
-            const cplx<double> d0 = sD[ix[j].x], d1 = sD[ix[j].y], d2 = sD[ix[j].z], d3 = sD[ix[j].w];
-            const cplx<double> z01 = cmul(z0, z1), z23 = cmul(z2, z3);
-            const cplx<double> Pt = cmul(z01, z23);
-            // product rule: d(z0 z1 z2 z3) = (d0 z1 + z0 d1) z23 + z01 (d2 z3 + z2 d3)
-            cplx<double> l = cmul(d0, z1), r = cmul(d2, z3);
-            cfma(l, z0, d1);
-            cfma(r, z2, d3);
-            cplx<double> Pd = cmul(l, z23);
-            cfma(Pd, z01, r);
-#pragma unroll
-            for (int d = 0; d < ND; ++d) {
-                accr[d][j] += al[d] * Pt.re + be[d] * Pd.re;
-                acci[d][j] += al[d] * Pt.im + be[d] * Pd.im;
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kFitMpt; ++j) {
-        const int t = t0 + j * blockDim.x;
-        if (t < nterms) {
-#pragma unroll
-            for (int d = 0; d < ND; ++d) {
-                atomicAdd(&M[2 * ((size_t)d * nterms + t)], accr[d][j]);
-                atomicAdd(&M[2 * ((size_t)d * nterms + t) + 1], acci[d][j]);
-            }
-        }
-    }
-}
-
 // gradient of the B1 coefficients: grad[d * nb_m + n] = sum_i alpha_{i,d} (g^m_n(mu_i) - 1)
 __global__ void k_fit_b1(DevParams<double> P, int natom, int nd, const double* __restrict__ dmomi,
                          const double* __restrict__ alpha, double* __restrict__ grad, int* err) {
@@ -1395,7 +1306,7 @@ __global__ void k_fit_b1(DevParams<double> P, int natom, int nd, const double* _
 }
 
 // gradient of the coefficients of orders 2..6: function k of the concatenated list (nb.n[0]
-// functions of order 2, ..., nb.n[4] of order 6), density d: Re sum_t u_{k,t} M_{t,d}, stored at
+// functions of order 2, ..., nb.n[4] of order 6), density d: sum_t u_{k,t} M_{t,d}, stored at
 // grad[nd * (functions of lower orders) + d * nb.n[o] + j] (the file's order: per body order,
 // density-major); grid.y = density
 struct OrderCounts {
@@ -1407,9 +1318,9 @@ __global__ void k_fit_grad(int nterms, OrderCounts nb, const int* __restrict__ p
     int lower = 0, o = 0;
     while (o < 5 && k >= lower + nb.n[o]) lower += nb.n[o++];
     if (o == 5) return;
-    const double* Md = M + 2 * (size_t)d * nterms;
+    const double* Md = M + (size_t)d * nterms;
     double s = 0.0;
-    for (int e = ptr[k]; e < ptr[k + 1]; ++e) s += uu[e] * Md[2 * (size_t)tt[e]];
+    for (int e = ptr[k]; e < ptr[k + 1]; ++e) s += uu[e] * Md[tt[e]];
     grad[nd * lower + d * nb.n[o] + (k - lower)] = s;
 }
 
@@ -1468,36 +1379,11 @@ hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int na
     else
         hipLaunchKernelGGL(k_fit_atom<1>, dim3(natom), dim3(256), 0, s, P, scaled, (const cplx<double>*)B.W,
                            (const cplx<double>*)F.Zdot, B.rho, B.ehc, F.ehc_dot, atom_struct, gE, F.alpha, F.beta);
-    const size_t nM = 2 * (size_t)nterms * nd;
+    const size_t nM = (size_t)nterms * nd;
     hipLaunchKernelGGL(k_fill_double, dim3((unsigned)((nM + 255) / 256)), dim3(256), 0, s, F.M, nM);
     const size_t ng = ((size_t)P.nb_m + nb234) * nd;
     hipLaunchKernelGGL(k_fill_double, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, s, grad, ng);
-    const int chunk = 64;
-    const size_t lds = 2 * (size_t)P.nzx * sizeof(cplx<double>);
-    {
-        // Z' and its derivative of one atom in LDS: beyond the default dynamic limit for long
-        // feature vectors
-        static bool set[2] = {false, false};
-        const void* k = nd == 2 ? (const void*)k_fit_accum<2> : (const void*)k_fit_accum<1>;
-        if (!set[nd - 1]) {
-            int dev = 0, maxsh = 0;
-            if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-            if ((e = hipDeviceGetAttribute(&maxsh, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) != hipSuccess)
-                return e;
-            if ((e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, maxsh)) != hipSuccess)
-                return e;
-            set[nd - 1] = true;
-        }
-    }
-    dim3 grid((unsigned)((nterms + 256 * kFitMpt - 1) / (256 * kFitMpt)), (unsigned)((natom + chunk - 1) / chunk));
-    if (nd == 2)
-        hipLaunchKernelGGL(k_fit_accum<2>, grid, dim3(256), lds, s, nterms, P.nz, P.zmap, P.ny, P.ypair, (const ushort4*)F.idx,
-                           (const cplx<double>*)B.Z, (const cplx<double>*)F.Zdot, F.alpha, F.beta, natom, chunk,
-                           F.M);
-    else
-        hipLaunchKernelGGL(k_fit_accum<1>, grid, dim3(256), lds, s, nterms, P.nz, P.zmap, P.ny, P.ypair, (const ushort4*)F.idx,
-                           (const cplx<double>*)B.Z, (const cplx<double>*)F.Zdot, F.alpha, F.beta, natom, chunk,
-                           F.M);
+    if ((e = fit_accumulate(F.plan, P.nz, nterms, nd, natom, B.Z, F.Zdot, F.alpha, F.beta, F.M, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_fit_b1, dim3((natom + 255) / 256), dim3(256), 0, s, P, natom, nd, dmomi, F.alpha, grad,
                        B.err);
     if (nb234 > 0)

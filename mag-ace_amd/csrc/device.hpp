@@ -171,15 +171,27 @@ struct Launch {
                           int nm3_class, hipEvent_t* ev, int dvar = -1, bool acc = false);
 };
 
+// FitPlan on the device (fit.hip)
+struct FitTab {
+    int groups = 0, slots = 0, most = 0;  // most: tiles of a wave
+    const int* head = nullptr;
+    const unsigned short* entry = nullptr;
+    const uint32_t *prod = nullptr, *node = nullptr, *place = nullptr;
+    const int4* t = nullptr;
+};
+// M[d][t] += sum_i alpha_{i,d} Re P_{t,i} + beta_{i,d} Re D_u P_{t,i}
+hipError_t fit_accumulate(const FitTab& F, int nz, int nterms, int nd, int natom, const void* Z, const void* Zdot,
+                          const double* alpha, const double* beta, double* M, hipStream_t s);
+
 // fitting (FP64): forward-mode density, per-atom adjoint scalars, monomial accumulation
 struct FitBuffers {
     void* Zdot = nullptr;        // [natom][nz] complex
     double* ehc_dot = nullptr;   // [natom]
     double* alpha = nullptr;     // [natom][nd]
     double* beta = nullptr;      // [natom][nd]
-    double* M = nullptr;         // [nd][nterms] complex
+    double* M = nullptr;         // [nd][nterms], real parts
     void* Wd = nullptr;          // [natom][2][nz] complex: per-density dRho/dZ (two densities)
-    unsigned short* idx = nullptr;  // [nterms][4] monomial factors
+    FitTab plan;                 // its arrays belong to the context
     int *ub_ptr = nullptr, *ub_t = nullptr;
     double* ub_u = nullptr;
     size_t cap_atoms = 0;
@@ -205,9 +217,6 @@ template <typename T>
 hipError_t run_forces(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
                       const double* dmomi, const double* emomi, const double* dmom, const double* emom, const Buffers& B,
                       bool scaled, double* flist, double* tlist, double* tlist0, hipStream_t s);
-// row of a 16x16x4 product's result in register r of lane group g, by the size of a value (matrix.hpp)
-inline int matrix_row(size_t bytes, int g, int r) { return bytes == 4 ? 4 * g + r : g + 4 * r; }
-
 hipError_t upload_legendre_constants();
 hipError_t clear_flags(int* p, hipStream_t s);
 int supported_nm3_class(int nm3, int nr2m, int nb_a, int l3a, int l2m, int nr3a);

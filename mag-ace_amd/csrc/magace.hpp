@@ -184,6 +184,23 @@ struct NodePlan {
     std::vector<int32_t> d_x, d_t;   // [kd][A0 entries][8]: A2 entry (ZLayout::half), monomial * 2 or -1
 };
 
+// The plan of the gradient in the coefficients (nodes.cpp, fit.hip): tiles of 16 pair products p (A0 entry times another
+// factor) by 16 pair products q, in groups that a workgroup has in LDS slots [entries of Z | 1 | products Y | p | q].
+constexpr int kFitWaves = 8, kFitTiles = 6;  // waves of a workgroup, tiles of a wave at most
+constexpr int kFitSlots = 2400;              // slots of a group (32 bytes each) unless one tile needs more
+constexpr int kFitEntries = 1024, kFitNodes = 1024, kFitProducts = 512;  // of a group at most (two, two and one a thread)
+constexpr int kFitHead = 12;
+struct FitPlan {
+    int groups = 0, slots = 0, tiles = 0;  // slots and tiles: of the largest group
+    // [groups][kFitHead]: first and number of the group's entries, of its products Y, first of its nodes, number of
+    // nodes p, of all nodes, first and number of its tiles
+    std::vector<int32_t> head;
+    std::vector<uint16_t> entry;   // ZLayout::half
+    std::vector<uint32_t> prod, node;  // slots of the two factors
+    std::vector<uint32_t> place;   // [tiles][64]: slots of node p and node q of row and column lane % 16
+    std::vector<int32_t> t;        // [tiles][64][4]: monomial * 2 + (1: minus) of a lane's results, -1: none
+};
+
 // Spline tables in node-major layout: row n holds [4 coeffs] for every function family.
 struct Splines {
     int nlut = 10000;                    // src/radial.F90:43
@@ -234,6 +251,9 @@ TermList build_terms(const Potential& pot, const ZLayout& z);
 // nodes.cpp: the adjoint's plan; not ok for monomials of other forms (body orders 5, 6), two densities,
 // or more than entry_limit LDS slots
 NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit);
+FitPlan build_fit_plan(const ZLayout& z, const TermList& T);
+// row of a 16x16x4 product's result in register r of lane group g, by the size of a value (matrix.hpp)
+inline int matrix_row(size_t bytes, int g, int r) { return bytes == 4 ? 4 * g + r : g + 4 * r; }
 // splines.cpp
 void radial_basis(int radtype, double lambda, int nb, double cut, double dcut, double r,
                   double* g, double* dg);

@@ -71,14 +71,15 @@ struct Row {
     std::vector<Entry> e;
 };
 
-// rows -> blocks of up to four rows with as many common columns as possible
-struct Block {
-    int slot[4] = {-1, -1, -1, -1};
+// rows -> blocks of up to G rows with as many common columns as possible
+template <int G> struct BlockOf {
+    std::array<int, G> slot;
     std::vector<int> col;
-    std::vector<std::array<int, 4>> t;  // monomial * 2 + minus, -1: none
+    std::vector<std::array<int, G>> t;  // monomial * 2 + minus, -1: none
 };
+using Block = BlockOf<4>;
 
-std::vector<Block> make_blocks(const std::vector<Row>& rows, int nslots) {
+template <int G> std::vector<BlockOf<G>> make_blocks(const std::vector<Row>& rows, int nslots) {
     const int n = (int)rows.size();
     std::vector<std::vector<int>> inv(nslots);
     for (int r = 0; r < n; ++r)
@@ -88,10 +89,13 @@ std::vector<Block> make_blocks(const std::vector<Row>& rows, int nslots) {
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return rows[a].e.size() > rows[b].e.size(); });
     std::vector<char> used(n, 0);
     std::vector<int> common(n, 0), touched, at(nslots, -1);
-    std::vector<Block> out;
+    std::vector<BlockOf<G>> out;
+    std::array<int, G> none;
+    none.fill(-1);
     for (int seed : order) {
         if (used[seed]) continue;
-        Block b;
+        BlockOf<G> b;
+        b.slot = none;
         std::vector<int> cols;
         int g = 0;
         auto take = [&](int r) {
@@ -101,7 +105,7 @@ std::vector<Block> make_blocks(const std::vector<Row>& rows, int nslots) {
                 if (at[e.col] < 0) {
                     at[e.col] = (int)cols.size();
                     cols.push_back(e.col);
-                    b.t.push_back({-1, -1, -1, -1});
+                    b.t.push_back(none);
                     for (int k : inv[e.col])
                         if (!used[k]) {
                             if (common[k]++ == 0) touched.push_back(k);
@@ -112,7 +116,7 @@ std::vector<Block> make_blocks(const std::vector<Row>& rows, int nslots) {
             ++g;
         };
         take(seed);
-        while (g < 4) {
+        while (g < G) {
             int best = -1;
             double score = 0;
             for (int k : touched) {
@@ -250,7 +254,7 @@ struct Side {
     Sched sc;
 };
 bool cut_side(const std::vector<Row>& rows, int nslots, int nw, size_t most, Side& S) {
-    S.blocks = make_blocks(rows, nslots);
+    S.blocks = make_blocks<4>(rows, nslots);
     std::vector<int> len;
     for (const Block& b : S.blocks) len.push_back((int)b.col.size());
     S.sc = best_schedule(len, nw, 40.0, 22.0, kNodeQuantum, most);
@@ -572,6 +576,156 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
         }
     N.ok = true;
     return N;
+}
+
+// The gradient in the coefficients is a sum over atoms of products X_p X_q of pair products, with p of an A0 entry and
+// another factor and q of the other two.  Rows p that share columns q are taken sixteen at a time, and their
+// columns sixteen at a time, so that a tile of 256 products is a matrix product over the atoms (FitPlan).
+FitPlan build_fit_plan(const ZLayout& z, const TermList& T) {
+    FitPlan F;
+    const int one = z.nz;
+    const Conj cj{T.fold, one};
+    const size_t nt = T.nterms();
+    auto product = [&](int x) { return x > one; };  // an entry Y, whose conjugate is not at hand
+    auto partner = [&](Pair p) { return ordered(cj.partner(p.first), cj.partner(p.second)); };
+    auto canon = [&](Pair p) { return product(p.first) || product(p.second) ? p : std::min(p, partner(p)); };
+    auto id_of = [](std::map<Pair, int>& m, std::vector<Pair>& v, Pair p) {
+        auto it = m.emplace(p, (int)v.size());
+        if (it.second) v.push_back(p);
+        return it.first->second;
+    };
+    // which two of the three factors behind A0 make q: monomials of three factors leave one alone
+    static const int rest3[3][3] = {{0, 1, 2}, {0, 2, 1}, {1, 2, 0}};
+    std::map<Pair, int> qid;
+    std::vector<Pair> qpair;
+    std::vector<std::vector<int>> options(nt);
+    for (size_t t = 0; t < nt; ++t) {
+        const uint16_t* f = &T.idx[4 * t + 1];
+        for (const auto& r : rest3) {
+            const Pair q = ordered(f[r[0]], f[r[1]]);
+            if (q != Pair(one, one)) options[t].push_back(id_of(qid, qpair, canon(q)));
+        }
+    }
+    const std::vector<int> pick = cover(options, (int)qpair.size(), std::vector<char>(qpair.size(), 0));
+    std::map<Pair, int> pid;
+    std::vector<Pair> P;
+    std::vector<Row> rows;
+    for (size_t t = 0; t < nt; ++t) {
+        const uint16_t* f = &T.idx[4 * t + 1];
+        for (const auto& r : rest3) {
+            const int x = f[r[0]], y = f[r[1]];
+            if (ordered(x, y) == Pair(one, one) || pick[t] != qid[canon(ordered(x, y))]) continue;
+            int c = T.idx[4 * t], k = f[r[2]], minus = 0;
+            // Re P = s Re P' of the conjugate monomial (an entry Y beside a pair that is not its own conjugate
+            // keeps the monomial as it is: its q then has a column of its own)
+            Pair q = ordered(x, y);
+            if (q != canon(q) && !product(k)) {
+                minus = cj.sign(c) * cj.sign(k) * cj.sign(x) * cj.sign(y) < 0;
+                c = cj.partner(c);
+                k = cj.partner(k);
+                q = canon(q);
+            }
+            const int p = id_of(pid, P, Pair(c, k)), qi = id_of(qid, qpair, q);
+            if (p == (int)rows.size()) rows.push_back({p, {}});
+            rows[p].e.push_back({qi, (int)(2 * t) + minus});
+            break;
+        }
+    }
+    // two monomials never share both nodes
+    const std::vector<BlockOf<16>> blocks = make_blocks<16>(rows, (int)qpair.size());
+    struct Tile {
+        const BlockOf<16>* b;
+        size_t c0;
+    };
+    std::vector<Tile> tiles;
+    for (const auto& b : blocks)
+        for (size_t c = 0; c < b.col.size(); c += 16) tiles.push_back({&b, c});
+    const size_t most = (size_t)kFitWaves * kFitTiles, want = std::max<size_t>(1, (tiles.size() + most - 1) / most);
+    const size_t per = (tiles.size() + want - 1) / want;
+    // a group of tiles with the entries and nodes that it needs
+    for (size_t i = 0; i < tiles.size();) {
+        std::map<int, int> entry;                  // Z entry -> slot; entries Y behind them
+        std::vector<int> entries, prods;
+        std::map<int, int> prow, pcol;             // node -> number
+        std::vector<int> nrow, ncol;
+        auto add_entry = [&](int x) {
+            if (x == one || entry.count(x)) return;
+            if (product(x)) {
+                for (int k = 0; k < 2; ++k) {
+                    const int a = T.ypair[2 * (x - one - 1) + k];
+                    if (!entry.count(a)) entry[a] = 0, entries.push_back(a);
+                }
+                entry[x] = 0;
+                prods.push_back(x);
+            } else {
+                entry[x] = 0;
+                entries.push_back(x);
+            }
+        };
+        const size_t i0 = i;
+        while (i < tiles.size() && i - i0 < per) {
+            const auto e0 = entry;
+            const auto r0 = prow, c0 = pcol;
+            const size_t ne = entries.size(), ny = prods.size(), nr = nrow.size(), nc = ncol.size();
+            const Tile& t = tiles[i];
+            for (int r : t.b->slot)
+                if (r >= 0 && !prow.count(r)) {
+                    prow[r] = (int)nrow.size();
+                    nrow.push_back(r);
+                    add_entry(P[r].first);
+                    add_entry(P[r].second);
+                }
+            for (size_t c = t.c0; c < std::min(t.c0 + 16, t.b->col.size()); ++c) {
+                const int q = t.b->col[c];
+                if (pcol.count(q)) continue;
+                pcol[q] = (int)ncol.size();
+                ncol.push_back(q);
+                add_entry(qpair[q].first);
+                add_entry(qpair[q].second);
+            }
+            const int ge = (int)entries.size(), gy = (int)prods.size(), gn = (int)(nrow.size() + ncol.size());
+            if (i > i0 && (ge > kFitEntries || gy > kFitProducts || gn > kFitNodes || ge + 1 + gy + gn > kFitSlots)) {
+                entry = e0, prow = r0, pcol = c0;
+                entries.resize(ne), prods.resize(ny), nrow.resize(nr), ncol.resize(nc);
+                break;
+            }
+            ++i;
+        }
+        // in the order of their places, so that neighbouring lanes load neighbouring entries
+        std::sort(entries.begin(), entries.end(), [&](int a, int b) {
+            return std::make_pair(z.half[a] & 0xfff, a) < std::make_pair(z.half[b] & 0xfff, b);
+        });
+        for (size_t k = 0; k < entries.size(); ++k) entry[entries[k]] = (int)k;
+        const int so = (int)entries.size();  // the slot of 1
+        for (size_t k = 0; k < prods.size(); ++k) entry[prods[k]] = so + 1 + (int)k;
+        entry[one] = so;
+        const int n0 = so + 1 + (int)prods.size(), nn = (int)(nrow.size() + ncol.size());
+        for (int v : {(int)F.entry.size(), so, (int)F.prod.size(), (int)prods.size(), (int)F.node.size(),
+                      (int)nrow.size(), nn, (int)(F.place.size() / 64), (int)(i - i0)})
+            F.head.push_back(v);
+        F.head.resize(F.head.size() + kFitHead - 9, 0);
+        for (int x : entries) F.entry.push_back(z.half[x]);
+        auto slots = [&](Pair p) { return (uint32_t)entry[p.first] | (uint32_t)entry[p.second] << 16; };
+        for (int x : prods) F.prod.push_back(slots({T.ypair[2 * (x - one - 1)], T.ypair[2 * (x - one - 1) + 1]}));
+        for (int r : nrow) F.node.push_back(slots(P[r]));
+        for (int q : ncol) F.node.push_back(slots(qpair[q]));
+        for (size_t k = i0; k < i; ++k) {
+            const Tile& t = tiles[k];
+            auto row = [&](int r) { return t.b->slot[r]; };
+            auto col = [&](int c) { return t.c0 + c < t.b->col.size() ? t.b->col[t.c0 + c] : -1; };
+            for (int lane = 0; lane < 64; ++lane) {
+                const int r = row(lane & 15), q = col(lane & 15);  // none: any node
+                F.place.push_back((uint32_t)(n0 + (r < 0 ? 0 : prow[r])) |
+                                  (uint32_t)(n0 + (int)nrow.size() + (q < 0 ? 0 : pcol[q])) << 16);
+                for (int u = 0; u < 4; ++u)
+                    F.t.push_back(q < 0 ? -1 : t.b->t[t.c0 + (lane & 15)][matrix_row(8, lane >> 4, u)]);
+            }
+        }
+        F.slots = std::max(F.slots, n0 + nn);
+        F.tiles = std::max(F.tiles, (int)(i - i0));
+        ++F.groups;
+    }
+    return F;
 }
 
 }  // namespace magace
