@@ -202,7 +202,9 @@ int magace_md_destroy(void *md);
  * offsets, nlist[p] = global 0-based neighbour atom) that also assembles per-atom forces
  * forces[3*natom] and per-structure energies estruct[nstruc] (atom_struct[natom] = structure
  * of each atom; may be NULL when nstruc = 0).
- * magace_fit_backward: right after magace_fit_forward on the same arrays, the gradient
+ * magace_fit_state: the part of magace_fit_forward that a following magace_fit_backward needs, without
+ * pair forces and without outputs (a backward that re-evaluates its own batch first).
+ * magace_fit_backward: right after magace_fit_forward or magace_fit_state on the same arrays, the gradient
  * grad[ncoef] = d/dc (sum_s gE[s] E_s + sum_j gF[3j..] . F_j) for cotangents gE (may be NULL)
  * and gF (device arrays), by forward-mode differentiation of the density along gF. */
 int magace_fit_ncoef(void);
@@ -212,6 +214,9 @@ int magace_fit_forward(int natom, int nei, const int *offsets, const int *nlist,
                        const double *elist, const double *dlist_momi, const double *elist_momi,
                        const double *dlist_mom, const double *elist_mom, const int *atom_struct,
                        int nstruc, double *estruct, double *forces, void *stream);
+int magace_fit_state(int natom, int nei, const int *offsets, const double *dlist, const double *elist,
+                     const double *dlist_momi, const double *elist_momi, const double *dlist_mom,
+                     const double *elist_mom, void *stream);
 int magace_fit_backward(int natom, int nei, const int *offsets, const int *nlist, const double *dlist,
                         const double *elist, const double *dlist_momi, const double *dlist_mom,
                         const double *elist_mom, const int *atom_struct, const double *gE,

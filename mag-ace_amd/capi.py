@@ -27,7 +27,7 @@ EXPORTS = ("acelibini_", "acelib_", "magace_last_error", "magace_error_string", 
            "magace_pair_compute", "magace_model_terms", "magace_profile", "magace_profile_read",
            "magace_neighbors_device", "magace_packstructures", "magace_md_create", "magace_md_run",
            "magace_md_read", "magace_md_destroy", "magace_fit_ncoef", "magace_fit_get_coefficients",
-           "magace_fit_set_coefficients", "magace_fit_forward", "magace_fit_backward", "magace_write_potential",
+           "magace_fit_set_coefficients", "magace_fit_forward", "magace_fit_state", "magace_fit_backward", "magace_write_potential",
            "magace_model_records", "magace_compute_device_noalloc", "magace_set_tuning", "magace_get_tuning",
            "magace_tune", "magace_model_products")
 
@@ -71,6 +71,7 @@ def lib():
     L.magace_fit_set_coefficients.argtypes = [_D, C.c_int]
     L.magace_fit_forward.argtypes = [C.c_int, C.c_int] + [C.c_void_p] * 9 + [C.c_int, C.c_void_p, C.c_void_p,
                                                                               C.c_void_p]
+    L.magace_fit_state.argtypes = [C.c_int, C.c_int] + [C.c_void_p] * 8
     L.magace_fit_backward.argtypes = [C.c_int, C.c_int] + [C.c_void_p] * 12
     L.magace_write_potential.argtypes = [C.c_char_p]
     L.magace_md_create.argtypes = [C.c_int, _D, C.c_double, C.c_double, C.c_double, C.c_int, _D, _D, _D, _D,
@@ -399,6 +400,11 @@ def fit_forward(natom, nei, offsets, nlist, dlist, elist, dmomi, emomi, dmom, em
     """magace_fit_forward on device pointers."""
     _check(lib().magace_fit_forward(natom, nei, offsets, nlist, dlist, elist, dmomi, emomi, dmom, emom,
                                     atom_struct or None, nstruc, estruct or None, forces, stream or None))
+
+
+def fit_state(natom, nei, offsets, dlist, elist, dmomi, emomi, dmom, emom, stream=0):
+    """magace_fit_state on device pointers."""
+    _check(lib().magace_fit_state(natom, nei, offsets, dlist, elist, dmomi, emomi, dmom, emom, stream or None))
 
 
 def fit_backward(natom, nei, offsets, nlist, dlist, elist, dmomi, dmom, emom, atom_struct, gE, gF, grad,

@@ -1607,23 +1607,13 @@ int magace_write_potential(const char* path) {
     return 0;
 }
 
-int magace_fit_forward(int natom, int nei, const int* offsets, const int* nlist, const double* dlist,
-                       const double* elist, const double* dlist_momi, const double* elist_momi,
-                       const double* dlist_mom, const double* elist_mom, const int* atom_struct, int nstruc,
-                       double* estruct, double* forces, void* stream) {
-    clear_error();
-    if (!g_ctx) {
-        set_error(MAGACE_ERR_STATE, "library not initialised");
-        return MAGACE_ERR_STATE;
-    }
-    Context& c = *g_ctx;
-    if (natom < 0 || nei < 0 || nstruc < 0 || ((nstruc > 0 || estruct) && !atom_struct) || !forces) {
-        set_error(MAGACE_ERR_INPUT, "magace_fit_forward: invalid sizes");
-        return MAGACE_ERR_INPUT;
-    }
+// The FP64 density and adjoint of a fit, and the pair forces where they are asked for; Z, W and the
+// atoms' energies stay in the context
+static int fit_evaluate(Context& c, int natom, int nei, const int* offsets, const double* dlist, const double* elist,
+                        const double* dlist_momi, const double* elist_momi, const double* dlist_mom,
+                        const double* elist_mom, bool forces, hipStream_t s) {
     if (int rc = upload(c)) return rc;
-    hipStream_t s = (hipStream_t)stream;  // NULL: the default (null) stream
-    if ((size_t)nei > c.fit_cap_pairs) {
+    if (forces && (size_t)nei > c.fit_cap_pairs) {
         dfree(c.f_fl); dfree(c.f_tl);
         const size_t cap = (size_t)nei + nei / 4 + 64;
         HIPCHK(hipMalloc((void**)&c.f_fl, 3 * cap * sizeof(double)));
@@ -1649,12 +1639,53 @@ int magace_fit_forward(int natom, int nei, const int* offsets, const int* nlist,
     const int saved = c.precision;
     c.precision = MAGACE_FP64;  // the adjoint runs on the FP64 Z and W of this evaluation
     c.buf.Wd = nd == 2 ? c.fit.Wd : nullptr;
+    c.buf.forces = forces;
     const int rc = run_device(c, natom, offsets, dlist, elist, dlist_momi, elist_momi, dlist_mom, elist_mom,
                               c.f_eout, c.f_fl, c.f_tl, c.f_t0, s);
     c.buf.Wd = nullptr;
+    c.buf.forces = true;
     c.precision = saved;
-    if (rc) return rc;
+    return rc;
+}
+
+int magace_fit_forward(int natom, int nei, const int* offsets, const int* nlist, const double* dlist,
+                       const double* elist, const double* dlist_momi, const double* elist_momi,
+                       const double* dlist_mom, const double* elist_mom, const int* atom_struct, int nstruc,
+                       double* estruct, double* forces, void* stream) {
+    clear_error();
+    if (!g_ctx) {
+        set_error(MAGACE_ERR_STATE, "library not initialised");
+        return MAGACE_ERR_STATE;
+    }
+    Context& c = *g_ctx;
+    if (natom < 0 || nei < 0 || nstruc < 0 || ((nstruc > 0 || estruct) && !atom_struct) || !forces) {
+        set_error(MAGACE_ERR_INPUT, "magace_fit_forward: invalid sizes");
+        return MAGACE_ERR_INPUT;
+    }
+    hipStream_t s = (hipStream_t)stream;  // NULL: the default (null) stream
+    if (int rc = fit_evaluate(c, natom, nei, offsets, dlist, elist, dlist_momi, elist_momi, dlist_mom, elist_mom, true, s))
+        return rc;
     HIPCHK(fit_assemble(natom, offsets, nlist, c.f_fl, c.f_eout, atom_struct, nstruc, forces, estruct, s));
+    c.fit_natom = natom;
+    return 0;
+}
+
+int magace_fit_state(int natom, int nei, const int* offsets, const double* dlist, const double* elist,
+                     const double* dlist_momi, const double* elist_momi, const double* dlist_mom,
+                     const double* elist_mom, void* stream) {
+    clear_error();
+    if (!g_ctx) {
+        set_error(MAGACE_ERR_STATE, "library not initialised");
+        return MAGACE_ERR_STATE;
+    }
+    if (natom < 0 || nei < 0) {
+        set_error(MAGACE_ERR_INPUT, "magace_fit_state: invalid sizes");
+        return MAGACE_ERR_INPUT;
+    }
+    Context& c = *g_ctx;
+    if (int rc = fit_evaluate(c, natom, nei, offsets, dlist, elist, dlist_momi, elist_momi, dlist_mom, elist_mom, false,
+                              (hipStream_t)stream))
+        return rc;
     c.fit_natom = natom;
     return 0;
 }

@@ -1518,7 +1518,7 @@ static hipError_t run_class(const DevParams<T>& P, const NodeTab<T>& N, int nato
                            B.dE, B.edf, B.rho);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[2], s);
-    if ((e = run_forces<T>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, B, !nodes, flist, tlist, tlist0, s)) !=
+    if (B.forces && (e = run_forces<T>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, B, !nodes, flist, tlist, tlist0, s)) !=
         hipSuccess)
         return e;
     if (ev) (void)hipEventRecord(ev[3], s);

@@ -107,6 +107,7 @@ struct Buffers {
                              // written by the adjoint when set
     int* err = nullptr;
     size_t cap_atoms = 0;
+    bool forces = true;      // false: a fit's gradient is to follow, which needs Z and W only
 };
 
 // bytes of Buffers::Pt per atom

@@ -76,3 +76,27 @@ def test_gradient_of_energies_and_forces(tmp_path, header, natom):
         want = np.concatenate([np.tile(want[cuts[k]:cuts[k + 1]], nd) for k in range(6)])
         err = np.abs(g.cpu().numpy() - want).max()
         assert err <= tol
+
+
+@pytest.mark.parametrize("header", ["H500", "H500ND2"])
+def test_state_serves_backward_as_forward_does(tmp_path, header):
+    pot = str(tmp_path / "Fe.pbe.in")
+    with open(pot, "w") as f:
+        f.write(potgen.render(HEADERS[header], capi.enumerate_basis(HEADERS[header]), 32, c_scale=1e-2))
+    capi.init_file(pot)
+    structs = structures(35, 6)
+    batch = fit.Batch(structs, 5.0)
+    rng = np.random.default_rng(7)
+    gE, gF = torch.tensor(rng.normal(size=len(structs)), device="cuda"), torch.tensor(rng.normal(size=(35, 3)), device="cuda")
+    grads = []
+    for forward in (True, False):
+        if forward:
+            batch.forward(torch.zeros(len(structs), dtype=torch.float64, device="cuda"),
+                          torch.zeros(35, 3, dtype=torch.float64, device="cuda"))
+        else:
+            batch.state()
+        g = torch.zeros(capi.fit_ncoef(), dtype=torch.float64, device="cuda")
+        batch.backward(gE, gF, g)
+        grads.append(g.cpu().numpy())
+    # the same sums; those over atoms meet in memory in any order
+    assert np.abs(grads[0] - grads[1]).max() <= 1e-12 * np.abs(grads[0]).max()
