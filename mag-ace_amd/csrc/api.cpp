@@ -924,6 +924,11 @@ struct ChunkLayout {
     }
 };
 
+constexpr size_t slots16(size_t bytes) { return (bytes + 15) / 16; }
+
+// An acelib_ call of one chunk whose inputs are up to this size runs in one stream and waits for the GPU once.
+constexpr size_t kOneStreamBytes = (size_t)4 << 20;
+
 // Atom boundaries of the chunks (cut[0] = 0, ..., cut.back() = natom).  Chunks hold whole
 // atoms and at most cmax pairs (unless one atom has more).  The first chunks grow from
 // cmax/4 and the last ones shrink by halves down to cmax/4, so that the host's first packing
@@ -947,10 +952,7 @@ std::vector<int> chunk_plan(const std::vector<int>& off, int cmax) {
     return cut;
 }
 
-int check_kernel_errors(Context& c, hipStream_t s) {
-    int err = 0;
-    HIPCHK(hipMemcpyAsync(&err, c.buf.err, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+int report_kernel_errors(int err) {
     if (err & kErrSmallDistance) {
         set_error(MAGACE_ERR_INPUT, "Encountered very small distance.");
         return MAGACE_ERR_INPUT;
@@ -960,6 +962,13 @@ int check_kernel_errors(Context& c, hipStream_t s) {
         return MAGACE_ERR_INPUT;
     }
     return 0;
+}
+
+int check_kernel_errors(Context& c, hipStream_t s) {
+    int err = 0;
+    HIPCHK(hipMemcpyAsync(&err, c.buf.err, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return report_kernel_errors(err);
 }
 
 // Per-atom buffers of the allocation-free entry point, carved from the fixed device scratch:
@@ -1343,8 +1352,9 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
     size_t need_in = 0, need_out = 0;
     for (size_t k = 0; k < nchunk; ++k) {
         const ChunkLayout L(cut[k + 1] - cut[k], c.h_off[cut[k + 1]] - c.h_off[cut[k]]);
-        need_in = std::max(need_in, L.in_bytes);
-        need_out = std::max(need_out, L.out_bytes);
+        // whole slots of 16 bytes, and one for the error flags
+        need_in = std::max(need_in, slots16(L.in_bytes) * 16);
+        need_out = std::max(need_out, slots16(L.out_bytes) * 16 + 16);
     }
     for (auto& sl : c.slots) {
         if (need_in > sl.cap_in) {
@@ -1370,11 +1380,9 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
     }
     hipStream_t s = c.stream;
     HostPool& pool = HostPool::get();
-    if (fail(clear_flags(c.buf.err, s), "clear")) return;
     // chunk k's outputs, once its kernels are done, into the caller's arrays
-    auto unpack = [&](size_t k) {
+    auto copy_back = [&](size_t k) {
         const Context::Slot& sl = c.slots[k & 1];
-        if (fail(hipEventSynchronize(sl.ev_done), "sync")) return false;
         const size_t a0 = cut[k], p0 = c.h_off[a0];
         const ChunkLayout L(cut[k + 1] - a0, c.h_off[cut[k + 1]] - p0);
         const char* o = sl.h_out;
@@ -1382,6 +1390,10 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
                              {tlist0 + 3 * a0, o + L.o_t0, 24 * L.na},
                              {flist + 3 * p0, o + L.o_fl, 24 * L.np},
                              {tlist + 3 * p0, o + L.o_tl, 24 * L.np}});
+    };
+    auto unpack = [&](size_t k) {
+        if (fail(hipEventSynchronize(c.slots[k & 1].ev_done), "sync")) return false;
+        copy_back(k);
         return true;
     };
     // Order of the host's work: chunk k's kernels and copy-back are enqueued, then chunk k + 1
@@ -1391,9 +1403,8 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
     // waits for chunk k's kernels (d_in), its kernels for chunk k's copy-back (d_out); its
     // copy-back is enqueued after chunk k is unpacked (h_out), its packing after chunk k's
     // upload has finished (h_in).
-    auto pack_upload = [&](size_t k) {
+    auto pack = [&](size_t k) {
         Context::Slot& sl = c.slots[k & 1];
-        if (k >= 2 && fail(hipEventSynchronize(sl.ev_in), "sync")) return false;  // h_in of chunk k - 2 sent
         const size_t a0 = cut[k], p0 = c.h_off[a0];
         const ChunkLayout L(cut[k + 1] - a0, c.h_off[cut[k + 1]] - p0);
         char* in = sl.h_in;
@@ -1405,10 +1416,45 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
                              {in + L.i_em, elist_mom + 3 * p0, 24 * L.np},
                              {in + L.i_dmi, dlist_momi + a0, 8 * L.na},
                              {in + L.i_emi, elist_momi + 3 * a0, 24 * L.na}});
+        return L.in_bytes;
+    };
+    auto pack_upload = [&](size_t k) {
+        Context::Slot& sl = c.slots[k & 1];
+        if (k >= 2 && fail(hipEventSynchronize(sl.ev_in), "sync")) return false;  // h_in of chunk k - 2 sent
+        const size_t bytes = pack(k);
         if (k >= 2 && fail(hipStreamWaitEvent(c.s_in, sl.ev_comp, 0), "event")) return false;  // d_in free
-        return !(fail(hipMemcpyAsync(sl.d_in, in, L.in_bytes, hipMemcpyHostToDevice, c.s_in), "copy") ||
+        return !(fail(hipMemcpyAsync(sl.d_in, sl.h_in, bytes, hipMemcpyHostToDevice, c.s_in), "copy") ||
                  fail(hipEventRecord(sl.ev_in, c.s_in), "event"));
     };
+    auto evaluate = [&](size_t k) {
+        const Context::Slot& sl = c.slots[k & 1];
+        const size_t a0 = cut[k], p0 = c.h_off[a0];
+        const ChunkLayout L(cut[k + 1] - a0, c.h_off[cut[k + 1]] - p0);
+        const char* d = sl.d_in;
+        char* o = sl.d_out;
+        return run_device(c, (int)L.na, (const int*)(d + L.i_off), (const double*)(d + L.i_dl),
+                          (const double*)(d + L.i_el), (const double*)(d + L.i_dmi), (const double*)(d + L.i_emi),
+                          (const double*)(d + L.i_dm), (const double*)(d + L.i_em), (double*)(o + L.o_eout),
+                          (double*)(o + L.o_fl), (double*)(o + L.o_tl), (double*)(o + L.o_t0), s, false, false, nullptr,
+                          cut[k]);
+    };
+    if (nchunk == 1 && need_in <= kOneStreamBytes) {
+        // Inputs and outputs cross by a kernel, the flags with them: the copy engine's transfers, the events between
+        // three streams and the copy of the flags cost a small call more than its evaluation does.  Here and by the
+        // pipeline (FP64, us): lmax 4 54 atoms 85 and 154, 432 atoms 184 and 235, 1024 atoms (3.9 MB) 328 and 383; lmax 6
+        // 395 and 438.  From 98304 pairs a call has several chunks, whose copies overlap.
+        const Context::Slot& sl = c.slots[0];
+        pack(0);
+        int* flag = (int*)(sl.h_out + need_out - 16);
+        if (fail(copy_slots(sl.h_in, sl.d_in, need_in / 16, c.buf.err, nullptr, s), "copy") || evaluate(0) ||
+            fail(copy_slots(sl.d_out, sl.h_out, need_out / 16 - 1, c.buf.err, flag, s), "copy") ||
+            fail(hipStreamSynchronize(s), "sync"))
+            return;
+        copy_back(0);
+        (void)report_kernel_errors(*flag);
+        return;
+    }
+    if (fail(clear_flags(c.buf.err, s), "clear")) return;
     if (nchunk > 0 && !pack_upload(0)) return;
     for (size_t k = 0; k < nchunk; ++k) {
         Context::Slot& sl = c.slots[k & 1];
@@ -1416,14 +1462,7 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
         const ChunkLayout L(cut[k + 1] - a0, c.h_off[cut[k + 1]] - p0);
         if (fail(hipStreamWaitEvent(s, sl.ev_in, 0), "event")) return;
         if (k >= 2 && fail(hipStreamWaitEvent(s, sl.ev_done, 0), "event")) return;  // d_out of chunk k - 2 copied
-        const char* d = sl.d_in;
-        char* o = sl.d_out;
-        if (run_device(c, (int)L.na, (const int*)(d + L.i_off), (const double*)(d + L.i_dl),
-                       (const double*)(d + L.i_el), (const double*)(d + L.i_dmi), (const double*)(d + L.i_emi),
-                       (const double*)(d + L.i_dm), (const double*)(d + L.i_em), (double*)(o + L.o_eout),
-                       (double*)(o + L.o_fl), (double*)(o + L.o_tl), (double*)(o + L.o_t0), s, false, false, nullptr,
-                       cut[k]))
-            return;
+        if (evaluate(k)) return;
         if (fail(hipEventRecord(sl.ev_comp, s), "event") || fail(hipStreamWaitEvent(c.s_out, sl.ev_comp, 0), "event") ||
             fail(hipMemcpyAsync(sl.h_out, sl.d_out, L.out_bytes, hipMemcpyDeviceToHost, c.s_out), "copy") ||
             fail(hipEventRecord(sl.ev_done, c.s_out), "event"))

@@ -1422,6 +1422,32 @@ hipError_t fit_assemble(int natom, const int* off, const int* nlist, const doubl
 // ============================================================================ launch
 __global__ void k_clear_flags(int* p) { *p = 0; }
 
+// n slots of 16 bytes; then *flag_out = *flag, or *flag = 0 where there is no flag_out
+__global__ void __launch_bounds__(256) k_copy_slots(const uint4* __restrict__ src, uint4* __restrict__ dst, int n, int* flag,
+                                                    int* flag_out) {
+    constexpr int U = 4;  // in flight a thread: a trip to host memory takes microseconds
+    const int i0 = blockIdx.x * (U * 256) + threadIdx.x;
+    uint4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = src[min(i0 + 256 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (i0 + 256 * u < n) dst[i0 + 256 * u] = v[u];
+    if (i0 == 0) {
+        if (flag_out)
+            *flag_out = *flag;
+        else
+            *flag = 0;
+    }
+}
+
+hipError_t copy_slots(const void* src, void* dst, size_t n, int* flag, int* flag_out, hipStream_t s) {
+    if (n == 0 || n > (size_t)1 << 24) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_copy_slots, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, (const uint4*)src, (uint4*)dst,
+                       (int)n, flag, flag_out);
+    return hipGetLastError();
+}
+
 hipError_t clear_flags(int* p, hipStream_t s) {
     // a kernel rather than hipMemsetAsync, so that the evaluation can be captured in a graph
     hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(1), 0, s, p);

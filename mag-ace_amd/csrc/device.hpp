@@ -220,6 +220,9 @@ hipError_t run_forces(const DevParams<T>& P, int natom, const int* off, const do
                       bool scaled, double* flist, double* tlist, double* tlist0, hipStream_t s);
 hipError_t upload_legendre_constants();
 hipError_t clear_flags(int* p, hipStream_t s);
+// n >= 1 slots of 16 bytes between device memory and pinned host memory; with flag_out its copy of *flag, without it
+// *flag is cleared
+hipError_t copy_slots(const void* src, void* dst, size_t n, int* flag, int* flag_out, hipStream_t s);
 int supported_nm3_class(int nm3, int nr2m, int nb_a, int l3a, int l2m, int nr3a);
 
 }  // namespace magace

@@ -103,6 +103,12 @@ void parallel_copy(HostPool& pool, const std::vector<CopyJob>& jobs) {
     size_t total = 0;
     for (const auto& j : jobs) total += j.bytes;
     if (total == 0) return;
+    // waking the other threads takes longer than copying this
+    if (total <= size_t(256) << 10) {
+        for (const auto& j : jobs)
+            if (j.bytes) std::memcpy(j.dst, j.src, j.bytes);
+        return;
+    }
     // pieces of at least 256 KiB, about four per thread
     const size_t piece = std::max<size_t>(size_t(256) << 10, total / (4 * (size_t)pool.size()) + 1);
     struct Piece {
