@@ -88,7 +88,7 @@ int magace_tune(int natom, int nei, const int *offsets, const double *dlist, con
 /* acelib_ on device-resident arrays (same meaning as acelib_, FP64), with 0-based CSR
  * offsets[natom+1] instead of nstart/nstop.  Enqueued on `stream` (a hipStream_t; NULL is the
  * default stream, as in HIP); no host synchronisation.  magace_check_errors() synchronises the
- * stream and reports geometry errors raised by the kernels.  From 2048 atoms the second half of
+ * stream and reports geometry errors raised by the kernels.  In FP64 from 12288 atoms the second half of
  * the atoms runs on the library's own stream, forked from `stream` and joined back to it before
  * the call's work on `stream` completes (not while `stream` is being captured into a graph;
  * MAGACE_SPLIT_STREAMS=0 turns this off).  Calls on different streams must not overlap. */

@@ -793,18 +793,22 @@ int ensure_atoms(Context& c, size_t natom) {
     return 0;
 }
 
-// Evaluations of at least kSplitAtoms atoms run as two halves of the atom range, the second on
+// FP64 evaluations of at least kSplitAtoms atoms run as two halves of the atom range, the second on
 // the context's own stream (used otherwise only by acelib_), forked from the caller's stream
 // and joined back to it; no further stream is created, since the process's streams share
 // four hardware queues and a fifth one slowed acelib_'s copy pipeline.  Every
 // kernel is independent per atom, so the halves only overlap: the tail of one half's launch
-// and the next kernel of the other share the CUs, and an LDS-bound adjoint runs beside the
-// VALU-bound forces.  The second half uses its own rows of the per-atom device buffers; pair
-// arrays are indexed by absolute pair index.  Not while per-kernel times are measured, nor
-// while the caller's stream is being captured into a graph, nor inside acelib_'s chunk
+// and the next kernel of the other share the CUs.  The second half uses its own rows of the per-atom
+// device buffers; pair arrays are indexed by absolute pair index.  Not while per-kernel times are
+// measured, nor while the caller's stream is being captured into a graph, nor inside acelib_'s chunk
 // pipeline, whose kernels run on that stream.  MAGACE_SPLIT_STREAMS=0 turns the split off
 // (read at every call).
-constexpr int kSplitAtoms = 2048;
+// The fork and the join take about 10 us, and kernels of one workgroup an atom or two have short tails, so little is
+// left to gain (split and one sequence, us): FP64 lmax 6 4394 atoms 542 and 543, 8192 1019 and 1023, 16000 1983 and 1995,
+// 54000 6581 and 6608; 27 magnetic columns 8192 1193 and 1188, 16000 2399 and 2419, 54000 8147 and 8246; lmax 4
+// 8192 428 and 420, 16000 equal.  Mixed: lmax 4 2662 atoms 124 and 115, 8192 268 and 252, 54000 1639 and 1620; lmax 6
+// 4394 291 and 275, 16000 949 and 946; 27 columns 4394 314 and 308, 54000 3363 and 3356.
+constexpr int kSplitAtoms = 12288;
 
 bool split_enabled() {
     const char* e = std::getenv("MAGACE_SPLIT_STREAMS");
@@ -860,7 +864,8 @@ int run_device(Context& c, int natom, const int* off, const double* dlist, const
         }
         ev = c.events[c.events_used++].data();
     }
-    bool split = allow_split && s != c.stream && !c.profiling && natom >= kSplitAtoms && split_enabled();
+    bool split = allow_split && s != c.stream && !c.profiling && c.precision == MAGACE_FP64 && natom >= kSplitAtoms &&
+                 split_enabled();
     if (split) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         HIPCHK(hipStreamIsCapturing(s, &cs));
