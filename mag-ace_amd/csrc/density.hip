@@ -58,6 +58,22 @@ struct DensityLds {  // strides and offsets (in T) of the staging arrays
     }
 };
 
+// harmonics() without a branch on l where the header has all of the instance's, in FP32 up to l = 4 always (rows have
+// room for them).  The conditions of the other case are not to be kept across the rounds: 40 to 77 scalars of masks,
+// spilled to vector registers, were up to a third of the staging's instructions.  27648 atoms lmax 4: mixed 295 -> 287
+// us, FP64 480 -> 470 us; 16000 atoms lmax 6 FP64 484 -> 465 us.  FP32 at l = 6 spills with the long straight code (267
+// us) and keeps its branches (264 us, 265 before).
+template <typename T, int L, typename F>
+__device__ __forceinline__ void row_of_harmonics(T x, T y, T z, int lmax, F&& put) {
+    if (sizeof(T) == 4 && L <= 4) lmax = L;
+    if (lmax == L && !(sizeof(T) == 4 && L > 4)) {
+        harmonics<T, L>(x, y, z, L, put);
+    } else {
+        asm volatile("" : "+s"(lmax));
+        harmonics<T, L>(x, y, z, lmax, put);
+    }
+}
+
 // functions first .. first + nf - 1 of a row: value(k, coefficients), some more than once
 template <typename T, typename F>
 __device__ __forceinline__ void spline_row(const T* __restrict__ row, int first, int nf, F&& value) {
@@ -149,7 +165,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                         z = live ? (T)elist[3 * p + 2] : (T)1;
                 const Coef<T> cc = coef_at(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g + 4 * P.nb_a);
                 if constexpr (!JVP) {
-                    harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
+                    row_of_harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
                         sY[lane * SY + k] = {pl * ph.re, pl * ph.im};
                     });
                     core += row < 0 ? 0.0 : (double)coef_value(cc, w);
@@ -165,7 +181,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                     const T invr = live ? (T)(1.0 / dlist[p]) : (T)0;
                     // the displacement's part across the bond, over r: D_u Y = grad Y . t
                     const T tx = (dx - rdot * x) * invr, ty = (dy - rdot * y) * invr, tz = (dz - rdot * z) * invr;
-                    harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T dpl, cplx<T> ph, cplx<T> ph1, int m) {
+                    row_of_harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T dpl, cplx<T> ph, cplx<T> ph1, int m) {
                         sY[lane * SY + k] = {pl * ph.re, pl * ph.im};
                         // Y = P(z) (x + iy)^m
                         const T a = dpl * tz, b = (T)m * pl;
@@ -188,7 +204,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 Coef<T> cm[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) cm[u] = coef_at(mrow + 4 * (u <= P.l3m ? u * P.nr2m : 0));
-                harmonics<T, L>(x, y, z, P.l2m, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
+                row_of_harmonics<T, L>(x, y, z, P.l2m, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
                     sYm[lane * SYM + k] = {pl * ph.re, pl * ph.im};
                 });
                 if (lane < nr)
