@@ -15,6 +15,7 @@
 #include <cstring>
 #include <array>
 #include <atomic>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -556,7 +557,13 @@ int upload_kept(std::vector<void*>& kept, D*& dst, const V& v) {
 
 // the fitting plan, built when a fit asks for its first gradient
 int upload_fit_plan(Context& c) {
-    const FitPlan F = build_fit_plan(c.model.z, c.model.terms);
+    FitPlan F;
+    try {
+        F = build_fit_plan(c.model.z, c.model.terms);
+    } catch (const std::exception& e) {  // no exception leaves a C entry point
+        set_error(MAGACE_ERR_DEVICE, std::string("fitting plan: ") + e.what());
+        return MAGACE_ERR_DEVICE;
+    }
     FitTab& D = c.fit.plan;
     D.groups = F.groups;
     D.slots = F.slots;
