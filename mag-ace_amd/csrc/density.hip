@@ -120,7 +120,8 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
     const int p0 = off[atom], nn = off[atom + 1] - p0;
     Zout += (size_t)atom * P.nz;
 
-    // this lane's columns (P.cols): wave w has the tiles w, w + 4, ... of those of A followed by those of A2
+    // this lane's columns (P.cols): wave w has the tiles w, w + 4, ... of those of A followed by those of A2.  There may
+    // be none of either: a potential of pair functions has A2 only, one of the moments' functions alone neither.
     const int nA = P.lha * P.nm3, nA2 = P.nr2m * P.lhm;
     const int tA = (nA + 15) >> 4, tAll = tA + ((nA2 + 15) >> 4);
     const int ci = lane & 15, g = lane >> 4;
@@ -131,13 +132,13 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
     for (int t = 0; t < TA; ++t) {
         ar[t] = (V)(T)0;
         ai[t] = (V)(T)0;
-        ca[t] = P.cols[min(wave + 4 * t, tA - 1) * 16 + ci];
+        ca[t] = tA > 0 ? P.cols[min(wave + 4 * t, tA - 1) * 16 + ci] : 0u;
     }
 #pragma unroll
     for (int t = 0; t < T2; ++t) {
         a2r[t] = (V)(T)0;
         a2i[t] = (V)(T)0;
-        c2[t] = P.cols[min(wave + 4 * (na + t), tAll - 1) * 16 + ci];
+        c2[t] = tAll > 0 ? P.cols[min(wave + 4 * (na + t), tAll - 1) * 16 + ci] : 0u;
     }
     // rows past nb_a of the base functions stay zero
     for (int i = tid; i < kPairs * kG; i += 256) {
@@ -470,7 +471,6 @@ hipError_t by_tiles(const DevParams<T>& P, A... a) {
         const int n2 = ((tAll - w + 3) >> 2) - na;
         t2 = t2 > n2 ? t2 : n2;
     }
-    if (tA < 1) return hipErrorInvalidValue;
     if (ta <= 1 && t2 <= 1) return launch_density<T, L, 1, 1, JVP>(P, a...);
     if (ta <= 2 && t2 <= 1) return launch_density<T, L, 2, 1, JVP>(P, a...);
     if (ta <= 4 && t2 <= 1) return launch_density<T, L, 4, 1, JVP>(P, a...);

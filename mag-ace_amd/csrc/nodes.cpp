@@ -294,6 +294,7 @@ NodePlan build_nodes(const ZLayout& z, const TermList& T, int entry_limit) {
     if (T.ny > 0 || T.nd != 1) return N;
     const Conj cj{T.fold, one};
     const size_t nt = T.nterms();
+    if (nt == 0) return N;  // the atoms' own moments alone: nothing to plan, and no entry of Z
     struct Mono {
         int a0, f[3], n;  // factors past n: none
     };
