@@ -127,12 +127,13 @@ __device__ __forceinline__ void spline_values(const T* __restrict__ row, const T
 }
 
 // Spline row and fraction for the atomic table (src/radial.F90:68-84).
-// Returns nullptr when the pair is beyond the table (all functions zero).
+// Returns nullptr when the pair is beyond the table (all functions zero).  A distance or moment that is
+// not a number is an error too: its row number would be -1, in front of the table.
 template <typename T>
 __device__ __forceinline__ const T* atomic_row(const DevParams<T>& P, double r, T& w, int* err) {
     const double x = r * P.rs_a;
     const double fl = floor(x);
-    if (fl <= 0.0) { atomicOr(err, kErrSmallDistance); return nullptr; }
+    if (!(fl > 0.0)) { atomicOr(err, kErrSmallDistance); return nullptr; }
     if (fl >= (double)P.nlut) return nullptr;
     const int nl = (int)fl;
     w = (T)(x - fl);
@@ -146,7 +147,7 @@ __device__ __forceinline__ const T* magnetic_row(const DevParams<T>& P, double m
     unit = false;
     const double x = mu * P.rs_m;
     const double fl = floor(x);
-    if (fl < 0.0 || fl > (double)P.nlut) { atomicOr(err, kErrMomentRange); return nullptr; }
+    if (!(fl >= 0.0 && fl <= (double)P.nlut)) { atomicOr(err, kErrMomentRange); return nullptr; }
     if (fl == 0.0) { unit = true; return nullptr; }
     w = (T)(x - fl);
     return P.lut_m + (size_t)((int)fl - 1) * P.stride_m;

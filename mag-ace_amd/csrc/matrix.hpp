@@ -95,13 +95,14 @@ __device__ __forceinline__ void harmonics(T x, T y, T z, int lmax, F&& put) {
 
 // ---------------------------------------------------------------- spline rows
 // Row number and fraction of a distance or moment (src/radial.F90:68-84, 126-158); row < 0: every function
-// is 0 (kRowZero: beyond the table) or, for moments below the first node, 1 (kRowOne)
+// is 0 (kRowZero: beyond the table) or, for moments below the first node, 1 (kRowOne).  A value that is not a number
+// is in no row: it takes the error's side of every comparison.
 constexpr int kRowZero = -1, kRowOne = -2;
 template <typename T>
 __device__ __forceinline__ int atomic_index(const DevParams<T>& P, double r, T& w, int* err) {
     const double x = r * P.rs_a, fl = floor(x);
     w = (T)(x - fl);
-    if (fl <= 0.0) {
+    if (!(fl > 0.0)) {
         atomicOr(err, kErrSmallDistance);
         return kRowZero;
     }
@@ -111,7 +112,7 @@ template <typename T>
 __device__ __forceinline__ int magnetic_index(const DevParams<T>& P, double mu, T& w, int* err) {
     const double x = mu * P.rs_m, fl = floor(x);
     w = (T)(x - fl);
-    if (fl < 0.0 || fl > (double)P.nlut) {
+    if (!(fl >= 0.0 && fl <= (double)P.nlut)) {
         atomicOr(err, kErrMomentRange);
         return kRowZero;
     }
