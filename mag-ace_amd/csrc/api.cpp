@@ -240,7 +240,9 @@ void fill_params(DevParams<T>& P, const Model& M) {
     const Header& h = M.pot.h;
     P.stride_a = M.spl.atomic_stride;
     P.stride_m = M.spl.magnetic_stride;
-    P.stride_g = 4 * (h.nb_a + 1);
+    P.og = sizeof(T) == 4 || M.factors.own ? M.factors.nf : 0;
+    P.nf = P.og > 0 ? P.og : h.nb_a;
+    P.stride_g = 4 * (P.og + h.nb_a + 1);
     P.nlut = M.spl.nlut;
     P.rs_a = M.spl.rs_a;
     P.rs_m = M.spl.rs_m;
@@ -285,17 +287,21 @@ int upload_table(T*& dst, const std::vector<double>& src) {
     return 0;
 }
 
-// the base functions' and the core term's part of the atomic table, and the radial coefficients as
-// operands of the matrix products
+// the factors', the base functions' and the core term's part of the atomic table, and the coefficients that make
+// R_{l,n} of the factors, or of the base functions where they are these, as operands of the matrix products
 template <typename T>
-int upload_base_tables(DevTables<T>& t, const Model& M) {
+int upload_base_tables(DevTables<T>& t, const DevParams<T>& P, const Model& M) {
     const Header& h = M.pot.h;
-    const int sg = 4 * (h.nb_a + 1), sa = M.spl.atomic_stride;
+    const int sg = P.stride_g, sa = M.spl.atomic_stride, nf = P.nf;
+    const RadialFactors& F = M.factors;
+    const std::vector<double>& u = P.og > 0 ? F.u : M.pot.crad_a;
     std::vector<double> g((size_t)M.spl.nlut * sg);
     for (int n = 0; n < M.spl.nlut; ++n) {
         const double* row = M.spl.atomic.data() + (size_t)n * sa;
-        std::copy(row, row + 4 * h.nb_a, g.begin() + (size_t)n * sg);
-        std::copy(row + sa - 4, row + sa, g.begin() + (size_t)n * sg + 4 * h.nb_a);
+        auto to = g.begin() + (size_t)n * sg;
+        if (P.og > 0) to = std::copy_n(F.table.begin() + (size_t)n * nf * 4, 4 * nf, to);
+        to = std::copy(row, row + 4 * h.nb_a, to);
+        std::copy(row + sa - 4, row + sa, to);
     }
     if (upload_table(t.lut_g, g)) return MAGACE_ERR_DEVICE;
     std::vector<double> c((size_t)(h.l3a + 1) * 256, 0.0);
@@ -303,15 +309,13 @@ int upload_base_tables(DevTables<T>& t, const Model& M) {
         for (int r = 0; r < 4; ++r)
             for (int lane = 0; lane < 64; ++lane) {
                 const int n = lane & 15, k = matrix_row(sizeof(T), lane >> 4, r);
-                if (n < h.nr3_a && k < h.nb_a)
-                    c[((size_t)l * 4 + r) * 64 + lane] = M.pot.crad_a[((size_t)n * (h.l3a + 1) + l) * h.nb_a + k];
+                if (n < h.nr3_a && k < nf) c[((size_t)l * 4 + r) * 64 + lane] = u[((size_t)n * (h.l3a + 1) + l) * nf + k];
             }
     if (upload_table(t.cperm, c)) return MAGACE_ERR_DEVICE;
     std::vector<double> r((size_t)(h.l3a + 1) * 8 * 16, 0.0);
     for (int l = 0; l <= h.l3a; ++l)
         for (int n = 0; n < h.nr3_a; ++n)
-            for (int k = 0; k < h.nb_a; ++k)
-                r[((size_t)l * 8 + n) * 16 + k] = M.pot.crad_a[((size_t)n * (h.l3a + 1) + l) * h.nb_a + k];
+            for (int k = 0; k < nf; ++k) r[((size_t)l * 8 + n) * 16 + k] = u[((size_t)n * (h.l3a + 1) + l) * nf + k];
     return upload_table(t.crow, r);
 }
 
@@ -474,6 +478,7 @@ int build_context(Potential&& pot, std::unique_ptr<Context>& out) {
     }
     M.nodes = build_nodes(M.z, M.terms, (int)((kNodeLdsMost - kNodeLdsTail) / 16));
     M.spl = build_splines(M.pot);
+    M.factors = radial_factors(M.pot, M.spl);
     fill_params(ctx->P64, M);
     fill_params(ctx->P32, M);
     apply_tuning_table(*ctx);
@@ -698,7 +703,7 @@ int upload(Context& c) {
     if (upload_table(c.t64.lut_m, M.spl.magnetic)) return MAGACE_ERR_DEVICE;
     if (upload_table(c.t32.lut_a, M.spl.atomic)) return MAGACE_ERR_DEVICE;
     if (upload_table(c.t32.lut_m, M.spl.magnetic)) return MAGACE_ERR_DEVICE;
-    if (upload_base_tables(c.t64, M) || upload_base_tables(c.t32, M)) return MAGACE_ERR_DEVICE;
+    if (upload_base_tables(c.t64, c.P64, M) || upload_base_tables(c.t32, c.P32, M)) return MAGACE_ERR_DEVICE;
     const size_t nc = M.terms.ncontrib(), nch = M.terms.chunks.size() / 2;
     HIPCHK(hipMalloc((void**)&c.crec64, nc * sizeof(uint4) + 64));
     HIPCHK(hipMalloc((void**)&c.crec32, nc * sizeof(uint4) + 64));

@@ -7,7 +7,8 @@
 // which is one product G^T F of the pairs' base functions (at most 16 rows) with all columns, and a small
 // one with C whose B operand is the first one's result as it lies in the registers.  Only the g_k (10 for
 // the lmax-6 header) are looked up for a pair, in a table of their own that stays in L2, where the 49
-// R_{l,n} had to come from a table six times as large.
+// R_{l,n} had to come from a table six times as large.  Where the C cancel, or where there are no more R than g, A is
+// summed over radial factors h_f in place of the g_k (RadialFactors), A = U B, and both are looked up.
 //
 // Measured against the kernel that staged all R_{l,n} and summed on the vector units (us): 16000 atoms
 // lmax 6 mixed 403 -> 328, FP64 735 -> 545; 27648 atoms lmax 4 mixed 494 -> 370, FP64 855 -> 535; 4394 atoms
@@ -34,6 +35,11 @@ template <typename T> constexpr int kChain = sizeof(T) == 4 ? 12 : kPairs;
 template <typename T> constexpr int kRound = sizeof(T) == 4 ? 12 : 4;  // pairs of an unrolled turn; divides kPairs
 
 constexpr int kG = 17;  // row of a pair's base functions: 16, and one for the banks
+// the same in FP32, where the radial factors come before them (the 16 rows of a product's operand may reach into what
+// lies behind: their results are not used)
+template <bool SEP> __host__ __device__ constexpr int functions_row(int og, int nb) {
+    return !SEP || og + nb < kG ? kG : (og + nb) | 1;
+}
 
 // Harmonics in a pair's row of Y or Y'.  In FP32 those of the instance's lmax, so that the rows' addresses are known
 // when it is compiled; in FP64 the longer rows of headers below it cost a workgroup of a compute unit (4394 atoms
@@ -43,18 +49,18 @@ template <typename T, int L> __host__ __device__ constexpr int harmonics_row(int
 }
 
 struct DensityLds {  // strides and offsets (in T) of the staging arrays
-    int sY, sYm, sH, sM;          // row lengths: Y, Y' and H in complex entries, M in values; odd
+    int sY, sYm, sH, sM, sG;      // row lengths: Y, Y' and H in complex entries, M and the functions in values; odd
     int oYm, oH, oG, oM, oYd, oGd, size;
-    // lha, lhm: harmonics_row
-    __host__ __device__ constexpr DensityLds(int lha, int lhm, int nm3, int nfm, bool jvp)
-        : sY(lha | 1), sYm(lhm | 1), sH(nm3 | 1), sM(nfm | 1), oYm(0), oH(0), oG(0), oM(0), oYd(0), oGd(0), size(0) {
+    // lha, lhm: harmonics_row; row: functions_row
+    __host__ __device__ constexpr DensityLds(int lha, int lhm, int nm3, int nfm, bool jvp, int row = kG)
+        : sY(lha | 1), sYm(lhm | 1), sH(nm3 | 1), sM(nfm | 1), sG(row), oYm(0), oH(0), oG(0), oM(0), oYd(0), oGd(0), size(0) {
         oYm = 2 * kPairs * sY;
         oH = oYm + 2 * (kPairs + 1) * sYm;
         oG = (oH + 2 * kPairs * sH + 3) & ~3;
-        oM = oG + kG * kPairs;
+        oM = oG + sG * kPairs + (sG > kG ? 16 : 0);  // 16: the last row's operands end here
         oYd = (oM + (kPairs + 1) * sM + 3) & ~3;
         oGd = oYd + (jvp ? 2 * kPairs * sY : 0);
-        size = oGd + (jvp ? kG * kPairs : 0);
+        size = oGd + (jvp ? oM - oG : 0);
     }
 };
 
@@ -94,9 +100,10 @@ __device__ __forceinline__ void spline_row(const T* __restrict__ row, int first,
 // bonds and the core term; Y_l'm' of the moments and H_q = M_{l',n'} Y_l'm'; the g_k; the M_{l',n'}.  Then
 // wave w takes the column tiles w, w + 4, ... (16 columns of A or A2, real and imaginary parts: two
 // products a step of four pairs).  TA, T2: tiles of A and of A2 of a wave at most.  JVP: the derivative of A and A2 along
-// the pairs' displacements u_i - u_j (k_density_jvp's work in a fit) in place of the values.
+// the pairs' displacements u_i - u_j (k_density_jvp's work in a fit) in place of the values.  SEP: radial factors of
+// A's own before the base functions (DevParams::og).
 // Waves per SIMD: what the LDS of the usual headers lets in.
-template <typename T, int L, int TA, int T2, bool JVP>
+template <typename T, int L, int TA, int T2, bool JVP, bool SEP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TA > 2 ? 2 : sizeof(T) == 4 ? 4 : L <= 4 ? 3 : 2, 8)))
 k_density_mm(DevParams<T> P, const int* __restrict__ off,
                                                     const double* __restrict__ dlist, const double* __restrict__ elist,
@@ -111,7 +118,8 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nfm = P.nr2m * (P.l2m + 1);
     const int SY = harmonics_row<T, L>(P.lha) | 1, SYM = harmonics_row<T, L>(P.lhm) | 1;  // DensityLds::sY and sYm
-    const DensityLds D(harmonics_row<T, L>(P.lha), harmonics_row<T, L>(P.lhm), P.nm3, nfm, JVP);
+    const int og = SEP ? P.og : 0, SG = functions_row<SEP>(og, P.nb_a);
+    const DensityLds D(harmonics_row<T, L>(P.lha), harmonics_row<T, L>(P.lhm), P.nm3, nfm, JVP, SG);
     T* lds = (T*)smem;
     cplx<T>*sY = (cplx<T>*)lds, *sYm = (cplx<T>*)(lds + D.oYm), *sH = (cplx<T>*)(lds + D.oH);
     T *sG = lds + D.oG, *sM = lds + D.oM;
@@ -140,8 +148,8 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
         a2i[t] = (V)(T)0;
         c2[t] = tAll > 0 ? P.cols[min(wave + 4 * (na + t), tAll - 1) * 16 + ci] : 0u;
     }
-    // rows past nb_a of the base functions stay zero
-    for (int i = tid; i < kPairs * kG; i += 256) {
+    // what lies behind a pair's functions stays zero
+    for (int i = tid; i < D.oM - D.oG; i += 256) {
         sG[i] = (T)0;
         if (JVP) sGd[i] = (T)0;
     }
@@ -164,7 +172,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 const int row = live ? atomic_index(P, dlist[p], w, err) : kRowZero;
                 const T x = live ? (T)elist[3 * p] : (T)0, y = live ? (T)elist[3 * p + 1] : (T)0,
                         z = live ? (T)elist[3 * p + 2] : (T)1;
-                const Coef<T> cc = coef_at(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g + 4 * P.nb_a);
+                const Coef<T> cc = coef_at(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g + 4 * (og + P.nb_a));
                 if constexpr (!JVP) {
                     row_of_harmonics<T, L>(x, y, z, P.l3a, [&](int k, T pl, T, cplx<T> ph, cplx<T>, int) {
                         sY[lane * SY + k] = {pl * ph.re, pl * ph.im};
@@ -237,12 +245,12 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 }
             }
             if (lane < nr)
-                spline_row<T>(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g, 0, P.nb_a,
+                spline_row<T>(P.lut_g + (size_t)(row < 0 ? 0 : row) * P.stride_g, 0, og + P.nb_a,
                               [&](int k, const Coef<T>& c) {
-                                  sG[lane * kG + k] = row < 0 ? (T)0 : coef_value(c, w);
+                                  sG[lane * SG + k] = row < 0 ? (T)0 : coef_value(c, w);
                                   // g'_k (u_i - u_j) . e
                                   if constexpr (JVP)
-                                      sGd[lane * kG + k] = row < 0 ? (T)0 : coef_slope(c, w, (T)P.rs_a) * rdot;
+                                      sGd[lane * SG + k] = row < 0 ? (T)0 : coef_slope(c, w, (T)P.rs_a) * rdot;
                               });
         } else {
             T w = 0;
@@ -302,7 +310,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                 iy2[t] = g * SYM + (c2[t] & 0xff);
                 im[t] = g * D.sM + (c2[t] >> 8 & 0xff);
             }
-            int ig = g * kG + ci;
+            int ig = g * SG + ci;
             for (int s0 = 0; s0 < nr; s0 += kRound<T>) {
                 V br[TA], bi[TA], b2r[T2], b2i[T2];
 #pragma unroll
@@ -318,9 +326,13 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
 #pragma unroll
                 for (int s = 0; s < kRound<T>; s += 4) {
                     // the step's operands of every tile first, so that one trip to LDS serves them all
-                    const T a = sG[ig + s * kG];
-                    T ad = 0;
-                    if constexpr (JVP) ad = sGd[ig + s * kG];
+                    const T a = sG[ig + s * SG];
+                    const T a2 = SEP && N2 > 0 ? sG[ig + s * SG + og] : a;
+                    T ad = 0, ad2 = 0;
+                    if constexpr (JVP) {
+                        ad = sGd[ig + s * SG];
+                        ad2 = SEP && N2 > 0 ? sGd[ig + s * SG + og] : ad;
+                    }
                     cplx<T> y[TA], h[TA], yd[JVP ? TA : 1], y2[T2];
                     T m2[T2];
 #pragma unroll
@@ -349,11 +361,11 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
                     }
 #pragma unroll
                     for (int t = 0; t < N2; ++t) {
-                        b2r[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].re, b2r[t]);
-                        b2i[t] = Mm<T>::mul(JVP ? ad : a, m2[t] * y2[t].im, b2i[t]);
+                        b2r[t] = Mm<T>::mul(JVP ? ad2 : a2, m2[t] * y2[t].re, b2r[t]);
+                        b2i[t] = Mm<T>::mul(JVP ? ad2 : a2, m2[t] * y2[t].im, b2i[t]);
                     }
                 }
-                ig += kRound<T> * kG;
+                ig += kRound<T> * SG;
 #pragma unroll
                 for (int t = 0; t < NA; ++t) {
                     ar[t] = kPart ? ar[t] + br[t] : br[t];
@@ -386,7 +398,7 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
 #pragma unroll
     for (int t = 0; t < TA; ++t)
         if (t < na) {
-            // A = C B for each l that the tile's columns have
+            // A = U B for each l that the tile's columns have
             const int l = ca[t] >> 16 & 15;
             const int l0 = __builtin_amdgcn_readlane(l, 0), l1 = __builtin_amdgcn_readlane(l, 15);
             V zr = (V)(T)0, zi = (V)(T)0;
@@ -435,14 +447,14 @@ k_density_mm(DevParams<T> P, const int* __restrict__ off,
 
 namespace {
 
-template <typename T, int L, int TA, int T2, bool JVP>
+template <typename T, int L, int TA, int T2, bool JVP, bool SEP>
 hipError_t launch_density(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
                           const double* dmomi, const double* emomi, const double* dmom, const double* emom,
                           const int* nlist, const double* du, void* Z, double* ehc, double* rho1, int* err,
                           hipStream_t s) {
-    auto k = k_density_mm<T, L, TA, T2, JVP>;
+    auto k = k_density_mm<T, L, TA, T2, JVP, SEP>;
     const size_t lds = (size_t)DensityLds(harmonics_row<T, L>(P.lha), harmonics_row<T, L>(P.lhm), P.nm3,
-                                         P.nr2m * (P.l2m + 1), JVP).size * sizeof(T);
+                                         P.nr2m * (P.l2m + 1), JVP, functions_row<SEP>(P.og, P.nb_a)).size * sizeof(T);
     static bool set = false;
     static size_t limit = 0;
     hipError_t e;
@@ -461,7 +473,7 @@ hipError_t launch_density(const DevParams<T>& P, int natom, const int* off, cons
     return hipGetLastError();
 }
 
-template <typename T, int L, bool JVP, typename... A>
+template <typename T, int L, bool JVP, bool SEP, typename... A>
 hipError_t by_tiles(const DevParams<T>& P, A... a) {
     const int tA = (P.lha * P.nm3 + 15) >> 4, tAll = tA + ((P.nr2m * P.lhm + 15) >> 4);
     int ta = 0, t2 = 0;
@@ -471,10 +483,10 @@ hipError_t by_tiles(const DevParams<T>& P, A... a) {
         const int n2 = ((tAll - w + 3) >> 2) - na;
         t2 = t2 > n2 ? t2 : n2;
     }
-    if (ta <= 1 && t2 <= 1) return launch_density<T, L, 1, 1, JVP>(P, a...);
-    if (ta <= 2 && t2 <= 1) return launch_density<T, L, 2, 1, JVP>(P, a...);
-    if (ta <= 4 && t2 <= 1) return launch_density<T, L, 4, 1, JVP>(P, a...);
-    if (ta <= 4 && t2 <= 3) return launch_density<T, L, 4, 3, JVP>(P, a...);
+    if (ta <= 1 && t2 <= 1) return launch_density<T, L, 1, 1, JVP, SEP>(P, a...);
+    if (ta <= 2 && t2 <= 1) return launch_density<T, L, 2, 1, JVP, SEP>(P, a...);
+    if (ta <= 4 && t2 <= 1) return launch_density<T, L, 4, 1, JVP, SEP>(P, a...);
+    if (ta <= 4 && t2 <= 3) return launch_density<T, L, 4, 3, JVP, SEP>(P, a...);
     return hipErrorInvalidValue;  // no header of the supported classes has more
 }
 
@@ -487,9 +499,13 @@ hipError_t run_density(const DevParams<T>& P, int natom, const int* off, const d
     const int l = P.l3a > P.l2m ? P.l3a : P.l2m;
     const int* no_list = nullptr;
     const double* no_u = nullptr;
-    if (l <= 2) return by_tiles<T, 2, false>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
-    if (l <= 4) return by_tiles<T, 4, false>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
-    return by_tiles<T, 6, false>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+    auto go = [&](auto sep) {
+        constexpr bool SEP = decltype(sep)::value;
+        if (l <= 2) return by_tiles<T, 2, false, SEP>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+        if (l <= 4) return by_tiles<T, 4, false, SEP>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+        return by_tiles<T, 6, false, SEP>(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, no_list, no_u, B.Z, B.ehc, B.rho1, B.err, s);
+    };
+    return P.og > 0 ? go(std::true_type()) : go(std::false_type());
 }
 
 hipError_t run_density_jvp(const DevParams<double>& P, int natom, const int* off, const int* nlist, const double* du,
@@ -498,9 +514,13 @@ hipError_t run_density_jvp(const DevParams<double>& P, int natom, const int* off
     const int l = P.l3a > P.l2m ? P.l3a : P.l2m;
     const double* none = nullptr;
     double* no_rho = nullptr;
-    if (l <= 2) return by_tiles<double, 2, true>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
-    if (l <= 4) return by_tiles<double, 4, true>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
-    return by_tiles<double, 6, true>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+    auto go = [&](auto sep) {
+        constexpr bool SEP = decltype(sep)::value;
+        if (l <= 2) return by_tiles<double, 2, true, SEP>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+        if (l <= 4) return by_tiles<double, 4, true, SEP>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+        return by_tiles<double, 6, true, SEP>(P, natom, off, dlist, elist, none, none, dmom, emom, nlist, du, Zdot, ehc_dot, no_rho, err, s);
+    };
+    return P.og > 0 ? go(std::true_type()) : go(std::false_type());
 }
 
 template hipError_t run_density<double>(const DevParams<double>&, int, const int*, const double*, const double*,

@@ -23,8 +23,11 @@ template <typename T>
 struct DevParams {
     const T* lut_a = nullptr;  // atomic spline rows [nlut][stride_a]
     const T* lut_m = nullptr;  // magnetic spline rows [nlut][stride_m]
-    const T* lut_g = nullptr;  // rows of the base functions g_1..g_nb and the core term alone [nlut][stride_g]
-    const T* cperm = nullptr;  // radial coefficients C_{nlk} as A operands, [l3a + 1][4][64] (density.hip)
+    // rows of the radial factors h_1..h_nf (RadialFactors), the base functions g_1..g_nb and the core term
+    // [nlut][stride_g]; the g begin at function og.  og = 0: the factors are the g, nf = nb_a.
+    const T* lut_g = nullptr;
+    int nf = 0, og = 0;
+    const T* cperm = nullptr;  // coefficients of the factors in R_{l,n} as A operands, [l3a + 1][4][64] (density.hip)
     // columns of the density's products, 16 a tile: of A (Y entry | q << 8 | l << 16), then of A2 (Y' entry | M
     // entry << 8)
     const uint32_t* cols = nullptr;
@@ -33,7 +36,7 @@ struct DevParams {
     // sth meet l' <= l3m): a, b, c, l | m << 8 | first of its order << 16 | harmonic << 17 |
     // l nr2m << 18, firsta and firstm the steps that are some group's first of an order; rows of the tiles of
     // V: column of A | l << 16 | it and y are a pair +m', -m' << 25 | its sine << 26 | its odd m' << 27, column of
-    // A2 | 1 << 24, or ~0; radial coefficients [l3a + 1][8][16]
+    // A2 | 1 << 24, or ~0; coefficients of the factors [l3a + 1][8][16]
     const double* steps = nullptr;
     const uint2* vcol = nullptr;
     const T* crow = nullptr;

@@ -3,7 +3,8 @@
 // k_forces_mm does the work of forcecompute and torquecompute (src/forces.F90:418-623, 688-961).  With
 // V[k][lm,q] = sum_n C_{nlk} W[n][lm][q] once an atom, the pair's weights are
 //   P[lm,q] = sum_k g_k V[k][lm,q],  Q[lm,q] = sum_k g'_k V[k][lm,q]
-// (and the same of A2's W2[k][n'][l'm']), matrix products over at most 16 base functions.  The columns q of a
+// (and the same of A2's W2[k][n'][l'm']), matrix products over at most 16 base functions, or for A over its radial
+// factors h_f with V[f] = sum_n U_{nlf} W[n] (RadialFactors).  The columns q of a
 // pair +m', -m' enter as the real and the imaginary part h of H_{m'} = M Y_{m'} (V of the two columns added and
 // subtracted), which halves the work behind the products:
 //   S = sum_q P h,  dE/dY = S;   dE/dr = Re sum Q h Y;   u_q = dE/dh_q = Re sum_lm P Y.
@@ -13,6 +14,8 @@
 // with four columns of its own.  So neither harmonics nor weights pass through LDS.  A wave holds 16
 // pairs; waves meet only for V.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "device.hpp"
 #include "kernels.hpp"
@@ -91,11 +94,11 @@ struct ForceLds {  // offsets in T
     // rows of n complex values that 16 lanes read at different banks (64 of four bytes)
     __host__ __device__ static int spread(int n, size_t t) { return t == 8 ? n | 1 : n % 4 ? n : n + 1; }
     int tiles, rounds, nqp, oStep, oWave, oM, oP, oE, wave, size;
-    __host__ __device__ ForceLds(int nk, int ta, int nq4, int tm, int steps, bool qsplit, int nfm, int waves, size_t t) {
+    __host__ __device__ ForceLds(int na, int nk, int ta, int nq4, int tm, int steps, bool qsplit, int nfm, int waves, size_t t) {
         rounds = qsplit ? (nq4 + 3) >> 2 : nq4;
         nqp = 4 * (qsplit ? 4 * rounds : nq4);  // columns q with their padding
         tiles = rounds * ta + tm;
-        oStep = 2 * tiles * nk * 64;            // operands of V, complex
+        oStep = 2 * (rounds * ta * na + tm * nk) * 64;  // operands of V, complex
         oWave = oStep + steps * 4;              // a ForceStep is four T
         // of a wave: h, then u [16][nqp], (M, M') [16][spread(nfm)], powers, then results [16][kPowers], directions [16][8]
         oM = 16 * nqp;
@@ -109,7 +112,7 @@ struct ForceLds {  // offsets in T
 }  // namespace
 
 // Workgroup: one atom, up to four waves of 16 pairs (fewer where their LDS does not fit).  NK: steps of four base
-// functions.
+// functions; NA: of four radial factors of A.  SEP: these are functions of their own (DevParams::og).
 //
 // Bound by issue: at 16000 atoms of lmax 6 a wave has 1670 vector instructions and 132 products of 32 cycles
 // (FP32; 64 in FP64), about 11000 cycles of a SIMD, which measures 294 us (FP64 622 us).  One lane a pair, with W
@@ -118,7 +121,7 @@ struct ForceLds {  // offsets in T
 // 320 us), at 128 atoms of lmax 4 in FP64, where a wave's length counts, 36 -> 15 us.  Five waves a SIMD in
 // FP32 need at most 96 registers and 32000 bytes of LDS a workgroup, which the layout below keeps at lmax 6;
 // loading the pairs' inputs before V is made costs the fifth wave and was slower (323 us).
-template <typename T, int NK>
+template <typename T, int NK, int NA, bool SEP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 2, sizeof(T) == 4 ? 5 : 3)))
 k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restrict__ dlist,
             const double* __restrict__ elist, const double* __restrict__ dmomi, const double* __restrict__ emomi,
@@ -134,7 +137,8 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
     const int nthr = blockDim.x, nw = nthr >> 6;
     const int nfm = P.nr2m * (P.l2m + 1), sMs = ForceLds::spread(nfm, sizeof(T));
     const int tm = (P.stm * P.nr2m + 3) >> 2, steps = 4 * (P.sta + P.stm);
-    const ForceLds D(NK, P.sta, (P.nm3 + 3) >> 2, tm, steps, P.qsplit, nfm, nw, sizeof(T));
+    const int og = SEP ? P.og : 0, nf = SEP ? P.nf : P.nb_a;
+    const ForceLds D(NA, NK, P.sta, (P.nm3 + 3) >> 2, tm, steps, P.qsplit, nfm, nw, sizeof(T));
     T* lds = (T*)smem;
     cplx<T>* sV = (cplx<T>*)lds;
     ForceStep<T>* sStep = (ForceStep<T>*)(lds + D.oStep);
@@ -229,21 +233,21 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
                 constexpr int NB = sizeof(T) == 4 ? 2 : 4;
                 for (int n0 = 0; n0 < P.nr3a; n0 += NB) {
                     cplx<T> w[NB], wb[NB];
-                    Coef<T> k[NB][NK];
+                    Coef<T> k[NB][NA];
 #pragma unroll
                     for (int n = 0; n < NB; ++n) {
                         const int o = (n0 + n < P.nr3a ? n0 + n : 0) * nA;
                         w[n] = W[o + c];
                         wb[n] = W[o + cb];
 #pragma unroll
-                        for (int s = 0; s < NK; ++s) k[n][s] = coef_at(cn + 16 * (n0 + n) + 4 * s);
+                        for (int s = 0; s < NA; ++s) k[n][s] = coef_at(cn + 16 * (n0 + n) + 4 * s);
                     }
 #pragma unroll
                     for (int n = 0; n < NB; ++n) {
                         const T ar = fma(sb, wb[n].re, sc * w[n].re), ai = fma(sb, wb[n].im, sc * w[n].im);
                         const T wr = sine ? -ai : ar, wi = sine ? ar : ai;
 #pragma unroll
-                        for (int u = 0; u < 4 * NK; ++u) {
+                        for (int u = 0; u < 4 * NA; ++u) {
                             re[u] = fma(k[n][u / 4].c[u % 4], wr, re[u]);
                             im[u] = fma(k[n][u / 4].c[u % 4], wi, im[u]);
                         }
@@ -251,9 +255,11 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
                 }
             }
         }
-        cplx<T>* o = sV + (x >> 4) * NK * 64 + (x & 15);
+        const int tile = x >> 4, tb = D.rounds * P.sta;
+        cplx<T>* o = sV + (tile < tb ? tile * NA : tb * NA + (tile - tb) * NK) * 64 + (x & 15);
 #pragma unroll
-        for (int u = 0; u < 4 * NK; ++u) o[16 * u] = {re[u], im[u]};
+        for (int u = 0; u < 4 * NK; ++u)
+            if (NA == NK || u < 4 * NA || tile >= tb) o[16 * u] = {re[u], im[u]};
     }
     __syncthreads();
 
@@ -275,21 +281,26 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
             T* o = sE + 8 * ji + 4 * g;
             o[0] = g ? sx : ex, o[1] = g ? sy : ey, o[2] = g ? sz : ez, o[3] = rowa >= 0 ? inv : (T)0;
         }
-        // base functions: lane group g has k = 4 s + g
+        // radial factors, and with SEP later the base functions (n of them from function `first` on): lane group g has
+        // k = 4 s + g
         T gv[NK], gd[NK];
         T fr = 0;  // dE/dr
-        {
-            const T* __restrict__ ga = P.lut_g + (size_t)(rowa < 0 ? 0 : rowa) * P.stride_g;
-            Coef<T> c[NK];
+        const T* __restrict__ ga = P.lut_g + (size_t)(rowa < 0 ? 0 : rowa) * P.stride_g;
+        auto functions = [&](auto steps, int first, int n) {
+            constexpr int N = decltype(steps)::value;
+            Coef<T> c[N];
 #pragma unroll
-            for (int s = 0; s < NK; ++s) c[s] = coef_at(ga + 4 * (4 * s + g < P.nb_a ? 4 * s + g : 0));
-            const Coef<T> cc = coef_at(ga + 4 * P.nb_a);
+            for (int s = 0; s < N; ++s) c[s] = coef_at(ga + 4 * (first + (4 * s + g < n ? 4 * s + g : 0)));
 #pragma unroll
-            for (int s = 0; s < NK; ++s) {
-                const bool on = rowa >= 0 && 4 * s + g < P.nb_a;
+            for (int s = 0; s < N; ++s) {
+                const bool on = rowa >= 0 && 4 * s + g < n;
                 gv[s] = on ? coef_value(c[s], wa) : (T)0;
                 gd[s] = on ? coef_slope(c[s], wa, rsa) : (T)0;
             }
+        };
+        {
+            const Coef<T> cc = coef_at(ga + 4 * (og + P.nb_a));
+            functions(std::integral_constant<int, NA>(), 0, nf);
             if (g == 0 && rowa >= 0) fr = edf * coef_slope(cc, wa, rsa);  // core term
         }
         // M and M' of the pair, spread over its four lanes
@@ -341,13 +352,13 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
                 h[r] = sH[q0 + r];
                 u[r] = 0;
             }
-            const cplx<T>* __restrict__ v = sV + (size_t)rd * P.sta * NK * 64 + lane;
+            const cplx<T>* __restrict__ v = sV + (size_t)rd * P.sta * NA * 64 + lane;
             Walk<T> k;
-            for (int t = 0; t < P.sta; ++t, v += NK * 64) {
+            for (int t = 0; t < P.sta; ++t, v += NA * 64) {
                 const ForceStep<T> st = sStep[4 * t + g];
                 V pr = (V)(T)0, pi = (V)(T)0, qr = (V)(T)0, qi = (V)(T)0;
 #pragma unroll
-                for (int s = 0; s < NK; ++s) {
+                for (int s = 0; s < NA; ++s) {
                     const cplx<T> a = v[64 * s];
                     pr = Mm<T>::mul(a.re, gv[s], pr);
                     pi = Mm<T>::mul(a.im, gv[s], pi);
@@ -375,13 +386,14 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
                 sH[q0 + g] = fold_groups(u);  // the four walks together
             }
         }
+        if constexpr (SEP) functions(std::integral_constant<int, NK>(), og, P.nb_a);
         wave_order();
         put_powers(sP, g, sx, sy);
         wave_order();
         // ---- moments: four (step, n') a tile
         T tr = 0, tx = 0, ty = 0, tz = 0;
         {
-            const cplx<T>* __restrict__ v = sV + (size_t)D.rounds * P.sta * NK * 64 + lane;
+            const cplx<T>* __restrict__ v = sV + (size_t)D.rounds * P.sta * NA * 64 + lane;
             Walk<T> k;
             ForceStep<T> st = {};
             T Sr = 0, Si = 0, S1r = 0, S1i = 0, Rr = 0, Ri = 0;  // sums over n' of M X, M' X, M Q
@@ -459,14 +471,14 @@ k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restric
 
 namespace {
 
-template <typename T, int NK>
+template <typename T, int NK, int NA, bool SEP>
 hipError_t launch_forces(const DevParams<T>& P, int natom, const int* off, const double* dlist, const double* elist,
                          const double* dmomi, const double* emomi, const double* dmom, const double* emom,
                          const Buffers& B, bool scaled, double* flist, double* tlist, double* tlist0, hipStream_t s) {
-    auto k = k_forces_mm<T, NK>;
+    auto k = k_forces_mm<T, NK, NA, SEP>;
     int waves = 4;
     auto bytes = [&] {
-        return (size_t)ForceLds(NK, P.sta, (P.nm3 + 3) >> 2, (P.stm * P.nr2m + 3) >> 2, 4 * (P.sta + P.stm), P.qsplit,
+        return (size_t)ForceLds(NA, NK, P.sta, (P.nm3 + 3) >> 2, (P.stm * P.nr2m + 3) >> 2, 4 * (P.sta + P.stm), P.qsplit,
                                 P.nr2m * (P.l2m + 1), waves, sizeof(T)).size * sizeof(T);
     };
     static bool set = false;
@@ -496,10 +508,16 @@ hipError_t run_forces(const DevParams<T>& P, int natom, const int* off, const do
                       const double* dmomi, const double* emomi, const double* dmom, const double* emom, const Buffers& B,
                       bool scaled, double* flist, double* tlist, double* tlist0, hipStream_t s) {
     auto go = [&](auto k) { return k(P, natom, off, dlist, elist, dmomi, emomi, dmom, emom, B, scaled, flist, tlist, tlist0, s); };
-    if (P.nb_a <= 4) return go(launch_forces<T, 1>);
-    if (P.nb_a <= 8) return go(launch_forces<T, 2>);
-    if (P.nb_a <= 12) return go(launch_forces<T, 3>);
-    return go(launch_forces<T, 4>);
+    if (P.og > 0) {
+        if (P.nb_a <= 4) return go(launch_forces<T, 1, 1, true>);
+        if (P.nb_a <= 8) return go(launch_forces<T, 2, 2, true>);
+        if (P.nb_a <= 12) return P.nf <= 8 ? go(launch_forces<T, 3, 2, true>) : go(launch_forces<T, 3, 3, true>);
+        return P.nf <= 8 ? go(launch_forces<T, 4, 2, true>) : go(launch_forces<T, 4, 4, true>);
+    }
+    if (P.nb_a <= 4) return go(launch_forces<T, 1, 1, false>);
+    if (P.nb_a <= 8) return go(launch_forces<T, 2, 2, false>);
+    if (P.nb_a <= 12) return go(launch_forces<T, 3, 3, false>);
+    return go(launch_forces<T, 4, 4, false>);
 }
 
 template hipError_t run_forces<double>(const DevParams<double>&, int, const int*, const double*, const double*,

@@ -213,12 +213,40 @@ struct Splines {
     std::vector<double> magnetic;
 };
 
+// The atomic radial functions R_{l,n} = sum_k C_{nlk} g_k as sums over at most nb_a factors h, R_{l,n} = sum_f U_{nlf}
+// h_f.  The C of a fitted potential cancel (sum |C g| is 21 times |R| in the example
+// potential, hundreds of times in a fit to narrow functions), so that g and C rounded to 32 bits lose what the sum in 64
+// bits behind a table of R keeps.  Where there are no more R than g the factors are the R themselves, in FP64
+// too, whose results then are those of the table of R (example potential, pair forces: 5e-15 from the reference and 5e-12
+// through g, which is what the reference's rounded table differs from its own g by).  Otherwise, in FP32, U
+// has orthonormal columns over the R, each scaled by its size (a QR decomposition of C), so that no term of
+// the sum is larger than the R together.  Relative rms errors of R in 32 bits (U and h rounded, sum in FP32):
+// table of R 3.6e-8; through g, random C 1.1e-7 to 2.0e-7, fits 1.2e-5 to 4.5e-5; through h 0.8e-7 to 0.9e-7 for
+// either.
+//
+// The factors stand beside the g, which A2 needs, and their lookups take 2 to 5% of an evaluation.  With more R than g
+// they are left out (nf = 0: the factors are the g) while the root mean square over the R of |terms C g| / |R| is at
+// most kFactorLine.  Errors of energies, forces, torques and self torques against 64 bits, 128 atoms, table of R /
+// through g / factors in 1e-7: lmax 4 at 2.4 2.3 2.5 2.9 2.3 / 2.0 2.2 2.2 1.8 / 2.0 2.3 2.2 2.1, at 4.3 3.1 2.5 2.6
+// 3.3 / 3.2 3.3 2.6 3.6 / 2.0 2.2 2.0 2.2; lmax 6 at 3.0 14.9 7.5 6.7 11.4 / 10.7 6.7 5.3 9.3 / 9.5 6.7 5.4 8.6, at 4.2
+// 4.1 4.1 3.6 4.4 / 3.8 4.5 3.1 4.2 / 2.4 3.7 2.7 3.0; a fit to narrow functions at lmax 6, 2.8 6.4 7.1 3.1 / 350 310
+// 360 320 / 2.3 5.3 5.7 2.3.  With no more R than g they always pay: example potential's shape at 2.8, 1.8 4.4 4.0 6.8 /
+// 2.1 7.9 7.3 16.9 / 0.9 1.8 1.6 1.8.
+constexpr double kFactorLine = 3.0;
+struct RadialFactors {
+    int nf = 0;
+    bool own = false;           // the factors are the R themselves
+    std::vector<double> u;      // [nr3_a][l3a + 1][nf]
+    std::vector<double> table;  // [nlut][nf][4], as Splines::atomic
+};
+
 struct Model {
     Potential pot;
     ZLayout z;
     TermList terms;
     NodePlan nodes;
     Splines spl;
+    RadialFactors factors;
 };
 
 // api.cpp: the library's last-error state (magace_last_error / magace_error_string)
@@ -259,5 +287,6 @@ void radial_basis(int radtype, double lambda, int nb, double cut, double dcut, d
                   double* g, double* dg);
 void core_repulsion(double r, double pre, double lambda, double cut, double& cr, double& dcr);
 Splines build_splines(const Potential& pot);
+RadialFactors radial_factors(const Potential& pot, const Splines& S);
 
 }  // namespace magace

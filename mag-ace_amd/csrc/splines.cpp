@@ -171,4 +171,76 @@ Splines build_splines(const Potential& pot) {
     return S;
 }
 
+RadialFactors radial_factors(const Potential& pot, const Splines& S) {
+    const Header& h = pot.h;
+    const int nb = h.nb_a, nr = h.nr3_a * (h.l3a + 1);
+    RadialFactors F;
+    if (nr == 0) return F;
+    const double* C = pot.crad_a.data();
+    // mean squares over the distances at which atoms have neighbours, a third of the cutoff and more, of each R and of
+    // the terms C g that it is the sum of
+    std::vector<double> size(nr, 0.0), terms(nr, 0.0);
+    const int first = S.nlut / 3;
+    for (int n = first; n < S.nlut; ++n) {
+        const double* g = S.atomic.data() + (size_t)n * S.atomic_stride;
+        for (int i = 0; i < nr; ++i) {
+            double r = 0.0;
+            for (int k = 0; k < nb; ++k) {
+                const double t = C[(size_t)i * nb + k] * g[4 * k];
+                r += t;
+                terms[i] += t * t;
+            }
+            size[i] += r * r;
+        }
+    }
+    double lost = 0.0;
+    for (int i = 0; i < nr; ++i) lost += size[i] > 0.0 ? terms[i] / size[i] : 1.0;
+    if (nr > nb && lost <= kFactorLine * kFactorLine * nr) return F;
+    F.nf = std::min(nb, nr);
+    F.own = nr <= nb;
+    F.u.assign((size_t)nr * F.nf, 0.0);
+    std::vector<double> q((size_t)nr * F.nf, 0.0);  // h_f = sum_i q[i][f] R_i
+    if (F.own) {
+        for (int i = 0; i < nr; ++i) F.u[(size_t)i * nr + i] = q[(size_t)i * nr + i] = 1.0;
+    } else {
+        for (double& v : size) v = v > 0.0 ? std::sqrt(v / (S.nlut - first)) : 1.0;
+        // Gram-Schmidt, each column twice: the columns of C / size; one in the span of those before it adds nothing
+        for (int f = 0; f < nb; ++f) {
+            std::vector<double> c(nr);
+            double whole = 0.0, rest = 0.0;
+            for (int i = 0; i < nr; ++i) {
+                c[i] = C[(size_t)i * nb + f] / size[i];
+                whole += c[i] * c[i];
+            }
+            for (int pass = 0; pass < 2; ++pass)
+                for (int e = 0; e < f; ++e) {
+                    double d = 0.0;
+                    for (int i = 0; i < nr; ++i) d += q[(size_t)i * nb + e] * c[i];
+                    for (int i = 0; i < nr; ++i) c[i] -= d * q[(size_t)i * nb + e];
+                }
+            for (int i = 0; i < nr; ++i) rest += c[i] * c[i];
+            if (rest <= 1e-28 * whole) continue;
+            for (int i = 0; i < nr; ++i) q[(size_t)i * nb + f] = c[i] / std::sqrt(rest);
+        }
+        for (int i = 0; i < nr; ++i)
+            for (int f = 0; f < nb; ++f) {
+                F.u[(size_t)i * nb + f] = q[(size_t)i * nb + f] * size[i];
+                q[(size_t)i * nb + f] /= size[i];
+            }
+    }
+    // from the rows of the R, so that the factors have their rounding and none of the cancelling sums'
+    F.table.assign((size_t)S.nlut * F.nf * 4, 0.0);
+    for (int n = 0; n < S.nlut; ++n)
+        for (int i = 0; i < nr; ++i) {
+            const double* r = S.atomic.data() + (size_t)n * S.atomic_stride + 4 * (nb + i % (h.l3a + 1) * h.nr3_a + i / (h.l3a + 1));
+            for (int f = 0; f < F.nf; ++f) {
+                const double v = q[(size_t)i * F.nf + f];
+                if (v == 0.0) continue;
+                double* o = F.table.data() + ((size_t)n * F.nf + f) * 4;
+                for (int u = 0; u < 4; ++u) o[u] += v * r[u];
+            }
+        }
+    return F;
+}
+
 }  // namespace magace
