@@ -75,8 +75,9 @@ int magace_get_precision(void);
  * 0..2; split 0 = automatic, 1..8.
  * magace_tune times MAGACE_TUNE_CANDIDATES (variant, split) candidates on the caller's
  * device-resident system (magace_compute_device arguments, reps evaluations each, on `stream`)
- * for the current precision, writes the average milliseconds per evaluation into ms[] (-1:
- * candidate not available for this potential), keeps the fastest and returns it in best[2]. */
+ * in MAGACE_MIXED_ACC, writes the average milliseconds per evaluation into ms[] (-1: candidate not
+ * available for this potential), keeps the fastest and returns it in best[2].  In the other precisions
+ * every candidate is the same evaluation: ms[] holds its time, the setting stays and is returned. */
 #define MAGACE_TUNE_CANDIDATES 9
 int magace_set_tuning(const int *v, int n);
 int magace_get_tuning(int *v, int n);

@@ -178,8 +178,8 @@ def get_tuning():
 
 def tune(natom, nei, offsets, dlist, elist, dmomi, emomi, dmom, emom, eout, flist, tlist, tlist0, reps=5,
          stream=0):
-    """Times the density variants on device arrays for the current precision and keeps the
-    fastest.  Returns (best (variant, split), {candidate: ms per evaluation or None})."""
+    """Times the density variants on device arrays and keeps the fastest, in MIXED_ACC (in the other
+    precisions there is nothing to choose and the setting stays).  Returns (best (variant, split), {candidate: ms per evaluation or None})."""
     ms = np.zeros(len(TUNE_CANDIDATES))
     best = np.zeros(2, np.int32)
     rc = lib().magace_tune(natom, nei, offsets, dlist, elist, dmomi, emomi, dmom, emom, eout, flist, tlist, tlist0,

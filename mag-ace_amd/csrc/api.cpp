@@ -148,9 +148,9 @@ struct Context {
 
 std::unique_ptr<Context> g_ctx;
 
-// Tuned density variants per potential header, measured on MI355X by mag-ace_amd/tune.py
-// (which writes tuning_table.inc and the record tuning.json); headers not listed use the
-// built-in rule.
+// Tuned variants of the accumulation recipe's density per potential header, measured on MI355X by
+// mag-ace_amd/tune.py (which writes tuning_table.inc and the record tuning.json); headers not listed use the
+// built-in rule.  FP64 has no variants: its column is kept for magace_get_tuning alone.
 struct TuneEntry {
     int hdr[12];  // nb_a nb_m nr2_m l2m nr3_a nr3_m l3a l3m nr4_a nr4_m l4a l4m
     int fp64[2];  // variant, neighbour split
@@ -1167,7 +1167,16 @@ int magace_tune(int natom, int nei, const int* offsets, const double* dlist, con
     }
     Context& c = *g_ctx;
     hipStream_t s = (hipStream_t)stream;
+    // Only the accumulation recipe's density has variants.  The others' setting changes nothing, so that there is
+    // nothing to choose: one measurement stands for every candidate and the setting stays, the recipe's above all.
+    const bool choose = c.precision == MAGACE_MIXED_ACC;
     const int p = c.precision == MAGACE_FP64 ? 0 : 1;
+    const int was[2] = {c.dvar[p], c.dsplit[p]};
+    auto set = [&](int variant, int split) {
+        c.dvar[p] = variant;
+        c.dsplit[p] = split;
+        (p ? c.P32.sa : c.P64.sa) = split;
+    };
     // (variant, neighbour split) candidates, MAGACE_TUNE_CANDIDATES of them
     static const int cand[MAGACE_TUNE_CANDIDATES][2] = {{0, 0}, {1, 1}, {1, 2}, {1, 3}, {1, 4},
                                                         {2, 1}, {2, 2}, {2, 3}, {2, 4}};
@@ -1176,10 +1185,9 @@ int magace_tune(int natom, int nei, const int* offsets, const double* dlist, con
     HIPCHK(hipEventCreate(&e1));
     int bi = -1;
     for (int k = 0; k < MAGACE_TUNE_CANDIDATES; ++k) {
-        c.dvar[p] = cand[k][0];
-        c.dsplit[p] = cand[k][1];
-        (p ? c.P32.sa : c.P64.sa) = cand[k][1];
-        ms[k] = -1.0;
+        ms[k] = choose || k == 0 ? -1.0 : ms[0];
+        if (!choose && k > 0) continue;
+        if (choose) set(cand[k][0], cand[k][1]);
         // a variant whose LDS does not fit this potential fails at launch and is skipped
         int rc = run_device(c, natom, offsets, dlist, elist, dlist_momi, elist_momi, dlist_mom, elist_mom, eout,
                             flist, tlist, tlist0, s);
@@ -1207,15 +1215,16 @@ int magace_tune(int natom, int nei, const int* offsets, const double* dlist, con
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (bi < 0) {
+        set(was[0], was[1]);
         set_error(MAGACE_ERR_DEVICE, "magace_tune: no variant ran");
         return MAGACE_ERR_DEVICE;
     }
-    c.dvar[p] = cand[bi][0];
-    c.dsplit[p] = cand[bi][1];
-    (p ? c.P32.sa : c.P64.sa) = cand[bi][1];
-    best[0] = cand[bi][0];
-    best[1] = cand[bi][1];
-    bump_generation();
+    if (choose) {
+        set(cand[bi][0], cand[bi][1]);
+        bump_generation();
+    }
+    best[0] = c.dvar[p];
+    best[1] = c.dsplit[p];
     return 0;
 }
 

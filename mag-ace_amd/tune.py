@@ -1,10 +1,10 @@
-"""Sweep of the density kernel's variants per potential header; writes the tuning table.
+"""Sweep of the variants of the accumulation recipe's density per potential header; writes the tuning table.
 
-For each header below and both precisions, magace_tune times every (variant, neighbour split)
-candidate on the 16000-atom bcc Fe workload (20x20x20 cells, jitter N(0, 0.05 A), cone spins,
+For each header below magace_tune times every (variant, neighbour split) candidate in MIXED_ACC, the one precision
+that has them, on the 16000-atom bcc Fe workload (20x20x20 cells, jitter N(0, 0.05 A), cone spins,
 r_c 5.0 A, seed 2028), twice; the per-candidate minimum decides.  Results go to
 
-  mag-ace_amd/tuning.json          the record: per header and precision, ms per evaluation of
+  mag-ace_amd/tuning.json          the record: per header, ms per evaluation of
                                    every candidate, the choice and the built-in rule's time;
   mag-ace_amd/csrc/tuning_table.inc the table compiled into libmagace.so (rebuild after).
 
@@ -62,8 +62,8 @@ def main():
         potgen.write(pot, h, capi.enumerate_basis(h), 2028)
         capi.init_file(pot)
         entry = {"header": [int(h[k]) for k in KEYS]}
-        choice = {}
-        for prec, mode in (("fp64", capi.FP64), ("mixed", capi.MIXED)):
+        choice = {"fp64": (-1, 0)}  # none to choose
+        for prec, mode in (("mixed_acc", capi.MIXED_ACC),):
             capi.set_precision(mode)
             # the built-in rule first, as the reference point
             capi.set_tuning()
@@ -85,13 +85,13 @@ def main():
         capi.set_precision(capi.FP64)
         record["headers"][name] = entry
         lines.append("{{%s}, {%d, %d}, {%d, %d}},  // %s" % (", ".join(str(v) for v in entry["header"]),
-                                                           *choice["fp64"], *choice["mixed"], name))
+                                                           *choice["fp64"], *choice["mixed_acc"], name))
     os.makedirs(os.path.join(args.out, "csrc"), exist_ok=True)
     with open(os.path.join(args.out, "tuning.json"), "w") as f:
         json.dump(record, f, indent=1)
     with open(os.path.join(args.out, "csrc", "tuning_table.inc"), "w") as f:
         f.write("// Written by mag-ace_amd/tune.py from measurements on MI355X (record: mag-ace_amd/tuning.json).\n"
-                "// One line per potential header: {header}, {FP64 variant, split}, {mixed variant, split}.\n")
+                "// One line per potential header: {header}, {FP64 variant, split} (none), {MIXED_ACC variant, split}.\n")
         f.write("\n".join(lines) + "\n")
 
 
