@@ -1467,8 +1467,10 @@ void acelib_(int* natom, int* nall, int* nei, int* nlist, int* occ, int* occlist
     if (nchunk == 1 && need_in <= kOneStreamBytes) {
         // Inputs and outputs cross by a kernel, the flags with them: the copy engine's transfers, the events between
         // three streams and the copy of the flags cost a small call more than its evaluation does.  Here and by the
-        // pipeline (FP64, us): lmax 4 54 atoms 85 and 154, 432 atoms 184 and 235, 1024 atoms (3.9 MB) 328 and 383; lmax 6
-        // 395 and 438.  From 98304 pairs a call has several chunks, whose copies overlap.
+        // pipeline (FP64, us): lmax 4 54 atoms 85 and 154, 432 atoms 197 and 256, 1024 atoms (3.9 MB) 337 and 391; lmax 6
+        // 407 and 458.  The line is the largest size that was measured when it was drawn, not where the two meet: at 1620
+        // atoms (92884 pairs, 6.2 MB) one stream would take 475 and 603 us, the pipeline takes 537 and 656.  From 98304
+        // pairs a call has several chunks, whose copies overlap.
         const Context::Slot& sl = c.slots[0];
         pack(0);
         int* flag = (int*)(sl.h_out + need_out - 16);
