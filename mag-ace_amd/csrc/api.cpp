@@ -560,8 +560,11 @@ int upload_kept(std::vector<void*>& kept, D*& dst, const V& v) {
     return 0;
 }
 
-// the fitting plan, built when a fit asks for its first gradient
+// the fitting plan, built when a fit asks for its first gradient; a call after one that failed on its way starts anew
 int upload_fit_plan(Context& c) {
+    for (void*& p : c.fit_mem) dfree(p);
+    c.fit_mem.clear();
+    dfree(c.fit.ub_ptr); dfree(c.fit.ub_t); dfree(c.fit.ub_u);
     FitPlan F;
     try {
         F = build_fit_plan(c.model.z, c.model.terms);
