@@ -1807,7 +1807,7 @@ int magace_fit_backward(int natom, int nei, const int* offsets, const int* nlist
                         (int)bs.b6.size()};
     Buffers B = c.buf;
     B.Wd = F.Wd;
-    HIPCHK(fit_backward(c.P64, !c.model.nodes.ok, c.shape_class, natom, offsets, nlist, gF, dlist, elist, dlist_momi, dlist_mom,
+    HIPCHK(fit_backward(c.P64, !c.model.nodes.ok, natom, offsets, nlist, gF, dlist, elist, dlist_momi, dlist_mom,
                         elist_mom, gE ? atom_struct : nullptr, gE, B, F, (int)T.nterms(), nbo, grad, s));
     return 0;
 }

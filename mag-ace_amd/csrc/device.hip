@@ -2,21 +2,20 @@
 //
 // One evaluation (the work of libace's acelib_, src/ace.F90:280-286) is three launches:
 //
-//   k_density  (prepA, src/a_basis.F90:59-359)   one workgroup per atom.  Pair radial
-//              functions and Y_lm of the bond and of the neighbour moment are staged in LDS
+//   density    (prepA, src/a_basis.F90:59-359) k_density_mm (density.hip), for the accumulation recipe k_density
+//              (here): one workgroup per atom writes Z = [A | A2 | A0], the core sum and the B1 part of rho.
+//              k_density stages pair radial functions and Y_lm of the bond and of the neighbour moment in LDS
 //              for a chunk of neighbours; threads then own (lm, n-block) columns of A and
-//              (l'm', n-block) columns of A2 and accumulate in registers.  Writes
-//              Z = [A | A2 | A0] per atom, the core sum and the B1 part of rho.
-//   k_adjoint_nodes (prepB + forceweights, src/b_basis.F90:62-307, src/forces.F90:84-349; adjoint.hip)
-//              for one density and body orders up to 4; otherwise, and for the accumulation recipe,
-//   k_adjoint  one workgroup per atom (two in FP32).  Z and dZ in LDS; each thread sums
-//              chunks of gradient records w*Z[a]Z[b]Z[c] per target (the transposed
+//              (l'm', n-block) columns of A2 and accumulate in registers.
+//   adjoint    (prepB + forceweights, src/b_basis.F90:62-307, src/forces.F90:84-349) k_adjoint_nodes (adjoint.hip)
+//              for one density and body orders up to 4; otherwise, and for the accumulation recipe, k_adjoint and
+//              k_adjoint_pair (here): one workgroup per atom, or two atoms in FP32.  Z and dZ in LDS; each thread
+//              sums chunks of gradient records w*Z[a]Z[b]Z[c] per target (the transposed
 //              monomial table), partial sums meet in a fixed order (no atomics); then rho,
 //              E_i, dE/drho and the scaled gradient W = dE/dZ are written.
-//   k_forces   (forcecompute + torquecompute, src/forces.F90:418-623, 688-961) one lane per
-//              pair.  Splines and Y_lm are recomputed in registers (nothing per pair is
-//              stored between launches); F_p = dE_i/du_p and T_p = dE_i/dm_j are
-//              contractions of W with the pair's derivatives; lane 0 adds T0_i = dE_i/dm_i.
+//   forces     (forcecompute + torquecompute, src/forces.F90:418-623, 688-961) k_forces_mm (forces.hip): nothing per
+//              pair is stored between launches; F_p = dE_i/du_p, T_p = dE_i/dm_j and T0_i = dE_i/dm_i are
+//              contractions of W with the pair's derivatives.
 //
 // T = double (FP64 path) or float (mixed path: FP32 splines, Y_lm, A, B products; FP64 for
 // rho, the energy and all outputs).
@@ -32,49 +31,27 @@ namespace magace {
 constexpr int kLmaxC = 12;
 constexpr int kLhC = (kLmaxC + 1) * (kLmaxC + 2) / 2;
 
-// Legendre recursion coefficients (src/spherical.F90:18-49): a_lm, b_lm (m <= l-2), c_l, d_l
-__constant__ double c_alm_d[kLhC], c_blm_d[kLhC], c_cl_d[kLmaxC + 1], c_dl_d[kLmaxC + 1];
-__constant__ float c_alm_f[kLhC], c_blm_f[kLhC], c_cl_f[kLmaxC + 1], c_dl_f[kLmaxC + 1];
-
-template <typename T> struct LegC;
-template <> struct LegC<double> {
-    __device__ static double a(int k) { return c_alm_d[k]; }
-    __device__ static double b(int k) { return c_blm_d[k]; }
-    __device__ static double c(int l) { return c_cl_d[l]; }
-    __device__ static double d(int l) { return c_dl_d[l]; }
-};
-template <> struct LegC<float> {
-    __device__ static float a(int k) { return c_alm_f[k]; }
-    __device__ static float b(int k) { return c_blm_f[k]; }
-    __device__ static float c(int l) { return c_cl_f[l]; }
-    __device__ static float d(int l) { return c_dl_f[l]; }
-};
+// Legendre recursion coefficients of k_density (src/spherical.F90:18-49): a_lm, b_lm (m <= l-2), c_l, d_l
+__constant__ float c_alm[kLhC], c_blm[kLhC], c_cl[kLmaxC + 1], c_dl[kLmaxC + 1];
 
 hipError_t upload_legendre_constants() {
-    double a[kLhC] = {0}, b[kLhC] = {0}, c[kLmaxC + 1] = {0}, d[kLmaxC + 1] = {0};
-    float af[kLhC], bf[kLhC], cf[kLmaxC + 1], df[kLmaxC + 1];
+    float a[kLhC] = {0}, b[kLhC] = {0}, c[kLmaxC + 1] = {0}, d[kLmaxC + 1] = {0};
     for (int l = 1; l <= kLmaxC; ++l) {
         const double lsq = (double)(l * l), l1 = 4.0 * lsq - 1.0, l2 = lsq - 2.0 * l + 1.0;
         for (int m = 0; m <= l - 2; ++m) {
             const double msq = (double)(m * m);
             const int k = l * (l + 1) / 2 + m;
-            a[k] = std::sqrt(l1 / (lsq - msq));
-            b[k] = -std::sqrt((l2 - msq) / (4.0 * l2 - 1.0));
+            a[k] = (float)std::sqrt(l1 / (lsq - msq));
+            b[k] = (float)-std::sqrt((l2 - msq) / (4.0 * l2 - 1.0));
         }
-        c[l] = -std::sqrt(1.0 + 0.5 / (double)l);
-        d[l] = std::sqrt(2.0 * (double)(l - 1) + 3.0);
+        c[l] = (float)-std::sqrt(1.0 + 0.5 / (double)l);
+        d[l] = (float)std::sqrt(2.0 * (double)(l - 1) + 3.0);
     }
-    for (int i = 0; i < kLhC; ++i) af[i] = (float)a[i], bf[i] = (float)b[i];
-    for (int i = 0; i <= kLmaxC; ++i) cf[i] = (float)c[i], df[i] = (float)d[i];
     hipError_t e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_alm_d), a, sizeof a))) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_blm_d), b, sizeof b))) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_cl_d), c, sizeof c))) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_dl_d), d, sizeof d))) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_alm_f), af, sizeof af))) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_blm_f), bf, sizeof bf))) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_cl_f), cf, sizeof cf))) return e;
-    return hipMemcpyToSymbol(HIP_SYMBOL(c_dl_f), df, sizeof df);
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_alm), a, sizeof a))) return e;
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_blm), b, sizeof b))) return e;
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_cl), c, sizeof c))) return e;
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_dl), d, sizeof d);
 }
 
 // ---------------------------------------------------------------- small helpers
@@ -96,28 +73,23 @@ __device__ __forceinline__ void horner(const T* __restrict__ c, T w, T rs, T& v,
     dv = fma(w, fma(w, (T)3 * c3, (T)2 * c2), c1) * rs;
 }
 
-// The four coefficients of one spline function as one or two 16-byte loads (rows and functions
-// are 16-byte aligned: 4 coefficients per function)
+// The four coefficients of one spline function as one 16-byte load (rows and functions are 16-byte aligned)
 __device__ __forceinline__ void load_coef(const float* __restrict__ p, float (&c)[4]) {
     const float4 v = *(const float4*)p;
     c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
 }
-__device__ __forceinline__ void load_coef(const double* __restrict__ p, double (&c)[4]) {
-    const double2 a = *(const double2*)p, b = *(const double2*)(p + 2);
-    c[0] = a.x; c[1] = a.y; c[2] = b.x; c[3] = b.y;
-}
 
 // Values of the spline functions koff + k, k0 <= k < k1, of one table row at fraction w
-// (horner's value, in the same operation order), with the coefficient loads of eight functions
-// (four in FP64) issued together so that one trip to L2 serves them all instead of one; dflt for every
-// function when the row is absent.  put(k, v) stores each.  `safe` is any readable coefficient
-// address, read in place of the row's where a function is past k1 or the row is absent.
-template <typename T, typename F>
-__device__ __forceinline__ void spline_values(const T* __restrict__ row, const T* __restrict__ safe, T w, int k0,
-                                              int k1, int koff, T dflt, F&& put) {
-    constexpr int B = sizeof(T) == 4 ? 8 : 4;  // FP64: four functions (32 registers) at a time
+// (horner's value, in the same operation order), with the coefficient loads of eight functions issued together
+// so that one trip to L2 serves them all instead of one; dflt for every function when the row is absent.
+// put(k, v) stores each.  `safe` is any readable coefficient address, read in place of the row's where a
+// function is past k1 or the row is absent.
+template <typename F>
+__device__ __forceinline__ void spline_values(const float* __restrict__ row, const float* __restrict__ safe, float w,
+                                              int k0, int k1, int koff, float dflt, F&& put) {
+    constexpr int B = 8;
     for (int k = k0; k < k1; k += B) {
-        T c[B][4];
+        float c[B][4];
 #pragma unroll
         for (int u = 0; u < B; ++u) load_coef(row && k + u < k1 ? row + 4 * (koff + k + u) : safe, c[u]);
 #pragma unroll
@@ -153,43 +125,36 @@ __device__ __forceinline__ const T* magnetic_row(const DevParams<T>& P, double m
     return P.lut_m + (size_t)((int)fl - 1) * P.stride_m;
 }
 
-// Normalised associated Legendre functions P[lh], dP[lh] = dP/dz for l <= L, m <= l
+// Normalised associated Legendre functions P[lh] for l <= L, m <= l
 // (src/spherical.F90:55-155); lh = l(l+1)/2 + m.  Y_lm(x,y,z) = P[lh] (x+iy)^m.
-template <typename T, int L>
-__device__ __forceinline__ void legendre(T z, T* P, T* dP) {
-    P[0] = (T)1;
-    dP[0] = (T)0;
+template <int L>
+__device__ __forceinline__ void legendre(float z, float* P) {
+    P[0] = 1.0f;
     if (L == 0) return;
-    const T sq3 = (T)1.73205080756887719318, sq3o2 = (T)1.22474487139158894067;
+    const float sq3 = (float)1.73205080756887719318, sq3o2 = (float)1.22474487139158894067;
     P[1] = sq3 * z;
-    dP[1] = sq3;
     P[2] = -sq3o2;
-    dP[2] = (T)0;
 #pragma unroll
     for (int l = 2; l <= L; ++l) {
 #pragma unroll
         for (int m = 0; m <= l - 2; ++m) {
             const int k = l * (l + 1) / 2 + m, k1 = (l - 1) * l / 2 + m, k2 = (l - 2) * (l - 1) / 2 + m;
-            const T a = LegC<T>::a(k), b = LegC<T>::b(k);
-            P[k] = a * fma(z, P[k1], b * P[k2]);
-            dP[k] = a * (P[k1] + fma(z, dP[k1], b * dP[k2]));
+            P[k] = c_alm[k] * fma(z, P[k1], c_blm[k] * P[k2]);
         }
         const int kp = (l - 1) * l / 2 + (l - 1);
-        const T t = LegC<T>::d(l) * P[kp];
+        const float t = c_dl[l] * P[kp];
         P[l * (l + 1) / 2 + l - 1] = t * z;
-        dP[l * (l + 1) / 2 + l - 1] = t;
-        P[l * (l + 1) / 2 + l] = LegC<T>::c(l) * P[kp];
-        dP[l * (l + 1) / 2 + l] = (T)0;
+        P[l * (l + 1) / 2 + l] = c_cl[l] * P[kp];
     }
 }
 
 // half set of Y_lm (m >= 0) written to out[lh]
-template <typename T, int L>
-__device__ __forceinline__ void ylm_half(T x, T y, T z, int lmax, cplx<T>* out) {
-    T P[(L + 1) * (L + 2) / 2], dP[(L + 1) * (L + 2) / 2];
-    legendre<T, L>(z, P, dP);
-    cplx<T> ph = {1, 0};
-    const cplx<T> e = {x, y};
+template <int L>
+__device__ __forceinline__ void ylm_half(float x, float y, float z, int lmax, cplx<float>* out) {
+    float P[(L + 1) * (L + 2) / 2];
+    legendre<L>(z, P);
+    cplx<float> ph = {1, 0};
+    const cplx<float> e = {x, y};
 #pragma unroll
     for (int m = 0; m <= L; ++m) {
 #pragma unroll
@@ -212,12 +177,8 @@ __device__ __forceinline__ cplx<T> yfull(const cplx<T>* half, int l, int m) {
 // ============================================================================ k_density
 // Shapes: NB n-block of A columns, NM3X max magnetic columns of A, NB2 n-block of A2,
 // NR2X max magnetic radial index of A2.
-// Shape class 0: 4 waves per SIMD in FP32 (128 registers; with the eight-function spline
-// batches 127 are used, and 5 waves at 96 registers spilled and ran no faster) and 3 in FP64
-// (168 registers; at 169 the occupancy halves and the kernel takes 1.85 instead of 1.39 ms).  Class 1 (27
-// magnetic columns): 3 waves per SIMD in FP32 (168 registers, a 12-byte spill; on the shape
-// of the example potential 0.75 -> 0.57 ms) and 2 in FP64 (256 registers with a 192-byte
-// spill instead of 302 registers at 1 wave: 2.06 -> 1.33 ms).
+// FP32 sums with Kahan compensation (the accumulation recipe): 153 to 156 registers in shape class 0, three waves
+// per SIMD; 239 to 256 in the others, two.
 // Stores of the m >= 0 density tasks: A[n][l,m][q] for the task's radial block, A2[n][n'][l',m'], in the
 // places of ZLayout::half.
 template <typename T, int NB, int NM3X, int NACC, int NQ>
@@ -294,7 +255,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
             sMc[k - P.nb_m] = v;
     }
     if (tid == nthr - 64) {
-        ylm_half<T, L>((T)emomi[3 * atom], (T)emomi[3 * atom + 1], (T)emomi[3 * atom + 2], P.l2m, sYc);
+        ylm_half<L>((T)emomi[3 * atom], (T)emomi[3 * atom + 1], (T)emomi[3 * atom + 2], P.l2m, sYc);
         *sEhc = 0.0;
     }
     __syncthreads();
@@ -362,8 +323,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
         if (isA) { lh = ta % P.lha; n0 = (ta / P.lha) * NB; }
         if (isA2) { lh = (task - a2base) % P.lhm; n0 = ((task - a2base) / P.lhm) * NB2; }
         while ((l + 1) * (l + 2) / 2 <= lh) ++l;
-        const int m = lh - l * (l + 1) / 2;  // >= 0
-        const int lm = l * l + l + m;
 
         for (int c0 = 0; c0 < nn; c0 += CH) {
             const int nj = nn - c0 < CH ? nn - c0 : CH;
@@ -399,7 +358,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
 #pragma unroll
                             for (int lp = 0; lp < 2; ++lp)
                                 load_coef(!bond && row && lp <= P.l3m ? row + 4 * (P.nb_m + lp * P.nr2m) : P.lut_m, cmh[lp]);
-                        ylm_half<T, L>((T)v3[3 * p], (T)v3[3 * p + 1], (T)v3[3 * p + 2], bond ? P.l3a : P.l2m, yo);
+                        ylm_half<L>((T)v3[3 * p], (T)v3[3 * p + 1], (T)v3[3 * p + 2], bond ? P.l3a : P.l2m, yo);
                         if (!bond) {
                             // H_q = M_{l',n'} Y_{l'm'} for the magnetic columns of A (l' <= l3m,
                             // q = n' lsm3 + l'^2 + l' + m'); the few M it needs are evaluated
@@ -431,7 +390,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         if (k0 < nf) {
                             T w = 0;
                             const T* row = atomic_row(P, dlist[p], w, err);
-                            spline_values<T>(row, P.lut_a, w, k0, min(k1, nf), 0, (T)0, [&](int k, T v) {
+                            spline_values(row, P.lut_a, w, k0, min(k1, nf), 0, (T)0, [&](int k, T v) {
                                 if (k < P.nb_a)
                                     sG[j * sGs + k] = v;
                                 else
@@ -442,7 +401,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                             T w = 0;
                             bool unit;
                             const T* row = magnetic_row(P, dmom[p], w, unit, err);
-                            spline_values<T>(row, P.lut_m, w, max(k0, nf), k1, P.nb_m - nf, unit ? (T)1 : (T)0,
+                            spline_values(row, P.lut_m, w, max(k0, nf), k1, P.nb_m - nf, unit ? (T)1 : (T)0,
                                              [&](int k, T v) { sM[j * sMs + (k - nf)] = v; });
                         }
                     }
@@ -456,7 +415,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         const int p = p0 + c0 + j;
                         T w = 0;
                         const T* row = atomic_row(P, dlist[p], w, err);
-                        spline_values<T>(row, P.lut_a, w, 0, P.nb_a + nfa, 0, (T)0, [&](int k, T v) {
+                        spline_values(row, P.lut_a, w, 0, P.nb_a + nfa, 0, (T)0, [&](int k, T v) {
                             if (k < P.nb_a)
                                 sG[j * sGs + k] = v;
                             else
@@ -465,7 +424,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         T cr = 0, dcr;
                         if (row) horner(row + 4 * (P.nb_a + nfa), w, (T)P.rs_a, cr, dcr);
                         sCr[j] = cr;
-                        ylm_half<T, L>((T)elist[3 * p], (T)elist[3 * p + 1], (T)elist[3 * p + 2], P.l3a,
+                        ylm_half<L>((T)elist[3 * p], (T)elist[3 * p + 1], (T)elist[3 * p + 2], P.l3a,
                                        sY + j * sYs);
                     } else {
                         sCr[j] = 0;
@@ -477,10 +436,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L == 6
                         T w = 0;
                         bool unit;
                         const T* row = magnetic_row(P, dmom[p], w, unit, err);
-                        spline_values<T>(row, P.lut_m, w, 0, nfm, P.nb_m, unit ? (T)1 : (T)0,
+                        spline_values(row, P.lut_m, w, 0, nfm, P.nb_m, unit ? (T)1 : (T)0,
                                          [&](int k, T v) { sM[j * sMs + k] = v; });
                         cplx<T>* yh = sYm + j * sYms;
-                        ylm_half<T, L>((T)emom[3 * p], (T)emom[3 * p + 1], (T)emom[3 * p + 2], P.l2m, yh);
+                        ylm_half<L>((T)emom[3 * p], (T)emom[3 * p + 1], (T)emom[3 * p + 2], P.l2m, yh);
                         // H_q = M_{l',n'} Y_{l'm'} for the magnetic columns of A (l' <= l3m)
                         for (int q = 0; q < P.nm3; ++q) {
                             const int np = q / P.lsm3, lmp = q % P.lsm3;
@@ -1376,7 +1335,7 @@ __global__ void k_fill_double(double* __restrict__ p, size_t n) {
     if (i < n) p[i] = 0.0;
 }
 
-hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int natom, const int* off, const int* nlist,
+hipError_t fit_backward(const DevParams<double>& P, bool scaled, int natom, const int* off, const int* nlist,
                         const double* du, const double* dlist, const double* elist, const double* dmomi,
                         const double* dmom, const double* emom, const int* atom_struct, const double* gE,
                         Buffers& B, FitBuffers& F, int nterms, const int* nbo5, double* grad, hipStream_t s) {

@@ -200,7 +200,7 @@ struct FitBuffers {
     double* ub_u = nullptr;
     size_t cap_atoms = 0;
 };
-hipError_t fit_backward(const DevParams<double>& P, bool scaled, int cls, int natom, const int* off, const int* nlist,
+hipError_t fit_backward(const DevParams<double>& P, bool scaled, int natom, const int* off, const int* nlist,
                         const double* du, const double* dlist, const double* elist, const double* dmomi,
                         const double* dmom, const double* emom, const int* atom_struct, const double* gE,
                         Buffers& B, FitBuffers& F, int nterms, const int* nbo5, double* grad, hipStream_t s);

@@ -10,7 +10,7 @@
 //   v += dt/2 f_n/m ; x += dt v ;
 //   s <- R(Omega(G_mid), dt) s with G_mid = 3/2 G_n - 1/2 G_{n-1} (the field extrapolated to
 //        the middle of the step, which makes the spin update second order) ;
-//   pair geometry from x, s ; evaluate (k_density, k_adjoint, k_forces) ; assemble f_{n+1},
+//   pair geometry from x, s ; evaluate (density, adjoint, forces) ; assemble f_{n+1},
 //   G_{n+1} = dE/dm ; v += dt/2 f_{n+1}/m
 // with Omega_i = -(g/hbar) G_i (rad/ps; g = 2, hbar in eV ps, G in eV/muB), so
 // ds_i/dt = Omega_i x s_i, which conserves |s_i| and, at fixed positions, the energy.  The
