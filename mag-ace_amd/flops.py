@@ -64,3 +64,29 @@ def flops_model(h: dict, basis: dict, raw: dict, nneigh: float) -> dict:
     forces = nneigh * (force_pair + torque_pair) + torque_atom
     return {k: float(v) for k, v in dict(density=density, adjoint=adjoint, forces=forces,
                                           total=density + adjoint + forces).items()}
+
+
+def _walk(lmax):
+    """Steps of the longest of four walks through the harmonics l <= lmax, m >= 0, the orders m spread over them
+    (csrc/forces.hip)."""
+    n = [0] * 4
+    for m in range(lmax + 1):
+        n[n.index(min(n))] += lmax + 1 - m
+    return max(n)
+
+
+def executed(h: dict, nterms: int, nneigh: float) -> dict:
+    """FLOPs per atom-step of the sums that the mixed-precision kernels execute, which are fewer than flops_model's:
+    density and forces as 16x16x4 matrix products (2048 each, padding included; csrc/density.hip, forces.hip), adjoint
+    as two real-by-complex multiply-adds a monomial (csrc/nodes.cpp).  Spline rows, harmonics, pair products and the
+    gradient of the entries are not in it."""
+    nm3, lha = h["nr3_m"] * (h["l3m"] + 1) ** 2, (h["l3a"] + 1) * (h["l3a"] + 2) // 2
+    ls = [l for l in range(h["l3a"] + 1) for _ in range((l + 1) * nm3)]
+    tiles = [ls[c:c + 16] for c in range(0, lha * nm3, 16)]
+    t2 = -(-h["nr2_m"] * (h["l2m"] + 1) * (h["l2m"] + 2) // 2 // 16)
+    steps = 3 * -(-int(nneigh) // 12)
+    density = 2 * steps * (len(tiles) + t2) + 8 * sum(t[-1] - t[0] + 1 for t in tiles)
+    nk, nq4 = -(-h["nb_a"] // 4), -(-nm3 // 4)
+    bonds = min(-(-nq4 // 4) * lha, nq4 * _walk(h["l3a"]))
+    forces = 4 * nk * (bonds + -(-_walk(h["l2m"]) * h["nr2_m"] // 4)) * -(-int(nneigh) // 16)
+    return dict(density=2048.0 * density, adjoint=8.0 * nterms, forces=2048.0 * forces)
