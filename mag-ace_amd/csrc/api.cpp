@@ -1105,9 +1105,15 @@ int magace_set_precision(int mode) {
         set_error(MAGACE_ERR_STATE, "library not initialised");
         return MAGACE_ERR_STATE;
     }
-    if (g_ctx->precision != mode) bump_generation();
+    const int was = g_ctx->precision;
     g_ctx->precision = mode;
-    return g_ctx->uploaded ? ensure_records(*g_ctx) : 0;
+    if (g_ctx->uploaded)
+        if (int rc = ensure_records(*g_ctx)) {
+            g_ctx->precision = was;  // not without the records that the new one reads
+            return rc;
+        }
+    if (was != mode) bump_generation();
+    return 0;
 }
 
 int magace_get_precision(void) { return g_ctx ? g_ctx->precision : -1; }
