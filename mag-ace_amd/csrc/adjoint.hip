@@ -12,10 +12,10 @@
 // a 2^s-th of its columns), and the tables stream from L2 once per workgroup.
 //
 // Measured on 16000 atoms of the lmax-6 header against the walk over three-factor gradient records
-// (k_adjoint, k_adjoint_pair): mixed 786 -> 478 us, FP64 1566 -> 1081 us; 4394 atoms of the example
-// potential's shape 214 -> 122 us and 369 -> 264 us; 27648 atoms of the lmax-4 header 346 -> 280 us
-// and 621 -> 555 us.  What bounds it: the tables' way from L2 (0.44 MB a workgroup in FP32, 0.83 MB in
-// FP64: 20 TB/s together) and the latency between the phases; the vector units are 40% busy in FP32.
+// (k_adjoint, k_adjoint_pair): mixed 786 -> 388 us, FP64 1566 -> 893 us; 4394 atoms of the example
+// potential's shape 214 -> 97 us and 369 -> 230 us; 27648 atoms of the lmax-4 header 346 -> 205 us
+// and 621 -> 414 us.  What bounds it: in FP32 the vector units, 63% busy, and the latency between the phases; in
+// FP64 (40%) also the tables' way from L2 (0.83 MB a workgroup, 15 TB/s together; 0.44 MB in FP32).
 #include <hip/hip_runtime.h>
 
 #include "device.hpp"

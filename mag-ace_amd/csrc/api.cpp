@@ -819,10 +819,11 @@ int ensure_atoms(Context& c, size_t natom) {
 // pipeline, whose kernels run on that stream.  MAGACE_SPLIT_STREAMS=0 turns the split off
 // (read at every call).
 // The fork and the join take about 10 us, and kernels of one workgroup an atom or two have short tails, so little is
-// left to gain (split and one sequence, us): FP64 lmax 6 4394 atoms 542 and 543, 8192 1019 and 1023, 16000 1983 and 1995,
-// 54000 6581 and 6608; 27 magnetic columns 8192 1193 and 1188, 16000 2399 and 2419, 54000 8147 and 8246; lmax 4
-// 8192 428 and 420, 16000 equal.  Mixed: lmax 4 2662 atoms 124 and 115, 8192 268 and 252, 54000 1639 and 1620; lmax 6
-// 4394 291 and 275, 16000 949 and 946; 27 columns 4394 314 and 308, 54000 3363 and 3356.
+// left to gain, and not with every header (split and one sequence, FP64, us): lmax 6 12800 atoms 1571 and 1581, 16000 1962
+// and 1977, 54000 6529 and 6557; 27 magnetic columns 12800 1585 and 1582, 16000 1996 and 1995, 54000 6646 and 6670; lmax 4,
+// where it loses, 12800 665 and 663, 16000 847 and 844, 27648 1472 and 1466, 54000 2854 and 2845.  The line stands
+// where lmax 6 began to gain.  Mixed, which never splits, lost up to 8%: lmax 4 2662 atoms 124 and 115, 8192 268 and 252,
+// 54000 1639 and 1620; lmax 6 4394 291 and 275, 16000 949 and 946.
 constexpr int kSplitAtoms = 12288;
 
 bool split_enabled() {

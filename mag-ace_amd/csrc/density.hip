@@ -11,9 +11,10 @@
 // summed over radial factors h_f in place of the g_k (RadialFactors), A = U B, and both are looked up.
 //
 // Measured against the kernel that staged all R_{l,n} and summed on the vector units (us): 16000 atoms
-// lmax 6 mixed 403 -> 328, FP64 735 -> 545; 27648 atoms lmax 4 mixed 494 -> 370, FP64 855 -> 535; 4394 atoms
-// of the example potential's shape 161 -> 89 and 338 -> 110; 128 atoms lmax 4 FP64 24.4 -> 14.5.  Of the 328
-// the staging is 90, the products 110 (69 at the matrix cores' rate) and the stores of Z 100.
+// lmax 6 mixed 403 -> 248, FP64 735 -> 470; 27648 atoms lmax 4 mixed 494 -> 268, FP64 855 -> 474; 4394 atoms
+// of the example potential's shape, with its factors, 161 -> 75 and 338 -> 132 (through the g 78 and 110); 128 atoms
+// lmax 4 FP64 24.4 -> 12.4.  Of the 248 the matrix cores issue for 90 and the vector units for 107: the phases of a
+// workgroup do not overlap, and a compute unit holds four workgroups (two in FP64).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -102,7 +103,9 @@ __device__ __forceinline__ void spline_row(const T* __restrict__ row, int first,
 // products a step of four pairs).  TA, T2: tiles of A and of A2 of a wave at most.  JVP: the derivative of A and A2 along
 // the pairs' displacements u_i - u_j (k_density_jvp's work in a fit) in place of the values.  SEP: radial factors of
 // A's own before the base functions (DevParams::og).
-// Waves per SIMD: what the LDS of the usual headers lets in.
+// Waves per SIMD: what the LDS of the usual headers lets in.  Under that bound the FP32 instances of two and one tiles
+// spill six registers (95 MB of writes at 16000 atoms of lmax 6, half as much again as Z), those of four and three tiles, which
+// class-2 headers with many magnetic radial functions run, 37 to 51, and 94 to 205 in FP64.
 template <typename T, int L, int TA, int T2, bool JVP, bool SEP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TA > 2 ? 2 : sizeof(T) == 4 ? 4 : L <= 4 ? 3 : 2, 8)))
 k_density_mm(DevParams<T> P, const int* __restrict__ off,

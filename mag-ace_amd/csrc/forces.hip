@@ -115,12 +115,15 @@ struct ForceLds {  // offsets in T
 // functions; NA: of four radial factors of A.  SEP: these are functions of their own (DevParams::og).
 //
 // Bound by issue: at 16000 atoms of lmax 6 a wave has 1670 vector instructions and 132 products of 32 cycles
-// (FP32; 64 in FP64), about 11000 cycles of a SIMD, which measures 294 us (FP64 622 us).  One lane a pair, with W
+// (FP32; 64 in FP64), about 11000 cycles of a SIMD, which measures 280 us (FP64 622 us).  One lane a pair, with W
 // in LDS and sums over n, columns and the harmonics in vector instructions, took 449 us (1093 us); at lmax 4
-// and 27648 atoms 419 -> 324 us (901 -> 590 us), with 27 magnetic columns and 4394 atoms 213 -> 130 us (454 ->
-// 320 us), at 128 atoms of lmax 4 in FP64, where a wave's length counts, 36 -> 15 us.  Five waves a SIMD in
+// and 27648 atoms 419 -> 316 us (901 -> 587 us), with 27 magnetic columns and 4394 atoms 213 -> 103 us (454 ->
+// 193 us; 130 and 320 with A's sixteen base functions in place of its eight factors), at 128 atoms of lmax 4 in FP64,
+// where a wave's length counts, 36 -> 15 us.  Five waves a SIMD in
 // FP32 need at most 96 registers and 32000 bytes of LDS a workgroup, which the layout below keeps at lmax 6;
-// loading the pairs' inputs before V is made costs the fifth wave and was slower (323 us).
+// loading the pairs' inputs before V is made costs the fifth wave and was slower (323 us).  The 96 registers are not
+// quite enough: with three steps of base functions two are spilled (34 MB of writes at 16000 atoms), with four three, and
+// up to fourteen with factors.
 template <typename T, int NK, int NA, bool SEP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 2, sizeof(T) == 4 ? 5 : 3)))
 k_forces_mm(DevParams<T> P, const int* __restrict__ off, const double* __restrict__ dlist,

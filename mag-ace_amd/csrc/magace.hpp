@@ -144,7 +144,7 @@ struct TermList {
 // entry and q = product of two A entries or one A entry, rho = Re sum w X_p X_q.  A workgroup keeps
 // the entries it needs in LDS slots: the core [the A and A0 entries in use | 1 | 0], the pair
 // products [p | q] and the sums over A2 entries.  The work is cut into tasks of one wave each,
-// assigned to the waves of a workgroup at build time (wave_ptr); records are stored step by step,
+// assigned to the waves of a workgroup at build time (head); records are stored step by step,
 // 64 lanes after one another.
 constexpr size_t kNodeLdsTail = 384;          // sums and scalars behind the slots
 constexpr size_t kNodeLdsMost = 160 * 1024;
@@ -159,7 +159,7 @@ struct NodePlan {
     int slot_one = 0, slot_zero = 0, first_node = 0, np = 0, nq = 0, nslots = 0;
     std::vector<uint16_t> core_z;    // Z entry of core slot i (ZLayout::half)
     std::vector<uint32_t> pair;      // nodes: slots of the two factors
-    // [waves][64][4]: headers of a wave's tasks (steps, even; log2 of the lanes per block; first row), p
+    // [waves][64][4]: headers of a wave's tasks (steps, multiples of four; log2 of the lanes per block; first row), p
     // tasks, then q tasks, then gradient tasks; entry 62: their numbers, entry 63: first steps of the
     // wave's two record streams, which run through its tasks in order
     std::vector<int32_t> head;
