@@ -36,7 +36,7 @@ template <typename T> constexpr int kChain = sizeof(T) == 4 ? 12 : kPairs;
 template <typename T> constexpr int kRound = sizeof(T) == 4 ? 12 : 4;  // pairs of an unrolled turn; divides kPairs
 
 constexpr int kG = 17;  // row of a pair's base functions: 16, and one for the banks
-// the same in FP32, where the radial factors come before them (the 16 rows of a product's operand may reach into what
+// the same where radial factors of A's own come before them (the 16 rows of a product's operand may reach into what
 // lies behind: their results are not used)
 template <bool SEP> __host__ __device__ constexpr int functions_row(int og, int nb) {
     return !SEP || og + nb < kG ? kG : (og + nb) | 1;
